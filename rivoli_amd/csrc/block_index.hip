@@ -17,8 +17,16 @@
 //
 // Scorer. score[t][c] = bf16(sum_h bf16(relu(bf16(q[t][h] . kv[c])) * w[t][h])), the dot a
 // sequential f32 fold of separately rounded products and the head sum a sequential f32 fold
-// (blockindex.hip:138-207 argues each). That order rules out the matrix cores and any split of
-// a dot over lanes; what is free is where the operands come from. A lane owns block c and
+// (blockindex.hip:138-207 argues each). In general that order rules out the matrix cores and
+// any split of a dot over lanes. But the rows the indexer hands over are spread rows: a handful
+// of significant bits each, over a few binades. Every product and every partial sum of two such
+// rows is a multiple of one power of two and fits 24 bits, so no addition rounds and EVERY order
+// gives the reference's bits. The matrix kernels (hd = 128, up to 64 heads) test that property
+// on the operands they hold (RowSpan) and take such tiles through v_mfma_f32_32x32x16_bf16; any
+// other tile of the same launch is folded term by term as below. 8 192 queries x 64 heads x
+// <= 2 048 blocks: 237 us against 3 680 term by term (the whole rectangle 363 against 7 970).
+// Operands of another kind (no such rows leave the indexer) take the same launches' fold: 4.8 ms.
+// Term by term, what is free is where the operands come from. A lane owns block c and
 // keeps its 128-value row in registers for the whole launch; a wave's 64 lanes share the query,
 // so q[t][h][i] and w[t][h] are wave-uniform and come through scalar loads straight into the
 // multiply's scalar operand. Per (t, h) a wave issues 128 multiplies and 128 adds for 64
@@ -44,8 +52,9 @@ constexpr int kSpreadMaxD = 256;   // blockindex.hip:40-42
 constexpr int kSpreadThreads = 256;
 constexpr int kSpreadInFlight = 4;  // row groups per wave, all requested before the first is used
 
+// bf16(x) as a float: the conversion of the pair (0, x) leaves it in the upper half, one instruction.
 __device__ __forceinline__ float round_bf16(float x) {
-    return __uint_as_float((uint32_t)f32_to_bf16(x) << 16);
+    return __builtin_bit_cast(float, __builtin_convertvector(f32x2{0.0f, x}, bf16x2));
 }
 
 // formats.hpp:285-293 followed by its decode, for |q| <= 6: the nearest of {0, .5, 1, 1.5, 2, 3,
@@ -239,7 +248,7 @@ __device__ __forceinline__ void walk_pairs(const float* __restrict__ q, const fl
     }
 }
 
-// hd = 128, many (query, block group) pairs: a lane owns a block for the workgroup's queries
+// hd = 128 past the matrix kernels' 64 heads, many (query, block group) pairs: a lane owns a block for the workgroup's queries
 // and folds the head terms itself, in head order.
 __global__ __launch_bounds__(kScoreThreads) void index_score_blocks_128_kernel(
     const float* __restrict__ q, const float* __restrict__ kv, const float* __restrict__ w,
@@ -263,7 +272,7 @@ __global__ __launch_bounds__(kScoreThreads) void index_score_blocks_128_kernel(
     });
 }
 
-// hd = 128, few (query, block group) pairs (a decode step: one query): the plain kernel would
+// hd = 128, 65 to 128 heads, few (query, block group) pairs (a decode step: one query): the plain kernel would
 // occupy n_comp / 256 compute units for 64 heads' worth of arithmetic each. Here a workgroup
 // owns 64 blocks and its eight waves each take an eighth of the heads: the dots of different
 // heads are independent, only their sum has an order. The head terms meet in LDS and the first
@@ -294,6 +303,311 @@ __global__ __launch_bounds__(kSplitWavesPerGroup* kWave) void index_score_blocks
             if (c < n_comp) score[(size_t)t * n_comp + c] = round_bf16(acc);
         }
         __syncthreads();
+    }
+}
+
+// ---- the matrix kernels -------------------------------------------------------------------------
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef f32x4 f32x4_u __attribute__((aligned(4)));  // q rows need no more than a float's alignment
+
+// When is q . kv the same in every order? Let the non-zero values of a row have exponents in
+// [lo, hi] and at most two significant bits (1 or 1.5 times a power of two: what e2m1 times a
+// power of two is). Its values are multiples of 2^(lo - 1) and at most 1.5 * 2^hi. A sum of up to
+// 128 products of two rows is then a multiple of u = 2^(lo_q + lo_kv - 2) below 288 * 2^(hi_q +
+// hi_kv), that is below 2^(10.2 + (hi_q - lo_q) + (hi_kv - lo_kv)) u: with (hi_q - lo_q) + (hi_kv -
+// lo_kv) <= 13 every partial sum is a whole number of u below 2^24 and every f32 addition is
+// exact. Exponents within +-60 keep u and the sums normal. A spread row spans 3 binades plus what
+// its four block scales differ by; 13 leaves 7 for those.
+constexpr int kExactSpan = 13;
+constexpr int kNoSpan = 99;  // not such a row: no partner makes it exact
+// The census of a row, two bf16 patterns per dword: largest magnitude in the low 16 bits' field,
+// 0xffff - (smallest non-zero magnitude - 1) in the high one, so both fold by a packed maximum.
+struct RowSpan {
+    u16x2 hi = {0, 0}, lo = {0xffff, 0xffff};
+    uint32_t low_bits = 0;
+    // p: two bf16 patterns; bits: the OR of the low mantissa halves of the f32 values they came from
+    __device__ __forceinline__ void add(uint32_t p, uint32_t bits) {
+        low_bits |= bits | (p & 0x003f003fu);
+        const u16x2 m = __builtin_bit_cast(u16x2, p & 0x7fff7fffu);
+        hi = __builtin_elementwise_max(hi, m);
+        lo = __builtin_elementwise_min(lo, (u16x2)(m - (u16x2){1, 1}));  // a zero wraps to 0xffff
+    }
+    __device__ __forceinline__ uint32_t folded() const {
+        const uint32_t h = hi.x > hi.y ? hi.x : hi.y, l = lo.x < lo.y ? lo.x : lo.y;
+        return low_bits ? 0xffffffffu : (h | ((0xffffu - l) << 16));
+    }
+};
+__device__ __forceinline__ uint32_t span_max(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a),
+                                                                  __builtin_bit_cast(u16x2, b)));
+}
+__device__ __forceinline__ int span_of(uint32_t folded) {
+    const int hi = (int)((folded & 0xffffu) >> 7), lo = (int)((0x10000u - (folded >> 16)) >> 7);
+    if (!(folded & 0xffffu)) return 0;  // a row of zeros
+    return hi > 127 + 60 || lo < 127 - 60 ? kNoSpan : hi - lo;
+}
+// Two f32 bit patterns to a dword of two bf16 patterns by truncation (exact when the census finds
+// no low bits).
+__device__ __forceinline__ uint32_t upper_halves(float a, float b) {
+    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+__device__ __forceinline__ uint32_t low_half_bits(const f32x4& v) {
+    return (__float_as_uint(v.x) | __float_as_uint(v.y) | __float_as_uint(v.z) | __float_as_uint(v.w)) & 0xffffu;
+}
+
+// A workgroup's four waves own two queries each and walk the split's blocks in tiles of 32, which
+// all four read from LDS; a wave's q rows stay in registers as matrix operands (64 heads x 2
+// queries x 128 values = 128 registers). The 32 rows of a matrix tile are 16 heads of the wave's
+// first query and the same 16 of its second, dealt so that a lane's sixteen results are sixteen
+// heads of ONE query in order (the result layout gives lanes 0-31 the rows with bit 2 clear): the
+// head sum, whose order the reference fixes, is then register arithmetic. What bounds it is
+// issue: per 64 dots of a lane 32 matrix instructions of 32 cycles and five vector instructions a
+// dot (round, relu, weight, round, sum). e4m3 operands would halve the matrix half, but that
+// instruction does not keep 24 bits of a sum (checked: it loses bits at a span of 13).
+constexpr int kPairWaves = 4;
+constexpr int kPairThreads = kPairWaves * kWave;
+constexpr int kPairQueries = kPairWaves * 2;
+constexpr int kPairHeads = 64;
+constexpr int kPairTile = 32;
+constexpr int kPairRow = 128 * 2 + 16;  // bytes of a bf16 row in LDS: 16-byte reads of 16 rows meet no bank twice
+constexpr int kPairSplitMax = 4096;     // blocks of a split: one bit of a 64-bit mask per 64
+
+__global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
+    const float* __restrict__ q, const float* __restrict__ kv, const float* __restrict__ w,
+    float* __restrict__ score, int s, int n_comp, int heads, int split_blocks, int ratio) {
+    // q rows on their way to operands (a wave's 32 at a time), then two kv tiles
+    __shared__ __align__(16) unsigned char stage[kPairWaves * 32 * kPairRow];
+    __shared__ __align__(16) float weights[kPairWaves][2][kPairHeads];
+    __shared__ int kv_spans[2][kPairTile];
+    const int lane = threadIdx.x & (kWave - 1), half = lane >> 5, row = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    // the last queries of a prefill rank the most blocks: they start first
+    const int group = ratio > 0 ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x;
+    const int tw = group * kPairQueries + wave * 2;  // the wave's first query
+    const int c0 = blockIdx.y * split_blocks;
+    // 64-block groups with a block that some query up to t_last may rank (first_query)
+    const auto groups_for = [&](int t_last) {
+        int end = min(n_comp, c0 + split_blocks);
+        if (ratio > 0) end = min(end, ((t_last + 1) / ratio + 63) & ~63);
+        return end > c0 ? (end - c0 + 63) >> 6 : 0;
+    };
+    const int all_groups = groups_for(min(s, (group + 1) * kPairQueries) - 1);
+    if (!all_groups) return;  // workgroup-uniform
+    const int my_groups = tw < s ? groups_for(min(s, tw + 2) - 1) : 0;
+
+    bf16x8 a[4][8];
+    int q_span = 0;
+    {
+        unsigned char* const mine = stage + wave * 32 * kPairRow;
+        for (int i = lane; i < 2 * kPairHeads; i += kWave) {
+            const int hh = i & (kPairHeads - 1), t = min(tw + (i >> 6), s - 1);
+            weights[wave][i >> 6][hh] = hh < heads ? w[(size_t)t * heads + hh] : 0.0f;
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (c * 16 >= heads) break;
+            uint32_t low = 0;
+#pragma unroll
+            for (int j0 = 0; j0 < 16; j0 += 8) {
+                f32x4 v[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {  // an instruction moves two whole rows
+                    const int m = 2 * (j0 + j) + half, hh = c * 16 + (m >> 3) * 4 + (m & 3);
+                    const int t = min(tw + ((m >> 2) & 1), s - 1);
+                    v[j] = *reinterpret_cast<const f32x4_u*>(q + ((size_t)t * heads + min(hh, heads - 1)) * 128 + row * 4);
+                    if (hh >= heads) v[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    low |= low_half_bits(v[j]);
+                    const u32x2 p = {upper_halves(v[j].x, v[j].y), upper_halves(v[j].z, v[j].w)};
+                    *reinterpret_cast<u32x2*>(mine + (2 * (j0 + j) + half) * kPairRow + row * 8) = p;
+                }
+                asm volatile("" ::: "memory");  // no more than eight rows' loads in registers at a time
+            }
+            if (__any(low != 0)) q_span = kNoSpan;
+            asm volatile("" ::: "memory");  // the rows cross lanes: LDS serves a wave in order, the compiler must keep to it
+            RowSpan span;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const u32x4 p = *reinterpret_cast<const u32x4*>(mine + row * kPairRow + k * 32 + half * 16);
+                span.add(p.x, 0), span.add(p.y, 0), span.add(p.z, 0), span.add(p.w, 0);
+                a[c][k] = __builtin_bit_cast(bf16x8, p);
+            }
+            asm volatile("" ::: "memory");
+            const uint32_t f = span.folded();
+            q_span = max(q_span, span_of(span_max(f, __shfl_xor(f, 32, kWave))));
+        }
+#pragma unroll
+        for (int m = 1; m < 32; m <<= 1) q_span = max(q_span, __shfl_xor(q_span, m, kWave));
+    }
+
+    // kv tiles: eight threads a row, 16-byte pieces; the next tile's are requested before this
+    // one's products and parked after them
+    const int kr = threadIdx.x >> 3, kp = threadIdx.x & 7;
+    f32x4 next[4];
+    const auto request = [&](int tile) {
+        const float* const p = kv + (size_t)min(c0 + tile * kPairTile + kr, n_comp - 1) * 128 + kp * 4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) next[j] = *reinterpret_cast<const f32x4*>(p + j * 32);
+    };
+    const auto park = [&](int tile) {
+        unsigned char* const to = stage + ((tile & 1) * kPairTile + kr) * kPairRow + kp * 8;
+        RowSpan span;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const u32x2 p = {upper_halves(next[j].x, next[j].y), upper_halves(next[j].z, next[j].w)};
+            span.add(p.x, low_half_bits(next[j]));
+            span.add(p.y, 0);
+            *reinterpret_cast<u32x2*>(to + j * 64) = p;
+        }
+        uint32_t f = span.folded();
+        f = span_max(f, __shfl_xor(f, 1, kWave));
+        f = span_max(f, __shfl_xor(f, 2, kWave));
+        f = span_max(f, __shfl_xor(f, 4, kWave));
+        if (kp == 0) kv_spans[tile & 1][kr] = span_of(f);
+    };
+    const int tiles = all_groups * 2;
+    request(0);
+    __syncthreads();  // every wave's q rows are out of the stage
+    park(0);
+    unsigned long long inexact = 0;  // one bit per 64-block group
+    const int t = tw + half;
+    for (int tile = 0; tile < tiles; ++tile) {
+        __syncthreads();  // this tile is parked and nobody reads the other buffer any more
+        if (tile + 1 < tiles) request(tile + 1);
+        if ((tile >> 1) < my_groups) {
+            if (__any(kv_spans[tile & 1][row] + q_span > kExactSpan)) {
+                inexact |= 1ull << (tile >> 1);
+            } else {
+                const unsigned char* const from = stage + ((tile & 1) * kPairTile + row) * kPairRow + half * 16;
+                bf16x8 b[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) b[k] = *reinterpret_cast<const bf16x8*>(from + k * 32);
+                float acc = 0.0f;
+                f32x16 d[2] = {};
+#pragma unroll
+                for (int k = 0; k < 8; ++k) d[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][k], b[k], d[0], 0, 0, 0);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    if (c * 16 >= heads) break;
+                    // the next sixteen heads' products run under these heads' terms
+                    if (c < 3 && (c + 1) * 16 < heads) {
+                        f32x16& n = d[(c + 1) & 1];
+                        n = f32x16{};
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) n = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[c + 1][k], b[k], n, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 16; i += 4) {
+                        const f32x4 wv = *reinterpret_cast<const f32x4*>(&weights[wave][half][c * 16 + i]);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc = acc + head_term(d[c & 1][i + j], wv[j]);
+                    }
+                }
+                const int c = c0 + tile * kPairTile + row;
+                const int cw = c & ~63;
+                if (c < n_comp && t < s && (ratio <= 0 || (cw + 1) * (long long)ratio - 1 <= t))
+                    score[(size_t)t * n_comp + c] = round_bf16(acc);
+            }
+        }
+        if (tile + 1 < tiles) park(tile + 1);
+    }
+    // what is left, term by term: a lane owns a block of the 64
+    while (inexact) {
+        const int g = __builtin_ctzll(inexact);
+        inexact &= inexact - 1;
+        const long long cw = (long long)c0 + g * 64, c = cw + lane;
+        const int t1 = min(s, tw + 2), t0 = first_query(tw, t1, ratio, cw);
+        float row_v[128];
+        load_row(row_v, kv + (size_t)(c < n_comp ? c : n_comp - 1) * 128);
+        float acc = 0.0f;
+        int hh = 0, tt = t0;
+        walk_pairs(q, w, row_v, (size_t)t0 * heads, (size_t)t1 * heads, [&](size_t, float term) {
+            acc = acc + term;
+            if (++hh == heads) {
+                if (c < n_comp) score[(size_t)tt * n_comp + c] = round_bf16(acc);
+                acc = 0.0f, hh = 0, ++tt;
+            }
+        });
+    }
+}
+
+// Few queries (a decode step: one). A workgroup owns one query's 64 heads against 64 blocks, a
+// wave 32 x 32 of them: one matrix tile, operands straight from memory (lane L holds half L >> 5
+// of row L & 31, contiguous: the contraction's terms may be dealt to its steps in any order), the
+// head terms through LDS, the first wave folding them in head order. Bound by latency.
+// 8 192 blocks: 7.8 us, 14.1 with every dot folded term by term.
+constexpr int kOneThreads = 4 * kWave;
+__global__ __launch_bounds__(kOneThreads) void score_blocks_one_kernel(
+    const float* __restrict__ q, const float* __restrict__ kv, const float* __restrict__ w,
+    float* __restrict__ score, int s, int n_comp, int heads, int ratio) {
+    __shared__ float terms[kPairHeads][kWave];
+    __shared__ int inexact;
+    const int lane = threadIdx.x & (kWave - 1), half = lane >> 5, row = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int t = blockIdx.y;
+    const long long cw = (long long)blockIdx.x * kWave, c = cw + lane;
+    if (first_query(t, t + 1, ratio, cw) > t) return;  // workgroup-uniform: no block of these is legal for t
+    if (threadIdx.x == 0) inexact = 0;
+    const size_t base = (size_t)t * heads;
+    const int h0 = (wave & 1) * 32, b0 = (wave >> 1) * 32;
+    __syncthreads();
+    if (h0 < heads) {
+        const auto operand = [&](const float* p, bool live, bf16x8 (&x)[8]) {
+            RowSpan span;
+            f32x4 v[16];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) v[j] = *reinterpret_cast<const f32x4_u*>(p + half * 64 + j * 4);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                u32x4 b;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    f32x4 u = v[2 * k + j];
+                    if (!live) u = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    b[2 * j] = upper_halves(u.x, u.y), b[2 * j + 1] = upper_halves(u.z, u.w);
+                    span.add(b[2 * j], low_half_bits(u));
+                    span.add(b[2 * j + 1], 0);
+                }
+                x[k] = __builtin_bit_cast(bf16x8, b);
+            }
+            const uint32_t f = span.folded();
+            return span_of(span_max(f, __shfl_xor(f, 32, kWave)));
+        };
+        bf16x8 a[8], b[8];
+        const int hr = h0 + row;
+        const long long cr = cw + b0 + row;
+        int q_span = operand(q + (base + min(hr, heads - 1)) * 128, hr < heads, a);
+        const int k_span = operand(kv + (size_t)(cr < n_comp ? cr : n_comp - 1) * 128, true, b);
+#pragma unroll
+        for (int m = 1; m < 32; m <<= 1) q_span = max(q_span, __shfl_xor(q_span, m, kWave));
+        if (__any(q_span + k_span > kExactSpan)) {
+            if (lane == 0) inexact = 1;
+        } else {
+            f32x16 d = {};
+#pragma unroll
+            for (int k = 0; k < 8; ++k) d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[k], b[k], d, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int hh = h0 + (i >> 2) * 8 + half * 4 + (i & 3);
+                if (hh < heads) terms[hh][b0 + row] = head_term(d[i], w[base + hh]);
+            }
+        }
+    }
+    __syncthreads();
+    if (inexact) {  // term by term: every wave a quarter of the heads for all 64 blocks
+        const int per = (heads + 3) / 4, g0 = min(wave * per, heads), g1 = min(g0 + per, heads);
+        float row_v[128];
+        load_row(row_v, kv + (size_t)(c < n_comp ? c : n_comp - 1) * 128);
+        walk_pairs(q, w, row_v, base + g0, base + g1, [&](size_t g, float term) { terms[g - base][lane] = term; });
+        __syncthreads();
+    }
+    if (wave == 0) {
+        float acc = 0.0f;
+        for (int hh = 0; hh < heads; ++hh) acc = acc + terms[hh][lane];
+        if (c < n_comp) score[(size_t)t * n_comp + c] = round_bf16(acc);
     }
 }
 
@@ -348,6 +662,10 @@ extern "C" int rivoli_act_quant_f4_rotated(float* x, int rows, int d, void* stre
 }
 
 namespace rk {
+// Up to here a workgroup per (query, 64 blocks) is the faster: 4 queries x 4 096 blocks 8 us against
+// 10 (4 x 8 192, 512 workgroups: 11.3 against 10.1; 300 queries x 75, 600: 15 against 10). One query
+// has no second for the many-query kernel's wave: 8 192 blocks 7.8 against 10.3, 65 536 20 against 25.
+constexpr int kOneGroups = 384;
 static int score_blocks_launch(const float* q, const float* kv, const float* w, float* score, int s,
                                int n_comp, int heads, int hd, int ratio, hipStream_t st) {
     if (s <= 0 || heads <= 0 || hd <= 0) return 1001;
@@ -356,6 +674,27 @@ static int score_blocks_launch(const float* q, const float* kv, const float* w, 
     if (n_comp <= 0) return 1005;
     if (!q || !kv || !w || !score) return 1001;
     (void)hipGetLastError();
+    if (hd == 128 && aligned16(kv) && heads <= kPairHeads) {
+        const unsigned groups = (unsigned)(((long long)n_comp + kWave - 1) / kWave);
+        if (s == 1 || (long long)s * groups <= kOneGroups) {
+            hipLaunchKernelGGL(score_blocks_one_kernel, dim3(groups, (unsigned)s), dim3(kOneThreads), 0, st, q, kv, w,
+                               score, s, n_comp, heads, ratio);
+            return launch_status();
+        }
+        // two workgroups per compute unit at a time; splits of the blocks while the queries alone
+        // give fewer than two rounds of those (a split reads its queries' rows again)
+        const unsigned t_groups = (unsigned)(((long long)s + kPairQueries - 1) / kPairQueries);
+        long long splits = t_groups >= 1024 ? 1 : 1024 / t_groups;
+        if (splits > groups) splits = groups;
+        int per = (int)((groups + splits - 1) / splits) * 64;
+        if (per > kPairSplitMax) per = kPairSplitMax;
+        const unsigned y = (unsigned)(((long long)n_comp + per - 1) / per);
+        if (y <= 65535u) {
+            hipLaunchKernelGGL(score_blocks_pair_kernel, dim3(t_groups, y), dim3(kPairThreads), 0, st, q, kv, w, score,
+                               s, n_comp, heads, per, ratio);
+            return launch_status();
+        }
+    }
     // enough workgroups to fill the part while a workgroup keeps its rows for several queries
     const unsigned c_groups = (unsigned)(((long long)n_comp + kScoreThreads - 1) / kScoreThreads);
     int t_per_group = kScoreQueriesPerGroup;

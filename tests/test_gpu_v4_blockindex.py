@@ -225,3 +225,42 @@ def test_prefill_form_writes_every_legal_entry_and_skips_whole_groups(oracle, s,
     assert np.array_equal(back(sel_a, np.int32), back(sel_b, np.int32))
     assert hip.lib().rivoli_index_score_blocks_prefill(qd.data_ptr(), kd.data_ptr(), wd.data_ptr(), out.data_ptr(),
                                                        s, n_comp, heads, hd, 0, None) == 1001
+
+
+def few_bit_rows(rng, rows, span):
+    """+-{1, 1.5} times powers of two over exactly `span` + 1 binades, with zeros; every third row
+    positive and mostly at its top binade, so that a sum comes near the largest the rule allows."""
+    e = rng.integers(0, span + 1, (rows, 128))
+    e[::3][rng.random((len(e[::3]), 128)) < 0.9] = span
+    e[:, 0], e[:, 1] = 0, span
+    x = rng.choice([-1.5, -1.0, 1.0, 1.5], (rows, 128)) * 2.0 ** (e - 7)
+    x[::3] = np.abs(x[::3])
+    x[:, 2:][rng.random((rows, 126)) < 0.1] = 0.0
+    return x.astype(np.float32)
+
+
+@pytest.mark.parametrize("s,n_comp,heads", [(1, 1, 64), (2, 65, 31), (4, 190, 17), (5, 33, 1), (9, 3100, 64), (16, 1600, 47),
+                                            (23, 1210, 16)])
+@pytest.mark.parametrize("q_span,kv_span", [(3, 4), (6, 7), (13, 0), (7, 7), (3, 20)])
+def test_score_of_rows_whose_sums_are_exact_up_to_the_last_span_and_past_it(oracle, s, n_comp, heads, q_span, kv_span):
+    """Rows of one- and two-bit values over q_span + kv_span = 7 and 13 binades, where every sum is
+    exact and the matrix cores take them, and 14 and 23, where they are folded term by term; then
+    the same launch with a single block, and a single head, that only the fold gets right. All bit
+    for bit, through the few-query and the many-query kernel and both forms of the call."""
+    rng = np.random.default_rng(s * 1000 + n_comp + q_span * 7 + kv_span)
+    q = few_bit_rows(rng, s * heads, q_span).reshape(s, heads, 128)
+    kv = few_bit_rows(rng, n_comp, kv_span)
+    w = bf16_round((rng.standard_normal((s, heads)) * 0.1).astype(np.float32))
+    for change in ("none", "block", "head"):
+        if change == "block":
+            kv[n_comp // 2] = rng.standard_normal(128).astype(np.float32)
+        if change == "head":
+            q[s // 2, heads // 2] = rng.standard_normal(128).astype(np.float32)
+        code, want = oracle.index_score_blocks(q, kv, w)
+        got = device_score(q, kv, w)
+        assert code == 0 and same_bits(got, want).size == 0, change
+        out = dzeros(s * n_comp * 4, 0x5A)
+        hip.launch_index_score_blocks_prefill(dev(q), dev(kv), dev(w), out, s, n_comp, heads, 128, 1)
+        part = back(out, np.float32).reshape(s, n_comp).view(np.uint32)
+        live = (np.arange(n_comp)[None, :] // 64) * 64 < np.minimum(np.arange(s) + 1, n_comp)[:, None]
+        assert np.array_equal(part[live], want.view(np.uint32)[live]) and (part[~live] == 0x5A5A5A5A).all(), change
