@@ -16,8 +16,10 @@
 // bf16 rounding of q would miss. With heads as the tile's ROWS a lane holds 16 heads of one
 // token, so ReLU, the head weights and the sum over heads are register arithmetic plus one
 // cross-half shuffle; nothing goes through LDS after the query is staged.
-// A workgroup stages its query once and walks 2048 tokens (4 waves x 16 blocks of 32). The
-// kernel reads hd*2 bytes per token and is bound by that stream, not by the matrix cores.
+// A workgroup stages its query once and walks up to 2048 tokens (4 waves x 16 blocks of 32), fewer
+// where that would leave compute units without one (score_blocks). The kernel reads hd*2 bytes per
+// token: large calls are bound by that stream, not by the matrix cores, small ones by the way from
+// launch to the first block's products and the blocks a wave walks one after another.
 // Launch-only; see include/rivoli_kvcache.h for the contract of every entry point.
 #include "topk_common.hpp"
 
@@ -30,8 +32,8 @@ constexpr int kScoreThreads = 256;
 constexpr int kScoreWaves = kScoreThreads / kWave;
 constexpr int kScoreMaxHeads = 64;   // active heads, padded to a multiple of 32
 constexpr int kScoreMaxHd = 128;     // head dimension, a multiple of 16
-constexpr int kScoreBlocks = 16;     // 32-token blocks per wave
-constexpr int kScoreTokensPerGroup = kScoreWaves * kScoreBlocks * 32;
+constexpr int kScoreMaxBlocks = 16;  // 32-token blocks per wave, at most
+constexpr int kScoreTokensPerBlock = kScoreWaves * 32;
 constexpr int kScoreRowPad = 8;      // bf16 of padding per staged query row
 
 // RB = 32-head row blocks (1 or 2). HD = the head dimension at compile time (128, the shipped
@@ -47,7 +49,8 @@ __global__ __launch_bounds__(kScoreThreads) void index_score_kernel(
     const uint16_t* __restrict__ kpool, const int* __restrict__ block_table,
     const int* __restrict__ nts, const unsigned int* __restrict__ heads, int max_blocks_per_seq,
     int stride, int nt_all, int nh, int nact, int hd_rt, int page_tokens, int n_pages, float wscale,
-    float dscale, float* __restrict__ scores, uint32_t* __restrict__ topk_ws, size_t ws_stride) {
+    float dscale, float* __restrict__ scores, uint32_t* __restrict__ topk_ws, size_t ws_stride,
+    int blocks) {
     const int hd = HD ? HD : hd_rt;
     __shared__ __attribute__((aligned(16))) uint16_t s_qh[RB * 32][kScoreMaxHd + kScoreRowPad];
     __shared__ __attribute__((aligned(16))) uint16_t s_ql[RB * 32][kScoreMaxHd + kScoreRowPad];
@@ -57,11 +60,11 @@ __global__ __launch_bounds__(kScoreThreads) void index_score_kernel(
     // With a top-k workspace: the histogram of this workgroup's scores by the top 12 bits of
     // their selection key, two 16-bit counters per word (a workgroup scores 2048 tokens).
     __shared__ uint32_t s_hist[kTopBins / 2];
-    static_assert(kScoreTokensPerGroup < 65536, "16-bit histogram counters");
+    static_assert(kScoreTokensPerBlock * kScoreMaxBlocks < 65536, "16-bit histogram counters");
 
     const int qi = blockIdx.y;
     const int nt = nts ? min(nts[qi], nt_all) : nt_all;
-    const int t0 = (int)blockIdx.x * kScoreTokensPerGroup;
+    const int t0 = (int)blockIdx.x * blocks * kScoreTokensPerBlock;
     if (t0 >= nt) return;
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -69,22 +72,70 @@ __global__ __launch_bounds__(kScoreThreads) void index_score_kernel(
     if (topk_ws)
         for (int i = tid; i < kTopBins / 2; i += kScoreThreads) s_hist[i] = 0u;
 
-    // ---- stage the active heads: q = hi + lo in bf16, and the per-head weight ----
-    // eight consecutive query values per step: two 16-byte loads in, two 16-byte LDS stores out
-    const int cpr = hd >> 3;
-    for (int c = tid; c < RB * 32 * cpr; c += kScoreThreads) {
-        const int a = c / cpr, d = (c - a * cpr) * 8;
-        float val[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        if (a < nact) {
-            const int h = heads ? (int)heads[a] : a;
-            if ((unsigned)h < (unsigned)nh) {
-                const float4* src =
-                    reinterpret_cast<const float4*>(q + ((size_t)qi * nh + h) * hd + d);
-                const float4 v0 = src[0], v1 = src[1];
-                val[0] = v0.x, val[1] = v0.y, val[2] = v0.z, val[3] = v0.w;
-                val[4] = v1.x, val[5] = v1.y, val[6] = v1.z, val[7] = v1.w;
+    // A block's 32 key rows are one contiguous run (consecutive tokens of one page, or of the
+    // linear cache), so the wave fetches it with fully coalesced 16-byte loads, parks it in its
+    // own LDS tile and reads it back in the matrix core's operand layout. Fetching each lane's
+    // operand straight from memory instead touches 32 different rows per instruction and was
+    // measured ~1.6x slower. The next block's fetch is issued before this block's MFMAs.
+    constexpr int kChunks = 32 * kScoreMaxHd / 8 / kWave;  // 16-byte chunks per lane per block
+    uint16_t(*tile)[kScoreMaxHd + kScoreRowPad] = s_k[wave];
+    const int cprk = hd >> 3;                               // 16-byte chunks per key row
+    // rows_ok < 0: the block's page is outside the pool, -rows_ok of its tokens are in range
+    auto block_base = [&](int tb, int& rows_ok) -> const uint16_t* {
+        rows_ok = min(32, nt - tb);
+        size_t slot = (size_t)tb;
+        if (block_table) {
+            const int page = block_table[(size_t)qi * max_blocks_per_seq + tb / page_tokens];
+            if ((unsigned)page >= (unsigned)n_pages) {
+                rows_ok = -rows_ok;  // nothing of this block is readable
+                return kpool;
             }
+            slot = (size_t)page * page_tokens + (size_t)(tb % page_tokens);
         }
+        return kpool + slot * hd;
+    };
+    auto fetch = [&](const uint16_t* base, int rows_ok, u32x4 (&raw)[kChunks]) {
+#pragma unroll
+        for (int j = 0; j < kChunks; ++j) {
+            const int c = lane + j * kWave;
+            raw[j] = (c < rows_ok * cprk) ? reinterpret_cast<const u32x4*>(base)[c]
+                                          : u32x4{0, 0, 0, 0};
+        }
+    };
+
+    // the first block's rows are on their way while the query is staged
+    int tb = t0 + wave * 32, rows_ok = 0;
+    u32x4 raw[kChunks];
+    if (tb < nt) fetch(block_base(tb, rows_ok), rows_ok, raw);
+
+    // ---- stage the active heads: q = hi + lo in bf16, and the per-head weight ----
+    // eight consecutive query values per step: two 16-byte loads in, two 16-byte LDS stores out.
+    // Every step's loads are requested before the first is used (unconditionally: a head that does
+    // not count reads head 0 and is zeroed).
+    const int cpr = hd >> 3;
+    constexpr int kStages = RB * 32 * (kScoreMaxHd / 8) / kScoreThreads;
+    float4 qv[kStages][2];
+    unsigned counted = 0;
+#pragma unroll
+    for (int j = 0; j < kStages; ++j) {
+        const int c = tid + j * kScoreThreads;
+        const int a = c / cpr, d = (c - a * cpr) * 8;
+        const int h = a < nact ? (heads ? (int)heads[a] : a) : -1;
+        const bool live = (unsigned)h < (unsigned)nh;
+        counted |= (live ? 1u : 0u) << j;
+        const float4* src = reinterpret_cast<const float4*>(q + ((size_t)qi * nh + (live ? h : 0)) * hd + d);
+        qv[j][0] = src[0], qv[j][1] = src[1];
+    }
+#pragma unroll
+    for (int j = 0; j < kStages; ++j) {
+        const int c = tid + j * kScoreThreads;
+        if (c >= RB * 32 * cpr) break;
+        const int a = c / cpr, d = (c - a * cpr) * 8;
+        const float4 v0 = qv[j][0], v1 = qv[j][1];
+        const bool live = ((counted >> j) & 1u) != 0u;
+        float val[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) val[i] = live ? val[i] : 0.0f;
         uint32_t hi[4], lo[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -126,41 +177,7 @@ __global__ __launch_bounds__(kScoreThreads) void index_score_kernel(
         for (int v = 0; v < 16; ++v)
             wv[rb][v] = s_w[rb * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)];
 
-    // A block's 32 key rows are one contiguous run (consecutive tokens of one page, or of the
-    // linear cache), so the wave fetches it with fully coalesced 16-byte loads, parks it in its
-    // own LDS tile and reads it back in the matrix core's operand layout. Fetching each lane's
-    // operand straight from memory instead touches 32 different rows per instruction and was
-    // measured ~1.6x slower. The next block's fetch is issued before this block's MFMAs.
-    constexpr int kChunks = 32 * kScoreMaxHd / 8 / kWave;  // 16-byte chunks per lane per block
-    uint16_t(*tile)[kScoreMaxHd + kScoreRowPad] = s_k[wave];
-    const int cprk = hd >> 3;                               // 16-byte chunks per key row
-    // rows_ok < 0: the block's page is outside the pool, -rows_ok of its tokens are in range
-    auto block_base = [&](int tb, int& rows_ok) -> const uint16_t* {
-        rows_ok = min(32, nt - tb);
-        size_t slot = (size_t)tb;
-        if (block_table) {
-            const int page = block_table[(size_t)qi * max_blocks_per_seq + tb / page_tokens];
-            if ((unsigned)page >= (unsigned)n_pages) {
-                rows_ok = -rows_ok;  // nothing of this block is readable
-                return kpool;
-            }
-            slot = (size_t)page * page_tokens + (size_t)(tb % page_tokens);
-        }
-        return kpool + slot * hd;
-    };
-    auto fetch = [&](const uint16_t* base, int rows_ok, u32x4 (&raw)[kChunks]) {
-#pragma unroll
-        for (int j = 0; j < kChunks; ++j) {
-            const int c = lane + j * kWave;
-            raw[j] = (c < rows_ok * cprk) ? reinterpret_cast<const u32x4*>(base)[c]
-                                          : u32x4{0, 0, 0, 0};
-        }
-    };
-
-    int tb = t0 + wave * 32, rows_ok = 0;
-    u32x4 raw[kChunks];
-    if (tb < nt) fetch(block_base(tb, rows_ok), rows_ok, raw);
-    for (int it = 0; it < kScoreBlocks && tb < nt; ++it) {
+    for (int it = 0; it < blocks && tb < nt; ++it) {
         // park this block; the wave's LDS operations execute in order, the fences only keep
         // the compiler from moving the reads above the writes (and the next writes above them)
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -177,7 +194,7 @@ __global__ __launch_bounds__(kScoreThreads) void index_score_kernel(
         const bool valid = col < rows_ok;
         const int tb_next = tb + kScoreWaves * 32;
         int rows_next = 0;
-        if (it + 1 < kScoreBlocks && tb_next < nt) fetch(block_base(tb_next, rows_next), rows_next, raw);
+        if (it + 1 < blocks && tb_next < nt) fetch(block_base(tb_next, rows_next), rows_next, raw);
 
         f32x16 acc[RB];
 #pragma unroll
@@ -340,6 +357,20 @@ __global__ __launch_bounds__(256) void index_append_paged_kernel(
     *reinterpret_cast<u32x4*>(kpool + (size_t)slot * hd + c * 8) = out;
 }
 
+// Blocks of 32 tokens a wave walks: as few as keep the launch within one round of workgroups (two
+// per compute unit, by LDS; the query is staged once per workgroup). With 16 blocks whatever the
+// call, 8 192 tokens of one query took 24 us on four compute units; with one block 5.2 us. 8 x
+// 16 384: 26 -> 10 us, 16 x 16 384: 28 -> 16 us. Half as many workgroups: 10.8 and 17.8 us; twice
+// as many (two rounds): 12.9 and 19.7 us; 16 x 40 000 tokens a workgroup or so past the round
+// (9 blocks, 560 workgroups): 43.6 us against 37.
+constexpr int kScoreTargetGroups = 512;
+static int score_blocks(int n_queries, int nt) {
+    const int per_query = n_queries < kScoreTargetGroups ? kScoreTargetGroups / n_queries : 1;
+    const int all = (nt + kScoreTokensPerBlock - 1) / kScoreTokensPerBlock;
+    const int blocks = (all + per_query - 1) / per_query;
+    return blocks > kScoreMaxBlocks ? kScoreMaxBlocks : blocks;
+}
+
 static int index_score_launch(const float* q, const float* w, const unsigned short* kpool,
                               const int* block_table, const int* nts, const unsigned int* heads,
                               int n_queries, int max_blocks_per_seq, int stride, int nt, int nh,
@@ -363,8 +394,9 @@ static int index_score_launch(const float* q, const float* w, const unsigned sho
     if (topk_workspace && !aligned16(topk_workspace)) return 1004;
     uint32_t* ws = topk_runs_split(n_queries, nt) ? (uint32_t*)topk_workspace : nullptr;
     const size_t ws_stride = topk_ws_words(topk_segments(nt));
-    dim3 grid((unsigned)((nt + kScoreTokensPerGroup - 1) / kScoreTokensPerGroup),
-              (unsigned)n_queries);
+    const int blocks = score_blocks(n_queries, nt);
+    const int group = blocks * kScoreTokensPerBlock;
+    dim3 grid((unsigned)((nt + group - 1) / group), (unsigned)n_queries);
     (void)hipGetLastError();
     if (plain) {
         const size_t q_bytes = (size_t)nact * hd * sizeof(float);
@@ -380,7 +412,7 @@ static int index_score_launch(const float* q, const float* w, const unsigned sho
 #define RK_SCORE(RBV, HDV)                                                                      \
     hipLaunchKernelGGL((index_score_kernel<RBV, HDV>), grid, dim3(kScoreThreads), 0, stream, q, w, \
                        kpool, block_table, nts, heads, max_blocks_per_seq, stride, nt, nh, nact,  \
-                       hd, page_tokens, n_pages, wscale, dscale, scores, ws, ws_stride)
+                       hd, page_tokens, n_pages, wscale, dscale, scores, ws, ws_stride, blocks)
     if (hd == 128) {
         if (nact <= 32) RK_SCORE(1, 128); else RK_SCORE(2, 128);
     } else {

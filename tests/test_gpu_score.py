@@ -149,3 +149,28 @@ def test_scores_feed_topk_like_the_oracle_chain(oracle):
     assert np.all(np.abs(want_scores[0][differ] - kth) <= tol), differ
     # and on the device's own scores the selection is exactly the oracle's rule
     assert np.array_equal(got, oracle.topk(back(sc, np.float32), k))
+
+
+@pytest.mark.parametrize("n_q,top", [(1, 129), (2, 128 * 3), (128, 513), (256, 257), (600, 300)])
+def test_workgroup_sizes_by_the_call(oracle, n_q, top):
+    """One block of 32 tokens per wave up to several (128, 256 and 600 queries leave 4, 2 and one
+    workgroup each): lengths one short of, at and one past a workgroup's tokens, an empty query,
+    tokens past a query's length untouched."""
+    nh, hd, pt = 5, 128, 32
+    rng = np.random.default_rng(n_q)
+    blocks = -(-top // pt)
+    tables = rng.permutation(n_q * blocks).astype(np.int32).reshape(n_q, blocks)
+    lens = rng.integers(0, top + 1, n_q).astype(np.int32)
+    edges = [top, 0, 127, 128, 129, 255, 256, 257, top - 1]
+    lens[:len(edges)] = np.minimum(edges, top)[:n_q]
+    q = rng.standard_normal((n_q, nh, hd), dtype=np.float32)
+    w = rng.standard_normal((n_q, nh), dtype=np.float32)
+    kpool = oracle.f32_to_bf16(rng.standard_normal((n_q * blocks * pt, hd), dtype=np.float32))
+    want = oracle.index_score_paged(q, w, kpool, tables, lens, None, top, hd, pt, 0.5, 0.25, n_threads=4)
+    out = dzeros(n_q * top * 4, 0x7F)
+    hip.launch_index_score_paged(dev(q), dev(w), dev(kpool), dev(tables), dev(lens), None, n_q, blocks, top, top, nh,
+                                 nh, hd, pt, n_q * blocks, 0.5, 0.25, out)
+    got = back(out, np.float32).reshape(n_q, top)
+    live = np.arange(top)[None, :] < lens[:, None]
+    assert rel(got[live], want[live]) < TOL
+    assert (got.view(np.uint32)[~live] == 0x7F7F7F7F).all()
