@@ -658,33 +658,31 @@ __device__ __forceinline__ void attend_part(const AttendArgs& a, int seq, int hb
 
 }  // namespace rk
 #include "mla_attend_f8.hpp"
+#include "mla_attend_heads16.hpp"
 namespace rk {
 
-// F8: the contractions run on the 8-bit matrix instructions with QSPLIT / PSPLIT e4m3 terms for
-// q / the softmax weights (mla_attend_f8.hpp); else on the bf16 ones.
-template <int QSPLIT, int PSPLIT, int MODE, bool ANY, bool F8 = false>
-__global__ __launch_bounds__(F8 ? kF8Threads : kAttThreads) void mla_attend_paged_kernel(const AttendArgs a) {
-    constexpr int THREADS = F8 ? kF8Threads : kAttThreads;
-    constexpr int PER = kDealMaxSeqs / THREADS;  // sequences per thread in the prefix below
-    __shared__ int pre[kDealMaxSeqs + 8];  // tiles before each sequence, when dealing
-    __shared__ int wave_total[THREADS / kWave];
+// Rows of sequence s that are attended.
+template <int MODE>
+__device__ __forceinline__ int attended_rows(const AttendArgs& a, int s) {
+    if (MODE == kLinear) return a.k;
+    if (MODE == kSparse) return a.n_rows ? max(min(a.n_rows[s], a.k), 0) : a.k;
+    return max(min(a.seq_lens[s], a.k), 0);
+}
+
+// Which rows of which sequences a workgroup attends: one sequence, all of it, when nothing is
+// dealt. Otherwise the tiles [t_lo, t_hi) of the batch-wide tile sequence, starting in sequence
+// `seq` (given: the sequence that is not dealt): the workgroup walks the sequences that range touches. pre[s] = tiles before sequence s.
+// False: nothing for this workgroup.
+template <int THREADS, int MODE>
+__device__ __forceinline__ bool dealt_range(const AttendArgs& a, int item, int (&pre)[kDealMaxSeqs + 8],
+                                            int (&wave_total)[THREADS / kWave], long long& t_lo, long long& t_hi,
+                                            int& seq) {
     constexpr bool SPARSE = MODE == kSparse;
-    const int hb = blockIdx.z;
+    constexpr int PER = kDealMaxSeqs / THREADS;  // sequences per thread in the prefix below
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-
-    auto attended = [&](int s) -> int {
-        if (MODE == kLinear) return a.k;
-        if (SPARSE) return a.n_rows ? max(min(a.n_rows[s], a.k), 0) : a.k;
-        return max(min(a.seq_lens[s], a.k), 0);
-    };
-
-    // ---- which rows of which sequences this workgroup attends ------------------------------
-    // One sequence, all of it, when nothing is dealt. Otherwise the tiles [t_lo, t_hi) of the
-    // batch-wide tile sequence: the workgroup walks the sequences that range touches.
-    long long t_lo = 0, t_hi = 0;
-    int seq = blockIdx.y;
+    t_lo = 0, t_hi = 0;
     if (a.n_items > 0) {
         // inclusive prefix of tiles per sequence, PER consecutive sequences per thread
         // (the lengths are read unconditionally, a sequence past the last re-reading the last
@@ -724,9 +722,9 @@ __global__ __launch_bounds__(F8 ? kF8Threads : kAttThreads) void mla_attend_page
         }
         __syncthreads();
         const long long total = pre[a.n_seqs];
-        t_lo = deal_lo(blockIdx.x, a.n_items, total);
-        t_hi = deal_lo(blockIdx.x + 1, a.n_items, total);
-        if (t_lo >= t_hi) return;
+        t_lo = deal_lo(item, a.n_items, total);
+        t_hi = deal_lo(item + 1, a.n_items, total);
+        if (t_lo >= t_hi) return false;
         // the sequence holding tile t_lo: the last one that starts at or before it
         int lo = 0, hi = a.n_seqs;  // pre[lo] <= t_lo < pre[hi]
         while (hi - lo > 1) {
@@ -736,6 +734,41 @@ __global__ __launch_bounds__(F8 ? kF8Threads : kAttThreads) void mla_attend_page
         }
         seq = lo;
     }
+    return true;
+}
+
+// The rows of sequence `seq` that [t_lo, t_hi) holds, and the record they go to; t_lo moves past
+// them. False: none (a sequence with nothing to attend).
+template <int MODE>
+__device__ __forceinline__ bool dealt_part(const AttendArgs& a, int item, const int (&pre)[kDealMaxSeqs + 8], int seq,
+                                           long long& t_lo, long long t_hi, int& r_begin, int& r_end, bool& whole,
+                                           float*& pa, float*& pml) {
+    const long long p0 = pre[seq], p1 = pre[seq + 1];
+    const long long e = t_hi < p1 ? t_hi : p1;
+    if (e <= t_lo) return false;
+    r_begin = (int)(t_lo - p0) * kTile;
+    r_end = min(attended_rows<MODE>(a, seq), (int)(e - p0) * kTile);
+    whole = t_lo == p0 && e == p1;
+    const size_t rec = (size_t)item + seq;  // unique: both only grow along the walk
+    pa = a.part_acc + rec * a.H * kKvl;
+    pml = a.part_ml + rec * a.H * 2;
+    t_lo = e;
+    return true;
+}
+
+// F8: the contractions run on the 8-bit matrix instructions with QSPLIT / PSPLIT e4m3 terms for
+// q / the softmax weights (mla_attend_f8.hpp); else on the bf16 ones.
+template <int QSPLIT, int PSPLIT, int MODE, bool ANY, bool F8 = false>
+__global__ __launch_bounds__(F8 ? kF8Threads : kAttThreads) void mla_attend_paged_kernel(const AttendArgs a) {
+    constexpr int THREADS = F8 ? kF8Threads : kAttThreads;
+    __shared__ int pre[kDealMaxSeqs + 8];  // tiles before each sequence, when dealing
+    __shared__ int wave_total[THREADS / kWave];
+    const int hb = blockIdx.z;
+    const int tid = threadIdx.x;
+
+    long long t_lo, t_hi;
+    int seq = blockIdx.y;
+    if (!dealt_range<THREADS, MODE>(a, blockIdx.x, pre, wave_total, t_lo, t_hi, seq)) return;
 
   for (;; ++seq) {
     int r_begin = 0, r_end;
@@ -743,19 +776,10 @@ __global__ __launch_bounds__(F8 ? kF8Threads : kAttThreads) void mla_attend_page
     float *pa = a.part_acc, *pml = a.part_ml;  // else this part's partial record
     if (a.n_items > 0) {
         if (t_lo >= t_hi || seq >= a.n_seqs) break;
-        const long long p0 = pre[seq], p1 = pre[seq + 1];
-        const long long e = t_hi < p1 ? t_hi : p1;
-        if (e <= t_lo) continue;  // a sequence with nothing to attend
-        r_begin = (int)(t_lo - p0) * kTile;
-        r_end = min(attended(seq), (int)(e - p0) * kTile);
-        whole = t_lo == p0 && e == p1;
-        const size_t rec = (size_t)blockIdx.x + seq;  // unique: both only grow along the walk
-        pa = a.part_acc + rec * a.H * kKvl;
-        pml = a.part_ml + rec * a.H * 2;
-        t_lo = e;
+        if (!dealt_part<MODE>(a, blockIdx.x, pre, seq, t_lo, t_hi, r_begin, r_end, whole, pa, pml)) continue;
         __syncthreads();  // the previous part is done with the LDS tiles and the prefix reads above
     } else {
-        r_end = attended(seq);
+        r_end = attended_rows<MODE>(a, seq);
         if (r_end <= 0) {
             // a sequence with nothing to attend gets zeros, like the reference's `l > 0 ? 1/l : 0`
             const int kvl = ANY ? a.kvl : kKvl;
@@ -770,6 +794,42 @@ __global__ __launch_bounds__(F8 ? kF8Threads : kAttThreads) void mla_attend_page
     else attend_part<QSPLIT, PSPLIT, MODE, ANY>(a, seq, hb, r_begin, r_end, whole, pa, pml);
     if (a.n_items == 0) break;
   }  // parts of this workgroup
+}
+
+// The same walk for 16 heads per workgroup (mla_attend_heads16.hpp).
+template <int QSPLIT, int PSPLIT, int MODE>
+__global__ __launch_bounds__(kH16Threads, 1) void mla_attend_heads16_kernel(const AttendArgs a) {
+    __shared__ int pre[kDealMaxSeqs + 8];
+    __shared__ int wave_total[kH16Waves];
+    // Workgroups are dealt to the eight dies in turn: the head groups of one work item follow each
+    // other on one die, whose cache then serves the item's rows to all but the first of them.
+    const int groups = (a.H + kH16Heads - 1) / kH16Heads, turn = (int)blockIdx.x >> 3;
+    const int item = (turn / groups) * 8 + ((int)blockIdx.x & 7), hg = turn % groups;
+    long long t_lo, t_hi;
+    int seq = item;
+    if (item >= (a.n_items > 0 ? a.n_items : a.n_seqs)) return;
+    if (!dealt_range<kH16Threads, MODE>(a, item, pre, wave_total, t_lo, t_hi, seq)) return;
+    for (;; ++seq) {
+        int r_begin = 0, r_end;
+        bool whole = true;
+        float *pa = a.part_acc, *pml = a.part_ml;
+        if (a.n_items > 0) {
+            if (t_lo >= t_hi || seq >= a.n_seqs) break;
+            if (!dealt_part<MODE>(a, item, pre, seq, t_lo, t_hi, r_begin, r_end, whole, pa, pml)) continue;
+            __syncthreads();
+        } else {
+            r_end = attended_rows<MODE>(a, seq);
+            if (r_end <= 0) {
+                for (int i = threadIdx.x; i < kH16Heads * kKvl; i += kH16Threads) {
+                    const int h = hg * kH16Heads + i / kKvl;
+                    if (h < a.H) a.clat[((size_t)seq * a.H + h) * kKvl + (i % kKvl)] = 0.0f;
+                }
+                return;
+            }
+        }
+        attend_part_heads16<QSPLIT, PSPLIT, MODE>(a, seq, hg, r_begin, r_end, whole, pa, pml);
+        if (a.n_items == 0) break;
+    }
 }
 
 // Dealt plan: clat[seq][head] = sum_r w_r acc_r / sum_r w_r l_r over the sequence's partial
@@ -852,11 +912,67 @@ __global__ __launch_bounds__(128) void mla_attend_combine_kernel(
     *dst = float4{sum.x * inv, sum.y * inv, sum.z * inv, sum.w * inv};
 }
 
+// After the attention launch: the merge of the partial records when the plan has any.
+static int attend_merge(const AttendArgs& a, const AttendPlan& plan, int n_seqs, int max_rows, const int* seq_lens,
+                        const int* n_rows, bool listed, hipStream_t st) {
+    const int rc = launch_status();
+    if (rc != 0 || plan.n_splits <= 1) return rc;
+    hipLaunchKernelGGL(mla_attend_combine_kernel, dim3((unsigned)a.H, (unsigned)n_seqs), dim3(128), 0, st,
+                       a.part_acc, a.part_ml, seq_lens, n_rows, listed ? 1 : 0, max_rows, n_seqs, plan.n_items,
+                       a.H, a.kvl, a.clat);
+    return launch_status();
+}
+
+// Whether a call goes to the workgroups of 16 heads: its 32-token tiles times its groups of 16
+// heads, before the lengths are known. Parity mode, 64 heads: 1 x 4 096 tokens (512) 21.5 us
+// against 34.5 in workgroups of 64 heads, 32 x 1 000 (4 096) 33 against 39, 6 x 9 000 (6 768) 47
+// both, 32 listed sets of 2 048 rows (8 192) 45 against 48, 32 x 4 096 (16 384) 73 against 64.
+// The 8-bit modes' kernel is the faster one sooner: 8 listed sets of 2 048 rows (2 048) 24 us in
+// the parity mode here against 34 at precise 4, 32 x 1 000 (4 096) 32 against 33, 32 listed sets
+// (8 192) 44 against 42; below the line they run in the parity mode. Up to 16 heads the other
+// kernels' workgroups are three quarters empty: 32 x 16 384 tokens 84 us against 163 (precise 2)
+// and 107 (4).
+constexpr long long kH16MaxWork = 8192, kH16MaxWork8Bit = 4096;
+static bool heads16_pays(int n_seqs, int H, int max_rows, int precise) {
+    const long long tiles = (long long)n_seqs * ((max_rows + kTile - 1) / kTile);
+    return H <= kH16Heads ||
+           tiles * ((H + kH16Heads - 1) / kH16Heads) <= (precise > 2 ? kH16MaxWork8Bit : kH16MaxWork);
+}
+// The splits of a call by 16 heads a workgroup: one workgroup per compute unit, at least a tile per
+// wave, and no more partial records than `plan` (which the caller's scratch was sized by) has.
+static void heads16_plan(AttendPlan& plan, int n_seqs, int H, int max_rows) {
+    const long long per_split = (long long)n_seqs * ((H + kH16Heads - 1) / kH16Heads);
+    const int tiles = (max_rows + kTile - 1) / kTile;
+    long long n = kAttTargetGroups / per_split;
+    if (n > tiles / kH16Waves) n = tiles / kH16Waves;
+    if (n > plan.n_splits) n = plan.n_splits;
+    plan.n_splits = n < 1 ? 1 : (int)n;
+    plan.n_items = plan.n_splits > 1 ? plan.n_splits * n_seqs : 0;
+    plan.n_records = plan.n_items ? plan.n_items + n_seqs : 0;
+}
+
 // What both launchers share once the arguments are in place: the attention kernel of the right
 // mode, then the merge of the partial records when the plan has any.
 template <int MODE>
-static int attend_launch(const AttendArgs& a, const AttendPlan& plan, int n_seqs, int max_rows, bool any,
+static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_rows, bool any,
                          int precise, const int* seq_lens, const int* n_rows, bool listed, hipStream_t st) {
+    if (!any && heads16_pays(n_seqs, a.H, max_rows, precise)) {
+        heads16_plan(plan, n_seqs, a.H, max_rows);
+        a.n_items = plan.n_items;
+        const int items = plan.n_items ? plan.n_items : n_seqs;
+        const dim3 grid((unsigned)(((items + 7) / 8 * 8) * (long long)((a.H + kH16Heads - 1) / kH16Heads)));
+        (void)hipGetLastError();
+        constexpr int M = MODE == kDensePaged ? kDense : MODE;  // the rows are looked up one by one
+        if (precise >= 2 || MODE == kLinear)
+            hipLaunchKernelGGL((mla_attend_heads16_kernel<2, 2, M>), grid, dim3(kH16Threads), 0, st, a);
+        else if constexpr (MODE != kLinear) {
+            if (precise == 1)
+                hipLaunchKernelGGL((mla_attend_heads16_kernel<2, 1, M>), grid, dim3(kH16Threads), 0, st, a);
+            else
+                hipLaunchKernelGGL((mla_attend_heads16_kernel<1, 1, M>), grid, dim3(kH16Threads), 0, st, a);
+        }
+        return attend_merge(a, plan, n_seqs, max_rows, seq_lens, n_rows, listed, st);
+    }
     const dim3 grid(plan.n_items ? (unsigned)plan.n_items : 1u, plan.n_items ? 1u : (unsigned)n_seqs,
                     (unsigned)((a.H + 63) / 64));
     (void)hipGetLastError();
@@ -877,12 +993,7 @@ static int attend_launch(const AttendArgs& a, const AttendPlan& plan, int n_seqs
         else
             hipLaunchKernelGGL((mla_attend_paged_kernel<1, 1, MODE, false>), grid, dim3(kAttThreads), 0, st, a);
     }
-    const int rc = launch_status();
-    if (rc != 0 || plan.n_splits <= 1) return rc;
-    hipLaunchKernelGGL(mla_attend_combine_kernel, dim3((unsigned)a.H, (unsigned)n_seqs), dim3(128), 0, st,
-                       a.part_acc, a.part_ml, seq_lens, n_rows, listed ? 1 : 0, max_rows, n_seqs, plan.n_items,
-                       a.H, a.kvl, a.clat);
-    return launch_status();
+    return attend_merge(a, plan, n_seqs, max_rows, seq_lens, n_rows, listed, st);
 }
 
 }  // namespace rk
@@ -1026,5 +1137,8 @@ extern "C" int rivoli_mla_attend(const float* qabs, const float* qrope, const un
     a.clat = clat;
     a.part_acc = plan.n_items ? partial : nullptr;
     a.part_ml = plan.n_items ? partial + (size_t)plan.n_records * H * kKvl : nullptr;
-    return attend_launch<kLinear>(a, plan, 1, nr, true, 2, nullptr, nullptr, rows != nullptr, nullptr);
+    // any row width but the shipped one (whole 16-byte pieces) takes the general form
+    const bool any = kvl != kKvl || rope != kRopeW || n_blocks != kKvl / 128 || !aligned16(Rc) || !aligned16(Lscale) ||
+                     !aligned16(qabs) || !aligned16(qrope);
+    return attend_launch<kLinear>(a, plan, 1, nr, any, 2, nullptr, nullptr, rows != nullptr, nullptr);
 }

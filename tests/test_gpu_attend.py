@@ -402,3 +402,31 @@ def test_linear_attend_rows_and_guards(oracle):
         hip.launch_attend(b, b, b, b, b, None, 0, 16, 512, 64, 4, 1.0, b, b)
     assert e.value.code == 1001
     assert hip.attend_scratch_floats(64, 512) == 16 * 64 * 514
+
+
+@pytest.mark.parametrize("precise", [2, 1, 0, 4, 3])
+@pytest.mark.parametrize("large", [True, False])
+def test_both_sides_of_the_line_between_workgroups_of_16_and_of_64_heads(oracle, precise, large):
+    """Lengths one short of, at and one past the tile and run sizes of every kernel, an empty
+    sequence, and 33 heads: few sequences go to the workgroups of 16 heads (a wave per tile: tiles
+    a wave has none of, or two), many to those of 64 (and to the 8-bit kernel)."""
+    edges = [31, 32, 33, 127, 128, 129, 255, 256, 257, 383, 384, 385, 0, 1, 64, 65, 160, 200]
+    H = 33
+    # tiles x groups of 16 heads: 13 x 3 a sequence, the line at 8192 (8-bit modes: 4096)
+    lens = (edges * 12)[:212] if large else edges[:12]
+    assert (len(lens) * 13 * 3 > 8192) == large
+    c = paged_case(oracle, lens, H=H, seed=900, outlier_frac=0.0)
+    want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], None, None,
+                                   KVL, ROPE, PT, c["scale"], n_threads=8)
+    got = run_paged(c, max(lens), precise=precise)
+    check(got, want, precise, "dense", mild=precise in (2, 4))
+    k = 70
+    rows = np.zeros((len(lens), k), np.uint32)
+    n_rows = np.zeros(len(lens), np.int32)
+    rng = np.random.default_rng(901)
+    for s, n in enumerate(lens):
+        n_rows[s] = min(n, (k, 64, 33, 32, 31, 1)[s % 6])
+        rows[s, :n_rows[s]] = np.sort(rng.permutation(max(n, 1))[:n_rows[s]])
+    want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], rows, n_rows,
+                                   KVL, ROPE, PT, c["scale"], n_threads=8)
+    check(run_paged(c, k, rows=rows, n_rows=n_rows, precise=precise), want, precise, "listed", mild=precise in (2, 4))
