@@ -129,6 +129,13 @@ def test_deposit_and_decode_follow_the_state_machine(oracle, ratio, d, rd, s, s0
     assert np.array_equal(blocks.view(np.uint32), whole.view(np.uint32))
 
 
+@pytest.mark.parametrize("d,rd", [(4, 2), (68, 2), (256, 256), (1020, 64), (1024, 64), (1028, 64)])
+def test_overlapping_decode_at_the_widths_of_a_lane_a_feature(oracle, d, rd):
+    """Less than a wave, a remainder of one, every dim rotated, the widest and one past it; the
+    block and the slid state are the other form's to the bit."""
+    test_deposit_and_decode_follow_the_state_machine(oracle, 4, d, rd, 21, 6)
+
+
 def test_compress_guards():
     hg = hip.CompGeom.build(4, 32, 8, 1e-6)
     b = dzeros(1 << 16)
