@@ -465,22 +465,42 @@ __global__ __launch_bounds__(128) void gather_attn_combine_kernel(
     const int head = blockIdx.x;
     const size_t t = blockIdx.y;
     const size_t rec0 = t * n_splits * h + head;
+    // Shares are fetched eight at a time, all loads of a batch in flight together (a share past
+    // the last re-reads the last and is left out), and the first batch's accumulators with its
+    // maxima: two round trips for up to eight shares instead of one per share. The sums run in
+    // ascending order. 64 heads, 10 shares: 6.0 -> 3.9 us.
+    constexpr int kBatch = 8;
+    float m_r[kBatch], l_r[kBatch];
+    float4 v[kBatch];
+    auto fetch = [&](int r0) {
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            const size_t rec = rec0 + (size_t)min(r0 + u, n_splits - 1) * h;
+            m_r[u] = part_ml[rec * 2], l_r[u] = part_ml[rec * 2 + 1];
+            v[u] = reinterpret_cast<const float4*>(part_acc + rec * kGaD)[threadIdx.x];
+        }
+    };
+    fetch(0);
+    const float sk = sink[head] * kLog2e;
     float m_g = -INFINITY;
-    for (int r = 0; r < n_splits; ++r) m_g = fmaxf(m_g, part_ml[(rec0 + (size_t)r * h) * 2]);
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) m_g = fmaxf(m_g, m_r[u]);
+    for (int r = kBatch; r < n_splits; ++r) m_g = fmaxf(m_g, part_ml[(rec0 + (size_t)r * h) * 2]);
     float4 sum = {0, 0, 0, 0};
     float l_g = NAN;
     if (m_g != -INFINITY) {
         l_g = 0.0f;
-        for (int r = 0; r < n_splits; ++r) {
-            const size_t rec = rec0 + (size_t)r * h;
-            const float m_r = part_ml[rec * 2];
-            if (m_r == -INFINITY) continue;
-            const float w = exp2f(m_r - m_g);
-            l_g += part_ml[rec * 2 + 1] * w;
-            const float4 v = reinterpret_cast<const float4*>(part_acc + rec * kGaD)[threadIdx.x];
-            sum.x += v.x * w, sum.y += v.y * w, sum.z += v.z * w, sum.w += v.w * w;
+        for (int r0 = 0; r0 < n_splits; r0 += kBatch) {
+            if (r0 > 0) fetch(r0);
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                if (r0 + u >= n_splits || m_r[u] == -INFINITY) continue;
+                const float w = exp2f(m_r[u] - m_g);
+                l_g += l_r[u] * w;
+                sum.x += v[u].x * w, sum.y += v[u].y * w, sum.z += v[u].z * w, sum.w += v[u].w * w;
+            }
         }
-        l_g += exp2f(sink[head] * kLog2e - m_g);
+        l_g += exp2f(sk - m_g);
     }
     float4* const dst = reinterpret_cast<float4*>(o + (t * h + head) * kGaD) + threadIdx.x;
     *dst = float4{(float)(__bf16)(sum.x / l_g), (float)(__bf16)(sum.y / l_g), (float)(__bf16)(sum.z / l_g),

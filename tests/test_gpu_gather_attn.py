@@ -227,6 +227,12 @@ def test_split_plan_matches_oracle_and_the_unsplit_kernel(oracle, m, h, topk, pr
         assert e.value.code == 1001
 
 
+@pytest.mark.parametrize("topk", [512, 576, 1024, 1088, 2100])
+def test_merge_of_a_batch_of_shares_and_one_more(oracle, topk):
+    """8, 9, 16, 17 and 32 shares."""
+    test_split_plan_matches_oracle_and_the_unsplit_kernel(oracle, 1, 64, topk, 2)
+
+
 def test_split_plan_with_a_fully_masked_query(oracle):
     d, h, rows, topk = 512, 64, 200, 320
     q, kv, sink = attend_inputs(oracle, 2, h, d, rows, seed=77)
