@@ -1478,18 +1478,30 @@ static int index_topk_launch(const float* scores, int n_queries, int stride, con
 // ties) is bisected over all the keys instead. The selection is then emitted in index order
 // by ballots and prefix counts.
 //
-constexpr int kSelBits = 10;               // key bits resolved by the histogram
-constexpr int kSelBins = 1 << kSelBits;
-constexpr int kSelLow = 32 - kSelBits;
+// Sixteen waves on one row (decode) hold their keys in 8 or 16 registers a lane and are bound by
+// what the row does one after the other: colliding atomics of the histogram (half of a row's keys
+// share a few exponents) and the one wave's bisection. They resolve 12 bits (three of the
+// mantissa), which quarters both; the walk over 4096 bins is then a scan by all threads, four bins
+// each. One row of 8192 keys: 17.8 us in four waves of 10 bits, 14.3 in sixteen, 11.9 with 12 bits, 8.8 with the agreeing bits left out (below).
+template <int WAVES>
+struct SelShapeOf {
+    static constexpr int kBits = WAVES == 16 ? 12 : 10;  // key bits resolved by the histogram
+    static constexpr int kBins = 1 << kBits;
+    static constexpr int kLow = 32 - kBits;
+};
 constexpr int kSelCand = 1024;             // pivot-bin members listed in LDS
 constexpr int kSelMisc = 4 * 16 + 8;       // per-wave slots (up to 16 waves) and the pivot record
-constexpr int kSelLdsWords = kSelMisc + (kSelBins > kSelCand ? kSelBins : kSelCand);
+template <int WAVES>
+constexpr int sel_lds_words() {
+    return kSelMisc + (SelShapeOf<WAVES>::kBins > kSelCand ? SelShapeOf<WAVES>::kBins : kSelCand);
+}
 
 template <int WAVES, int ITEMS, class KEY>
 __device__ __forceinline__ void select_bisect(const float* __restrict__ s, int nt, uint32_t kq,
                                               uint32_t* __restrict__ out, uint32_t* lds,
                                               uint32_t add) {
-    // requires 1 <= kq < nt <= WAVES * 64 * ITEMS; lds holds kSelLdsWords words
+    // requires 1 <= kq < nt <= WAVES * 64 * ITEMS; lds (16-byte aligned) holds sel_lds_words words
+    constexpr int kSelBins = SelShapeOf<WAVES>::kBins, kSelLow = SelShapeOf<WAVES>::kLow;
     for (int i = threadIdx.x; i < kSelBins; i += WAVES * kWave) lds[kSelMisc + i] = 0u;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1522,7 +1534,7 @@ __device__ __forceinline__ void select_bisect(const float* __restrict__ s, int n
             fetch(std::integral_constant<int, 16>{});
         else
             fetch(std::integral_constant<int, 8>{});
-        // ---- the top kSelBits of the k-th largest key, by one LDS histogram -------------------
+        // ---- the top kBits of the k-th largest key, by one LDS histogram -------------------
         // (sign, exponent and the first mantissa bit of a score): one atomic per key instead
         // of a bisection step per bit. The atomic sits with the key's conversion so that the
         // per-element "exists" masks do not stay live (32 of them overflow the scalar file).
@@ -1565,7 +1577,36 @@ __device__ __forceinline__ void select_bisect(const float* __restrict__ s, int n
     uint32_t* s_cand = s_hist;  // the list reuses the histogram once the pivot bin is known
     uint32_t* s_pv = lds + 4 * WAVES;  // [0] pivot bin, [1] keys in higher bins, [2] keys in it, [3] list fill
     __syncthreads();
-    if (wave == 0) {
+    if constexpr (WAVES * kWave * 4 == kSelBins) {
+        // a thread owns four consecutive bins: suffix sums over the wave, then over the waves, find
+        // the thread where the running count from the top reaches kq
+        const uint4 c4 = *reinterpret_cast<const uint4*>(s_hist + 4 * threadIdx.x);
+        const uint32_t c[4] = {c4.x, c4.y, c4.z, c4.w};
+        const uint32_t mine = c[0] + c[1] + c[2] + c[3];
+        uint32_t suffix = mine;
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+            const uint32_t v = __shfl_down(suffix, off, kWave);
+            if (lane + off < kWave) suffix += v;
+        }
+        if (lane == 0) lds[wave] = suffix;  // (the count_ge slots are idle here)
+        __syncthreads();
+        uint32_t above = suffix - mine;
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) above += w > wave ? lds[w] : 0u;
+        if (above < kq && kq <= above + mine) {
+            uint32_t acc = above;
+            int i = 3;
+#pragma unroll
+            for (int j = 3; j > 0; --j) {
+                if (i == j && acc + c[j] < kq) acc += c[j], i = j - 1;
+            }
+            s_pv[0] = 4 * threadIdx.x + (uint32_t)i;
+            s_pv[1] = acc;
+            s_pv[2] = i == 3 ? c[3] : i == 2 ? c[2] : i == 1 ? c[1] : c[0];
+            s_pv[3] = 0u;
+        }
+    } else if (wave == 0) {
         // a lane owns 16 consecutive bins; suffix sums over the lanes find the lane where the
         // running count from the top reaches kq, which then walks its own bins
         uint32_t c[kSelBins / kWave], mine = 0;
@@ -1649,10 +1690,28 @@ __device__ __forceinline__ void select_bisect(const float* __restrict__ s, int n
                     if (i < csteps) c += (uint32_t)__popcll(__ballot(ck[i] >= cand));
                 return c;
             };
-            uint32_t p = pbin << kSelLow, t = 0, nd = 0;
+            // Bits in which every member agrees need no step, and scores rounded to bf16 (the block
+            // scorer's) agree in their low sixteen: p starts as the members' common ones, which
+            // changes no count — a member that matches the candidate above has them too.
+            uint32_t ones = 0xffffffffu, any = 0u;
+#pragma unroll
+            for (int i = 0; i < CP; ++i) {
+                if (i >= csteps) break;
+                any |= ck[i];
+                ones &= (i * kWave + lane) < (int)in_bin ? ck[i] : 0xffffffffu;
+            }
+#pragma unroll
+            for (int off = 1; off < kWave; off <<= 1) {
+                any |= (uint32_t)__shfl_xor((int)any, off, kWave);
+                ones &= (uint32_t)__shfl_xor((int)ones, off, kWave);
+            }
+            uint32_t open = __builtin_amdgcn_readfirstlane((int)(any & ~ones));
+            uint32_t p = __builtin_amdgcn_readfirstlane((int)ones), t = 0, nd = 0;
             bool exact = false;
-            for (int b = kSelLow - 1; b >= 0; --b) {
-                const uint32_t cand = p | (1u << b);
+            while (open) {
+                const uint32_t bit = 0x80000000u >> __builtin_clz(open);
+                open ^= bit;
+                const uint32_t cand = p | bit;
                 const uint32_t c = cand_ge(cand);
                 if (c >= need_in_bin) p = cand;
                 if (c == need_in_bin) {
@@ -1780,7 +1839,7 @@ template <int WAVES, int ITEMS>
 __global__ __launch_bounds__(WAVES* kWave) void block_select_bisect_kernel(
     const float* __restrict__ scores, int n_comp, int ratio, int prefill, int k, int offset,
     int32_t* __restrict__ out, int out_stride) {
-    __shared__ uint32_t lds[kSelLdsWords];
+    __shared__ __attribute__((aligned(16))) uint32_t lds[sel_lds_words<WAVES>()];
     const int t = blockIdx.x;
     const int limit = select_row_limit(t, n_comp, ratio, prefill);
     int32_t* o = out + (size_t)t * out_stride;
@@ -1807,6 +1866,8 @@ __global__ __launch_bounds__(THREADS) void block_select_kernel(const float* __re
                                               (uint32_t)offset);
 }
 
+constexpr int kSelFewRows = 256;  // a workgroup of sixteen waves per compute unit
+
 // `out_stride` (>= k) is the distance between the rows of `out`: k for a bare selection, the
 // rectangle's width when the selection is the tail of a [window | compressed] row.
 static int block_select_launch(const float* scores, int rows, int n_comp, int ratio,
@@ -1825,8 +1886,14 @@ static int block_select_launch(const float* scores, int rows, int n_comp, int ra
 #define RK_SELECT(T, I)                                                                       \
     hipLaunchKernelGGL((block_select_kernel<T, I>), grid, dim3(T), 0, stream, scores, n_comp, \
                        ratio, prefill ? 1 : 0, k, offset, out, out_stride)
-    // up to 32 keys per lane; a row takes as few waves as hold it
-    if (n_comp <= 64 * 8)
+    // Few rows (decode: one) leave the chip to one workgroup each, and a row's time is its
+    // longest wave's: sixteen waves, 8 keys a lane. One row of 8192: 17.8 -> 8.8 us.
+    if (rows <= kSelFewRows && n_comp > 64 * 8 && n_comp <= 1024 * 8)
+        RK_BISECT(16, 8);
+    else if (rows <= kSelFewRows && n_comp > 1024 * 8 && n_comp <= 1024 * 16)
+        RK_BISECT(16, 16);
+    // otherwise up to 32 keys per lane; a row takes as few waves as hold it
+    else if (n_comp <= 64 * 8)
         RK_BISECT(1, 8);
     else if (n_comp <= 64 * 32)
         RK_BISECT(1, 32);

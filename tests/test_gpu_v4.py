@@ -179,6 +179,23 @@ def test_select_matches_oracle(oracle, rows, n_comp, ratio, topk, prefill):
         assert np.array_equal(want, brute_force_rows(s, ratio, topk, prefill, 4096))
 
 
+@pytest.mark.parametrize("rows,n_comp,topk", [(1, 513, 512), (2, 1024, 3), (256, 700, 512), (257, 700, 512),
+                                              (1, 8191, 512), (2, 8192, 1), (1, 8193, 512), (3, 16384, 16383)])
+@pytest.mark.parametrize("kind", ["any", "bf16", "one value", "one bin"])
+def test_select_of_few_rows(oracle, rows, n_comp, topk, kind):
+    """Both sides of the line between few rows and many, of the keys a lane holds; scores whose low
+    halves agree, that all agree, and more of them in one bin than the list takes."""
+    s = adversarial_scores(rows, n_comp, seed=rows + n_comp)
+    if kind == "bf16":
+        s = (s.view(np.uint32) & 0xffff0000).view(np.float32)
+    elif kind == "one value":
+        s[:] = -2.5
+    elif kind == "one bin":
+        s = (np.uint32(0x3f800000) + np.random.default_rng(5).integers(0, 1 << 19, s.shape, dtype=np.uint32)).view(np.float32)
+    got = device_select(s, 4, topk, False, 128)
+    assert np.array_equal(got, oracle.v4_scored_rows(s, 4, topk, False, 128))
+
+
 def test_select_prefill_at_scale(oracle):
     """A 8192-token prefill at ratio 4 with a cap of 512: rows below the cap are positional,
     rows above it ranked; every row is ascending, legal, and -1 padded only at its tail."""
