@@ -1849,6 +1849,20 @@ __global__ __launch_bounds__(WAVES* kWave) void block_select_bisect_kernel(
                                                (uint32_t)offset);
 }
 
+// Few rows: sixteen waves each.
+template <int ITEMS>
+__global__ __launch_bounds__(1024) void block_select_few_kernel(
+    const float* __restrict__ scores, int n_comp, int ratio, int prefill, int k, int offset,
+    int32_t* __restrict__ out, int out_stride) {
+    __shared__ __attribute__((aligned(16))) uint32_t lds[sel_lds_words<16>()];
+    const int t = blockIdx.x;
+    const int limit = select_row_limit(t, n_comp, ratio, prefill);
+    int32_t* o = out + (size_t)t * out_stride;
+    if (select_positional<1024>(o, limit, k, offset)) return;
+    select_bisect<16, ITEMS, TotalOrderKey>(scores + (size_t)t * n_comp, limit, (uint32_t)k,
+                                            reinterpret_cast<uint32_t*>(o), lds, (uint32_t)offset);
+}
+
 // Rows too long for the register form: the single-query radix select, one workgroup per row.
 template <int THREADS, int ITEMS>
 __global__ __launch_bounds__(THREADS) void block_select_kernel(const float* __restrict__ scores,
@@ -1883,15 +1897,18 @@ static int block_select_launch(const float* scores, int rows, int n_comp, int ra
 #define RK_BISECT(WV, I)                                                                     \
     hipLaunchKernelGGL((block_select_bisect_kernel<WV, I>), grid, dim3(WV* kWave), 0, stream, \
                        scores, n_comp, ratio, prefill ? 1 : 0, k, offset, out, out_stride)
+#define RK_FEW(I)                                                                             \
+    hipLaunchKernelGGL((block_select_few_kernel<I>), grid, dim3(1024), 0, stream, scores, n_comp, \
+                       ratio, prefill ? 1 : 0, k, offset, out, out_stride)
 #define RK_SELECT(T, I)                                                                       \
     hipLaunchKernelGGL((block_select_kernel<T, I>), grid, dim3(T), 0, stream, scores, n_comp, \
                        ratio, prefill ? 1 : 0, k, offset, out, out_stride)
     // Few rows (decode: one) leave the chip to one workgroup each, and a row's time is its
     // longest wave's: sixteen waves, 8 keys a lane. One row of 8192: 17.8 -> 8.8 us.
     if (rows <= kSelFewRows && n_comp > 64 * 8 && n_comp <= 1024 * 8)
-        RK_BISECT(16, 8);
+        RK_FEW(8);
     else if (rows <= kSelFewRows && n_comp > 1024 * 8 && n_comp <= 1024 * 16)
-        RK_BISECT(16, 16);
+        RK_FEW(16);
     // otherwise up to 32 keys per lane; a row takes as few waves as hold it
     else if (n_comp <= 64 * 8)
         RK_BISECT(1, 8);
@@ -1910,6 +1927,7 @@ static int block_select_launch(const float* scores, int rows, int n_comp, int ra
     else
         RK_SELECT(1024, 0);
 #undef RK_BISECT
+#undef RK_FEW
 #undef RK_SELECT
     return launch_status();
 }
