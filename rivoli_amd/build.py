@@ -10,10 +10,12 @@ import os
 import re
 import subprocess
 import sys
+import sysconfig
 
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_PATH = os.path.join(CSRC, "librivoli_kvcache.so")
 HOST_LIB_PATH = os.path.join(CSRC, "librivoli_pagepool.so")
+LAUNCH_PATH = os.path.join(CSRC, "pylaunch.so")
 KERNELS = ["kv_append.hip", "kv_gather.hip", "index_topk.hip", "index_score.hip", "mla_attend.hip",
            "act_quant.hip", "kv_compress.hip", "kv_ring.hip", "gather_attn.hip", "hash_rows.hip",
            "block_index.hip"]
@@ -109,12 +111,28 @@ def build_host(verbose: bool = False) -> str:
     return HOST_LIB_PATH
 
 
+def build_launch(verbose: bool = False) -> str:
+    """The Python module of the launchers, beside the library it is linked against."""
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wextra",
+           "-I", os.path.join(os.path.dirname(CSRC), "..", "include"), "-I", sysconfig.get_paths()["include"],
+           "-o", LAUNCH_PATH, os.path.join(CSRC, "pylaunch.cpp"),
+           "-L", CSRC, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if verbose or res.returncode != 0:
+        sys.stderr.write(res.stdout + res.stderr)
+    if res.returncode != 0:
+        raise RuntimeError("g++ failed building " + LAUNCH_PATH)
+    return LAUNCH_PATH
+
+
 def build_all(verbose: bool = False) -> None:
     build_kernels(verbose)
     build_host(verbose)
+    build_launch(verbose)
 
 
 if __name__ == "__main__":
     build_all(verbose=True)
     print(LIB_PATH)
     print(HOST_LIB_PATH)
+    print(LAUNCH_PATH)

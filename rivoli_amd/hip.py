@@ -10,9 +10,11 @@ There is no fallback: if the HIP library has not been built, importing a launche
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
-from .build import LIB_PATH
+from .build import LAUNCH_PATH, LIB_PATH
 
 NULL_STREAM = None
 
@@ -132,16 +134,27 @@ def _p(x):
     return x.data_ptr()  # torch tensor
 
 
-def _s(stream):
-    if stream is None:
-        return None
-    if isinstance(stream, int):
-        return stream
-    return stream.cuda_stream  # torch.cuda.Stream
+class _Entries:
+    """The entry points as Python functions (csrc/pylaunch.cpp), loaded with the library on the
+    first use of one: tensors, ints, None and streams go in as they are, the status comes out."""
+
+    def __getattr__(self, name):
+        if name not in _SIGNATURES:
+            raise AttributeError(name)
+        lib()
+        if not os.path.exists(LAUNCH_PATH):
+            raise FileNotFoundError(f"{LAUNCH_PATH} is missing: build it with `python -m rivoli_amd.build`")
+        loader = importlib.machinery.ExtensionFileLoader("pylaunch", LAUNCH_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("pylaunch", loader))
+        self.__dict__.update((n, getattr(module, n)) for n in _SIGNATURES)
+        return self.__dict__[name]
+
+
+entry = _Entries()
 
 
 def device_sync() -> None:
-    ensure_hip_status(lib().rivoli_device_sync(), "device_sync")
+    ensure_hip_status(entry.rivoli_device_sync(), "device_sync")
 
 
 def kv_page_bytes(page_tokens: int, width: int) -> int:
@@ -151,60 +164,60 @@ def kv_page_bytes(page_tokens: int, width: int) -> int:
 # ---- reference-signature launchers --------------------------------------------------------
 
 def launch_append_kv(latent, rope, lc8, lscale, rc, pos, kvl, ropn, n_blocks) -> None:
-    ensure_hip_status(lib().rivoli_append_kv(_p(latent), _p(rope), _p(lc8), _p(lscale), _p(rc),
+    ensure_hip_status(entry.rivoli_append_kv(latent, rope, lc8, lscale, rc,
                                              pos, kvl, ropn, n_blocks), "append_kv")
 
 
 def launch_append_kv_rows(latent, rope, lc8, lscale, rc, pos0, n_tokens, kvl, ropn, n_blocks,
                           stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_append_kv_rows(_p(latent), _p(rope), _p(lc8), _p(lscale),
-                                                  _p(rc), pos0, n_tokens, kvl, ropn, n_blocks,
-                                                  _s(stream)), "append_kv_rows")
+    ensure_hip_status(entry.rivoli_append_kv_rows(latent, rope, lc8, lscale,
+                                                  rc, pos0, n_tokens, kvl, ropn, n_blocks,
+                                                  stream), "append_kv_rows")
 
 
 def launch_index_append(k, kcache, pos, hd) -> None:
-    ensure_hip_status(lib().rivoli_index_append(_p(k), _p(kcache), pos, hd), "index_append")
+    ensure_hip_status(entry.rivoli_index_append(k, kcache, pos, hd), "index_append")
 
 
 def launch_index_topk(scores, nt, k, rows) -> None:
-    ensure_hip_status(lib().rivoli_index_topk(_p(scores), nt, k, _p(rows)), "index_topk")
+    ensure_hip_status(entry.rivoli_index_topk(scores, nt, k, rows), "index_topk")
 
 
 def launch_index_score(q, w, kcache, heads, nt, nh, nact, hd, wscale, dscale, scores) -> None:
-    ensure_hip_status(lib().rivoli_index_score(_p(q), _p(w), _p(kcache), _p(heads), nt, nh, nact,
-                                               hd, wscale, dscale, _p(scores)), "index_score")
+    ensure_hip_status(entry.rivoli_index_score(q, w, kcache, heads, nt, nh, nact,
+                                               hd, wscale, dscale, scores), "index_score")
 
 
 def launch_index_score_paged(q, w, kpool, block_table, nts, heads, n_queries, max_blocks_per_seq,
                              stride, nt, nh, nact, hd, page_tokens, n_pages, wscale, dscale,
                              scores, stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_index_score_paged(
-        _p(q), _p(w), _p(kpool), _p(block_table), _p(nts), _p(heads), n_queries,
+    ensure_hip_status(entry.rivoli_index_score_paged(
+        q, w, kpool, block_table, nts, heads, n_queries,
         max_blocks_per_seq, stride, nt, nh, nact, hd, page_tokens, n_pages, wscale, dscale,
-        _p(scores), _s(stream)), "index_score_paged")
+        scores, stream), "index_score_paged")
 
 
 def launch_index_score_paged_hist(q, w, kpool, block_table, nts, heads, n_queries, max_blocks_per_seq,
                                   stride, nt, nh, nact, hd, page_tokens, n_pages, wscale, dscale,
                                   scores, topk_workspace, stream=NULL_STREAM) -> None:
     """index_score_paged that also counts the selection histogram into the top-k workspace."""
-    ensure_hip_status(lib().rivoli_index_score_paged_hist(
-        _p(q), _p(w), _p(kpool), _p(block_table), _p(nts), _p(heads), n_queries,
+    ensure_hip_status(entry.rivoli_index_score_paged_hist(
+        q, w, kpool, block_table, nts, heads, n_queries,
         max_blocks_per_seq, stride, nt, nh, nact, hd, page_tokens, n_pages, wscale, dscale,
-        _p(scores), _p(topk_workspace), _s(stream)), "index_score_paged_hist")
+        scores, topk_workspace, stream), "index_score_paged_hist")
 
 
 def launch_index_append_paged(k, slot_mapping, kpool, n_tokens, hd, page_tokens, n_pages,
                               bad_slots=None, stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_index_append_paged(_p(k), _p(slot_mapping), _p(kpool), n_tokens,
-                                                      hd, page_tokens, n_pages, _p(bad_slots),
-                                                      _s(stream)), "index_append_paged")
+    ensure_hip_status(entry.rivoli_index_append_paged(k, slot_mapping, kpool, n_tokens,
+                                                      hd, page_tokens, n_pages, bad_slots,
+                                                      stream), "index_append_paged")
 
 
 def launch_hash_rows(x, n, stride, i_base, out, stream=NULL_STREAM) -> None:
     if n > 2 ** 31 - 1:
         raise LaunchError("hash_rows", 1002)  # exceeds the i32 ABI, crates/backend/src/hip.rs:595-598
-    ensure_hip_status(lib().rivoli_hash_rows(_p(x), n, stride, i_base, _p(out), _s(stream)),
+    ensure_hip_status(entry.rivoli_hash_rows(x, n, stride, i_base, out, stream),
                       "hash_rows")
 
 
@@ -212,27 +225,27 @@ def launch_hash_rows(x, n, stride, i_base, out, stream=NULL_STREAM) -> None:
 
 def launch_kv_append_paged(rows, slot_mapping, pool, n_tokens, width, page_tokens, n_pages,
                            bad_slots=None, stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_kv_append_paged(_p(rows), _p(slot_mapping), _p(pool), n_tokens,
-                                                   width, page_tokens, n_pages, _p(bad_slots),
-                                                   _s(stream)), "kv_append_paged")
+    ensure_hip_status(entry.rivoli_kv_append_paged(rows, slot_mapping, pool, n_tokens,
+                                                   width, page_tokens, n_pages, bad_slots,
+                                                   stream), "kv_append_paged")
 
 
 def launch_kv_gather_paged(pool, block_table, seq_lens, cu_seqlens, out, n_seqs,
                            max_blocks_per_seq, width, page_tokens, n_pages, bad_pages=None,
                            stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_kv_gather_paged(_p(pool), _p(block_table), _p(seq_lens),
-                                                   _p(cu_seqlens), _p(out), n_seqs,
+    ensure_hip_status(entry.rivoli_kv_gather_paged(pool, block_table, seq_lens,
+                                                   cu_seqlens, out, n_seqs,
                                                    max_blocks_per_seq, width, page_tokens, n_pages,
-                                                   _p(bad_pages), _s(stream)), "kv_gather_paged")
+                                                   bad_pages, stream), "kv_gather_paged")
 
 
 def launch_kv_gather_paged_packed(pool, block_table, seq_lens, cu_seqlens, out, n_seqs,
                                   max_blocks_per_seq, total_tokens, width, page_tokens, n_pages,
                                   bad_pages=None, stream=NULL_STREAM) -> None:
     """launch_kv_gather_paged sized by the batch's real token count (>= sum of seq_lens)."""
-    ensure_hip_status(lib().rivoli_kv_gather_paged_packed(
-        _p(pool), _p(block_table), _p(seq_lens), _p(cu_seqlens), _p(out), n_seqs, max_blocks_per_seq,
-        total_tokens, width, page_tokens, n_pages, _p(bad_pages), _s(stream)), "kv_gather_paged_packed")
+    ensure_hip_status(entry.rivoli_kv_gather_paged_packed(
+        pool, block_table, seq_lens, cu_seqlens, out, n_seqs, max_blocks_per_seq,
+        total_tokens, width, page_tokens, n_pages, bad_pages, stream), "kv_gather_paged_packed")
 
 
 def launch_kv_append_gather_paged(new_rows, slot_mapping, pool, block_table, seq_lens, cu_seqlens, out, n_seqs,
@@ -240,19 +253,19 @@ def launch_kv_append_gather_paged(new_rows, slot_mapping, pool, block_table, seq
                                   bad_slots=None, bad_pages=None, stream=NULL_STREAM) -> None:
     """One launch for a decode step's cache work: append one new row per sequence (seq_lens already
     counts it; slot_mapping[s] is that token's slot), then gather every context."""
-    ensure_hip_status(lib().rivoli_kv_append_gather_paged(
-        _p(new_rows), _p(slot_mapping), _p(pool), _p(block_table), _p(seq_lens), _p(cu_seqlens), _p(out), n_seqs,
-        max_blocks_per_seq, total_tokens, width, page_tokens, n_pages, _p(bad_slots), _p(bad_pages),
-        _s(stream)), "kv_append_gather_paged")
+    ensure_hip_status(entry.rivoli_kv_append_gather_paged(
+        new_rows, slot_mapping, pool, block_table, seq_lens, cu_seqlens, out, n_seqs,
+        max_blocks_per_seq, total_tokens, width, page_tokens, n_pages, bad_slots, bad_pages,
+        stream), "kv_append_gather_paged")
 
 
 def launch_kv_gather_rows_paged(pool, block_table, rows, n_rows, out, n_queries, k,
                                 max_blocks_per_seq, width, page_tokens, n_pages, bad_rows=None,
                                 stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_kv_gather_rows_paged(_p(pool), _p(block_table), _p(rows),
-                                                        _p(n_rows), _p(out), n_queries, k,
+    ensure_hip_status(entry.rivoli_kv_gather_rows_paged(pool, block_table, rows,
+                                                        n_rows, out, n_queries, k,
                                                         max_blocks_per_seq, width, page_tokens,
-                                                        n_pages, _p(bad_rows), _s(stream)),
+                                                        n_pages, bad_rows, stream),
                       "kv_gather_rows_paged")
 
 
@@ -264,8 +277,8 @@ def launch_index_topk_batched(scores, n_queries, stride, nts, nt, k, rows, works
                               stream=NULL_STREAM) -> None:
     """`workspace`: a zero-filled device buffer of index_topk_workspace_bytes(n_queries, nt)
     bytes (left zero-filled by every call), or None for one workgroup per query."""
-    ensure_hip_status(lib().rivoli_index_topk_batched(_p(scores), n_queries, stride, _p(nts), nt,
-                                                      k, _p(rows), _p(workspace), _s(stream)),
+    ensure_hip_status(entry.rivoli_index_topk_batched(scores, n_queries, stride, nts, nt,
+                                                      k, rows, workspace, stream),
                       "index_topk_batched")
 
 
@@ -273,19 +286,19 @@ def launch_dsa_select_gather_paged(scores, n_queries, stride, nts, nt, k, rows, 
                                    pool, block_table, out, max_blocks_per_seq, width, page_tokens,
                                    n_pages, bad_rows=None, stream=NULL_STREAM) -> None:
     """Top-k selection and the sparse gather of the selected rows in one call."""
-    ensure_hip_status(lib().rivoli_dsa_select_gather_paged(
-        _p(scores), n_queries, stride, _p(nts), nt, k, _p(rows), _p(workspace), 1 if hist_ready else 0,
-        _p(pool), _p(block_table), _p(out), max_blocks_per_seq, width, page_tokens, n_pages,
-        _p(bad_rows), _s(stream)), "dsa_select_gather_paged")
+    ensure_hip_status(entry.rivoli_dsa_select_gather_paged(
+        scores, n_queries, stride, nts, nt, k, rows, workspace, 1 if hist_ready else 0,
+        pool, block_table, out, max_blocks_per_seq, width, page_tokens, n_pages,
+        bad_rows, stream), "dsa_select_gather_paged")
 
 
 def launch_dsa_select_gather_paged_noalloc(scores, n_queries, stride, nts, nt, k, rows, pool, block_table,
                                            out, max_blocks_per_seq, width, page_tokens, n_pages,
                                            bad_rows=None, stream=NULL_STREAM) -> None:
     """launch_dsa_select_gather_paged over the library's own workspace: allocates nothing."""
-    ensure_hip_status(lib().rivoli_dsa_select_gather_paged_noalloc(
-        _p(scores), n_queries, stride, _p(nts), nt, k, _p(rows), _p(pool), _p(block_table), _p(out),
-        max_blocks_per_seq, width, page_tokens, n_pages, _p(bad_rows), _s(stream)),
+    ensure_hip_status(entry.rivoli_dsa_select_gather_paged_noalloc(
+        scores, n_queries, stride, nts, nt, k, rows, pool, block_table, out,
+        max_blocks_per_seq, width, page_tokens, n_pages, bad_rows, stream),
         "dsa_select_gather_paged_noalloc")
 
 
@@ -299,8 +312,8 @@ def attend_scratch_floats(H: int, kvl: int) -> int:
 def launch_attend(qabs, qrope, lc8, lscale, rc, rows, H, nr, kvl, rope, n_blocks, scale, clat,
                   partial) -> None:
     """crates/backend/src/hip_attn.rs:113-128 (launch_attend -> rivoli_mla_attend)."""
-    ensure_hip_status(lib().rivoli_mla_attend(_p(qabs), _p(qrope), _p(lc8), _p(lscale), _p(rc), _p(rows),
-                                              H, nr, kvl, rope, n_blocks, scale, _p(clat), _p(partial)),
+    ensure_hip_status(entry.rivoli_mla_attend(qabs, qrope, lc8, lscale, rc, rows,
+                                              H, nr, kvl, rope, n_blocks, scale, clat, partial),
                       "mla_attend")
 
 
@@ -313,10 +326,10 @@ def mla_attend_paged_scratch_floats(n_seqs: int, H: int, max_rows: int) -> int:
 def launch_mla_attend_paged(qabs, qrope, pool, block_table, seq_lens, rows, n_rows, n_seqs, H,
                             max_rows, max_blocks_per_seq, kvl, rope, page_tokens, n_pages, scale,
                             precise, clat, partial, bad_rows=None, stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_mla_attend_paged(
-        _p(qabs), _p(qrope), _p(pool), _p(block_table), _p(seq_lens), _p(rows), _p(n_rows), n_seqs,
+    ensure_hip_status(entry.rivoli_mla_attend_paged(
+        qabs, qrope, pool, block_table, seq_lens, rows, n_rows, n_seqs,
         H, max_rows, max_blocks_per_seq, kvl, rope, page_tokens, n_pages, scale, int(precise),
-        _p(clat), _p(partial), _p(bad_rows), _s(stream)), "mla_attend_paged")
+        clat, partial, bad_rows, stream), "mla_attend_paged")
 
 
 # ---- the second cache format: simulated-fp8 rows, scored block selection -------------------
@@ -324,44 +337,44 @@ def launch_mla_attend_paged(qabs, qrope, pool, block_table, seq_lens, rows, n_ro
 def launch_act_quant_f8_prefix(src, dst, rows, row_stride, n, block, stream=NULL_STREAM) -> None:
     """crates/backend/src/hip_attn.rs launch_act_quant_f8_prefix: quantize-dequantize dims
     [0, n) of every row in blocks of `block`; src may be dst."""
-    ensure_hip_status(lib().rivoli_act_quant_f8_prefix(_p(src), _p(dst), rows, row_stride, n, block,
-                                                       _s(stream)), "act_quant_f8_prefix")
+    ensure_hip_status(entry.rivoli_act_quant_f8_prefix(src, dst, rows, row_stride, n, block,
+                                                       stream), "act_quant_f8_prefix")
 
 
 def launch_act_quant_f4_rotated(x, rows, d, stream=NULL_STREAM) -> None:
     """crates/backend/src/hip_linalg.rs:620 launch_act_quant_f4_rotated: the Hadamard + fp4
     spread of every row of x [rows][d], in place."""
-    ensure_hip_status(lib().rivoli_act_quant_f4_rotated(_p(x), rows, d, _s(stream)), "act_quant_f4_rotated")
+    ensure_hip_status(entry.rivoli_act_quant_f4_rotated(x, rows, d, stream), "act_quant_f4_rotated")
 
 
 def launch_index_score_blocks(q, kv, w, score, s, n_comp, heads, hd, stream=NULL_STREAM) -> None:
     """crates/backend/src/hip.rs:497-520 launch_index_score_blocks: block scores [s][n_comp]."""
-    ensure_hip_status(lib().rivoli_index_score_blocks(_p(q), _p(kv), _p(w), _p(score), s, n_comp, heads, hd,
-                                                      _s(stream)), "index_score_blocks")
+    ensure_hip_status(entry.rivoli_index_score_blocks(q, kv, w, score, s, n_comp, heads, hd,
+                                                      stream), "index_score_blocks")
 
 
 def launch_index_score_blocks_prefill(q, kv, w, score, s, n_comp, heads, hd, ratio, stream=NULL_STREAM) -> None:
     """launch_index_score_blocks for a prefill: only entries a row's selection can rank
     (block < (t + 1) / ratio, in groups of 64 blocks) are computed."""
-    ensure_hip_status(lib().rivoli_index_score_blocks_prefill(_p(q), _p(kv), _p(w), _p(score), s, n_comp, heads,
-                                                              hd, ratio, _s(stream)), "index_score_blocks_prefill")
+    ensure_hip_status(entry.rivoli_index_score_blocks_prefill(q, kv, w, score, s, n_comp, heads,
+                                                              hd, ratio, stream), "index_score_blocks_prefill")
 
 
 def launch_index_select_blocks(scores, rows, n_comp, ratio, index_topk, prefill, offset, out,
                                stream=NULL_STREAM) -> None:
     """crates/engine/src/v4/select.rs scored_rows on the device: out is int32
     [rows][min(index_topk, n_comp)]."""
-    ensure_hip_status(lib().rivoli_index_select_blocks(_p(scores), rows, n_comp, ratio, index_topk,
-                                                       1 if prefill else 0, offset, _p(out),
-                                                       _s(stream)), "index_select_blocks")
+    ensure_hip_status(entry.rivoli_index_select_blocks(scores, rows, n_comp, ratio, index_topk,
+                                                       1 if prefill else 0, offset, out,
+                                                       stream), "index_select_blocks")
 
 
 def sel_shape(win, ratio, index_topk, seqlen, start_pos):
     """crates/engine/src/v4/select.rs Sel::shape: (rows, cols) of the positional rectangle;
     raises LaunchError with the guard code where the reference refuses."""
     rows, cols = C.c_int(0), C.c_int(0)
-    ensure_hip_status(lib().rivoli_sel_shape(win, ratio, index_topk, seqlen, start_pos, C.byref(rows),
-                                             C.byref(cols)), "sel_shape")
+    ensure_hip_status(entry.rivoli_sel_shape(win, ratio, index_topk, seqlen, start_pos, C.addressof(rows),
+                                             C.addressof(cols)), "sel_shape")
     return rows.value, cols.value
 
 
@@ -387,7 +400,7 @@ def compress_dst(ratio, region_base, seqlen, start_pos):
 def launch_sel_gather(win, ratio, index_topk, seqlen, start_pos, out, stream=NULL_STREAM):
     """Sel::gather on the device: out is int32 [rows][cols] of sel_shape. Returns (rows, cols)."""
     shape = sel_shape(win, ratio, index_topk, seqlen, start_pos)
-    ensure_hip_status(lib().rivoli_sel_gather(win, ratio, index_topk, seqlen, start_pos, _p(out), _s(stream)),
+    ensure_hip_status(entry.rivoli_sel_gather(win, ratio, index_topk, seqlen, start_pos, out, stream),
                       "sel_gather")
     return shape
 
@@ -396,15 +409,15 @@ def launch_sel_gather_scored(scores, n_comp, win, ratio, index_topk, seqlen, sta
                              stream=NULL_STREAM):
     """Sel::gather_scored over scored_rows on the device. Returns (rows, cols)."""
     cols = C.c_int(0)
-    ensure_hip_status(lib().rivoli_sel_gather_scored(_p(scores), n_comp, win, ratio, index_topk, seqlen,
-                                                     start_pos, _p(out), C.byref(cols), _s(stream)),
+    ensure_hip_status(entry.rivoli_sel_gather_scored(scores, n_comp, win, ratio, index_topk, seqlen,
+                                                     start_pos, out, C.addressof(cols), stream),
                       "sel_gather_scored")
     return (seqlen if start_pos == 0 else 1), cols.value
 
 
 def launch_kv_ring_write(kv, cache, win, hd, seqlen, start_pos, stream=NULL_STREAM) -> None:
     """crates/engine/src/v4/attn.rs write_ring as one launch."""
-    ensure_hip_status(lib().rivoli_kv_ring_write(_p(kv), _p(cache), win, hd, seqlen, start_pos, _s(stream)),
+    ensure_hip_status(entry.rivoli_kv_ring_write(kv, cache, win, hd, seqlen, start_pos, stream),
                       "kv_ring_write")
 
 
@@ -419,16 +432,16 @@ def launch_gather_attn_shared_kv(q, kv, sink, idxs, m, h, d, topk, scale, o, str
     bounded entry point runs: indices at or past it are treated as masked. With partial (a
     buffer of gather_attn_scratch_floats f32) a query's list may be shared among workgroups."""
     if partial is not None:
-        code = lib().rivoli_gather_attn_shared_kv_split(_p(q), _p(kv), _p(sink), _p(idxs), m, h, d, topk,
+        code = entry.rivoli_gather_attn_shared_kv_split(q, kv, sink, idxs, m, h, d, topk,
                                                         0x7fffffff if n_kv is None else n_kv, scale, precise,
-                                                        _p(o), _p(partial), _s(stream))
+                                                        o, partial, stream)
     elif n_kv is None and precise == 2:
-        code = lib().rivoli_gather_attn_shared_kv(_p(q), _p(kv), _p(sink), _p(idxs), m, h, d, topk, scale, _p(o),
-                                                  _s(stream))
+        code = entry.rivoli_gather_attn_shared_kv(q, kv, sink, idxs, m, h, d, topk, scale, o,
+                                                  stream)
     else:
-        code = lib().rivoli_gather_attn_shared_kv_bounded(_p(q), _p(kv), _p(sink), _p(idxs), m, h, d, topk,
+        code = entry.rivoli_gather_attn_shared_kv_bounded(q, kv, sink, idxs, m, h, d, topk,
                                                           0x7fffffff if n_kv is None else n_kv, scale, precise,
-                                                          _p(o), _s(stream))
+                                                          o, stream)
     ensure_hip_status(code, "gather_attn_shared_kv")
 
 
@@ -454,42 +467,42 @@ class CompFinish(C.Structure):
         return cls(_p(norm), _p(freqs), _p(out))
 
 
-def _ref_or_null(struct):
-    return None if struct is None else C.byref(struct)
+def _addr_or_null(struct):
+    return None if struct is None else C.addressof(struct)
 
 
 def launch_kv_compress_deposit(kv, score, ape, kv_state, score_state, geom, s, slot0,
                                stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_kv_compress_deposit(
-        _p(kv), _p(score), _p(ape), _p(kv_state), _p(score_state), _ref_or_null(geom), s, slot0,
-        _s(stream)), "kv_compress_deposit")
+    ensure_hip_status(entry.rivoli_kv_compress_deposit(
+        kv, score, ape, kv_state, score_state, _addr_or_null(geom), s, slot0,
+        stream), "kv_compress_deposit")
 
 
 def launch_kv_compress_prefill(kv, score, ape, finish, geom, nblk, stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_kv_compress_prefill(
-        _p(kv), _p(score), _p(ape), _ref_or_null(finish), _ref_or_null(geom), nblk, _s(stream)),
+    ensure_hip_status(entry.rivoli_kv_compress_prefill(
+        kv, score, ape, _addr_or_null(finish), _addr_or_null(geom), nblk, stream),
         "kv_compress_prefill")
 
 
 def launch_kv_compress_decode(kv_state, score_state, finish, geom, start_pos,
                               stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_kv_compress_decode(
-        _p(kv_state), _p(score_state), _ref_or_null(finish), _ref_or_null(geom), start_pos,
-        _s(stream)), "kv_compress_decode")
+    ensure_hip_status(entry.rivoli_kv_compress_decode(
+        kv_state, score_state, _addr_or_null(finish), _addr_or_null(geom), start_pos,
+        stream), "kv_compress_decode")
 
 
 # ---- element codecs -----------------------------------------------------------------------
 
 def launch_codec_e4m3_encode(x, out, n, stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_codec_e4m3_encode(_p(x), _p(out), n, _s(stream)),
+    ensure_hip_status(entry.rivoli_codec_e4m3_encode(x, out, n, stream),
                       "codec_e4m3_encode")
 
 
 def launch_codec_e4m3_dequant_bf16(codes, scale, out, n, stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_codec_e4m3_dequant_bf16(_p(codes), scale, _p(out), n,
-                                                           _s(stream)), "codec_e4m3_dequant_bf16")
+    ensure_hip_status(entry.rivoli_codec_e4m3_dequant_bf16(codes, scale, out, n,
+                                                           stream), "codec_e4m3_dequant_bf16")
 
 
 def launch_codec_bf16_encode(x, out, n, stream=NULL_STREAM) -> None:
-    ensure_hip_status(lib().rivoli_codec_bf16_encode(_p(x), _p(out), n, _s(stream)),
+    ensure_hip_status(entry.rivoli_codec_bf16_encode(x, out, n, stream),
                       "codec_bf16_encode")
