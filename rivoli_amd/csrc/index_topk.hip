@@ -1835,14 +1835,35 @@ __device__ __forceinline__ bool select_positional(int32_t* o, int limit, int k, 
     return true;
 }
 
+// The window rule of a selection rectangle (select.rs:195-216): column j of row t.
+__device__ __forceinline__ int window_entry(int t, int j, int win, int start_pos) {
+    if (start_pos == 0) {
+        const int first = t > win - 1 ? t - (win - 1) : 0;
+        return first + j <= t ? first + j : -1;
+    }
+    if (start_pos >= win - 1) return (start_pos % win + 1 + j) % win;  // oldest first, from just past the newest slot
+    return j <= start_pos ? j : -1;
+}
+// The window columns in front of a selection (none: cols = 0), written by the workgroup that
+// selects for the row: a launch of their own cost a prompt of 8 192 rows 5.1 us and a decode step 1.3
+// (and the host a launch), in here they are a store or two per lane ahead of the selection's loads.
+struct SelWindow {
+    int win, start_pos, cols;
+};
+template <int THREADS>
+__device__ __forceinline__ void write_window(const SelWindow& w, int t, int32_t* o) {
+    for (int j = threadIdx.x; j < w.cols; j += THREADS) o[j - w.cols] = window_entry(t, j, w.win, w.start_pos);
+}
+
 template <int WAVES, int ITEMS>
 __global__ __launch_bounds__(WAVES* kWave) void block_select_bisect_kernel(
     const float* __restrict__ scores, int n_comp, int ratio, int prefill, int k, int offset,
-    int32_t* __restrict__ out, int out_stride) {
+    int32_t* __restrict__ out, int out_stride, SelWindow window) {
     __shared__ __attribute__((aligned(16))) uint32_t lds[sel_lds_words<WAVES>()];
     const int t = blockIdx.x;
     const int limit = select_row_limit(t, n_comp, ratio, prefill);
     int32_t* o = out + (size_t)t * out_stride;
+    write_window<WAVES * kWave>(window, t, o);
     if (select_positional<WAVES * kWave>(o, limit, k, offset)) return;
     select_bisect<WAVES, ITEMS, TotalOrderKey>(scores + (size_t)t * n_comp, limit, (uint32_t)k,
                                                reinterpret_cast<uint32_t*>(o), lds,
@@ -1853,11 +1874,12 @@ __global__ __launch_bounds__(WAVES* kWave) void block_select_bisect_kernel(
 template <int ITEMS>
 __global__ __launch_bounds__(1024) void block_select_few_kernel(
     const float* __restrict__ scores, int n_comp, int ratio, int prefill, int k, int offset,
-    int32_t* __restrict__ out, int out_stride) {
+    int32_t* __restrict__ out, int out_stride, SelWindow window) {
     __shared__ __attribute__((aligned(16))) uint32_t lds[sel_lds_words<16>()];
     const int t = blockIdx.x;
     const int limit = select_row_limit(t, n_comp, ratio, prefill);
     int32_t* o = out + (size_t)t * out_stride;
+    write_window<1024>(window, t, o);
     if (select_positional<1024>(o, limit, k, offset)) return;
     select_bisect<16, ITEMS, TotalOrderKey>(scores + (size_t)t * n_comp, limit, (uint32_t)k,
                                             reinterpret_cast<uint32_t*>(o), lds, (uint32_t)offset);
@@ -1869,11 +1891,12 @@ __global__ __launch_bounds__(THREADS) void block_select_kernel(const float* __re
                                                                int n_comp, int ratio, int prefill,
                                                                int k, int offset,
                                                                int32_t* __restrict__ out,
-                                                               int out_stride) {
+                                                               int out_stride, SelWindow window) {
     __shared__ uint32_t lds[topk_block_lds_words<THREADS>()];
     const int t = blockIdx.x;
     const int limit = select_row_limit(t, n_comp, ratio, prefill);
     int32_t* o = out + (size_t)t * out_stride;
+    write_window<THREADS>(window, t, o);
     if (select_positional<THREADS>(o, limit, k, offset)) return;
     topk_block<THREADS, ITEMS, TotalOrderKey>(scores + (size_t)t * n_comp, limit, (uint32_t)k,
                                               reinterpret_cast<uint32_t*>(o), lds,
@@ -1886,7 +1909,7 @@ constexpr int kSelFewRows = 256;  // a workgroup of sixteen waves per compute un
 // rectangle's width when the selection is the tail of a [window | compressed] row.
 static int block_select_launch(const float* scores, int rows, int n_comp, int ratio,
                                int index_topk, int prefill, int offset, int* out, int out_stride,
-                               hipStream_t stream) {
+                               const SelWindow& window, hipStream_t stream) {
     if (!scores || !out) return 1001;
     if (rows <= 0 || n_comp <= 0 || ratio <= 0 || index_topk <= 0 || offset < 0) return 1001;
     if ((long long)offset + n_comp > 0x7fffffffLL) return 1002;
@@ -1896,13 +1919,13 @@ static int block_select_launch(const float* scores, int rows, int n_comp, int ra
     const dim3 grid((unsigned)rows);
 #define RK_BISECT(WV, I)                                                                     \
     hipLaunchKernelGGL((block_select_bisect_kernel<WV, I>), grid, dim3(WV* kWave), 0, stream, \
-                       scores, n_comp, ratio, prefill ? 1 : 0, k, offset, out, out_stride)
+                       scores, n_comp, ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
 #define RK_FEW(I)                                                                             \
     hipLaunchKernelGGL((block_select_few_kernel<I>), grid, dim3(1024), 0, stream, scores, n_comp, \
-                       ratio, prefill ? 1 : 0, k, offset, out, out_stride)
+                       ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
 #define RK_SELECT(T, I)                                                                       \
     hipLaunchKernelGGL((block_select_kernel<T, I>), grid, dim3(T), 0, stream, scores, n_comp, \
-                       ratio, prefill ? 1 : 0, k, offset, out, out_stride)
+                       ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
     // Few rows (decode: one) leave the chip to one workgroup each, and a row's time is its
     // longest wave's: sixteen waves, 8 keys a lane. One row of 8192: 17.8 -> 8.8 us.
     if (rows <= kSelFewRows && n_comp > 64 * 8 && n_comp <= 1024 * 8)
@@ -1952,27 +1975,16 @@ static SelShape sel_shape(int win, int ratio, int seqlen, int start_pos) {
 }
 
 // One thread per cell of the first `win_cols + n_pos` columns of a `cols`-wide row: the window
-// rule (select.rs:195-216), then the positional block rule (:224-241) for n_pos columns.
+// rule, then the positional block rule (select.rs:224-241) for n_pos columns.
 __global__ __launch_bounds__(256) void sel_fill_kernel(int win, int ratio, int start_pos,
                                                        int win_cols, int n_pos, int offset,
                                                        int cols, int32_t* __restrict__ out) {
     const int j = blockIdx.y * 256 + threadIdx.x, t = blockIdx.x;  // rows on x: no 65 535 limit
     if (j >= win_cols + n_pos) return;
-    int v;
-    if (j < win_cols) {
-        if (start_pos == 0) {
-            const int first = t > win - 1 ? t - (win - 1) : 0;
-            v = first + j <= t ? first + j : -1;
-        } else if (start_pos >= win - 1) {
-            v = (start_pos % win + 1 + j) % win;  // oldest first, from just past the newest slot
-        } else {
-            v = j <= start_pos ? j : -1;
-        }
-    } else {
-        const int c = j - win_cols;
-        v = (start_pos != 0 || c < (t + 1) / ratio) ? c + offset : -1;
-    }
-    out[(size_t)t * cols + j] = v;
+    const int c = j - win_cols;
+    out[(size_t)t * cols + j] = j < win_cols ? window_entry(t, j, win, start_pos)
+                                : start_pos != 0 || c < (t + 1) / ratio ? c + offset
+                                                                        : -1;
 }
 
 static int sel_fill_launch(const SelShape& s, int win, int ratio, int start_pos, int n_pos,
@@ -2068,10 +2080,11 @@ extern "C" int rivoli_sel_gather_scored(const float* scores, int n_comp, int win
     const int k = index_topk < n_comp ? index_topk : n_comp;
     const int cols = s.win_cols + k;
     if (cols_out) *cols_out = cols;
-    const int code = rk::sel_fill_launch(s, win, ratio, start_pos, 0, cols, out, (hipStream_t)stream);
-    if (code || k == 0) return code;
-    return rk::block_select_launch(scores, s.rows, n_comp, ratio, index_topk, start_pos == 0,
-                                   s.offset, out + s.win_cols, cols, (hipStream_t)stream);
+    if (k == 0) return rk::sel_fill_launch(s, win, ratio, start_pos, 0, cols, out, (hipStream_t)stream);
+    if ((s.win_cols + 255) / 256 > 65535) return 1002;  // as the fill's launch
+    return rk::block_select_launch(scores, s.rows, n_comp, ratio, index_topk, start_pos == 0, s.offset,
+                                   out + s.win_cols, cols, rk::SelWindow{win, start_pos, s.win_cols},
+                                   (hipStream_t)stream);
 }
 
 extern "C" int rivoli_index_select_blocks(const float* scores, int rows, int n_comp, int ratio,
@@ -2079,7 +2092,7 @@ extern "C" int rivoli_index_select_blocks(const float* scores, int rows, int n_c
                                           void* stream) {
     const int k = index_topk < n_comp ? index_topk : n_comp;
     return rk::block_select_launch(scores, rows, n_comp, ratio, index_topk, prefill, offset, out,
-                                   k, (hipStream_t)stream);
+                                   k, rk::SelWindow{0, 0, 0}, (hipStream_t)stream);
 }
 
 extern "C" size_t rivoli_index_topk_workspace_bytes(int n_queries, int nt) {
