@@ -50,7 +50,11 @@ constexpr float kFp4MaxInv = 1.0f / kFp4Max;
 constexpr float kFp4AmaxFloor = kFp4Max * 1.17549435082228750797e-38f;  // 6 * 2^-126 (actquant.hpp:51)
 constexpr int kSpreadMaxD = 256;   // blockindex.hip:40-42
 constexpr int kSpreadThreads = 256;
-constexpr int kSpreadInFlight = 4;  // row groups per wave, all requested before the first is used
+// Row groups per wave, all requested before the first is used: 4, or 1 where that leaves fewer
+// workgroups than compute units (a wave's row groups are worked on one after the other: 64 rows of
+// 128, a decode step's, 5.0 -> 3.0 us; one row 3.4 -> 1.8).
+constexpr int kSpreadInFlight = 4;
+constexpr int kSpreadFewGroups = 256;
 
 // bf16(x) as a float: the conversion of the pair (0, x) leaves it in the upper half, one instruction.
 __device__ __forceinline__ float round_bf16(float x) {
@@ -74,25 +78,25 @@ __device__ __forceinline__ float e2m1_round_trip(float q) {
 
 // LPR: lanes per row (d / 4). scale = 1 / sqrt(d), taken on the host (a correctly rounded
 // square root and a true divide, blockindex.hip:107-113).
-template <int LPR>
+template <int LPR, int IN_FLIGHT>
 __global__ __launch_bounds__(kSpreadThreads) void f4_rotated_kernel(float* __restrict__ x,
                                                                      long long rows, float scale) {
     constexpr int kRowsPerWave = kWave / LPR;
     constexpr int d = LPR * 4;
     const int lane = threadIdx.x & (kWave - 1);
     const long long wave = (long long)blockIdx.x * (kSpreadThreads / kWave) + (threadIdx.x >> 6);
-    const long long row0 = wave * (kRowsPerWave * kSpreadInFlight) + lane / LPR;
+    const long long row0 = wave * (kRowsPerWave * IN_FLIGHT) + lane / LPR;
     const int col = (lane % LPR) * 4;
 
-    f32x4 v[kSpreadInFlight];
+    f32x4 v[IN_FLIGHT];
 #pragma unroll
-    for (int u = 0; u < kSpreadInFlight; ++u) {
+    for (int u = 0; u < IN_FLIGHT; ++u) {
         const long long r = row0 + (long long)u * kRowsPerWave;
         // unconditional: a row past the end re-reads the last row and is not stored
         v[u] = *reinterpret_cast<const f32x4*>(x + (r < rows ? r : rows - 1) * d + col);
     }
 #pragma unroll
-    for (int u = 0; u < kSpreadInFlight; ++u) {
+    for (int u = 0; u < IN_FLIGHT; ++u) {
         float e[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
         // stages h = 1, 2: inside the lane
         {
@@ -534,38 +538,50 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
     }
 }
 
-// Few queries (a decode step: one). A workgroup owns one query's 64 heads against 64 blocks, a
-// wave 32 x 32 of them: one matrix tile, operands straight from memory (lane L holds half L >> 5
-// of row L & 31, contiguous: the contraction's terms may be dealt to its steps in any order), the
-// head terms through LDS, the first wave folding them in head order. Bound by latency.
-// 8 192 blocks: 7.8 us, 14.1 with every dot folded term by term.
+// Few queries (a decode step: one). A workgroup owns one query's 64 heads against 32 HT blocks, a
+// wave 16 HT heads and 32 blocks of them: 16 x 16 matrix tiles, operands straight from memory (lane
+// group g holds the eight dims at 32 j + 8 g of row n16: four lanes take a line of a row, where a
+// lane per row takes a line each), the head terms through LDS, the first wave folding them in head
+// order. Bound by latency. 8 192 blocks: 14.1 us with every dot folded term by term, 8.0 as 32 x 32
+// tiles of 64-block workgroups with a lane per row, 6.0 so.
 constexpr int kOneThreads = 4 * kWave;
+template <int HT>
 __global__ __launch_bounds__(kOneThreads) void score_blocks_one_kernel(
     const float* __restrict__ q, const float* __restrict__ kv, const float* __restrict__ w,
     float* __restrict__ score, int s, int n_comp, int heads, int ratio) {
-    __shared__ float terms[kPairHeads][kWave];
+    constexpr int BLOCKS = 32 * HT;
+    __shared__ float terms[kPairHeads][BLOCKS];
     __shared__ int inexact;
-    const int lane = threadIdx.x & (kWave - 1), half = lane >> 5, row = lane & 31;
+    const int lane = threadIdx.x & (kWave - 1), g = lane >> 4, n16 = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int t = blockIdx.y;
-    const long long cw = (long long)blockIdx.x * kWave, c = cw + lane;
-    if (first_query(t, t + 1, ratio, cw) > t) return;  // workgroup-uniform: no block of these is legal for t
+    const long long cw = (long long)blockIdx.x * BLOCKS, c = cw + (lane & (BLOCKS - 1));
+    if (first_query(t, t + 1, ratio, cw & ~63ll) > t) return;  // workgroup-uniform: no block of the 64 is legal for t
     if (threadIdx.x == 0) inexact = 0;
     const size_t base = (size_t)t * heads;
-    const int h0 = (wave & 1) * 32, b0 = (wave >> 1) * 32;
+    const int h0 = HT == 1 ? wave * 16 : (wave & 1) * 32, c0 = HT == 1 ? 0 : (wave >> 1) * 32;
     __syncthreads();
     if (h0 < heads) {
-        const auto operand = [&](const float* p, bool live, bf16x8 (&x)[8]) {
+        struct Row {
+            f32x4 v[8];
+        };
+        const auto fetch = [&](const float* p) {
+            Row r;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                r.v[2 * j] = *reinterpret_cast<const f32x4_u*>(p + 32 * j + 8 * g);
+                r.v[2 * j + 1] = *reinterpret_cast<const f32x4_u*>(p + 32 * j + 8 * g + 4);
+            }
+            return r;
+        };
+        const auto operand = [&](const Row& r, bool live, bf16x8 (&x)[4]) {
             RowSpan span;
-            f32x4 v[16];
 #pragma unroll
-            for (int j = 0; j < 16; ++j) v[j] = *reinterpret_cast<const f32x4_u*>(p + half * 64 + j * 4);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
+            for (int k = 0; k < 4; ++k) {
                 u32x4 b;
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
-                    f32x4 u = v[2 * k + j];
+                    f32x4 u = r.v[2 * k + j];
                     if (!live) u = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                     b[2 * j] = upper_halves(u.x, u.y), b[2 * j + 1] = upper_halves(u.z, u.w);
                     span.add(b[2 * j], low_half_bits(u));
@@ -573,38 +589,55 @@ __global__ __launch_bounds__(kOneThreads) void score_blocks_one_kernel(
                 }
                 x[k] = __builtin_bit_cast(bf16x8, b);
             }
-            const uint32_t f = span.folded();
+            uint32_t f = span.folded();
+            f = span_max(f, __shfl_xor(f, 16, kWave));
             return span_of(span_max(f, __shfl_xor(f, 32, kWave)));
         };
-        bf16x8 a[8], b[8];
-        const int hr = h0 + row;
-        const long long cr = cw + b0 + row;
-        int q_span = operand(q + (base + min(hr, heads - 1)) * 128, hr < heads, a);
-        const int k_span = operand(kv + (size_t)(cr < n_comp ? cr : n_comp - 1) * 128, true, b);
+        const long long last = n_comp - 1;
+        Row rq[HT], rk[2];
+        float wv[HT][4];
 #pragma unroll
-        for (int m = 1; m < 32; m <<= 1) q_span = max(q_span, __shfl_xor(q_span, m, kWave));
+        for (int u = 0; u < HT; ++u) rq[u] = fetch(q + (base + min(h0 + 16 * u + n16, heads - 1)) * 128);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) rk[u] = fetch(kv + (size_t)min(cw + c0 + 16 * u + n16, last) * 128);
+#pragma unroll
+        for (int u = 0; u < HT; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) wv[u][i] = w[base + min(h0 + 16 * u + 4 * g + i, heads - 1)];
+        bf16x8 a[HT][4], b[2][4];
+        int q_span = 0;
+#pragma unroll
+        for (int u = 0; u < HT; ++u) q_span = max(q_span, operand(rq[u], h0 + 16 * u + n16 < heads, a[u]));
+        const int k_span = max(operand(rk[0], true, b[0]), operand(rk[1], true, b[1]));
+#pragma unroll
+        for (int m = 1; m < 16; m <<= 1) q_span = max(q_span, __shfl_xor(q_span, m, kWave));
         if (__any(q_span + k_span > kExactSpan)) {
             if (lane == 0) inexact = 1;
         } else {
-            f32x16 d = {};
 #pragma unroll
-            for (int k = 0; k < 8; ++k) d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[k], b[k], d, 0, 0, 0);
+            for (int v = 0; v < 2 * HT; ++v) {
+                f32x4 d = {0, 0, 0, 0};
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int hh = h0 + (i >> 2) * 8 + half * 4 + (i & 3);
-                if (hh < heads) terms[hh][b0 + row] = head_term(d[i], w[base + hh]);
+                for (int k = 0; k < 4; ++k)
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[v >> 1][k], b[v & 1][k], d, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int hh = h0 + 16 * (v >> 1) + 4 * g + i;
+                    if (hh < heads) terms[hh][c0 + 16 * (v & 1) + n16] = head_term(d[i], wv[v >> 1][i]);
+                }
             }
         }
     }
     __syncthreads();
-    if (inexact) {  // term by term: every wave a quarter of the heads for all 64 blocks
+    if (inexact) {  // term by term: every wave a quarter of the heads for all blocks (32 of them: twice, the same values)
         const int per = (heads + 3) / 4, g0 = min(wave * per, heads), g1 = min(g0 + per, heads);
         float row_v[128];
         load_row(row_v, kv + (size_t)(c < n_comp ? c : n_comp - 1) * 128);
-        walk_pairs(q, w, row_v, base + g0, base + g1, [&](size_t g, float term) { terms[g - base][lane] = term; });
+        walk_pairs(q, w, row_v, base + g0, base + g1,
+                   [&](size_t h, float term) { terms[h - base][lane & (BLOCKS - 1)] = term; });
         __syncthreads();
     }
-    if (wave == 0) {
+    if (threadIdx.x < BLOCKS) {
         float acc = 0.0f;
         for (int hh = 0; hh < heads; ++hh) acc = acc + terms[hh][lane];
         if (c < n_comp) score[(size_t)t * n_comp + c] = round_bf16(acc);
@@ -648,23 +681,31 @@ extern "C" int rivoli_act_quant_f4_rotated(float* x, int rows, int d, void* stre
     (void)hipGetLastError();
     const float scale = 1.0f / std::sqrt((float)d);
     const int lpr = d / 4;
-    const long long rows_per_group = (long long)(rk::kWave / lpr) * rk::kSpreadInFlight *
-                                     (rk::kSpreadThreads / rk::kWave);
+    const long long rows_per_step = (long long)(rk::kWave / lpr) * (rk::kSpreadThreads / rk::kWave);
+    const bool few = rows <= rows_per_step * rk::kSpreadInFlight * rk::kSpreadFewGroups;
+    const long long rows_per_group = few ? rows_per_step : rows_per_step * rk::kSpreadInFlight;
     const dim3 grid((unsigned)((rows + rows_per_group - 1) / rows_per_group)), block(rk::kSpreadThreads);
     hipStream_t st = (hipStream_t)stream;
+#define RK_SPREAD(LPR)                                                                                      \
+    if (few)                                                                                                \
+        hipLaunchKernelGGL((rk::f4_rotated_kernel<LPR, 1>), grid, block, 0, st, x, (long long)rows, scale); \
+    else                                                                                                    \
+        hipLaunchKernelGGL((rk::f4_rotated_kernel<LPR, rk::kSpreadInFlight>), grid, block, 0, st, x,        \
+                           (long long)rows, scale)
     switch (lpr) {
-        case 8: hipLaunchKernelGGL(rk::f4_rotated_kernel<8>, grid, block, 0, st, x, (long long)rows, scale); break;
-        case 16: hipLaunchKernelGGL(rk::f4_rotated_kernel<16>, grid, block, 0, st, x, (long long)rows, scale); break;
-        case 32: hipLaunchKernelGGL(rk::f4_rotated_kernel<32>, grid, block, 0, st, x, (long long)rows, scale); break;
-        default: hipLaunchKernelGGL(rk::f4_rotated_kernel<64>, grid, block, 0, st, x, (long long)rows, scale); break;
+        case 8: RK_SPREAD(8); break;
+        case 16: RK_SPREAD(16); break;
+        case 32: RK_SPREAD(32); break;
+        default: RK_SPREAD(64); break;
     }
+#undef RK_SPREAD
     return rk::launch_status();
 }
 
 namespace rk {
-// Up to here a workgroup per (query, 64 blocks) is the faster: 4 queries x 4 096 blocks 8 us against
-// 10 (4 x 8 192, 512 workgroups: 11.3 against 10.1; 300 queries x 75, 600: 15 against 10). One query
-// has no second for the many-query kernel's wave: 8 192 blocks 7.8 against 10.3, 65 536 20 against 25.
+// Up to here a workgroup per (query, 64 blocks) is the faster: 4 queries x 4 096 blocks 7 us against
+// 10 (4 x 8 192, 512 workgroups: 11.3 against 10.4; 300 queries x 75, 600: 15 against 10). One query
+// has no second for the many-query kernel's wave: 65 536 blocks 18 us against 25.
 constexpr int kOneGroups = 384;
 static int score_blocks_launch(const float* q, const float* kv, const float* w, float* score, int s,
                                int n_comp, int heads, int hd, int ratio, hipStream_t st) {
@@ -677,8 +718,14 @@ static int score_blocks_launch(const float* q, const float* kv, const float* w, 
     if (hd == 128 && aligned16(kv) && heads <= kPairHeads) {
         const unsigned groups = (unsigned)(((long long)n_comp + kWave - 1) / kWave);
         if (s == 1 || (long long)s * groups <= kOneGroups) {
-            hipLaunchKernelGGL(score_blocks_one_kernel, dim3(groups, (unsigned)s), dim3(kOneThreads), 0, st, q, kv, w,
-                               score, s, n_comp, heads, ratio);
+            // half the blocks a workgroup while there is a compute unit for each (8 192 blocks 6.1 us, 7.1 in
+            // 64s; 16 384 blocks 7.1 us in 64s, 8.5 in 32s)
+            if ((long long)s * 2 * groups <= 256)
+                hipLaunchKernelGGL(score_blocks_one_kernel<1>, dim3((unsigned)(((long long)n_comp + 31) / 32), (unsigned)s),
+                                   dim3(kOneThreads), 0, st, q, kv, w, score, s, n_comp, heads, ratio);
+            else
+                hipLaunchKernelGGL(score_blocks_one_kernel<2>, dim3(groups, (unsigned)s), dim3(kOneThreads), 0, st, q,
+                                   kv, w, score, s, n_comp, heads, ratio);
             return launch_status();
         }
         // two workgroups per compute unit at a time; splits of the blocks while the queries alone

@@ -48,6 +48,13 @@ def test_spread_matches_the_oracle(oracle, rows, d):
     assert bad.size == 0, [(int(i) // d, int(i) % d, got.ravel()[i], want.ravel()[i]) for i in bad[:6]]
 
 
+@pytest.mark.parametrize("rows,d", [(8192, 128), (8193, 128), (16385, 64)])
+def test_spread_across_the_change_of_rows_in_flight(oracle, rows, d):
+    """Up to 8192 rows of 128 (16 384 of 64) a wave has one row group in flight, past them four."""
+    x = spread_rows(rows, d, rows)
+    assert same_bits(device_spread(x), oracle.act_quant_f4_rotated(x)[1]).size == 0
+
+
 def sixty_binades():
     rng = np.random.default_rng(60)
     base = bf16_round(rng.standard_normal((60, 128)).astype(np.float32))
@@ -131,6 +138,18 @@ def test_score_matches_the_oracle(oracle, s, n_comp, heads, hd, spread):
     bad = same_bits(got, want)
     assert bad.size == 0, [(int(i) // n_comp, int(i) % n_comp, got.ravel()[i], want.ravel()[i]) for i in bad[:6]]
     assert np.count_nonzero(want) > 0 or n_comp * s < 4
+
+
+@pytest.mark.parametrize("n_comp", [1, 16, 17, 31, 32, 33, 65, 8192, 8193, 8225])
+@pytest.mark.parametrize("heads", [1, 15, 16, 17, 64])
+def test_one_query_at_the_edges_of_its_tiles(oracle, n_comp, heads):
+    """Workgroups of 32 blocks (64 past 8192), waves of 16 or 32 heads; where `mixed`, some blocks' rows are not spread
+    rows, so exact and folded workgroups meet in one launch."""
+    for mixed in (False, True):
+        q, kv, w = score_case(1, n_comp, heads, 128, n_comp + heads, oracle)
+        if mixed:
+            kv[40::97] *= np.float32(1.2345678)
+        assert same_bits(device_score(q, kv, w), oracle.index_score_blocks(q, kv, w)[1]).size == 0, mixed
 
 
 def test_score_known_answer(oracle):
