@@ -288,8 +288,8 @@ int rivoli_index_append_paged(const float* k, const int* slot_mapping, unsigned 
  * power-of-two block scales: 3 = two terms each (the accuracy class of 0), 4 = three terms for
  * q and two for the weights (the class of 1; inside the reference's bar on the test caches).
  * They are the fastest modes for large calls: about 30 % less time per launch than 0 / 2. Calls
- * whose 32-token tiles times groups of 16 heads number 4096 or fewer, and calls of up to 16 heads,
- * run as 2 instead, which is faster there.
+ * whose 32-token tiles times groups of 16 heads number 4096 or fewer (up to 16384 for dense calls of
+ * few sequences), and calls of up to 16 heads, run as 2 instead, which is faster there.
  * Other row widths (kvl a multiple of 128 up to 512, rope a multiple of 8 up to 64) always run
  * as 2.
  * Guards: 1001 null / non-positive, or a null `partial` when scratch is needed; 1002

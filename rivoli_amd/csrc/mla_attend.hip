@@ -137,6 +137,7 @@ struct AttendArgs {
     size_t page_bytes;
     float qscale;                 // softmax scale * log2(e)
     int n_seqs, n_items;          // n_items > 0: tiles are dealt to that many work items
+    int by_seq;                   // and no work item has tiles of two sequences (SeqDeal)
     float* clat;                  // [n_seqs][H][512]
     float* part_acc;              // [n_records][H][512]
     float* part_ml;               // [n_records][H][2]
@@ -756,6 +757,65 @@ __device__ __forceinline__ bool dealt_part(const AttendArgs& a, int item, const 
     return true;
 }
 
+// The deal of the workgroups of 16 heads: every sequence's tiles in runs of about one length, a work
+// item each, numbered through the batch, so that no work item meets two sequences. A second part costs
+// such a workgroup its query, its first rows' latency and its waves' merge again, as much as two
+// tiles a wave, and the call lasts as long as its slowest workgroup. The longest run is the shortest whole
+// number of tiles a wave with which the work items suffice. Each wave finds it for itself, a
+// sequence a lane for the lengths and then a candidate a lane, with no barrier.
+// 64 heads, parity mode, ragged, the tiles dealt evenly -> so (workgroups of 64 heads): 16 x up to
+// 2 959 tokens 50.9 -> 37.5 us (47.5), 25 x 1 422 45.8 -> 32.8 (44.4),
+// 24 x 934 52.0 -> 29.4 (50.1).
+constexpr int kSeqDealMax = 64;             // sequences: one a lane
+constexpr int kSeqDealMaxTiles = 1 << 19;   // of a sequence: the quotients below stay under 2^24
+struct SeqDeal {
+    int tiles, parts, first;  // of the lane's sequence: its tiles, its work items, the first of them
+};
+__device__ __forceinline__ int ceil_quotient(int t, int c, float inv) {
+    const int n = t + c - 1;
+    int q = (int)((float)n * inv);  // off by one at most
+    q -= q * c > n;
+    q += (q + 1) * c <= n;
+    return q;
+}
+// Needs n_items >= 2 * n_seqs. `lens` null: every sequence has k rows.
+__device__ __forceinline__ SeqDeal seq_deal(const int* lens, int k, int n_seqs, int n_items) {
+    const int lane = threadIdx.x & (kWave - 1);
+    SeqDeal d;
+    const int rows = lens ? max(min(lens[min(lane, n_seqs - 1)], k), 0) : k;
+    d.tiles = lane < n_seqs ? (rows + kTile - 1) / kTile : 0;
+    int total = d.tiles, longest = d.tiles;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        total += __shfl_xor(total, off, kWave);
+        longest = max(longest, __shfl_xor(longest, off, kWave));
+    }
+    // `rounds` tiles a wave: at least what an even deal gives, and then the first that suffices
+    const int least = max((total + kH16Waves * n_items - 1) / (kH16Waves * n_items), 1);
+    const int c = (least + lane) * kH16Waves;
+    const float c_inv = 1.0f / (float)c;
+    int items = 0;
+    for (int s = 0; s < n_seqs; ++s) items += ceil_quotient(__builtin_amdgcn_readlane(d.tiles, s), c, c_inv);
+    const unsigned long long enough = __ballot(items <= n_items);
+    int rounds;
+    if (enough) {
+        rounds = least + __builtin_ctzll(enough);
+    } else {  // sum of ceil(t / run) <= total / run + n_seqs; and a run that holds the longest is one item each
+        const int spare = kH16Waves * (n_items - n_seqs);
+        rounds = max(min((total + spare - 1) / spare, (longest + kH16Waves - 1) / kH16Waves), 1);
+    }
+    const int run = __builtin_amdgcn_readfirstlane(rounds * kH16Waves);
+    d.parts = ceil_quotient(d.tiles, run, 1.0f / (float)run);
+    int upto = d.parts;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int up = __shfl_up(upto, off, kWave);
+        if (lane >= off) upto += up;
+    }
+    d.first = upto - d.parts;
+    return d;
+}
+
 // F8: the contractions run on the 8-bit matrix instructions with QSPLIT / PSPLIT e4m3 terms for
 // q / the softmax weights (mla_attend_f8.hpp); else on the bf16 ones.
 template <int QSPLIT, int PSPLIT, int MODE, bool ANY, bool F8 = false>
@@ -808,6 +868,21 @@ __global__ __launch_bounds__(kH16Threads, 1) void mla_attend_heads16_kernel(cons
     long long t_lo, t_hi;
     int seq = item;
     if (item >= (a.n_items > 0 ? a.n_items : a.n_seqs)) return;
+    if (a.by_seq) {
+        const SeqDeal d = seq_deal(MODE == kLinear ? nullptr : (MODE == kSparse ? a.n_rows : a.seq_lens), a.k, a.n_seqs, a.n_items);
+        const unsigned long long past = __ballot(d.first + d.parts > item);
+        if (!past) return;  // more work items than runs
+        seq = __builtin_ctzll(past);
+        const int first = __builtin_amdgcn_readlane(d.first, seq), parts = __builtin_amdgcn_readlane(d.parts, seq);
+        // of a sequence's work items none is longer than the run: its tiles in `parts` even shares
+        const int tiles = __builtin_amdgcn_readlane(d.tiles, seq), part = item - first;
+        const int r_begin = (int)((unsigned)(part * tiles) / (unsigned)parts) * kTile;
+        const int r_end = min(attended_rows<MODE>(a, seq), (int)((unsigned)((part + 1) * tiles) / (unsigned)parts) * kTile);
+        const size_t rec = (size_t)item + seq;
+        attend_part_heads16<QSPLIT, PSPLIT, MODE>(a, seq, hg, r_begin, r_end, parts == 1, a.part_acc + rec * a.H * kKvl,
+                                                  a.part_ml + rec * a.H * 2);
+        return;
+    }
     if (!dealt_range<kH16Threads, MODE>(a, item, pre, wave_total, t_lo, t_hi, seq)) return;
     for (;; ++seq) {
         int r_begin = 0, r_end;
@@ -838,40 +913,49 @@ __global__ __launch_bounds__(kH16Threads, 1) void mla_attend_heads16_kernel(cons
 // whole was written by it directly; one with nothing to attend gets zeros.
 __global__ __launch_bounds__(128) void mla_attend_combine_kernel(
     const float* __restrict__ part_acc, const float* __restrict__ part_ml, const int* __restrict__ seq_lens,
-    const int* __restrict__ n_rows, int sparse, int k, int n_seqs, int n_items, int H, int kvl,
+    const int* __restrict__ n_rows, int sparse, int k, int n_seqs, int n_items, int by_seq, int H, int kvl,
     float* __restrict__ clat) {
     __shared__ long long s_sum[3][2];  // per wave: tiles before seq, tiles of seq .. end
     const int head = blockIdx.x, seq = blockIdx.y;
-    // tiles before this sequence, of this sequence, and in all
-    long long before = 0, mine = 0, total = 0;
-    for (int s = threadIdx.x; s < n_seqs; s += 128) {
-        int n = (sparse || !seq_lens) ? (n_rows ? min(n_rows[s], k) : k) : min(seq_lens[s], k);
-        n = max(n, 0);
-        const long long t = (n + kTile - 1) / kTile;
-        total += t;
-        if (s < seq) before += t;
-        if (s == seq) mine = t;
+    int first, last;       // the sequence's work items
+    long long mine = 0;    // its tiles
+    if (by_seq) {
+        const SeqDeal d = seq_deal(sparse ? n_rows : seq_lens, k, n_seqs, n_items);
+        mine = __builtin_amdgcn_readlane(d.tiles, seq);
+        first = __builtin_amdgcn_readlane(d.first, seq);
+        last = first + __builtin_amdgcn_readlane(d.parts, seq) - 1;
+    } else {
+        // tiles before this sequence, of this sequence, and in all
+        long long before = 0, total = 0;
+        for (int s = threadIdx.x; s < n_seqs; s += 128) {
+            int n = (sparse || !seq_lens) ? (n_rows ? min(n_rows[s], k) : k) : min(seq_lens[s], k);
+            n = max(n, 0);
+            const long long t = (n + kTile - 1) / kTile;
+            total += t;
+            if (s < seq) before += t;
+            if (s == seq) mine = t;
+        }
+        for (int off = 32; off > 0; off >>= 1) {
+            before += __shfl_xor(before, off, kWave);
+            mine += __shfl_xor(mine, off, kWave);
+            total += __shfl_xor(total, off, kWave);
+        }
+        if ((threadIdx.x & 63) == 0) {
+            s_sum[0][threadIdx.x >> 6] = before;
+            s_sum[1][threadIdx.x >> 6] = mine;
+            s_sum[2][threadIdx.x >> 6] = total;
+        }
+        __syncthreads();
+        before = s_sum[0][0] + s_sum[0][1], mine = s_sum[1][0] + s_sum[1][1], total = s_sum[2][0] + s_sum[2][1];
+        first = mine ? deal_item_of(before, n_items, total) : 0;
+        last = mine ? deal_item_of(before + mine - 1, n_items, total) : 0;
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        before += __shfl_xor(before, off, kWave);
-        mine += __shfl_xor(mine, off, kWave);
-        total += __shfl_xor(total, off, kWave);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        s_sum[0][threadIdx.x >> 6] = before;
-        s_sum[1][threadIdx.x >> 6] = mine;
-        s_sum[2][threadIdx.x >> 6] = total;
-    }
-    __syncthreads();
-    before = s_sum[0][0] + s_sum[0][1], mine = s_sum[1][0] + s_sum[1][1], total = s_sum[2][0] + s_sum[2][1];
     if (4 * (int)threadIdx.x >= kvl) return;  // the records are 512 wide whatever the cache's width
     float4* const dst = reinterpret_cast<float4*>(clat + ((size_t)seq * H + head) * kvl) + threadIdx.x;
     if (mine == 0) {
         *dst = float4{0, 0, 0, 0};
         return;
     }
-    const int first = deal_item_of(before, n_items, total);
-    const int last = deal_item_of(before + mine - 1, n_items, total);
     if (first == last) return;  // one work item had the whole sequence and wrote it
     // Records are fetched eight at a time, every load of a batch issued before the first use
     // (a record past the last re-reads the last and is left out): one round trip per batch
@@ -919,36 +1003,56 @@ static int attend_merge(const AttendArgs& a, const AttendPlan& plan, int n_seqs,
     if (rc != 0 || plan.n_splits <= 1) return rc;
     hipLaunchKernelGGL(mla_attend_combine_kernel, dim3((unsigned)a.H, (unsigned)n_seqs), dim3(128), 0, st,
                        a.part_acc, a.part_ml, seq_lens, n_rows, listed ? 1 : 0, max_rows, n_seqs, plan.n_items,
-                       a.H, a.kvl, a.clat);
+                       a.by_seq, a.H, a.kvl, a.clat);
     return launch_status();
 }
 
 // Whether a call goes to the workgroups of 16 heads: its 32-token tiles times its groups of 16
 // heads, before the lengths are known. Parity mode, 64 heads: 1 x 4 096 tokens (512) 21.5 us
-// against 34.5 in workgroups of 64 heads, 32 x 1 000 (4 096) 33 against 39, 6 x 9 000 (6 768) 47
-// both, 32 listed sets of 2 048 rows (8 192) 45 against 48, 32 x 4 096 (16 384) 73 against 64.
+// against 34.5 in workgroups of 64 heads, 32 x 1 000 (4 096) 33 against 39, 6 ragged of up
+// to 9 000 (6 768) 39 against 51 with the append, 32 listed sets of 2 048 rows (8 192) 45 against 48, 32 x 4 096 (16 384) 73 against 64.
 // The 8-bit modes' kernel is the faster one sooner: 8 listed sets of 2 048 rows (2 048) 24 us in
 // the parity mode here against 34 at precise 4, 32 x 1 000 (4 096) 32 against 33, 32 listed sets
 // (8 192) 44 against 42; below the line they run in the parity mode. Up to 16 heads the other
 // kernels' workgroups are three quarters empty: 32 x 16 384 tokens 84 us against 163 (precise 2)
 // and 107 (4).
 constexpr long long kH16MaxWork = 8192, kH16MaxWork8Bit = 4096;
-static bool heads16_pays(int n_seqs, int H, int max_rows, int precise) {
-    const long long tiles = (long long)n_seqs * ((max_rows + kTile - 1) / kTile);
-    return H <= kH16Heads ||
-           tiles * ((H + kH16Heads - 1) / kH16Heads) <= (precise > 2 ? kH16MaxWork8Bit : kH16MaxWork);
+// Above that line, dense calls of few enough sequences for SeqDeal to cut them well (two and a half
+// work items a sequence; at 2, 32 x 2 989 ragged tokens 57 us against 52) still go there while the
+// workgroups of 64 heads would need a second, nearly empty round: they are dealt as ceil(256 / per
+// split) splits, so 18 sequences are 270 workgroups for 256 compute units. Ragged, parity mode: 7 x
+// 11 360 tokens 38 us against 64, 17 x 10 161 (21 624) 63 against 83, 11 x 12 613 of 128 heads
+// (34 760) 178 against 174; precise 4: 13 x 7 584 (12 324) 41 against 66, 17 x 7 255 (15 436) 57
+// against 69, 18 x 10 262 (23 112) 107 against 102. Calls that those workgroups fill in one round
+// change sides sooner: 8 x 11 058 (11 072) 49 against 52, 4 x 32 768 (16 384) 74 against 71; precise
+// 4: 1 x 32 768 (4 096) 43 against 51, 4 x 32 768 70 against 59.
+constexpr long long kH16MaxWorkFull = 12288, kH16MaxWorkFull8Bit = 8192;
+constexpr long long kH16MaxWorkSpill = 24576, kH16MaxWorkSpill8Bit = 16384;
+static bool heads16_pays(const AttendPlan& plan, int n_seqs, int H, int max_rows, int precise, bool dense) {
+    const long long groups = (H + kH16Heads - 1) / kH16Heads;
+    const long long work = n_seqs * ((long long)max_rows / kTile + (max_rows % kTile != 0)) * groups;
+    const bool f8 = precise > 2;
+    if (groups == 1 || work <= (f8 ? kH16MaxWork8Bit : kH16MaxWork)) return true;
+    if (!dense || 5 * n_seqs * groups > 2 * kAttTargetGroups) return false;
+    const bool spills = (long long)plan.n_items * ((H + 63) / 64) > kAttTargetGroups;
+    return work <= (spills ? (f8 ? kH16MaxWorkSpill8Bit : kH16MaxWorkSpill) : (f8 ? kH16MaxWorkFull8Bit : kH16MaxWorkFull));
 }
-// The splits of a call by 16 heads a workgroup: one workgroup per compute unit, at least a tile per
-// wave, and no more partial records than `plan` (which the caller's scratch was sized by) has.
-static void heads16_plan(AttendPlan& plan, int n_seqs, int H, int max_rows) {
-    const long long per_split = (long long)n_seqs * ((H + kH16Heads - 1) / kH16Heads);
-    const int tiles = (max_rows + kTile - 1) / kTile;
-    long long n = kAttTargetGroups / per_split;
-    if (n > tiles / kH16Waves) n = tiles / kH16Waves;
-    if (n > plan.n_splits) n = plan.n_splits;
-    plan.n_splits = n < 1 ? 1 : (int)n;
-    plan.n_items = plan.n_splits > 1 ? plan.n_splits * n_seqs : 0;
-    plan.n_records = plan.n_items ? plan.n_items + n_seqs : 0;
+// The work items of a call by 16 heads a workgroup: one workgroup per compute unit, at least a tile
+// per wave, and no more partial records than `plan` (which the caller's scratch was sized by) has.
+// Up to 64 sequences no work item meets two of them, so their number need not be a multiple of the
+// sequences'; more sequences, or longer ones than SeqDeal counts, share the tiles evenly.
+static void heads16_plan(AttendPlan& plan, int n_seqs, int H, int max_rows, bool& by_seq) {
+    const int tiles = max_rows / kTile + (max_rows % kTile != 0);
+    const long long most = (long long)n_seqs * (tiles / kH16Waves);
+    by_seq = n_seqs <= kSeqDealMax && tiles <= kSeqDealMaxTiles;
+    long long n = kAttTargetGroups / ((H + kH16Heads - 1) / kH16Heads);
+    if (n > most) n = most;
+    if (n > plan.n_items) n = plan.n_items;
+    if (!by_seq) n = n / n_seqs * n_seqs;
+    if (n < 2 * n_seqs) n = 0, by_seq = false;
+    plan.n_items = (int)n;
+    plan.n_splits = n ? (int)((n + n_seqs - 1) / n_seqs) : 1;
+    plan.n_records = n ? plan.n_items + n_seqs : 0;
 }
 
 // What both launchers share once the arguments are in place: the attention kernel of the right
@@ -956,9 +1060,10 @@ static void heads16_plan(AttendPlan& plan, int n_seqs, int H, int max_rows) {
 template <int MODE>
 static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_rows, bool any,
                          int precise, const int* seq_lens, const int* n_rows, bool listed, hipStream_t st) {
-    if (!any && heads16_pays(n_seqs, a.H, max_rows, precise)) {
-        heads16_plan(plan, n_seqs, a.H, max_rows);
-        a.n_items = plan.n_items;
+    if (!any && heads16_pays(plan, n_seqs, a.H, max_rows, precise, MODE == kDense || MODE == kDensePaged)) {
+        bool by_seq;
+        heads16_plan(plan, n_seqs, a.H, max_rows, by_seq);
+        a.n_items = plan.n_items, a.by_seq = by_seq;
         const int items = plan.n_items ? plan.n_items : n_seqs;
         const dim3 grid((unsigned)(((items + 7) / 8 * 8) * (long long)((a.H + kH16Heads - 1) / kH16Heads)));
         (void)hipGetLastError();

@@ -430,3 +430,23 @@ def test_both_sides_of_the_line_between_workgroups_of_16_and_of_64_heads(oracle,
     want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], rows, n_rows,
                                    KVL, ROPE, PT, c["scale"], n_threads=8)
     check(run_paged(c, k, rows=rows, n_rows=n_rows, precise=precise), want, precise, "listed", mild=precise in (2, 4))
+
+
+@pytest.mark.parametrize("lens,H", [([2100, 31, 0, 33, 1], 64), ([257, 2049, 0, 0, 128, 1930], 33), ([0, 4000], 64),
+                                    ([640, 1, 129, 511] * 16, 16), ([640, 1, 129, 511] * 16 + [300], 16),
+                                    ([1850, 40, 0, 900, 385, 384] * 3, 64), ([0, 0, 5], 64)])
+def test_sequences_cut_into_work_items_of_their_own(oracle, lens, H):
+    """One long sequence among short and empty ones, 64 sequences (a lane each) and 65 (the even
+    deal), and 18 sequences that a call at precise 4 sends here past the line of its own kernel;
+    dense, and listed with as many rows."""
+    c = paged_case(oracle, lens, H=H, seed=950 + len(lens), outlier_frac=0.0)
+    k = max(max(lens), 512)
+    args = (c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"])
+    want = oracle.mla_attend_paged(*args, None, None, KVL, ROPE, PT, c["scale"], n_threads=8)
+    for precise in (2, 4):
+        check(run_paged(c, k, precise=precise), want, precise, "dense", mild=True)
+    rows = np.zeros((len(lens), k), np.uint32)
+    for s, n in enumerate(lens):
+        rows[s, :n] = np.arange(n)[::-1]
+    got = run_paged(c, k, rows=rows, n_rows=np.asarray(lens, np.int32))
+    check(got, want, 2, "listed", mild=True)
