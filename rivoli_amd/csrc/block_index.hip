@@ -321,8 +321,9 @@ typedef f32x4 f32x4_u __attribute__((aligned(4)));  // q rows need no more than 
 // 128 products of two rows is then a multiple of u = 2^(lo_q + lo_kv - 2) below 288 * 2^(hi_q +
 // hi_kv), that is below 2^(10.2 + (hi_q - lo_q) + (hi_kv - lo_kv)) u: with (hi_q - lo_q) + (hi_kv -
 // lo_kv) <= 13 every partial sum is a whole number of u below 2^24 and every f32 addition is
-// exact. Exponents within +-60 keep u and the sums normal. A spread row spans 3 binades plus what
-// its four block scales differ by; 13 leaves 7 for those.
+// exact. Exponents within +-59 keep u a normal number and every sum below 288 * 2^118 < 2^127 (at
+// 60 a fold may pass the largest float where another order does not). A spread row spans 3
+// binades plus what its four block scales differ by; 13 leaves 7 for those.
 constexpr int kExactSpan = 13;
 constexpr int kNoSpan = 99;  // not such a row: no partner makes it exact
 // The census of a row, two bf16 patterns per dword: largest magnitude in the low 16 bits' field,
@@ -349,7 +350,7 @@ __device__ __forceinline__ uint32_t span_max(uint32_t a, uint32_t b) {
 __device__ __forceinline__ int span_of(uint32_t folded) {
     const int hi = (int)((folded & 0xffffu) >> 7), lo = (int)((0x10000u - (folded >> 16)) >> 7);
     if (!(folded & 0xffffu)) return 0;  // a row of zeros
-    return hi > 127 + 60 || lo < 127 - 60 ? kNoSpan : hi - lo;
+    return hi > 127 + 59 || lo < 127 - 59 ? kNoSpan : hi - lo;
 }
 // Two f32 bit patterns to a dword of two bf16 patterns by truncation (exact when the census finds
 // no low bits).

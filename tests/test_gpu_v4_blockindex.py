@@ -283,3 +283,19 @@ def test_score_of_rows_whose_sums_are_exact_up_to_the_last_span_and_past_it(orac
         part = back(out, np.float32).reshape(s, n_comp).view(np.uint32)
         live = (np.arange(n_comp)[None, :] // 64) * 64 < np.minimum(np.arange(s) + 1, n_comp)[:, None]
         assert np.array_equal(part[live], want.view(np.uint32)[live]) and (part[~live] == 0x5A5A5A5A).all(), change
+
+
+@pytest.mark.parametrize("s,n_comp", [(1, 70), (9, 3100)])
+@pytest.mark.parametrize("exponent", [59, 60, -59, -60])
+def test_score_at_the_largest_and_smallest_exponents_whose_sums_are_exact(oracle, s, n_comp, exponent):
+    """112 products of 2.25 * 2^120, two more and then fourteen of the other sign: a fold passes the
+    largest float at the 114th and stays infinite, a sum in another order never reaches it. Rows of
+    exponent 60 have to be folded; at 59 (and at -59, below which products leave the normal
+    numbers' exact range) every order agrees."""
+    q = np.full((s, 16, 128), 1.5 * 2.0 ** exponent, np.float32)
+    kv = q[0, :1].repeat(n_comp, 0)
+    q[:, :, 114:] *= np.float32(-1.0)
+    w = np.full((s, 16), 0.25, np.float32)
+    code, want = oracle.index_score_blocks(q, kv, w)
+    assert code == 0 and np.isinf(want).all() == (exponent == 60)
+    assert same_bits(device_score(q, kv, w), want).size == 0
