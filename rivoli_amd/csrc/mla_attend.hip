@@ -1242,8 +1242,8 @@ extern "C" int rivoli_mla_attend(const float* qabs, const float* qrope, const un
     a.clat = clat;
     a.part_acc = plan.n_items ? partial : nullptr;
     a.part_ml = plan.n_items ? partial + (size_t)plan.n_records * H * kKvl : nullptr;
-    // any row width but the shipped one (whole 16-byte pieces) takes the general form
-    const bool any = kvl != kKvl || rope != kRopeW || n_blocks != kKvl / 128 || !aligned16(Rc) || !aligned16(Lscale) ||
-                     !aligned16(qabs) || !aligned16(qrope);
+    // any row width but the shipped one, and slabs that are not whole 16-byte pieces, take the general form
+    const bool any = kvl != kKvl || rope != kRopeW || n_blocks != kKvl / 128 || !aligned16(Lc8) || !aligned16(Rc) ||
+                     !aligned16(Lscale) || !aligned16(qabs) || !aligned16(qrope);
     return attend_launch<kLinear>(a, plan, 1, nr, any, 2, nullptr, nullptr, rows != nullptr, nullptr);
 }

@@ -323,12 +323,13 @@ def test_guards():
 
 # ---- the reference's single-token launcher over its linear slabs --------------------------
 
-def run_linear(case, h, nt, kvl, rope, rows=None, scratch=True, launch=None):
+def run_linear(case, h, nt, kvl, rope, rows=None, scratch=True, launch=None, lc8_offset=0):
     qabs, qrope, lc8, lscale, rc, nb, scale = case
     nr = nt if rows is None else rows.size
     clat = dzeros(h * kvl * 4, 0xFF)
     part = dzeros(hip.attend_scratch_floats(h, kvl) * 4, 0xFF) if scratch else None
-    args = (dev(qabs), dev(qrope), dev(lc8), dev(lscale), dev(rc), None if rows is None else dev(rows))
+    codes = dev(np.concatenate([np.zeros(lc8_offset, np.uint8), lc8]))[lc8_offset:]
+    args = (dev(qabs), dev(qrope), codes, dev(lscale), dev(rc), None if rows is None else dev(rows))
     if launch is None:
         hip.launch_attend(*args, h, nr, kvl, rope, nb, scale, clat, part)
     else:
@@ -450,3 +451,21 @@ def test_sequences_cut_into_work_items_of_their_own(oracle, lens, H):
         rows[s, :n] = np.arange(n)[::-1]
     got = run_paged(c, k, rows=rows, n_rows=np.asarray(lens, np.int32))
     check(got, want, 2, "listed", mild=True)
+
+
+@pytest.mark.parametrize("lc8_offset", [0, 8])
+@pytest.mark.parametrize("h,nt,nr", [(64, 3000, 2048), (20, 900, 333), (64, 700, 31), (5, 2500, 2500)])
+def test_linear_row_lists_and_code_slabs_on_an_8_byte_boundary(oracle, h, nt, nr, lc8_offset):
+    """Rows of 512 + 64 through an unsorted list and without one, several splits, one (null scratch)
+    and less than a tile. A code slab need be no more than 8-byte aligned: the kernel whose
+    transfers are of 16 bytes must leave such a one to the general form."""
+    from tests.attend_cases import reference_attend_case
+
+    case = reference_attend_case(oracle, 0x51E0 + h, h, nt, KVL, ROPE)
+    rows = np.random.default_rng(nr).permutation(nt)[:nr].astype(np.uint32)
+    for r in (rows, None):
+        code, want = oracle.mla_attend(*case[:5], r, h, nr, KVL, ROPE, case[5], case[6])
+        assert code == 0
+        for scratch in (True, False):
+            got = run_linear(case, h, nr if r is None else nt, KVL, ROPE, rows=r, scratch=scratch, lc8_offset=lc8_offset)
+            check_linear(got, want, f"rows={r is not None} scratch={scratch}")
