@@ -1060,7 +1060,8 @@ static void heads16_plan(AttendPlan& plan, int n_seqs, int H, int max_rows, bool
 template <int MODE>
 static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_rows, bool any,
                          int precise, const int* seq_lens, const int* n_rows, bool listed, hipStream_t st) {
-    if (!any && heads16_pays(plan, n_seqs, a.H, max_rows, precise, MODE == kDense || MODE == kDensePaged)) {
+    // (its 16-byte transfers want every page to start on 16 bytes: page_tokens a multiple of 4)
+    if (!any && a.page_bytes % 16 == 0 && heads16_pays(plan, n_seqs, a.H, max_rows, precise, MODE == kDense || MODE == kDensePaged)) {
         bool by_seq;
         heads16_plan(plan, n_seqs, a.H, max_rows, by_seq);
         a.n_items = plan.n_items, a.by_seq = by_seq;

@@ -170,6 +170,27 @@ def test_other_page_sizes(oracle, pt, precise):
           f"rows, pages of {pt}")
 
 
+@pytest.mark.parametrize("precise", [2, 1, 0])
+@pytest.mark.parametrize("pt", [6, 7, 2, 1])
+def test_pages_that_do_not_start_on_16_bytes(oracle, pt, precise):
+    """A page of 580 * page_tokens bytes puts the next one's rows on 4 or 8 bytes: such a call must
+    keep off the kernel whose transfers are of 16 bytes. Dense and listed. Rows without outliers: a
+    wrong address shows whatever the rows hold, and with q rounded once (0) a row 30 times as long
+    moves its score by 720 * 2^-9 / 24, a standard deviation of 0.06, which is no matter of pages."""
+    lens = [130, 33, 1]
+    c = paged_case(oracle, lens, H=64, seed=740 + pt, page_tokens=pt, outlier_frac=0.0)
+    want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], None, None,
+                                   KVL, ROPE, pt, c["scale"], n_threads=3)
+    check(run_paged(c, max(lens), pt=pt, precise=precise), want, precise, f"dense, pages of {pt}")
+    k = 100
+    rows = np.stack([np.random.default_rng(pt).choice(n, k, replace=n < k) for n in lens]).astype(np.uint32)
+    n_rows = np.array([100, 20, 33], np.int32)
+    want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], None, rows, n_rows,
+                                   KVL, ROPE, pt, c["scale"], n_threads=3)
+    check(run_paged(c, k, rows=rows, n_rows=n_rows, use_lens=False, pt=pt, precise=precise), want, precise,
+          f"rows, pages of {pt}")
+
+
 @pytest.mark.parametrize("kvl,rope", [(256, 64), (384, 32), (128, 8), (512, 24)])
 def test_other_row_widths(oracle, kvl, rope):
     """Latent widths the reference's launcher accepts (multiples of 128 up to 512,
