@@ -57,9 +57,9 @@ int rivoli_hash_rows(const float* x, int n, int stride, unsigned long long i_bas
  * launch_attend, crates/backend/src/hip_attn.rs:113-128): MLA decode attention for one token
  * over the LINEAR slabs — clat[h] = sum_t softmax_t((qabs_h . L_t + qrope_h . R_t) * scale) *
  * L_t with L_t the e4m3 latent times its per-128 f32 scales, R_t the bf16 roped key, token =
- * rows ? rows[j] : j for j < nr. `partial` is scratch of rivoli_mla_attend_scratch_floats(H,
- * kvl) floats, or null for a single split. Null stream. Guards as the reference: 1001
- * non-positive dim; 1002 (kvl + rope) > 1024; 1004 kvl > 512 or kvl % 128. */
+ * rows ? rows[j] : j for j < nr (an entry of 0xffffffff is left out). `partial` is scratch of
+ * rivoli_mla_attend_scratch_floats(H, kvl) floats, or null for a single split. Null stream. Guards
+ * as the reference: 1001 non-positive dim; 1002 (kvl + rope) > 1024; 1004 kvl > 512 or kvl % 128. */
 size_t rivoli_mla_attend_scratch_floats(int H, int kvl);
 int rivoli_mla_attend(const float* qabs, const float* qrope, const unsigned char* Lc8,
                       const float* Lscale, const unsigned short* Rc, const unsigned int* rows, int H,
@@ -271,7 +271,8 @@ int rivoli_index_append_paged(const float* k, const int* slot_mapping, unsigned 
  * null (dense); otherwise rows[s*max_rows + j] for j < n_rows[s] (max_rows when n_rows is
  * null) — the DSA selection, as rivoli_index_topk_batched emits it with k = max_rows.
  * Tokens whose page id is outside [0, n_pages) are left out of the softmax and counted in
- * *bad_rows when non-null. A sequence with nothing to attend gets zeros.
+ * *bad_rows when non-null; a list entry of 0xffffffff is left out too and counted by `precise` 3
+ * and 4 alone. A sequence with nothing to attend gets zeros.
  * `partial` is caller-owned scratch of rivoli_mla_attend_paged_scratch_floats(n_seqs, H,
  * max_rows) floats (the split-KV partials; may be null when that returns 0). When scratch is
  * used, the 32-token tiles of the whole batch are dealt evenly to the workgroups from the

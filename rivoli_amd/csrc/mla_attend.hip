@@ -138,6 +138,7 @@ struct AttendArgs {
     float qscale;                 // softmax scale * log2(e)
     int n_seqs, n_items;          // n_items > 0: tiles are dealt to that many work items
     int by_seq;                   // and no work item has tiles of two sequences (SeqDeal)
+    int count_ones;               // list entries of 0xffffffff count among bad_rows
     float* clat;                  // [n_seqs][H][512]
     float* part_acc;              // [n_records][H][512]
     float* part_ml;               // [n_records][H][2]
@@ -1064,7 +1065,7 @@ static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_row
     if (!any && a.page_bytes % 16 == 0 && heads16_pays(plan, n_seqs, a.H, max_rows, precise, MODE == kDense || MODE == kDensePaged)) {
         bool by_seq;
         heads16_plan(plan, n_seqs, a.H, max_rows, by_seq);
-        a.n_items = plan.n_items, a.by_seq = by_seq;
+        a.n_items = plan.n_items, a.by_seq = by_seq, a.count_ones = precise > 2;
         const int items = plan.n_items ? plan.n_items : n_seqs;
         const dim3 grid((unsigned)(((items + 7) / 8 * 8) * (long long)((a.H + kH16Heads - 1) / kH16Heads)));
         (void)hipGetLastError();
@@ -1177,6 +1178,7 @@ __global__ __launch_bounds__(256) void mla_attend_rowwise_kernel(
     float m = -INFINITY, l = 0.0f;
     for (int j = 0; j < nr; ++j) {
         const size_t t = rows ? rows[j] : (unsigned)j;
+        if (t == 0xffffffffu) continue;  // nobody's token, as in the tile kernels
         float lat[8], dot = 0.0f;
 #pragma unroll
         for (int c = 0; c < 8; ++c) {

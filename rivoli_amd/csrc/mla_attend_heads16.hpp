@@ -96,6 +96,8 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
     auto resolve = [&](int tile, unsigned int tok, int page) -> Where {
         Where w = {kNone, 0};
         if (lane >= kTile || tile >= n_tiles || r_begin + tile * kTile + lane >= r_end) return w;
+        // a list entry of all ones is nobody's token, and only the 8-bit modes count it (as attend_part)
+        if (MODE != kDense && tok == 0xffffffffu && (LINEAR || !a.count_ones)) return w;
         if (LINEAR) {
             w.code = (unsigned long long)tok * kKvl, w.scale = tok;
             return w;

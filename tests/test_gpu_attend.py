@@ -175,8 +175,8 @@ def test_other_page_sizes(oracle, pt, precise):
 def test_pages_that_do_not_start_on_16_bytes(oracle, pt, precise):
     """A page of 580 * page_tokens bytes puts the next one's rows on 4 or 8 bytes: such a call must
     keep off the kernel whose transfers are of 16 bytes. Dense and listed. Rows without outliers: a
-    wrong address shows whatever the rows hold, and with q rounded once (0) a row 30 times as long
-    moves its score by 720 * 2^-9 / 24, a standard deviation of 0.06, which is no matter of pages."""
+    wrong address shows whatever the rows hold, and with q rounded once (0) the score of a row 30
+    times as long is off by 30 * 2^-9 / sqrt(3) = 0.03 at one deviation, which is no matter of pages."""
     lens = [130, 33, 1]
     c = paged_case(oracle, lens, H=64, seed=740 + pt, page_tokens=pt, outlier_frac=0.0)
     want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], None, None,
@@ -490,3 +490,47 @@ def test_linear_row_lists_and_code_slabs_on_an_8_byte_boundary(oracle, h, nt, nr
         for scratch in (True, False):
             got = run_linear(case, h, nr if r is None else nt, KVL, ROPE, rows=r, scratch=scratch, lc8_offset=lc8_offset)
             check_linear(got, want, f"rows={r is not None} scratch={scratch}")
+
+
+@pytest.mark.parametrize("n_seqs,H", [(3, 64), (24, 128)])
+@pytest.mark.parametrize("precise", [2, 1, 0, 4, 3])
+def test_list_entries_of_all_ones_are_left_out(oracle, precise, n_seqs, H):
+    """0xffffffff in a row list is nobody's token: it takes no part, whichever kernel the call takes
+    (24 lists of 2 200 at 128 heads go to those of 64 heads a workgroup); the 8-bit modes count it
+    like any other token past the table, the others do not."""
+    k = 2200 if n_seqs > 3 else 200
+    assert (n_seqs * -(-k // 32) * (H // 16) > 8192) == (n_seqs > 3)
+    c = paged_case(oracle, [600] * n_seqs, H=H, seed=630, outlier_frac=0.0)
+    rng = np.random.default_rng(63)
+    rows = np.full((n_seqs, k), 0xFFFFFFFF, np.uint32)
+    n_rows = np.zeros(n_seqs, np.int32)
+    kept = np.zeros((n_seqs, k), np.uint32)
+    for s in range(n_seqs):
+        n = (130, 33, 200)[s % 3]
+        kept[s, :n] = rng.choice(600, n, replace=False)
+        at = np.sort(rng.choice(min(k, 2 * n), n, replace=False))
+        rows[s, at] = kept[s, :n]
+        n_rows[s] = n
+    want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], None, kept, n_rows,
+                                   KVL, ROPE, PT, c["scale"], n_threads=8)
+    bad = dzeros(4)
+    got = run_paged(c, k, rows=rows, use_lens=False, precise=precise, bad=bad)
+    # weights rounded once (0, 1) or to 8 bits (3): 2^-9 of what a row differs from the result by, that
+    # is of 6 + |result| for N(0,1) rows, and as much again for the scores
+    bar = {2: 1e-4, 4: 2e-3}.get(precise, 2.0 ** -8) * (np.abs(want).max() + (0.0 if precise in (2, 4) else 6.0))
+    assert np.abs(got.astype(np.float64) - want).max() <= bar, "entries of all ones"
+    assert back(bad, np.uint32)[0] == (int((rows == 0xFFFFFFFF).sum()) if precise > 2 else 0)
+
+
+def test_linear_list_entries_of_all_ones_are_left_out(oracle):
+    """The same over the linear slabs, where such an entry is an address 2 TB past the slab."""
+    from tests.attend_cases import reference_attend_case
+
+    for h, kvl, rope in ((64, KVL, ROPE), (20, 384, 24), (3, 256, 200)):
+        case = reference_attend_case(oracle, 0x51F0 + h, h, 500, kvl, rope)
+        kept = np.random.default_rng(h).permutation(500)[:300].astype(np.uint32)
+        rows = np.insert(kept, [0, 0, 31, 64, 150, 150, 150, 300], 0xFFFFFFFF).astype(np.uint32)
+        code, want = oracle.mla_attend(*case[:5], kept, h, kept.size, kvl, rope, case[5], case[6])
+        assert code == 0
+        for scratch in (True, False):
+            check_linear(run_linear(case, h, 500, kvl, rope, rows=rows, scratch=scratch), want, f"h={h} scratch={scratch}")
