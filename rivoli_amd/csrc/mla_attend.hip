@@ -50,13 +50,13 @@
 #include <type_traits>
 
 #include "attend_common.hpp"
+#include "mla_attend_plan.hpp"
 
 namespace rk {
 
 constexpr int kKvl = 512, kRopeW = 64, kRowW = kKvl + kRopeW;
 constexpr int kAttThreads = 512;
 constexpr int kAttWaves = kAttThreads / kWave;
-constexpr int kTile = 32;                  // tokens per LDS tile
 constexpr int kKSteps = kRowW / 32;        // 18 K-steps of the score contraction ...
 constexpr int kKStepsHalf = kKSteps / 2;   // ... 9 per wave of a pair
 constexpr int kColTilesHalf = kKvl / 16 / 2;  // 16 output column tiles per wave of a pair
@@ -69,37 +69,6 @@ constexpr int kBlockScaleBytes = kBufs * kTile * 16;  // linear slabs: four bloc
 constexpr int kAttSmemBytes =
     kBufs * kKrBytes + 2 * kBufs * kTile * 4 + kXchBytes + kTableLds * 4 + kBlockScaleBytes;
 static_assert(kAttSmemBytes + (1024 + 8 + 8) * 4 <= 160 * 1024, "one workgroup per CU must fit the 160 KiB of LDS");
-
-// Work plan. `n_splits` is a pure function of the call's shape; with more than one split the
-// attended rows of ALL sequences, in tiles, are dealt evenly to n_seqs * n_splits work items
-// from the device-side lengths (a work item may cover parts of several sequences, a sequence
-// several work items), so ragged batches keep every CU busy.
-constexpr int kAttTargetGroups = 256;      // one workgroup per CU of a 256-CU part
-constexpr int kAttMinTilesPerSplit = 8;    // below 256 rows a split costs more than it buys
-constexpr int kAttMaxSplits = 64;
-constexpr int kDealMaxSeqs = 1024;         // dealing keeps a prefix sum over the sequences in LDS
-
-struct AttendPlan {
-    int n_splits;
-    int n_items;    // work items per head block when dealing (0 = one workgroup per sequence)
-    int n_records;  // partial records when dealing: a (work item, sequence) pair is item + seq
-};
-
-static inline AttendPlan attend_plan(int n_seqs, int H, int max_rows) {
-    const int head_blocks = (H + 63) / 64;
-    const int tiles = (max_rows + kTile - 1) / kTile;
-    const long long per_split = (long long)n_seqs * head_blocks;
-    int by_grid = (int)((kAttTargetGroups + per_split - 1) / per_split);
-    int by_work = tiles / kAttMinTilesPerSplit;
-    int n = by_grid < by_work ? by_grid : by_work;
-    if (n > kAttMaxSplits) n = kAttMaxSplits;
-    if (n < 1 || n_seqs > kDealMaxSeqs) n = 1;
-    AttendPlan p;
-    p.n_splits = n;
-    p.n_items = n > 1 ? n * n_seqs : 0;
-    p.n_records = n > 1 ? p.n_items + n_seqs : 0;
-    return p;
-}
 
 // The tiles of work item `item` of `n_items` over `total` tiles: [lo, hi).
 __host__ __device__ __forceinline__ long long deal_lo(long long item, long long n_items, long long total) {
@@ -767,8 +736,6 @@ __device__ __forceinline__ bool dealt_part(const AttendArgs& a, int item, const 
 // 64 heads, parity mode, ragged, the tiles dealt evenly -> so (workgroups of 64 heads): 16 x up to
 // 2 959 tokens 50.9 -> 37.5 us (47.5), 25 x 1 422 45.8 -> 32.8 (44.4),
 // 24 x 934 52.0 -> 29.4 (50.1).
-constexpr int kSeqDealMax = 64;             // sequences: one a lane
-constexpr int kSeqDealMaxTiles = 1 << 19;   // of a sequence: the quotients below stay under 2^24
 struct SeqDeal {
     int tiles, parts, first;  // of the lane's sequence: its tiles, its work items, the first of them
 };
@@ -1008,64 +975,17 @@ static int attend_merge(const AttendArgs& a, const AttendPlan& plan, int n_seqs,
     return launch_status();
 }
 
-// Whether a call goes to the workgroups of 16 heads: its 32-token tiles times its groups of 16
-// heads, before the lengths are known. Parity mode, 64 heads: 1 x 4 096 tokens (512) 21.5 us
-// against 34.5 in workgroups of 64 heads, 32 x 1 000 (4 096) 33 against 39, 6 ragged of up
-// to 9 000 (6 768) 39 against 51 with the append, 32 listed sets of 2 048 rows (8 192) 45 against 48, 32 x 4 096 (16 384) 73 against 64.
-// The 8-bit modes' kernel is the faster one sooner: 8 listed sets of 2 048 rows (2 048) 24 us in
-// the parity mode here against 34 at precise 4, 32 x 1 000 (4 096) 32 against 33, 32 listed sets
-// (8 192) 44 against 42; below the line they run in the parity mode. Up to 16 heads the other
-// kernels' workgroups are three quarters empty: 32 x 16 384 tokens 84 us against 163 (precise 2)
-// and 107 (4).
-constexpr long long kH16MaxWork = 8192, kH16MaxWork8Bit = 4096;
-// Above that line, dense calls of few enough sequences for SeqDeal to cut them well (two and a half
-// work items a sequence; at 2, 32 x 2 989 ragged tokens 57 us against 52) still go there while the
-// workgroups of 64 heads would need a second, nearly empty round: they are dealt as ceil(256 / per
-// split) splits, so 18 sequences are 270 workgroups for 256 compute units. Ragged, parity mode: 7 x
-// 11 360 tokens 38 us against 64, 17 x 10 161 (21 624) 63 against 83, 11 x 12 613 of 128 heads
-// (34 760) 178 against 174; precise 4: 13 x 7 584 (12 324) 41 against 66, 17 x 7 255 (15 436) 57
-// against 69, 18 x 10 262 (23 112) 107 against 102. Calls that those workgroups fill in one round
-// change sides sooner: 8 x 11 058 (11 072) 49 against 52, 4 x 32 768 (16 384) 74 against 71; precise
-// 4: 1 x 32 768 (4 096) 43 against 51, 4 x 32 768 70 against 59.
-constexpr long long kH16MaxWorkFull = 12288, kH16MaxWorkFull8Bit = 8192;
-constexpr long long kH16MaxWorkSpill = 24576, kH16MaxWorkSpill8Bit = 16384;
-static bool heads16_pays(const AttendPlan& plan, int n_seqs, int H, int max_rows, int precise, bool dense) {
-    const long long groups = (H + kH16Heads - 1) / kH16Heads;
-    const long long work = n_seqs * ((long long)max_rows / kTile + (max_rows % kTile != 0)) * groups;
-    const bool f8 = precise > 2;
-    if (groups == 1 || work <= (f8 ? kH16MaxWork8Bit : kH16MaxWork)) return true;
-    if (!dense || 5 * n_seqs * groups > 2 * kAttTargetGroups) return false;
-    const bool spills = (long long)plan.n_items * ((H + 63) / 64) > kAttTargetGroups;
-    return work <= (spills ? (f8 ? kH16MaxWorkSpill8Bit : kH16MaxWorkSpill) : (f8 ? kH16MaxWorkFull8Bit : kH16MaxWorkFull));
-}
-// The work items of a call by 16 heads a workgroup: one workgroup per compute unit, at least a tile
-// per wave, and no more partial records than `plan` (which the caller's scratch was sized by) has.
-// Up to 64 sequences no work item meets two of them, so their number need not be a multiple of the
-// sequences'; more sequences, or longer ones than SeqDeal counts, share the tiles evenly.
-static void heads16_plan(AttendPlan& plan, int n_seqs, int H, int max_rows, bool& by_seq) {
-    const int tiles = max_rows / kTile + (max_rows % kTile != 0);
-    const long long most = (long long)n_seqs * (tiles / kH16Waves);
-    by_seq = n_seqs <= kSeqDealMax && tiles <= kSeqDealMaxTiles;
-    long long n = kAttTargetGroups / ((H + kH16Heads - 1) / kH16Heads);
-    if (n > most) n = most;
-    if (n > plan.n_items) n = plan.n_items;
-    if (!by_seq) n = n / n_seqs * n_seqs;
-    if (n < 2 * n_seqs) n = 0, by_seq = false;
-    plan.n_items = (int)n;
-    plan.n_splits = n ? (int)((n + n_seqs - 1) / n_seqs) : 1;
-    plan.n_records = n ? plan.n_items + n_seqs : 0;
-}
-
 // What both launchers share once the arguments are in place: the attention kernel of the right
 // mode, then the merge of the partial records when the plan has any.
 template <int MODE>
 static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_rows, bool any,
                          int precise, const int* seq_lens, const int* n_rows, bool listed, hipStream_t st) {
-    // (its 16-byte transfers want every page to start on 16 bytes: page_tokens a multiple of 4)
-    if (!any && a.page_bytes % 16 == 0 && heads16_pays(plan, n_seqs, a.H, max_rows, precise, MODE == kDense || MODE == kDensePaged)) {
-        bool by_seq;
-        heads16_plan(plan, n_seqs, a.H, max_rows, by_seq);
-        a.n_items = plan.n_items, a.by_seq = by_seq, a.count_ones = precise > 2;
+    // (16-byte transfers want every page to start on 16 bytes: page_tokens a multiple of 4)
+    const AttendRoute route = attend_route(plan, n_seqs, a.H, max_rows, precise, MODE == kDense || MODE == kDensePaged,
+                                           MODE == kLinear);
+    if (!any && a.page_bytes % 16 == 0 && route.heads16) {
+        plan = route.plan;
+        a.n_items = plan.n_items, a.by_seq = route.by_seq, a.count_ones = precise > 2;
         const int items = plan.n_items ? plan.n_items : n_seqs;
         const dim3 grid((unsigned)(((items + 7) / 8 * 8) * (long long)((a.H + kH16Heads - 1) / kH16Heads)));
         (void)hipGetLastError();

@@ -25,9 +25,7 @@
 
 namespace rk {
 
-constexpr int kH16Threads = 256;
-constexpr int kH16Waves = kH16Threads / kWave;
-constexpr int kH16Heads = 16;
+constexpr int kH16Threads = kH16Waves * kWave;
 constexpr int kH16ColTiles = kKvl / 16;
 constexpr int kH16Chunks = kKSteps / 2;  // 16-byte pieces of a row per lane group: two K-steps each
 

@@ -1,0 +1,145 @@
+// Which kernel an MLA attention call takes and how its 32-token tiles become work items: host
+// arithmetic on the call's shape alone (no length is known there), shared by the launchers of
+// mla_attend.hip and the tests that hold the rules.
+#pragma once
+
+namespace rk {
+
+constexpr int kTile = 32;                  // tokens per tile
+constexpr int kAttTargetGroups = 256;      // one workgroup per CU of a 256-CU part
+constexpr int kAttDies = 8;                // workgroups are dealt to the dies in turn
+constexpr int kAttMinTilesPerSplit = 8;    // below 256 rows a split costs more than it buys
+constexpr int kAttMaxSplits = 64;
+constexpr int kDealMaxSeqs = 1024;         // dealing keeps a prefix sum over the sequences in LDS
+constexpr int kH16Heads = 16;              // mla_attend_heads16.hpp: heads and waves of a workgroup
+constexpr int kH16Waves = 4;
+constexpr int kSeqDealMax = 64;            // SeqDeal: sequences, one a lane
+constexpr int kSeqDealMaxTiles = 1 << 19;  // of a sequence: its quotients stay under 2^24
+
+// Work plan of the workgroups of 64 heads. `n_splits` is a pure function of the call's shape; with
+// more than one split the attended rows of ALL sequences, in tiles, are dealt evenly to n_seqs *
+// n_splits work items from the device-side lengths (a work item may cover parts of several
+// sequences, a sequence several work items), so ragged batches keep every CU busy.
+struct AttendPlan {
+    int n_splits;
+    int n_items;    // work items per head block when dealing (0 = one workgroup per sequence)
+    int n_records;  // partial records when dealing: a (work item, sequence) pair is item + seq
+};
+
+static inline AttendPlan attend_plan(int n_seqs, int H, int max_rows) {
+    const int head_blocks = (H + 63) / 64;
+    const int tiles = (max_rows + kTile - 1) / kTile;
+    const long long per_split = (long long)n_seqs * head_blocks;
+    int by_grid = (int)((kAttTargetGroups + per_split - 1) / per_split);
+    int by_work = tiles / kAttMinTilesPerSplit;
+    int n = by_grid < by_work ? by_grid : by_work;
+    if (n > kAttMaxSplits) n = kAttMaxSplits;
+    if (n < 1 || n_seqs > kDealMaxSeqs) n = 1;
+    AttendPlan p;
+    p.n_splits = n;
+    p.n_items = n > 1 ? n * n_seqs : 0;
+    p.n_records = n > 1 ? p.n_items + n_seqs : 0;
+    return p;
+}
+
+// The work items of a call by 16 heads a workgroup: one workgroup per compute unit, at least a tile
+// per wave, and no more partial records than `plan` (which the caller's scratch was sized by) has.
+// Up to 64 sequences no work item meets two of them, so their number need not be a multiple of the
+// sequences'; more sequences, or longer ones than SeqDeal counts, share the tiles evenly.
+static inline AttendPlan heads16_plan(const AttendPlan& plan, int n_seqs, int H, int max_rows, bool& by_seq) {
+    const int tiles = max_rows / kTile + (max_rows % kTile != 0);
+    const long long most = (long long)n_seqs * (tiles / kH16Waves);
+    by_seq = n_seqs <= kSeqDealMax && tiles <= kSeqDealMaxTiles;
+    long long n = kAttTargetGroups / ((H + kH16Heads - 1) / kH16Heads);
+    if (n > most) n = most;
+    if (n > plan.n_items) n = plan.n_items;
+    if (!by_seq) n = n / n_seqs * n_seqs;
+    if (n < 2 * n_seqs) n = 0, by_seq = false;
+    AttendPlan p;
+    p.n_items = (int)n;
+    p.n_splits = n ? (int)((n + n_seqs - 1) / n_seqs) : 1;
+    p.n_records = n ? p.n_items + n_seqs : 0;
+    return p;
+}
+
+// Rounds of workgroups a die's 32 compute units take for `items` work items: the head groups of an
+// item sit on one die (mla_attend_heads16_kernel).
+static inline long long heads16_rounds(long long items, long long groups) {
+    const long long per_die = (items + kAttDies - 1) / kAttDies * groups, units = kAttTargetGroups / kAttDies;
+    return (per_die + units - 1) / units;
+}
+
+// Whether a call goes to the workgroups of 16 heads: its 32-token tiles times its groups of 16
+// heads, before the lengths are known. Parity mode, 64 heads: 1 x 4 096 tokens (512) 21.5 us
+// against 34.5 in workgroups of 64 heads, 32 x 1 000 (4 096) 33 against 39, 6 ragged of up
+// to 9 000 (6 768) 39 against 51 with the append, 32 listed sets of 2 048 rows (8 192) 45 against 48, 32 x 4 096 (16 384) 73 against 64.
+// The 8-bit modes' kernel is the faster one sooner: 8 listed sets of 2 048 rows (2 048) 24 us in
+// the parity mode here against 34 at precise 4, 32 x 1 000 (4 096) 32 against 33, 32 listed sets
+// (8 192) 44 against 42; below the line they run in the parity mode. Up to 16 heads the other
+// kernels' workgroups are three quarters empty: 32 x 16 384 tokens 84 us against 163 (precise 2)
+// and 107 (4).
+constexpr long long kH16MaxWork = 8192, kH16MaxWork8Bit = 4096;
+// Above that line, dense calls of few enough sequences for SeqDeal to cut them well (two and a half
+// work items a sequence; at 2, 32 x 2 989 ragged tokens 57 us against 52) still go there while the
+// workgroups of 64 heads would need a second, nearly empty round: they are dealt as ceil(256 / per
+// split) splits, so 18 sequences are 270 workgroups for 256 compute units. Ragged, parity mode: 7 x
+// 11 360 tokens 38 us against 64, 17 x 10 161 (21 624) 63 against 83, 11 x 12 613 of 128 heads
+// (34 760) 178 against 174; precise 4: 13 x 7 584 (12 324) 41 against 66, 17 x 7 255 (15 436) 57
+// against 69, 18 x 10 262 (23 112) 107 against 102. Calls that those workgroups fill in one round
+// change sides sooner: 8 x 11 058 (11 072) 49 against 52, 4 x 32 768 (16 384) 74 against 71; precise
+// 4: 1 x 32 768 (4 096) 43 against 51, 4 x 32 768 70 against 59.
+constexpr long long kH16MaxWorkFull = 12288, kH16MaxWorkFull8Bit = 8192;
+constexpr long long kH16MaxWorkSpill = 24576, kH16MaxWorkSpill8Bit = 16384;
+// Calls whose sequences stay whole (one workgroup a sequence and head group) go there while that
+// takes no more rounds of workgroups than a workgroup a sequence and 64 heads does. A round costs 11
+// us and 2.6 per four tiles here, 7 us and 2.4 per tile there: 128 heads, parity mode, 32 x 128
+// tokens 13 us against 19, 64 x 128 (two rounds) 23 against 21, 128 x 128 (four) 45 against 24; 64
+// heads, 256 x 256 tokens 59 against 34; precise 4, 128 x 256 tokens 32 against 22. Two rounds are
+// still the faster at 15 to 20 tiles (64 x 512 tokens of 128 heads 44 against 50, ragged 41 against
+// 56; 15 tiles 43 against 44, ragged 40 against 41; 10 tiles 36 against 33), where the other kernel
+// starts to split and merge, and past them (34 x 960 tokens 67 against 49) where its splits are more
+// than a round themselves (32 heads, 136 x 960 tokens 67 against 93). One tile, two of up to 16
+// heads and two dense ones of up to 32 leave half the waves and more without any: 16 heads, 32 tokens
+// 11 us against 8, 64 tokens 11.0 against 10.0; 64 heads, one token 12.7 against 10.8, 32 tokens 11.0
+// against 11.0. (The 8-bit kernel is not faster there, 12 us against 16, nor is the general form of
+// the linear slabs, 10.9 against 24.8.)
+constexpr int kH16TwoRoundTiles = 15, kH16TwoRoundMaxTiles = 20;
+static inline bool heads16_whole_pays(const AttendPlan& plan, int n_seqs, int H, int tiles, bool f8, bool dense,
+                                      bool linear) {
+    if (!f8 && !linear && tiles <= (H <= 16 || (dense && H <= 32) ? 2 : 1)) return false;
+    const long long blocks = (H + 63) / 64;
+    const long long rounds = heads16_rounds(n_seqs, (H + kH16Heads - 1) / kH16Heads);
+    if (rounds <= (n_seqs * blocks + kAttTargetGroups - 1) / kAttTargetGroups) return true;
+    return !f8 && rounds == 2 && tiles >= kH16TwoRoundTiles &&
+           (tiles <= kH16TwoRoundMaxTiles || plan.n_items * blocks > kAttTargetGroups);
+}
+// `cut`: heads16_plan shares the sequences among work items.
+static inline bool heads16_pays(const AttendPlan& plan, bool cut, int n_seqs, int H, int max_rows, int precise,
+                                bool dense, bool linear) {
+    const long long groups = (H + kH16Heads - 1) / kH16Heads;
+    const int tiles = max_rows / kTile + (max_rows % kTile != 0);
+    const long long work = (long long)n_seqs * tiles * groups;
+    const bool f8 = precise > 2;
+    if (!cut && !heads16_whole_pays(plan, n_seqs, H, tiles, f8, dense, linear)) return false;
+    if (groups == 1 || work <= (f8 ? kH16MaxWork8Bit : kH16MaxWork)) return true;
+    if (!dense || 5 * n_seqs * groups > 2 * kAttTargetGroups) return false;
+    const bool spills = (long long)plan.n_items * ((H + 63) / 64) > kAttTargetGroups;
+    return work <= (spills ? (f8 ? kH16MaxWorkSpill8Bit : kH16MaxWorkSpill) : (f8 ? kH16MaxWorkFull8Bit : kH16MaxWorkFull));
+}
+
+// A call of the shipped row widths whose rows are whole 16-byte pieces. `plan`: attend_plan's, or
+// the linear launcher's cut of it.
+struct AttendRoute {
+    bool heads16;  // workgroups of 16 heads; else of 64
+    bool by_seq;   // no work item has tiles of two sequences (SeqDeal)
+    AttendPlan plan;
+};
+static inline AttendRoute attend_route(const AttendPlan& plan, int n_seqs, int H, int max_rows, int precise, bool dense,
+                                       bool linear) {
+    bool by_seq;
+    const AttendPlan p = heads16_plan(plan, n_seqs, H, max_rows, by_seq);
+    if (!heads16_pays(plan, p.n_items > 0, n_seqs, H, max_rows, precise, dense, linear)) return {false, false, plan};
+    return {true, by_seq, p};
+}
+
+}  // namespace rk

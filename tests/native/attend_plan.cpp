@@ -1,0 +1,12 @@
+// The attention launchers' routing rules (rivoli_amd/csrc/mla_attend_plan.hpp) as a C function.
+#include "../../rivoli_amd/csrc/mla_attend_plan.hpp"
+
+// 1: workgroups of 16 heads, 0: of 64. out: items, by_seq, records of the route; items, records the
+// caller's scratch is sized by.
+extern "C" int attend_route(int n_seqs, int H, int max_rows, int precise, int listed, int out[5]) {
+    const rk::AttendPlan plan = rk::attend_plan(n_seqs, H, max_rows);
+    const rk::AttendRoute r = rk::attend_route(plan, n_seqs, H, max_rows, precise, !listed, false);
+    out[0] = r.plan.n_items, out[1] = r.by_seq, out[2] = r.plan.n_records;
+    out[3] = plan.n_items, out[4] = plan.n_records;
+    return r.heads16;
+}

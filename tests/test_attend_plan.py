@@ -1,0 +1,44 @@
+"""Which kernel an attention call takes and how its tiles are shared
+(rivoli_amd/csrc/mla_attend_plan.hpp, compiled for the host by tests/native/Makefile)."""
+import pytest
+
+from tests.util import attend_route
+
+
+@pytest.mark.parametrize("listed", [False, True])
+@pytest.mark.parametrize("precise", [0, 2, 4])
+def test_a_plan_fits_the_scratch_and_the_chip(precise, listed):
+    """Over head counts, batches and lengths: never more records than the caller's scratch was sized
+    for, every work item with a tile a wave, and whole sequences where there is nothing to deal."""
+    for H in (1, 16, 17, 33, 48, 64, 80, 128, 200, 528, 4096):
+        for n in (1, 2, 7, 16, 33, 64, 65, 100, 128, 129, 200, 255, 256, 1024, 1025, 5000):
+            for rows in (1, 32, 33, 64, 255, 256, 300, 512, 1000, 1984, 4096, 40000, 2 ** 25):
+                r = attend_route(n, H, rows, precise, listed)
+                tiles = -(-rows // 32)
+                if not r.heads16:
+                    assert r.items == r.scratch_items and r.records == r.scratch_records
+                    continue
+                assert r.items <= r.scratch_items and r.records <= r.scratch_records
+                assert r.records == (r.items + n if r.items else 0)
+                assert r.items == 0 or (r.items >= n and r.items <= n * (tiles // 4))
+                assert not r.by_seq or (n <= 64 and r.items > n)
+
+
+@pytest.mark.parametrize("precise", [2, 4])
+def test_batches_of_short_sequences_keep_to_the_kernel_of_fewer_rounds(precise):
+    """Sequences that stay whole are a workgroup for every 16 heads in one kernel and for every 64 in
+    the other: where the first need more rounds of the 256 compute units, short calls are the
+    other's (128 sequences of 128 tokens at 128 heads: four rounds against one)."""
+    for H, n in ((128, 64), (128, 128), (64, 128), (64, 256), (32, 256), (48, 85), (80, 51)):
+        for rows in (32, 64, 128, 256, 320):
+            for listed in (False, True):
+                assert not attend_route(n, H, rows, precise, listed).heads16, (H, n, rows)
+    for H, n in ((128, 32), (64, 64), (32, 128), (16, 256), (48, 80), (80, 48)):
+        assert attend_route(n, H, 128, precise).heads16, (H, n)
+    # one round more is made good where the other kernel splits
+    assert attend_route(128, 64, 512, 2).heads16 and not attend_route(34, 128, 960, 2).heads16
+    assert attend_route(136, 32, 960, 2).heads16 and not attend_route(128, 64, 512, 4).heads16
+    # nothing for most of the four waves to do
+    for H, rows in ((16, 1), (16, 64), (32, 33), (64, 1), (128, 32)):
+        assert attend_route(4, H, rows, precise).heads16 == (precise == 4), (H, rows)
+    assert attend_route(4, 32, 64, 2, listed=True).heads16 and attend_route(4, 64, 64, 2).heads16

@@ -1,4 +1,8 @@
 """Seeded synthetic inputs shared by the oracle and GPU parity tests (numpy only)."""
+import ctypes
+import os
+import subprocess
+
 import numpy as np
 
 
@@ -39,3 +43,27 @@ def shuffled_block_tables(n_seqs, blocks_per_seq, n_pages, seed):
 def slots_for(table_row, positions, page_tokens=64):
     positions = np.asarray(positions)
     return (table_row[positions // page_tokens] * page_tokens + positions % page_tokens).astype(np.int32)
+
+
+class AttendRoute:
+    """attend_route of rivoli_amd/csrc/mla_attend_plan.hpp: which workgroups a paged call of the
+    shipped row widths takes, and its work items."""
+
+    def __init__(self, heads16, out):
+        self.heads16 = bool(heads16)
+        self.items, self.by_seq, self.records, self.scratch_items, self.scratch_records = list(out)
+
+
+def attend_route(n_seqs, H, max_rows, precise, listed=False):
+    global _PLAN
+    if _PLAN is None:
+        here = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native")
+        path = os.path.join(here, "attend_plan.so")
+        if not os.path.exists(path):
+            subprocess.run(["make", "-C", here, path], check=True, capture_output=True)
+        _PLAN = ctypes.CDLL(path)
+    out = (ctypes.c_int * 5)()
+    return AttendRoute(_PLAN.attend_route(n_seqs, H, max_rows, precise, int(listed), out), out)
+
+
+_PLAN = None
