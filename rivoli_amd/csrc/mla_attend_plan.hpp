@@ -42,15 +42,27 @@ static inline AttendPlan attend_plan(int n_seqs, int H, int max_rows) {
     return p;
 }
 
+// Rounds of workgroups a die's 32 compute units take for `items` work items: the head groups of an
+// item sit on one die (mla_attend_heads16_kernel).
+constexpr int kAttDieUnits = kAttTargetGroups / kAttDies;
+static inline long long heads16_rounds(long long items, long long groups) {
+    const long long per_die = (items + kAttDies - 1) / kAttDies * groups;
+    return (per_die + kAttDieUnits - 1) / kAttDieUnits;
+}
+
 // The work items of a call by 16 heads a workgroup: one workgroup per compute unit, at least a tile
 // per wave, and no more partial records than `plan` (which the caller's scratch was sized by) has.
+// A die takes whole items, so three groups of heads make 8 x 10 items, not 85: with 85 five of the
+// dies had 33 workgroups for their 32 units and the call two rounds (21 x 1 600 tokens 50 us, with 80
+// 33; 112 heads, 5 x 4 000 55 and 36).
 // Up to 64 sequences no work item meets two of them, so their number need not be a multiple of the
 // sequences'; more sequences, or longer ones than SeqDeal counts, share the tiles evenly.
 static inline AttendPlan heads16_plan(const AttendPlan& plan, int n_seqs, int H, int max_rows, bool& by_seq) {
     const int tiles = max_rows / kTile + (max_rows % kTile != 0);
+    const int groups = (H + kH16Heads - 1) / kH16Heads;
     const long long most = (long long)n_seqs * (tiles / kH16Waves);
     by_seq = n_seqs <= kSeqDealMax && tiles <= kSeqDealMaxTiles;
-    long long n = kAttTargetGroups / ((H + kH16Heads - 1) / kH16Heads);
+    long long n = groups <= kAttDieUnits ? kAttDieUnits / groups * kAttDies : kAttTargetGroups / groups;
     if (n > most) n = most;
     if (n > plan.n_items) n = plan.n_items;
     if (!by_seq) n = n / n_seqs * n_seqs;
@@ -60,13 +72,6 @@ static inline AttendPlan heads16_plan(const AttendPlan& plan, int n_seqs, int H,
     p.n_splits = n ? (int)((n + n_seqs - 1) / n_seqs) : 1;
     p.n_records = n ? p.n_items + n_seqs : 0;
     return p;
-}
-
-// Rounds of workgroups a die's 32 compute units take for `items` work items: the head groups of an
-// item sit on one die (mla_attend_heads16_kernel).
-static inline long long heads16_rounds(long long items, long long groups) {
-    const long long per_die = (items + kAttDies - 1) / kAttDies * groups, units = kAttTargetGroups / kAttDies;
-    return (per_die + units - 1) / units;
 }
 
 // Whether a call goes to the workgroups of 16 heads: its 32-token tiles times its groups of 16

@@ -20,6 +20,8 @@ def test_a_plan_fits_the_scratch_and_the_chip(precise, listed):
                     continue
                 assert r.items <= r.scratch_items and r.records <= r.scratch_records
                 assert r.records == (r.items + n if r.items else 0)
+                groups = -(-H // 16)    # the groups of an item sit on one of the eight dies of 32 units
+                assert groups > 32 or -(-r.items // 8) * groups <= 32, (H, n, rows, r.items)
                 assert r.items == 0 or (r.items >= n and r.items <= n * (tiles // 4))
                 assert not r.by_seq or (n <= 64 and r.items > n)
 
