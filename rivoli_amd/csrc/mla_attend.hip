@@ -968,7 +968,7 @@ __global__ __launch_bounds__(128) void mla_attend_combine_kernel(
 static int attend_merge(const AttendArgs& a, const AttendPlan& plan, int n_seqs, int max_rows, const int* seq_lens,
                         const int* n_rows, bool listed, hipStream_t st) {
     const int rc = launch_status();
-    if (rc != 0 || plan.n_splits <= 1) return rc;
+    if (rc != 0 || plan.n_items == 0) return rc;
     hipLaunchKernelGGL(mla_attend_combine_kernel, dim3((unsigned)a.H, (unsigned)n_seqs), dim3(128), 0, st,
                        a.part_acc, a.part_ml, seq_lens, n_rows, listed ? 1 : 0, max_rows, n_seqs, plan.n_items,
                        a.by_seq, a.H, a.kvl, a.clat);

@@ -13,6 +13,7 @@ constexpr int kAttMaxSplits = 64;
 constexpr int kDealMaxSeqs = 1024;         // dealing keeps a prefix sum over the sequences in LDS
 constexpr int kH16Heads = 16;              // mla_attend_heads16.hpp: heads and waves of a workgroup
 constexpr int kH16Waves = 4;
+constexpr int kH16WholeTiles = 32;         // past these a whole sequence is a workgroup's for too long
 constexpr int kSeqDealMax = 64;            // SeqDeal: sequences, one a lane
 constexpr int kSeqDealMaxTiles = 1 << 19;  // of a sequence: its quotients stay under 2^24
 
@@ -56,7 +57,11 @@ static inline long long heads16_rounds(long long items, long long groups) {
 // dies had 33 workgroups for their 32 units and the call two rounds (21 x 1 600 tokens 50 us, with 80
 // 33; 112 heads, 5 x 4 000 55 and 36).
 // Up to 64 sequences no work item meets two of them, so their number need not be a multiple of the
-// sequences'; more sequences, or longer ones than SeqDeal counts, share the tiles evenly.
+// sequences'; more sequences, or longer ones than SeqDeal counts, share the tiles evenly. Fewer than
+// two work items a sequence are not worth the merge, but for one thing: up to 16 heads a call has
+// nowhere else to go, and one long sequence must not keep a workgroup to itself. Past 32 tiles a work
+// item a sequence shares those batches' tiles too: 200 sequences, one of 32 768 tokens and the others
+// of 100, 769 -> 72 us (one of 4 096 106 -> 36; all of 4 096 111 -> 118, the merge's launch).
 static inline AttendPlan heads16_plan(const AttendPlan& plan, int n_seqs, int H, int max_rows, bool& by_seq) {
     const int tiles = max_rows / kTile + (max_rows % kTile != 0);
     const int groups = (H + kH16Heads - 1) / kH16Heads;
@@ -66,7 +71,8 @@ static inline AttendPlan heads16_plan(const AttendPlan& plan, int n_seqs, int H,
     if (n > most) n = most;
     if (n > plan.n_items) n = plan.n_items;
     if (!by_seq) n = n / n_seqs * n_seqs;
-    if (n < 2 * n_seqs) n = 0, by_seq = false;
+    const int least = groups == 1 && tiles > kH16WholeTiles ? n_seqs : 2 * n_seqs;
+    if (n < least) n = 0, by_seq = false;
     AttendPlan p;
     p.n_items = (int)n;
     p.n_splits = n ? (int)((n + n_seqs - 1) / n_seqs) : 1;
@@ -107,16 +113,20 @@ constexpr long long kH16MaxWorkSpill = 24576, kH16MaxWorkSpill8Bit = 16384;
 // heads and two dense ones of up to 32 leave half the waves and more without any: 16 heads, 32 tokens
 // 11 us against 8, 64 tokens 11.0 against 10.0; 64 heads, one token 12.7 against 10.8, 32 tokens 11.0
 // against 11.0. (The 8-bit kernel is not faster there, 12 us against 16, nor is the general form of
-// the linear slabs, 10.9 against 24.8.)
+// the linear slabs, 10.9 against 24.8.) Past 32 tiles the call lasts as long as its longest sequence
+// in one workgroup, and the other kernel deals them out: 64 heads, 33 x 1 984 tokens 60 us against 46,
+// one of 1 984 among 32 of 100 58 against 36; unless its splits, again, are more than a round (32
+// heads, 80 x 1 600 tokens 50 against 80).
 constexpr int kH16TwoRoundTiles = 15, kH16TwoRoundMaxTiles = 20;
 static inline bool heads16_whole_pays(const AttendPlan& plan, int n_seqs, int H, int tiles, bool f8, bool dense,
                                       bool linear) {
     if (!f8 && !linear && tiles <= (H <= 16 || (dense && H <= 32) ? 2 : 1)) return false;
     const long long blocks = (H + 63) / 64;
+    const bool spills = plan.n_items * blocks > kAttTargetGroups;
+    if (!linear && H > kH16Heads && tiles > kH16WholeTiles) return spills;
     const long long rounds = heads16_rounds(n_seqs, (H + kH16Heads - 1) / kH16Heads);
     if (rounds <= (n_seqs * blocks + kAttTargetGroups - 1) / kAttTargetGroups) return true;
-    return !f8 && rounds == 2 && tiles >= kH16TwoRoundTiles &&
-           (tiles <= kH16TwoRoundMaxTiles || plan.n_items * blocks > kAttTargetGroups);
+    return !f8 && rounds == 2 && tiles >= kH16TwoRoundTiles && (tiles <= kH16TwoRoundMaxTiles || spills);
 }
 // `cut`: heads16_plan shares the sequences among work items.
 static inline bool heads16_pays(const AttendPlan& plan, bool cut, int n_seqs, int H, int max_rows, int precise,

@@ -23,7 +23,7 @@ def test_a_plan_fits_the_scratch_and_the_chip(precise, listed):
                 groups = -(-H // 16)    # the groups of an item sit on one of the eight dies of 32 units
                 assert groups > 32 or -(-r.items // 8) * groups <= 32, (H, n, rows, r.items)
                 assert r.items == 0 or (r.items >= n and r.items <= n * (tiles // 4))
-                assert not r.by_seq or (n <= 64 and r.items > n)
+                assert not r.by_seq or (n <= 64 and r.items >= 2 * n)
 
 
 @pytest.mark.parametrize("precise", [2, 4])
@@ -44,3 +44,18 @@ def test_batches_of_short_sequences_keep_to_the_kernel_of_fewer_rounds(precise):
     for H, rows in ((16, 1), (16, 64), (32, 33), (64, 1), (128, 32)):
         assert attend_route(4, H, rows, precise).heads16 == (precise == 4), (H, rows)
     assert attend_route(4, 32, 64, 2, listed=True).heads16 and attend_route(4, 64, 64, 2).heads16
+
+
+@pytest.mark.parametrize("precise", [0, 2])
+def test_no_batch_of_long_sequences_is_left_whole(precise):
+    """Past 32 tiles the lengths may differ widely, and the host does not know them: whichever kernel
+    takes such a call deals its tiles out, also with fewer than two work items a sequence (129 to 255
+    sequences of 16 heads, where one of 32 768 tokens took 769 us on a workgroup of its own)."""
+    for H in (8, 16, 17, 32, 64, 96, 128):
+        for n in list(range(1, 256, 6)) + [128, 129, 200, 254, 255]:
+            for rows in (1025, 1984, 4096, 32768):
+                r = attend_route(n, H, rows, precise)
+                # (whole only where there is no scratch to merge from, or the other kernel's splits are
+                # more than a round of workgroups themselves)
+                assert r.items or not r.scratch_items or (r.scratch_items * -(-H // 64) > 256 and H > 16 and rows < 2048), \
+                    (H, n, rows)

@@ -14,6 +14,7 @@ import pytest
 from rivoli_amd import hip
 from tests.attend_cases import paged_case
 from tests.gpu_util import back, dev, dzeros
+from tests.util import attend_route
 
 pytestmark = pytest.mark.gpu
 KVL, ROPE, PT = 512, 64, 64
@@ -534,3 +535,20 @@ def test_linear_list_entries_of_all_ones_are_left_out(oracle):
         assert code == 0
         for scratch in (True, False):
             check_linear(run_linear(case, h, 500, kvl, rope, rows=rows, scratch=scratch), want, f"h={h} scratch={scratch}")
+
+
+@pytest.mark.parametrize("H", [16, 5])
+def test_few_heads_and_more_sequences_than_half_the_work_items(oracle, H):
+    """129 to 255 sequences of up to 16 heads past 32 tiles: a work item a sequence, sharing the
+    batch's tiles (long ones cut, short ones several to an item); even lengths stay whole."""
+    lens = [40, 0, 33, 70] * 33
+    lens[50], lens[131] = 1500, 1100
+    c = paged_case(oracle, lens, H=H, seed=970, outlier_frac=0.0, page_tokens=16)
+    route = attend_route(len(lens), H, max(lens), 2)
+    assert route.heads16 and route.items == len(lens)
+    args = (c["qabs"], c["qrope"], c["pool"], c["table"])
+    for claimed in (c["lens"], np.full(len(lens), 32, np.int32)):
+        claimed = np.minimum(claimed, c["lens"])
+        want = oracle.mla_attend_paged(*args, claimed, None, None, KVL, ROPE, 16, c["scale"], n_threads=8)
+        got = run_paged(dict(c, lens=claimed), max(lens), pt=16)
+        check(got, want, 2, "dense", mild=True)
