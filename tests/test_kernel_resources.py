@@ -91,13 +91,57 @@ def test_block_scorer_keeps_its_row_and_both_chunk_buffers_in_registers():
     assert seen == 2
 
 
+@pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
+def test_kernels_of_16_heads_a_workgroup_do_not_spill():
+    """One wave per SIMD with the whole register file, transfers into LDS ordered by hand
+    (rivoli_amd/csrc/mla_attend_heads16.hpp): dense, listed and linear, in each of the bf16 modes."""
+    seen = 0
+    for b in _resource_blocks("mla_attend.hip"):
+        name = b.split()[0]
+        if "mla_attend_heads16_kernel" not in name:
+            continue
+        seen += 1
+        assert int(re.search(r"VGPRs Spill: (\d+)", b).group(1)) == 0, name
+        assert int(re.search(r"ScratchSize \[bytes/lane\]: (\d+)", b).group(1)) == 0, name
+        assert int(re.search(r"Occupancy \[waves/SIMD\]: (\d+)", b).group(1)) == 1, name
+        assert int(re.search(r"LDS Size \[bytes/block\]: (\d+)", b).group(1)) <= 160 * 1024, name
+    assert seen == 7
+
+
+@pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
+def test_the_block_scorers_matrix_kernels_and_the_few_row_selection_do_not_spill():
+    """Two waves per SIMD of 252 registers in the many-query scorer (scalar registers do spill
+    there, in the fold), three in the one-query scorers; a row's keys in registers and its masks
+    out of memory in the few-row selection, as in the many-row one."""
+    seen = []
+    for src, part, waves in (("block_index.hip", "score_blocks_pair_kernel", 2),
+                             ("block_index.hip", "score_blocks_one_kernel", 3),
+                             ("index_topk.hip", "block_select_few_kernel", 8)):
+        for b in _resource_blocks(src):
+            name = b.split()[0]
+            if part not in name:
+                continue
+            seen.append(part)
+            if part == "block_select_few_kernel":
+                assert int(re.search(r"SGPRs Spill: (\d+)", b).group(1)) == 0, name
+            assert int(re.search(r"VGPRs Spill: (\d+)", b).group(1)) == 0, name
+            assert int(re.search(r"ScratchSize \[bytes/lane\]: (\d+)", b).group(1)) == 0, name
+            assert int(re.search(r"Occupancy \[waves/SIMD\]: (\d+)", b).group(1)) >= waves, name
+    assert len(seen) == 5
+
+
 def test_the_build_refuses_an_attention_object_that_spills():
     """build.check_resources is what build_kernels applies to mla_attend.hip's resource report:
-    scratch memory or too much LDS in an 8-bit attention kernel raises instead of linking."""
+    scratch memory or too much LDS in an 8-bit attention kernel, or in one of 16 heads a workgroup,
+    raises instead of linking, and so does a report without them."""
+    figures = "    ScratchSize [bytes/lane]: 0\n    LDS Size [bytes/block]: 85632\n"
     head = "x.hip:1:1: remark: Function Name: _ZN2rk23mla_attend_paged_kernelILi2ELi2ELi0ELb0ELb1EEEvNS_10AttendArgsE\n"
-    fine = head + "    ScratchSize [bytes/lane]: 0\n    LDS Size [bytes/block]: 85632\n"
+    heads16 = "x.hip:1:1: remark: Function Name: _ZN2rk25mla_attend_heads16_kernelILi2ELi2ELi3EEEvNS_10AttendArgsE\n"
+    fine = head + figures + heads16 + figures.replace("85632", "161328")
     build.check_resources("mla_attend.hip", fine)
     build.check_resources("kv_gather.hip", "")                        # other files are not held to it
-    for bad in (fine.replace("lane]: 0", "lane]: 44"), fine.replace("85632", "170000"), ""):
+    for bad in (fine.replace("lane]: 0", "lane]: 44", 1), fine.replace("85632", "170000"), "", head + figures,
+                head + figures + heads16 + figures.replace("lane]: 0", "lane]: 8"),
+                fine.replace("161328", "163856")):
         with pytest.raises(RuntimeError):
             build.check_resources("mla_attend.hip", bad)
