@@ -7,7 +7,11 @@ hi + lo (precise = 2, the parity mode) the tests also hold the kernel to a purel
 2e-5 of the largest output, on caches with x30 outlier rows whose softmax is sharply peaked.
 With only q carried that way (1) the bound is 2e-3; with q rounded to bf16 once (0) a score
 is off by ~2^-10 of |q||k|, which is held to 3e-2 on the outlier caches. Both lighter modes
-meet the reference's bar on N(0,1) rows."""
+meet the reference's bar on N(0,1) rows.
+
+Short calls run in workgroups of 16 heads, at `precise` 3 and 4 too: what a case below says of the
+tiles and runs of the workgroups of 64 heads or of the 8-bit kernel is reached at its size only
+where it asserts the route (the batches that do are at the end of the file)."""
 import numpy as np
 import pytest
 
@@ -438,6 +442,8 @@ def test_both_sides_of_the_line_between_workgroups_of_16_and_of_64_heads(oracle,
     # tiles x groups of 16 heads: 13 x 3 a sequence, the line at 8192 (8-bit modes: 4096)
     lens = (edges * 12)[:212] if large else edges[:12]
     assert (len(lens) * 13 * 3 > 8192) == large
+    assert attend_route(len(lens), H, max(lens), precise).heads16 != large
+    assert attend_route(len(lens), H, 70, precise, listed=True).heads16 != large
     c = paged_case(oracle, lens, H=H, seed=900, outlier_frac=0.0)
     want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], None, None,
                                    KVL, ROPE, PT, c["scale"], n_threads=8)
@@ -552,3 +558,84 @@ def test_few_heads_and_more_sequences_than_half_the_work_items(oracle, H):
         want = oracle.mla_attend_paged(*args, claimed, None, None, KVL, ROPE, 16, c["scale"], n_threads=8)
         got = run_paged(dict(c, lens=claimed), max(lens), pt=16)
         check(got, want, 2, "dense", mild=True)
+
+
+def listed(tokens, width):
+    """Row lists of the sequences' token arrays, and their lengths."""
+    rows = np.zeros((len(tokens), width), np.uint32)
+    for s, t in enumerate(tokens):
+        rows[s, :len(t)] = t
+    return rows, np.array([len(t) for t in tokens], np.int32)
+
+
+@pytest.mark.parametrize("precise", [2, 1, 0, 4, 3])
+@pytest.mark.parametrize("pt", [64, 128, 16, 48, 4])
+def test_workgroups_of_64_heads_over_a_ragged_batch(oracle, pt, precise):
+    """A batch the workgroups of 64 heads (and the 8-bit kernel) take and deal out, dense and listed:
+    lengths around every tile and run size, an empty sequence, a second block of 6 heads; then the
+    same with pages the table does not have, lengths past the table and listed tokens past it, left
+    out and counted once each."""
+    H, top = 70, 700
+    lens = ([31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 255, 256, 257, 383, 384, 385, 0, 1, 511, 700] * 3)[:56]
+    n = len(lens)
+    for is_listed in (False, True):
+        route = attend_route(n, H, top, precise, is_listed)
+        assert not route.heads16 and route.items > n
+    c = paged_case(oracle, lens, H=H, seed=980 + pt, page_tokens=pt, outlier_frac=0.0)
+    rng = np.random.default_rng(98)
+
+    def want_of(tokens):
+        rows, n_rows = listed(tokens, top)
+        return oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], None, rows, n_rows,
+                                       KVL, ROPE, pt, c["scale"], n_threads=8)
+
+    mild = precise in (2, 4)
+    every = [np.arange(k) for k in lens]
+    want = want_of(every)
+    check(run_paged(c, top, precise=precise, pt=pt), want, precise, "dense", mild=mild)
+    rows, n_rows = listed([rng.permutation(t) for t in every], top)
+    check(run_paged(c, top, rows=rows, n_rows=n_rows, use_lens=False, precise=precise, pt=pt), want, precise, "listed",
+          mild=mild)
+    # pages that are not there, in the longest sequences and a short one
+    table = c["table"].copy()
+    blocks = table.shape[1]
+    gone = {(21, 0): -1, (21, blocks - 1): c["n_pages"], (43, 128 // pt): c["n_pages"] + 9, (0, 0): -7}
+    for at, page in gone.items():
+        table[at] = page
+    kept = [t[[(s, b) not in gone for b in t // pt]] for s, t in enumerate(every)]
+    missing = sum(lens) - sum(len(t) for t in kept)
+    want = want_of(kept)
+    bad = dzeros(4)
+    check(run_paged(dict(c, table=table), top, precise=precise, pt=pt, bad=bad), want, precise, "dense, missing pages",
+          mild=mild)
+    assert back(bad, np.uint32)[0] == missing
+    bad = dzeros(4)
+    tokens = [rng.permutation(t) for t in every]
+    tokens[4][:3], tokens[22] = [blocks * pt, 2 ** 31, 2 ** 32 - 2], np.array([blocks * pt + 5])
+    kept_listed = [np.array([k for k in t if k < blocks * pt and (s, k // pt) not in gone], np.int64)
+                   for s, t in enumerate(tokens)]
+    rows, n_rows = listed(tokens, top)
+    got = run_paged(dict(c, table=table), top, rows=rows, n_rows=n_rows, use_lens=False, precise=precise, pt=pt, bad=bad)
+    check(got, want_of(kept_listed), precise, "listed, missing pages and tokens past the table", mild=mild)
+    assert not got[22].any()
+    assert back(bad, np.uint32)[0] == sum(len(t) for t in tokens) - sum(len(t) for t in kept_listed)
+    # lengths past the table (what the table does have past a sequence's end are rows never written)
+    bad = dzeros(4)
+    claimed = np.array(lens, np.int32)
+    claimed[[7, 21]] = blocks * pt + 40, blocks * pt + 1
+    got = run_paged(dict(c, lens=claimed), blocks * pt + 64, precise=precise, pt=pt, bad=bad)
+    check(got, want_of(every), precise, "lengths past the table", mild=mild)
+    assert back(bad, np.uint32)[0] == 41
+
+
+@pytest.mark.parametrize("lists", [False, True])
+def test_peaked_softmax_in_workgroups_of_64_heads(oracle, lists):
+    """As test_peaked_softmax, where that kernel's own rescaling and masked tail run."""
+    lens = [1100, 777, 1000, 1] * 20
+    assert not attend_route(80, 64, 1100, 2, lists).heads16
+    c = paged_case(oracle, lens, H=64, seed=990, q_gain=6.0, page_tokens=16)
+    want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], None, None,
+                                   KVL, ROPE, 16, c["scale"], n_threads=8)
+    rows, n_rows = listed([np.arange(k)[::-1] for k in lens], 1100)
+    got = run_paged(c, 1100, rows=rows, n_rows=n_rows, pt=16) if lists else run_paged(c, 1100, pt=16)
+    check(got, want, 2, "peaked", tight_bound=False)
