@@ -78,8 +78,9 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
     const int* const table_g = LINEAR ? nullptr : a.block_table + (size_t)seq * a.max_blocks;
     // the list entry (or position) of the lane's row; the read is unconditional and clamped
     auto token_of = [&](int tile) -> unsigned int {
-        const int pos = min(r_begin + tile * kTile + (lane & 31), r_end - 1);
-        return rows_g ? rows_g[pos] : (unsigned)pos;
+        // (unsigned: three rounds of tiles past the end of 2^31 - 32 rows is past what an int holds)
+        const unsigned int pos = min((unsigned)r_begin + (unsigned)tile * kTile + (lane & 31), (unsigned)r_end - 1u);
+        return rows_g ? rows_g[pos] : pos;
     };
     // the row's page, likewise (-1: the block table has no entry for it)
     auto page_of = [&](unsigned int tok) -> int {

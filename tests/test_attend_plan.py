@@ -59,3 +59,22 @@ def test_no_batch_of_long_sequences_is_left_whole(precise):
                 # more than a round of workgroups themselves)
                 assert r.items or not r.scratch_items or (r.scratch_items * -(-H // 64) > 256 and H > 16 and rows < 2048), \
                     (H, n, rows)
+
+
+@pytest.mark.parametrize("r_end", [1, 33, 2 ** 20, 2 ** 31 - 400, 2 ** 31 - 32])
+def test_list_positions_looked_up_ahead_stay_in_the_list(r_end):
+    """Host-side restatement of token_of in mla_attend_heads16.hpp: which list entries a wave asks for
+    while it walks every fourth tile and looks up three of its own ahead. In 32 bits, unsigned; as
+    ints the last rounds of the longest lists would wrap to entries in front of the list."""
+    def wrapped(x, signed):
+        x &= 0xFFFFFFFF
+        return x - 2 ** 32 if signed and x >= 2 ** 31 else x
+
+    n_tiles = -(-r_end // 32)
+    for wave in range(4):
+        last = wave + (n_tiles - 1 - wave) // 4 * 4 if n_tiles > wave else wave
+        for tile in {wave, wave + 4, wave + 8, last, last + 4, last + 8, last + 12}:
+            for lane in (0, 31):
+                assert min(wrapped(tile * 32 + lane, False), r_end - 1) in range(r_end)
+    if r_end > 2 ** 31 - 384:
+        assert min(wrapped((n_tiles + 11) * 32, True), r_end - 1) < 0
