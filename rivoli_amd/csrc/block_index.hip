@@ -24,8 +24,8 @@
 // gives the reference's bits. The matrix kernels (hd = 128, up to 64 heads) test that property
 // on the operands they hold (RowSpan) and take such tiles through v_mfma_f32_32x32x16_bf16; any
 // other tile of the same launch is folded term by term as below. 8 192 queries x 64 heads x
-// <= 2 048 blocks: 237 us against 3 680 term by term (the whole rectangle 363 against 7 970).
-// Operands of another kind (no such rows leave the indexer) take the same launches' fold: 4.8 ms.
+// <= 2 048 blocks: 209 us against 3 640 term by term (the whole rectangle 361 against 7 500).
+// Operands of another kind (no such rows leave the indexer) take the same launches' fold: 3 430.
 // Term by term, what is free is where the operands come from. A lane owns block c and
 // keeps its 128-value row in registers for the whole launch; a wave's 64 lanes share the query,
 // so q[t][h][i] and w[t][h] are wave-uniform and come through scalar loads straight into the
@@ -36,6 +36,7 @@
 #include "codec.hpp"
 
 #include <cmath>
+#include <type_traits>
 
 #include "rivoli_kvcache.h"
 
@@ -361,6 +362,64 @@ __device__ __forceinline__ uint32_t low_half_bits(const f32x4& v) {
     return (__float_as_uint(v.x) | __float_as_uint(v.y) | __float_as_uint(v.z) | __float_as_uint(v.w)) & 0xffffu;
 }
 
+// The fold of rows that are not exact in every order. Scalar operands (walk_pairs) want waves that
+// share their q rows and three of them a SIMD; the matrix kernels' fold has neither, and waited for
+// the scalar cache a quarter of its time. Here every sixteen lanes hold a q row in eight registers,
+// lane j of them dims 4 j + e and 64 + 4 j + e, and a multiply takes dim i from lane (i % 64) / 4 of
+// its own sixteen (row_newbcast: an operand modifier, no instruction). Vector loads return in order,
+// so a row is requested a whole dot (256 instructions) before it is used, and the halves of a wave may
+// fold different rows. f32 values of no particular kind, 64 heads, prefill form, us: folded by
+// scalar operands in kernels of their own (walk_pairs) / by them in the matrix kernels / so:
+// 8 192 x 2 048 3 640 / 4 800 / 3 430, 4 096 x 1 024 1 050 / 1 290 / 970, 2 000 x 500 282 / 472 / 422,
+// 1 000 x 250 83 / 157 / 120, 300 x 75 39 / 88 / 44; the full form, 5 x 8 192 39 / 83 / 44, 1 x 8 192 14 /
+// 18 / 13. Not reached: 2 x 16 384 21 / 78 / 73 and 1 x 16 384 14 / 18.6 / 18.6, whose eight waves a
+// workgroup shared the heads, and 5 heads, 8 192 x 2 048 256 / 431 / 507, where fetching a row outweighs it.
+struct QRow {
+    f32x4 v[2];
+};
+__device__ __forceinline__ QRow load_q(const float* __restrict__ at) {  // at: the row + 4 * (lane & 15)
+    return {{*reinterpret_cast<const f32x4_u*>(at), *reinterpret_cast<const f32x4_u*>(at + 64)}};
+}
+template <int I>
+__device__ __forceinline__ float q_dim(const QRow& q) {
+    constexpr int kRowNewBcast = 0x150;  // | lane of the sixteen
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(q.v[I / 64][I % 4]), kRowNewBcast | (I % 64) / 4, 0xf, 0xf, true));
+}
+// Every addition needs the one before it, so the next dim's product is taken between two of them.
+// SHARED: another wave is on the SIMD. Two waves without a pause take 4.6 cycles an instruction
+// between them, with an empty slot after each addition 4.0; a wave alone 5.0, and 6.8 with the slot.
+template <bool SHARED, int I = 0>
+__device__ __forceinline__ float fold_dot(float dot, float prod, const QRow& q, const float (&row)[128]) {
+    if constexpr (I == 127) {
+        return dot + prod;
+    } else {
+        const float next = q_dim<I + 1>(q) * row[I + 1];
+        __builtin_amdgcn_sched_barrier(0);
+        dot = dot + prod;
+        __builtin_amdgcn_sched_barrier(0);
+        if (SHARED) asm volatile("s_nop 0");
+        return fold_dot<SHARED, I + 1>(dot, next, q, row);
+    }
+}
+// The head terms of `n` >= 1 consecutive heads from the lane's first on, whose q row and weight are at
+// q and w. on_term(i, term) receives them in order. All lanes of the wave must be here.
+template <bool SHARED, class OnTerm>
+__device__ __forceinline__ void fold_heads(const float* __restrict__ q, const float* __restrict__ w, int n,
+                                           const float (&row)[128], OnTerm&& on_term) {
+    q += 4 * (threadIdx.x & 15);
+    QRow next = load_q(q);
+    float next_w = *w;
+    for (int i = 0; i < n; ++i) {
+        const QRow now = next;
+        const float weight = next_w;
+        if (i + 1 < n) q += 128, ++w;  // the last re-reads its own
+        next = load_q(q);
+        next_w = *w;
+        __builtin_amdgcn_sched_barrier(0);
+        on_term(i, head_term(fold_dot<SHARED>(0.0f, q_dim<0>(now) * row[0], now, row), weight));
+    }
+}
+
 // A workgroup's four waves own two queries each and walk the split's blocks in tiles of 32, which
 // all four read from LDS; a wave's q rows stay in registers as matrix operands (64 heads x 2
 // queries x 128 values = 128 registers). The 32 rows of a matrix tile are 16 heads of the wave's
@@ -376,7 +435,7 @@ constexpr int kPairQueries = kPairWaves * 2;
 constexpr int kPairHeads = 64;
 constexpr int kPairTile = 32;
 constexpr int kPairRow = 128 * 2 + 16;  // bytes of a bf16 row in LDS: 16-byte reads of 16 rows meet no bank twice
-constexpr int kPairSplitMax = 4096;     // blocks of a split: one bit of a 64-bit mask per 64
+constexpr int kPairSplitMax = 4096;     // blocks of a split: one bit of a 128-bit mask per tile
 
 __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
     const float* __restrict__ q, const float* __restrict__ kv, const float* __restrict__ w,
@@ -391,15 +450,18 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
     const int group = ratio > 0 ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x;
     const int tw = group * kPairQueries + wave * 2;  // the wave's first query
     const int c0 = blockIdx.y * split_blocks;
-    // 64-block groups with a block that some query up to t_last may rank (first_query)
-    const auto groups_for = [&](int t_last) {
+    // tiles of 64-block groups with a block that some query up to t_last may rank (first_query)
+    const auto tiles_for = [&](int t_last) {
         int end = min(n_comp, c0 + split_blocks);
         if (ratio > 0) end = min(end, ((t_last + 1) / ratio + 63) & ~63);
-        return end > c0 ? (end - c0 + 63) >> 6 : 0;
+        return end > c0 ? (end - c0 + kPairTile - 1) / kPairTile : 0;
     };
-    const int all_groups = groups_for(min(s, (group + 1) * kPairQueries) - 1);
-    if (!all_groups) return;  // workgroup-uniform
-    const int my_groups = tw < s ? groups_for(min(s, tw + 2) - 1) : 0;
+    const int tiles = tiles_for(min(s, (group + 1) * kPairQueries) - 1);
+    if (!tiles) return;  // workgroup-uniform
+    const int my_tiles = tw < s ? tiles_for(min(s, tw + 2) - 1) : 0;
+
+    // query t exists and its selection may rank a block of c's 64
+    const auto may_rank = [&](int t, int c) { return t < s && (ratio <= 0 || ((c & ~63) + 1) * (long long)ratio - 1 <= t); };
 
     bf16x8 a[4][8];
     int q_span = 0;
@@ -421,10 +483,12 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
                     const int m = 2 * (j0 + j) + half, hh = c * 16 + (m >> 3) * 4 + (m & 3);
                     const int t = min(tw + ((m >> 2) & 1), s - 1);
                     v[j] = *reinterpret_cast<const f32x4_u*>(q + ((size_t)t * heads + min(hh, heads - 1)) * 128 + row * 4);
-                    if (hh >= heads) v[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 }
+                __builtin_amdgcn_sched_barrier(0);  // all eight requested before the first is waited for
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
+                    const int m = 2 * (j0 + j) + half, hh = c * 16 + (m >> 3) * 4 + (m & 3);
+                    if (hh >= heads) v[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                     low |= low_half_bits(v[j]);
                     const u32x2 p = {upper_halves(v[j].x, v[j].y), upper_halves(v[j].z, v[j].w)};
                     *reinterpret_cast<u32x2*>(mine + (2 * (j0 + j) + half) * kPairRow + row * 8) = p;
@@ -473,18 +537,17 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
         f = span_max(f, __shfl_xor(f, 4, kWave));
         if (kp == 0) kv_spans[tile & 1][kr] = span_of(f);
     };
-    const int tiles = all_groups * 2;
     request(0);
     __syncthreads();  // every wave's q rows are out of the stage
     park(0);
-    unsigned long long inexact = 0;  // one bit per 64-block group
+    unsigned long long inexact[2] = {0, 0};  // one bit per tile
     const int t = tw + half;
     for (int tile = 0; tile < tiles; ++tile) {
         __syncthreads();  // this tile is parked and nobody reads the other buffer any more
         if (tile + 1 < tiles) request(tile + 1);
-        if ((tile >> 1) < my_groups) {
+        if (tile < my_tiles) {
             if (__any(kv_spans[tile & 1][row] + q_span > kExactSpan)) {
-                inexact |= 1ull << (tile >> 1);
+                inexact[tile >> 6] |= 1ull << (tile & 63);
             } else {
                 const unsigned char* const from = stage + ((tile & 1) * kPairTile + row) * kPairRow + half * 16;
                 bf16x8 b[8];
@@ -512,31 +575,42 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
                     }
                 }
                 const int c = c0 + tile * kPairTile + row;
-                const int cw = c & ~63;
-                if (c < n_comp && t < s && (ratio <= 0 || (cw + 1) * (long long)ratio - 1 <= t))
+                if (c < n_comp && may_rank(t, c))
                     score[(size_t)t * n_comp + c] = round_bf16(acc);
             }
         }
         if (tile + 1 < tiles) park(tile + 1);
     }
-    // what is left, term by term: a lane owns a block of the 64
-    while (inexact) {
-        const int g = __builtin_ctzll(inexact);
-        inexact &= inexact - 1;
-        const long long cw = (long long)c0 + g * 64, c = cw + lane;
-        const int t1 = min(s, tw + 2), t0 = first_query(tw, t1, ratio, cw);
-        float row_v[128];
-        load_row(row_v, kv + (size_t)(c < n_comp ? c : n_comp - 1) * 128);
-        float acc = 0.0f;
-        int hh = 0, tt = t0;
-        walk_pairs(q, w, row_v, (size_t)t0 * heads, (size_t)t1 * heads, [&](size_t, float term) {
-            acc = acc + term;
-            if (++hh == heads) {
-                if (c < n_comp) score[(size_t)tt * n_comp + c] = round_bf16(acc);
-                acc = 0.0f, hh = 0, ++tt;
+    // What is left, term by term: a lane owns a block of a 64-block group for both of the wave's
+    // queries, or where only one of the group's tiles is left a block of that for one of them.
+    const auto fold = [&](auto shared) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            while (inexact[k]) {
+                const int bit = __builtin_ctzll(inexact[k]);
+                const bool both = !(bit & 1) && (inexact[k] >> bit & 2);
+                inexact[k] &= ~((both ? 3ull : 1ull) << bit);
+                const int c = c0 + (64 * k + bit) * kPairTile + (both ? lane : row);
+                float row_v[128];
+                load_row(row_v, kv + (size_t)min(c, n_comp - 1) * 128);
+                const int first = both ? tw : tw + half;
+                const size_t at = (size_t)min(first, s - 1) * heads;
+                // (both sums first, then the stores: 8 192 x 2 048 3 475 -> 3 425 us)
+                float sum = 0.0f, acc = 0.0f;
+                fold_heads<shared>(q + at * 128, w + at, both ? min(2, s - tw) * heads : heads, row_v, [&](int i, float term) {
+                    acc = acc + term;
+                    if (i + 1 == heads) sum = acc, acc = 0.0f;
+                });
+                if (c < n_comp && may_rank(first, c)) score[(size_t)first * n_comp + c] = round_bf16(sum);
+                if (c < n_comp && both && may_rank(tw + 1, c)) score[(size_t)(tw + 1) * n_comp + c] = round_bf16(acc);
             }
-        });
-    }
+        }
+    };
+    // (a prefill's grid has a third and more workgroups without a legal block)
+    if (gridDim.x * gridDim.y <= (ratio > 0 ? 384u : 256u))
+        fold(std::false_type{});
+    else
+        fold(std::true_type{});
 }
 
 // Few queries (a decode step: one). A workgroup owns one query's 64 heads against 32 HT blocks, a
@@ -630,12 +704,18 @@ __global__ __launch_bounds__(kOneThreads) void score_blocks_one_kernel(
         }
     }
     __syncthreads();
-    if (inexact) {  // term by term: every wave a quarter of the heads for all blocks (32 of them: twice, the same values)
+    if (inexact) {  // term by term: every wave a quarter of the heads
         const int per = (heads + 3) / 4, g0 = min(wave * per, heads), g1 = min(g0 + per, heads);
         float row_v[128];
         load_row(row_v, kv + (size_t)(c < n_comp ? c : n_comp - 1) * 128);
-        walk_pairs(q, w, row_v, base + g0, base + g1,
-                   [&](size_t h, float term) { terms[h - base][lane & (BLOCKS - 1)] = term; });
+        if constexpr (HT == 1) {  // each half of the wave half of those (of an odd number the middle one twice)
+            const int n = (g1 - g0 + 1) / 2, first = lane < 32 ? g0 : g1 - n;
+            if (n > 0)
+                fold_heads<false>(q + (base + first) * 128, w + base + first, n, row_v,
+                                  [&](int i, float term) { terms[first + i][lane & (BLOCKS - 1)] = term; });
+        } else {
+            walk_pairs(q, w, row_v, base + g0, base + g1, [&](size_t h, float term) { terms[h - base][lane] = term; });
+        }
         __syncthreads();
     }
     if (threadIdx.x < BLOCKS) {
@@ -732,9 +812,15 @@ static int score_blocks_launch(const float* q, const float* kv, const float* w, 
         // two workgroups per compute unit at a time; splits of the blocks while the queries alone
         // give fewer than two rounds of those (a split reads its queries' rows again)
         const unsigned t_groups = (unsigned)(((long long)s + kPairQueries - 1) / kPairQueries);
+        const long long tiles = ((long long)n_comp + kPairTile - 1) / kPairTile;
         long long splits = t_groups >= 1024 ? 1 : 1024 / t_groups;
         if (splits > groups) splits = groups;
         int per = (int)((groups + splits - 1) / splits) * 64;
+        // A tile each where that leaves compute units over, or is still one round and the q rows (32 KB
+        // a query) stay in a die's 4 MB of cache, which every one of a query's workgroups reads them
+        // through: 300 x 75 (114 workgroups) 11.7 -> 10.5 us, 5 x 8 192 (256) 10.1 -> 8.8; but 150 x 300 (190,
+        // 4.9 MB) 10.1 -> 11.9.
+        if (t_groups * tiles <= 128 || (t_groups * tiles <= 256 && t_groups <= 13)) per = kPairTile;
         if (per > kPairSplitMax) per = kPairSplitMax;
         const unsigned y = (unsigned)(((long long)n_comp + per - 1) / per);
         if (y <= 65535u) {

@@ -285,6 +285,31 @@ def test_score_of_rows_whose_sums_are_exact_up_to_the_last_span_and_past_it(orac
         assert np.array_equal(part[live], want.view(np.uint32)[live]) and (part[~live] == 0x5A5A5A5A).all(), change
 
 
+@pytest.mark.parametrize("s,n_comp,heads,ratio", [(113, 300, 64, 0), (113, 300, 5, 4), (8185, 2100, 3, 0), (8185, 2100, 2, 4)])
+def test_score_where_single_tiles_of_a_group_are_folded_and_past_64_tiles_of_a_split(oracle, s, n_comp, heads, ratio):
+    """Blocks that only the fold gets right in the upper 32 of a group of 64, in the lower, in both and
+    in none: a wave folds whole groups for its two queries and single tiles a half for each. 8 185
+    queries by 2 100 blocks walk 66 tiles in one workgroup. Bit for bit on sampled queries."""
+    rng = np.random.default_rng(s + n_comp + heads)
+    q = few_bit_rows(rng, s * heads, 3).reshape(s, heads, 128)
+    kv = few_bit_rows(rng, n_comp, 4)
+    for c in (40, 64 + 3, 128 + 1, 160 + 1, 299, 2060, 2099):
+        if c < n_comp:
+            kv[c] = rng.standard_normal(128).astype(np.float32)
+    w = bf16_round((rng.standard_normal((s, heads)) * 0.1).astype(np.float32))
+    out = dzeros(s * n_comp * 4, 0x5A)
+    if ratio:
+        hip.launch_index_score_blocks_prefill(dev(q), dev(kv), dev(w), out, s, n_comp, heads, 128, ratio)
+    else:
+        hip.launch_index_score_blocks(dev(q), dev(kv), dev(w), out, s, n_comp, heads, 128)
+    got = back(out, np.uint32).reshape(s, n_comp)
+    for t in (0, 1, 7, 8, s // 2, s // 2 + 1, s - 2, s - 1):
+        code, want = oracle.index_score_blocks(q[t:t + 1], kv, w[t:t + 1])
+        live = (np.arange(n_comp) // 64) * 64 < (min((t + 1) // ratio, n_comp) if ratio else n_comp)
+        assert code == 0 and np.array_equal(got[t][live], want[0].view(np.uint32)[live]), t
+        assert (got[t][~live] == 0x5A5A5A5A).all(), t
+
+
 @pytest.mark.parametrize("s,n_comp", [(1, 70), (9, 3100)])
 @pytest.mark.parametrize("exponent", [59, 60, -59, -60])
 def test_score_at_the_largest_and_smallest_exponents_whose_sums_are_exact(oracle, s, n_comp, exponent):
