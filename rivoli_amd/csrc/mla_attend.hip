@@ -1081,8 +1081,6 @@ extern "C" int rivoli_mla_attend_paged(const float* qabs, const float* qrope,
 // 16 * H * (kvl + 2) floats) holds as many 512-wide partial records as fit it.
 // ---------------------------------------------------------------------------------------------
 namespace rk {
-constexpr int kRefMaxSplits = 16;  // what rivoli_mla_attend_scratch_floats prices (attn.hip:66,98-103)
-
 // Shapes the tile kernel does not take (a roped key wider than 64, slabs that are not 8-byte
 // aligned): a wave per head walks the rows one at a time, lanes over the dims, online softmax.
 __global__ __launch_bounds__(256) void mla_attend_rowwise_kernel(
@@ -1148,13 +1146,7 @@ extern "C" int rivoli_mla_attend(const float* qabs, const float* qrope, const un
                            qrope, Lc8, Lscale, Rc, rows, H, nr, kvl, rope, n_blocks, scale * kLog2e, clat);
         return launch_status();
     }
-    // split plan: as the batched launcher's for one sequence, capped by what the scratch holds
-    AttendPlan plan = attend_plan(1, H, nr);
-    const int fit = (int)((size_t)kRefMaxSplits * ((size_t)kvl + 2) / (kKvl + 2)) - 1;  // records - 1
-    if (plan.n_splits > fit) plan.n_splits = fit;
-    if (!partial || plan.n_splits < 2) plan.n_splits = 1;
-    plan.n_items = plan.n_splits > 1 ? plan.n_splits : 0;
-    plan.n_records = plan.n_items ? plan.n_items + 1 : 0;
+    const AttendPlan plan = linear_plan(H, nr, (int)((size_t)kRefMaxSplits * ((size_t)kvl + 2) / (kKvl + 2)), partial != nullptr);
     AttendArgs a = {};
     a.qabs = qabs, a.qrope = qrope, a.rows = rows, a.k = nr, a.H = H;
     a.lc8 = Lc8, a.lscale = Lscale, a.rc = Rc, a.n_blocks = n_blocks;

@@ -10,6 +10,7 @@ constexpr int kAttTargetGroups = 256;      // one workgroup per CU of a 256-CU p
 constexpr int kAttDies = 8;                // workgroups are dealt to the dies in turn
 constexpr int kAttMinTilesPerSplit = 8;    // below 256 rows a split costs more than it buys
 constexpr int kAttMaxSplits = 64;
+constexpr int kRefMaxSplits = 16;          // what rivoli_mla_attend_scratch_floats prices (attn.hip:66,98-103)
 constexpr int kDealMaxSeqs = 1024;         // dealing keeps a prefix sum over the sequences in LDS
 constexpr int kH16Heads = 16;              // mla_attend_heads16.hpp: heads and waves of a workgroup
 constexpr int kH16Waves = 4;
@@ -40,6 +41,17 @@ static inline AttendPlan attend_plan(int n_seqs, int H, int max_rows) {
     p.n_splits = n;
     p.n_items = n > 1 ? n * n_seqs : 0;
     p.n_records = n > 1 ? p.n_items + n_seqs : 0;
+    return p;
+}
+
+// The same for the linear slabs' one sequence, cut to what the caller's scratch holds: `fit` records of
+// which one is spare.
+static inline AttendPlan linear_plan(int H, int nr, int fit, bool scratch) {
+    AttendPlan p = attend_plan(1, H, nr);
+    if (p.n_splits > fit - 1) p.n_splits = fit - 1;
+    if (!scratch || p.n_splits < 2) p.n_splits = 1;
+    p.n_items = p.n_splits > 1 ? p.n_splits : 0;
+    p.n_records = p.n_items ? p.n_items + 1 : 0;
     return p;
 }
 
@@ -128,6 +140,13 @@ static inline bool heads16_whole_pays(const AttendPlan& plan, int n_seqs, int H,
     if (rounds <= (n_seqs * blocks + kAttTargetGroups - 1) / kAttTargetGroups) return true;
     return !f8 && rounds == 2 && tiles >= kH16TwoRoundTiles && (tiles <= kH16TwoRoundMaxTiles || spills);
 }
+// The head groups of a work item are a die's 32 units at most, or the item takes rounds of its own: past
+// 512 heads calls stay with the other kernel (2 048 heads, parity mode, 1 024 listed rows 92 us here
+// against 44; 768 dense, 1 638 rows 44 against 40, precise 3, 857 rows 43 against 31; 520 with two
+// sequences listed 34 against 40). The general form of the linear slabs is slower than that kernel: 1 024
+// heads 512 rows 36 us here against 53, 2 048 rows 53 against 60, 4 096 rows 82 against 68; 1 536 heads 1 024
+// rows 75 against 59, 2 048 heads 2 048 rows 153 against 67.
+constexpr int kH16ManyHeadsTiles = 64;  // linear slabs, up to two rounds of head groups
 // `cut`: heads16_plan shares the sequences among work items.
 static inline bool heads16_pays(const AttendPlan& plan, bool cut, int n_seqs, int H, int max_rows, int precise,
                                 bool dense, bool linear) {
@@ -136,14 +155,15 @@ static inline bool heads16_pays(const AttendPlan& plan, bool cut, int n_seqs, in
     const long long work = (long long)n_seqs * tiles * groups;
     const bool f8 = precise > 2;
     if (!cut && !heads16_whole_pays(plan, n_seqs, H, tiles, f8, dense, linear)) return false;
+    if (groups > kAttDieUnits && !(linear && groups <= 2 * kAttDieUnits && tiles <= kH16ManyHeadsTiles)) return false;
     if (groups == 1 || work <= (f8 ? kH16MaxWork8Bit : kH16MaxWork)) return true;
     if (!dense || 5 * n_seqs * groups > 2 * kAttTargetGroups) return false;
     const bool spills = (long long)plan.n_items * ((H + 63) / 64) > kAttTargetGroups;
     return work <= (spills ? (f8 ? kH16MaxWorkSpill8Bit : kH16MaxWorkSpill) : (f8 ? kH16MaxWorkFull8Bit : kH16MaxWorkFull));
 }
 
-// A call of the shipped row widths whose rows are whole 16-byte pieces. `plan`: attend_plan's, or
-// the linear launcher's cut of it.
+// A call of the shipped row widths whose rows are whole 16-byte pieces. `plan`: attend_plan's or
+// linear_plan's.
 struct AttendRoute {
     bool heads16;  // workgroups of 16 heads; else of 64
     bool by_seq;   // no work item has tiles of two sequences (SeqDeal)

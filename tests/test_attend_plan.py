@@ -61,6 +61,23 @@ def test_no_batch_of_long_sequences_is_left_whole(precise):
                     (H, n, rows)
 
 
+def test_calls_of_more_head_groups_than_a_die_has_units_stay_with_the_other_kernel():
+    """Past 512 heads the groups of one work item are more than the 32 units of the die they sit on: a
+    call of 2 048 heads took twice its time so. The linear slabs' other kernel is slow enough for two
+    rounds of them over few rows."""
+    for rows in (64, 512, 1024, 2048, 4096, 40000):
+        for n in (1, 2, 7):
+            for precise in (0, 2, 4):
+                for listed in (False, True):
+                    assert not any(attend_route(n, H, rows, precise, listed).heads16 for H in (513, 768, 1024, 2048, 8192))
+        for linear in (1, 2):
+            assert not any(attend_route(1, H, rows, 2, linear=linear).heads16 for H in (1025, 1536, 2048, 8192))
+    for H in (520, 768, 1024):
+        assert all(attend_route(1, H, rows, 2, linear=1).heads16 for rows in (512, 1024, 2048))
+        assert not attend_route(1, H, 2049, 2, linear=1).heads16
+    assert attend_route(1, 512, 2048, 2).heads16 and attend_route(1, 512, 2048, 4, listed=True).heads16
+
+
 @pytest.mark.parametrize("r_end", [1, 33, 2 ** 20, 2 ** 31 - 400, 2 ** 31 - 32])
 def test_list_positions_looked_up_ahead_stay_in_the_list(r_end):
     """Host-side restatement of token_of in mla_attend_heads16.hpp: which list entries a wave asks for

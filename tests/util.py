@@ -46,15 +46,15 @@ def slots_for(table_row, positions, page_tokens=64):
 
 
 class AttendRoute:
-    """attend_route of rivoli_amd/csrc/mla_attend_plan.hpp: which workgroups a paged call of the
-    shipped row widths takes, and its work items."""
+    """attend_route of rivoli_amd/csrc/mla_attend_plan.hpp: which workgroups a call of the shipped row
+    widths takes, and its work items. `linear`: over the linear slabs, 1 with scratch, 2 without."""
 
     def __init__(self, heads16, out):
         self.heads16 = bool(heads16)
         self.items, self.by_seq, self.records, self.scratch_items, self.scratch_records = list(out)
 
 
-def attend_route(n_seqs, H, max_rows, precise, listed=False):
+def attend_route(n_seqs, H, max_rows, precise, listed=False, linear=0):
     global _PLAN
     if _PLAN is None:
         here = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native")
@@ -63,7 +63,7 @@ def attend_route(n_seqs, H, max_rows, precise, listed=False):
             subprocess.run(["make", "-C", here, path], check=True, capture_output=True)
         _PLAN = ctypes.CDLL(path)
     out = (ctypes.c_int * 5)()
-    return AttendRoute(_PLAN.attend_route(n_seqs, H, max_rows, precise, int(listed), out), out)
+    return AttendRoute(_PLAN.attend_route(n_seqs, H, max_rows, precise, int(listed), linear, out), out)
 
 
 _PLAN = None
