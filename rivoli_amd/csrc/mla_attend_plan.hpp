@@ -111,6 +111,9 @@ constexpr long long kH16MaxWork = 8192, kH16MaxWork8Bit = 4096;
 // against 69, 18 x 10 262 (23 112) 107 against 102. Calls that those workgroups fill in one round
 // change sides sooner: 8 x 11 058 (11 072) 49 against 52, 4 x 32 768 (16 384) 74 against 71; precise
 // 4: 1 x 32 768 (4 096) 43 against 51, 4 x 32 768 70 against 59.
+// Neither line holds for the linear slabs: their other kernel is the general form of the 64-head one and
+// their scratch gives it 15 work items. 64 heads: 512 rows 19 us against 50, 65 536 rows 139 against 484,
+// 200 000 rows 385 against 1 420; 512 heads, 20 000 rows 92 against 172.
 constexpr long long kH16MaxWorkFull = 12288, kH16MaxWorkFull8Bit = 8192;
 constexpr long long kH16MaxWorkSpill = 24576, kH16MaxWorkSpill8Bit = 16384;
 // Calls whose sequences stay whole (one workgroup a sequence and head group) go there while that
@@ -156,7 +159,7 @@ static inline bool heads16_pays(const AttendPlan& plan, bool cut, int n_seqs, in
     const bool f8 = precise > 2;
     if (!cut && !heads16_whole_pays(plan, n_seqs, H, tiles, f8, dense, linear)) return false;
     if (groups > kAttDieUnits && !(linear && groups <= 2 * kAttDieUnits && tiles <= kH16ManyHeadsTiles)) return false;
-    if (groups == 1 || work <= (f8 ? kH16MaxWork8Bit : kH16MaxWork)) return true;
+    if (linear || groups == 1 || work <= (f8 ? kH16MaxWork8Bit : kH16MaxWork)) return true;
     if (!dense || 5 * n_seqs * groups > 2 * kAttTargetGroups) return false;
     const bool spills = (long long)plan.n_items * ((H + 63) / 64) > kAttTargetGroups;
     return work <= (spills ? (f8 ? kH16MaxWorkSpill8Bit : kH16MaxWorkSpill) : (f8 ? kH16MaxWorkFull8Bit : kH16MaxWorkFull));

@@ -75,6 +75,9 @@ def test_calls_of_more_head_groups_than_a_die_has_units_stay_with_the_other_kern
     for H in (520, 768, 1024):
         assert all(attend_route(1, H, rows, 2, linear=1).heads16 for rows in (512, 1024, 2048))
         assert not attend_route(1, H, 2049, 2, linear=1).heads16
+    for linear in (1, 2):                   # ... and for any number of rows where the groups fit
+        assert all(attend_route(1, H, rows, 2, linear=linear).heads16
+                   for H in (1, 17, 64, 128, 512) for rows in (1, 300, 20000, 65537, 2 ** 24))
     assert attend_route(1, 512, 2048, 2).heads16 and attend_route(1, 512, 2048, 4, listed=True).heads16
 
 

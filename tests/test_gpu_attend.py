@@ -499,6 +499,24 @@ def test_linear_row_lists_and_code_slabs_on_an_8_byte_boundary(oracle, h, nt, nr
             check_linear(got, want, f"rows={r is not None} scratch={scratch}")
 
 
+@pytest.mark.parametrize("scratch", [True, False])
+def test_linear_rows_past_the_lines_of_the_paged_calls(oracle, scratch):
+    """131 100 rows at 17 heads (8 194 tiles times groups of 16 heads): the linear slabs know no line.
+    Against float64, a token's weight times how often the list names it: the oracle adds 131 100 terms
+    in f32, one after the other, and is off by 8.3e-7 here, 1.3e-4 of the largest output."""
+    from tests.attend_cases import reference_attend_case, widen_linear
+
+    h, nt, nr = 17, 500, 131100
+    assert -(-nr // 32) * 2 > 8192 and attend_route(1, h, nr, 2, linear=1).heads16 and attend_route(1, h, nr, 2, linear=2).heads16
+    case = reference_attend_case(oracle, 0x5200, h, nt, KVL, ROPE)
+    rows = np.random.default_rng(17).integers(0, nt, nr).astype(np.uint32)
+    lat, rk = (x.astype(np.float64) for x in widen_linear(oracle, *case[2:5], nt, KVL, ROPE, case[5]))
+    logit = (case[0].astype(np.float64) @ lat.T + case[1].astype(np.float64) @ rk.T) * case[6]
+    p = np.exp(logit - logit.max(axis=1, keepdims=True)) * np.bincount(rows, minlength=nt)
+    want = (p / p.sum(axis=1, keepdims=True)) @ lat
+    check_linear(run_linear(case, h, nt, KVL, ROPE, rows=rows, scratch=scratch), want, f"scratch={scratch}")
+
+
 @pytest.mark.parametrize("n_seqs,H", [(3, 64), (24, 128)])
 @pytest.mark.parametrize("precise", [2, 1, 0, 4, 3])
 def test_list_entries_of_all_ones_are_left_out(oracle, precise, n_seqs, H):
