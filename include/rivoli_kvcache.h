@@ -289,9 +289,9 @@ int rivoli_index_append_paged(const float* k, const int* slot_mapping, unsigned 
  * cache codes going into them untouched and q / the weights as sums of e4m3 terms under
  * power-of-two block scales: 3 = two terms each (the accuracy class of 0), 4 = three terms for
  * q and two for the weights (the class of 1; inside the reference's bar on the test caches).
- * They are the fastest modes for large calls: about 30 % less time per launch than 0 / 2. Calls
- * whose 32-token tiles times groups of 16 heads number 4096 or fewer (up to 16384 for dense calls of
- * few sequences), and calls of up to 16 heads, run as 2 instead, which is faster there.
+ * They are the fastest modes for large calls: about 30 % less time per launch than 0 / 2. Most calls
+ * of up to 512 heads whose 32-token tiles times groups of 16 heads number 4096 or fewer (up to 16384
+ * for dense calls of few sequences), and of up to 16 heads, run as 2 instead, which is faster there.
  * Other row widths (kvl a multiple of 128 up to 512, rope a multiple of 8 up to 64) always run
  * as 2.
  * Guards: 1001 null / non-positive, or a null `partial` when scratch is needed; 1002
@@ -339,8 +339,9 @@ int rivoli_act_quant_f4_rotated(float* x, int rows, int d, void* stream);
  * dot is a sequential f32 fold of separately rounded products and the head sum a sequential
  * f32 fold rounded once, exactly as the reference's kernel, so the result is bit-identical
  * to it. hd = 128 (the shipped width) with a 16-byte-aligned kv takes the register-resident
- * kernels (one for prefill-sized calls, one that splits the heads of a decode step's single
- * query over a workgroup's waves); any other width a slower one. Guards as the reference's: 1001 non-positive s, heads
+ * kernels; up to 64 heads, those run rows whose sums are exact in any order (what
+ * rivoli_act_quant_f4_rotated makes) on the matrix cores, the same bits some 15 times as fast. Any other
+ * width takes a slower one. Guards as the reference's: 1001 non-positive s, heads
  * or hd (also null pointers); 1005 n_comp <= 0 (no block has completed: the caller must not
  * rank an unwritten buffer). */
 int rivoli_index_score_blocks(const float* q, const float* kv, const float* w, float* score,

@@ -18,9 +18,9 @@
 // was bound by (16 heads use a tile a quarter as often as 64 do).
 // Measured, parity mode, 64 heads, with the merge of the records: one sequence of 4 096 tokens
 // 34.5 -> 21 us, 8 x 2 048 listed rows 38 -> 24 us, one token over 2 048 rows of the linear slabs
-// 52 -> 20.7 us. What a pass takes (27 000 cycles for two tiles a wave): 6 000 until the first
-// rows are asked for and the query is in, 6 000 a tile (136 matrix instructions 2 200, ~700 vector
-// instructions 2 800, 19 transfers 1 400: a wave's instructions add up), 6 500 the merge.
+// 52 -> 20.7 us. A wave of two listed tiles lives 39 500 cycles, by counter: matrix instructions (272)
+// 4 350, vector instructions 11 700, waits 17 100 (the first rows, the merge), the rest transfers, LDS and
+// scalar instructions.
 #pragma once
 
 namespace rk {
