@@ -127,15 +127,19 @@ constexpr long long kH16MaxWorkSpill = 24576, kH16MaxWorkSpill8Bit = 16384;
 // than a round themselves (32 heads, 136 x 960 tokens 67 against 93). One tile, two of up to 16
 // heads and two dense ones of up to 32 leave half the waves and more without any: 16 heads, 32 tokens
 // 11 us against 8, 64 tokens 11.0 against 10.0; 64 heads, one token 12.7 against 10.8, 32 tokens 11.0
-// against 11.0. (The 8-bit kernel is not faster there, 12 us against 16, nor is the general form of
-// the linear slabs, 10.9 against 24.8.) Past 32 tiles the call lasts as long as its longest sequence
+// against 11.0. Three tiles of more than a round of sequences are worth it where all are as long, and not
+// in a ragged batch (8 heads, 257 sequences, even 20 against 23, lengths to 96 from 3 on 21 against 18, one
+// of 96 among 6s 21 against 14; four tiles 20 against 28, 22 against 20 and 21 against 14; in one round 11
+// against 13, 12.4 against 12.3 and 12.2 against 11.8). (The 8-bit kernel is not faster there, 12 us
+// against 16, nor is the general form of the linear slabs, 10.9 against 24.8.) Past 32 tiles the call lasts as long as its longest sequence
 // in one workgroup, and the other kernel deals them out: 64 heads, 33 x 1 984 tokens 60 us against 46,
 // one of 1 984 among 32 of 100 58 against 36; unless its splits, again, are more than a round (32
 // heads, 80 x 1 600 tokens 50 against 80).
 constexpr int kH16TwoRoundTiles = 15, kH16TwoRoundMaxTiles = 20;
 static inline bool heads16_whole_pays(const AttendPlan& plan, int n_seqs, int H, int tiles, bool f8, bool dense,
                                       bool linear) {
-    if (!f8 && !linear && tiles <= (H <= 16 || (dense && H <= 32) ? 2 : 1)) return false;
+    const int few = H <= 16 && n_seqs > kAttTargetGroups ? 3 : H <= 16 || (dense && H <= 32) ? 2 : 1;
+    if (!f8 && !linear && tiles <= few) return false;
     const long long blocks = (H + 63) / 64;
     const bool spills = plan.n_items * blocks > kAttTargetGroups;
     if (!linear && H > kH16Heads && tiles > kH16WholeTiles) return spills;

@@ -44,6 +44,9 @@ def test_batches_of_short_sequences_keep_to_the_kernel_of_fewer_rounds(precise):
     for H, rows in ((16, 1), (16, 64), (32, 33), (64, 1), (128, 32)):
         assert attend_route(4, H, rows, precise).heads16 == (precise == 4), (H, rows)
     assert attend_route(4, 32, 64, 2, listed=True).heads16 and attend_route(4, 64, 64, 2).heads16
+    # three tiles of a second round of few-head sequences: the other's where most are shorter than that
+    for n, rows, there in ((256, 96, True), (257, 96, False), (257, 97, True), (1000, 65, False), (1000, 128, True)):
+        assert attend_route(n, 16, rows, precise).heads16 == (there or precise == 4), (n, rows)
 
 
 @pytest.mark.parametrize("precise", [0, 2])
