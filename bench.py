@@ -660,17 +660,14 @@ def bench_v4_index(a, torch, hip):
            "tokens_per_s": round(s / (ms * 1e-3), 1),
            "kernels": {"f4_rotated_kernel": {"avg_launch_ms": round(per["spread"], 5), "bytes_per_launch": spread_bytes,
                                              "GBps": round(spread_bytes / (per["spread"] * 1e-3) / 1e9, 1)},
-                       "index_score_blocks_kernel": {"avg_launch_ms": round(per["score"], 5),
+                       "score_blocks_pair_kernel": {"avg_launch_ms": round(per["score"], 5),
                                                      "flops_per_launch": score_flops, "bytes_per_launch": score_bytes,
                                                      "TFLOPps": round(score_flops / (per["score"] * 1e-3) / 1e12, 2)}},
-           # the scorer is bound by vector issue, not by memory or the matrix cores: the published
-           # fp32 vector peak counts a fused multiply-add on packed pairs as four operations per lane
-           # and cycle; the reference's two roundings per term allow one
-           "roofline": {"bound": "fp32", "kernel": "index_score_blocks_kernel",
-                        "achieved": round(score_flops / (per["score"] * 1e-3) / 1e12, 2), "peak": 157.3,
-                        "unit": "TFLOP/s", "frac": round(score_flops / (per["score"] * 1e-3) / 157.3e12, 4),
-                        "unfused_unpacked_peak": 39.3,
-                        "frac_of_unfused_unpacked_peak": round(score_flops / (per["score"] * 1e-3) / 39.3e12, 4),
+           # rows whose sums are exact in any order, which spread rows are, go through the bf16 matrix
+           # instructions; issue of the reference's roundings, five vector instructions a dot, is the larger half
+           "roofline": {"bound": "mfma", "kernel": "score_blocks_pair_kernel",
+                        "achieved": round(score_flops / (per["score"] * 1e-3) / 1e12, 2), "peak": 2500.0,
+                        "unit": "TFLOP/s", "frac": round(score_flops / (per["score"] * 1e-3) / 2.5e15, 4),
                         "avg_launch_ms": round(per["score"], 5), "traffic": None}}
     # a decode step of the same layer: one query against the ctx / ratio blocks of a long context
     d_comp = max(a.ctx // ratio, 1)
@@ -933,7 +930,10 @@ def bench_dsa(a, torch, hip, scored=False, attend=False):
            "layer_us": round(ms * 1e3 / L, 2), "hbm_peak_frac": round(L * layer_bytes / (ms * 1e-3) / HBM_PEAK, 4),
            "kernels_ms": {n: round(v, 5) for n, v in per.items()},
            "roofline": {"bound": "hbm",
-                        "kernel": "mla_attend_paged_kernel" if attend else
+                        # (short calls run in workgroups of 16 heads: rivoli_amd/csrc/mla_attend_plan.hpp)
+                        "kernel": ("mla_attend_heads16_kernel"
+                                   if B * -(-k // 32) * -(-H // 16) <= (4096 if a.precise > 2 else 8192)
+                                   else "mla_attend_paged_kernel") if attend else
                                   ("topk_hist + topk_cand + topk_finish_bits (select and gather)" if fused
                                    else "kv_gather_rows_kernel"),
                         "achieved": round(dom_bytes / (per[rows_kernel] * 1e-3) / 1e9, 2),
