@@ -174,3 +174,27 @@ def test_workgroup_sizes_by_the_call(oracle, n_q, top):
     live = np.arange(top)[None, :] < lens[:, None]
     assert rel(got[live], want[live]) < TOL
     assert (got.view(np.uint32)[~live] == 0x7F7F7F7F).all()
+
+
+@pytest.mark.parametrize("nact,hd", [(1, 128), (16, 128), (17, 128), (33, 128), (64, 128), (32, 64), (49, 48), (8, 16)])
+def test_head_lists_where_the_query_goes_ahead_of_the_keys(oracle, nact, hd):
+    """520 queries are more than a round of workgroups: the query's rows are staged before the first
+    keys are asked for, and steps of the staging without a head that counts are left out."""
+    n_q, top, nh, pt = 520, 140, 64, 32
+    rng = np.random.default_rng(nact * 1000 + hd)
+    blocks = -(-top // pt)
+    tables = rng.permutation(n_q * blocks).astype(np.int32).reshape(n_q, blocks)
+    lens = rng.integers(0, top + 1, n_q).astype(np.int32)
+    lens[:6] = [top, 0, 127, 128, 129, 1]
+    q = rng.standard_normal((n_q, nh, hd), dtype=np.float32)
+    w = rng.standard_normal((n_q, nh), dtype=np.float32)
+    heads = rng.permutation(nh)[:nact].astype(np.uint32)
+    kpool = oracle.f32_to_bf16(rng.standard_normal((n_q * blocks * pt, hd), dtype=np.float32))
+    want = oracle.index_score_paged(q, w, kpool, tables, lens, heads, top, hd, pt, 0.5, 0.25, n_threads=4)
+    out = dzeros(n_q * top * 4, 0x7F)
+    hip.launch_index_score_paged(dev(q), dev(w), dev(kpool), dev(tables), dev(lens), dev(heads), n_q, blocks, top, top,
+                                 nh, nact, hd, pt, n_q * blocks, 0.5, 0.25, out)
+    got = back(out, np.float32).reshape(n_q, top)
+    live = np.arange(top)[None, :] < lens[:, None]
+    assert rel(got[live], want[live]) < TOL
+    assert (got.view(np.uint32)[~live] == 0x7F7F7F7F).all()
