@@ -27,6 +27,8 @@
 // LDS tiles rotate so one barrier per tile suffices. Other widths (and rows that must not be
 // rounded to bf16) take an f32 kernel: a wave per (query, head), lanes over the dims, one
 // online-softmax pass over the list.
+// Calls of more than 256 such workgroups take another kernel, 32 heads a wave (gather_attn_wide.hpp), and this
+// one the queries that it leaves.
 // Launch-only; see include/rivoli_kvcache.h for the contract.
 #include "attend_common.hpp"
 
@@ -91,17 +93,21 @@ static inline int gather_attn_splits(int m, int h, int topk) {
     return n < 2 ? 1 : (int)n;
 }
 
+}  // namespace rk
+
+#include "gather_attn_wide.hpp"
+
+namespace rk {
+
+// One query's block of 64 heads (and share of its list), by the whole workgroup.
 template <int QSPLIT, int PSPLIT>
-__global__ __launch_bounds__(kGaThreads) void gather_attn_d512_kernel(const GatherAttnArgs a) {
+__device__ __forceinline__ void gather_attn_d512(const GatherAttnArgs& a, uint8_t* smem, size_t t, int hb, int split) {
     constexpr int kFragBlock = QSPLIT == 2 ? 2 : 4;   // score side, K-steps requested together
     constexpr int kValueAhead = QSPLIT == 2 ? 4 : 8;  // value side, fragments requested together
-    __shared__ __attribute__((aligned(16))) uint8_t smem[kGaSmemBytes];
     const lds_ptr<uint8_t> kr = (lds_ptr<uint8_t>)smem;                     // [kGaBufs] row-major tiles
     const lds_ptr<float> sbias = (lds_ptr<float>)(kr + kGaBufs * kGaTileBytes);  // [kGaBufs][32]: 0 or -inf
     const lds_ptr<f32x4> xch = (lds_ptr<f32x4>)(sbias + kGaBufs * kGaTile);  // [2 parities][8 waves][64 lanes][2]
 
-    const size_t t = blockIdx.x;
-    const int hb = blockIdx.y;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -109,7 +115,6 @@ __global__ __launch_bounds__(kGaThreads) void gather_attn_d512_kernel(const Gath
     const int half = wave >> 2;  // which half of the contraction dims / of the output columns
     const int g = lane >> 4, n16 = lane & 15;
     const int all_tiles = (a.topk + kGaTile - 1) / kGaTile;
-    const int split = blockIdx.z;
     const int tile0 = (int)((long long)split * all_tiles / a.n_splits);  // this workgroup's tiles
     const int n_tiles = (int)((long long)(split + 1) * all_tiles / a.n_splits) - tile0;
     const int* const ix = a.idxs + t * a.topk;
@@ -439,10 +444,11 @@ __global__ __launch_bounds__(kGaThreads) void gather_attn_d512_kernel(const Gath
         // nothing live: m_ref is still -inf and the query's output is NaN
         l_sum = m_ref == -INFINITY ? NAN : l_sum + exp2f(sk * kLog2e - m_ref);
     }
-    // the lane's accumulators are heads 4g+i; their denominators live in lanes with n16 == 4g+i
-    float l_h[4];
+    // The lane's accumulators are heads 4g+i; their denominators live in lanes with n16 == 4g+i. One division a head
+    // (64 quotients a lane were 3 % of a query): a product's error is far below the bf16 rounding that follows.
+    float l_inv[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) l_h[i] = __shfl(l_sum, 4 * g + i, kWave);
+    for (int i = 0; i < 4; ++i) l_inv[i] = 1.0f / __shfl(l_sum, 4 * g + i, kWave);
     const int head0 = hb * 64 + 16 * hw;
     const int col0 = half * (kGaD / 2) + n16;
 #pragma unroll
@@ -452,7 +458,44 @@ __global__ __launch_bounds__(kGaThreads) void gather_attn_d512_kernel(const Gath
             float* const dst = a.o + (t * a.h + head) * kGaD;
 #pragma unroll
             for (int nt = 0; nt < kGaColTilesHalf; ++nt)
-                dst[col0 + 16 * nt] = (float)(__bf16)(o[nt][i] / l_h[i]);
+                dst[col0 + 16 * nt] = (float)(__bf16)(o[nt][i] * l_inv[i]);
+        }
+    }
+}
+
+template <int QSPLIT, int PSPLIT>
+__global__ __launch_bounds__(kGaThreads) void gather_attn_d512_kernel(const GatherAttnArgs a) {
+    __shared__ __attribute__((aligned(16))) uint8_t smem[kGaSmemBytes];
+    gather_attn_d512<QSPLIT, PSPLIT>(a, smem, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// The blocks that the kernel of 32 heads a wave marked, one after another: a workgroup looks at 512 marks at a time,
+// which is all that it does when there are none (8192 queries: 3 us).
+template <int QSPLIT, int PSPLIT>
+__global__ __launch_bounds__(kGaThreads) void gather_attn_marked_kernel(const GatherAttnArgs a, long long blocks, int per_query) {
+    __shared__ __attribute__((aligned(16))) uint8_t smem[kGaSmemBytes];
+    __shared__ uint64_t marked[kGaWaves];
+    for (long long base = 0; base < blocks; base += (long long)gridDim.x * kGaThreads) {
+        const long long mine = base + (long long)threadIdx.x * gridDim.x + blockIdx.x;
+        bool is = false;
+        if (mine < blocks) {
+            const size_t t = mine / per_query;
+            const int hb = mine % per_query;
+            is = reinterpret_cast<const uint32_t*>(a.o)[(t * a.h + hb * 64) * kGaD] == kGwMark;
+        }
+        const uint64_t word = __builtin_amdgcn_ballot_w64(is);
+        __syncthreads();  // the words of the round before are read
+        if ((threadIdx.x & 63) == 0) marked[threadIdx.x >> 6] = word;
+        __syncthreads();
+        for (int w = 0; w < kGaWaves; ++w) {
+            uint64_t todo = marked[w];
+            while (todo != 0) {
+                const int bit = __builtin_ctzll(todo);
+                todo &= todo - 1;
+                const long long block = base + (long long)(64 * w + bit) * gridDim.x + blockIdx.x;
+                gather_attn_d512<QSPLIT, PSPLIT>(a, smem, block / per_query, (int)(block % per_query), 0);
+                __syncthreads();  // its LDS is read
+            }
         }
     }
 }
@@ -581,7 +624,27 @@ static int gather_attn_launch(const float* q, const float* kv, const float* sink
         a.part_acc = partial;
         a.part_ml = partial ? partial + (size_t)m * a.n_splits * h * kGaD : nullptr;
         const dim3 grid((unsigned)m, (unsigned)((h + 63) / 64), (unsigned)a.n_splits);
-        if (precise >= 2)
+        // Past a workgroup of 64 heads a compute unit, two of half the waves fit one (gather_attn_wide.hpp): 300 queries of
+        // 640 slots 101 -> 62 us, 520 153 -> 127, 8192 1624 -> 1044. Up to there a query is the faster the more waves it
+        // has (200 queries 54 us against 58, one 47 against 50), and a list of one tile has nothing to overlap (520 queries of
+        // 20 slots 43 us against 44). A scale of 0 gives a masked slot's -inf no weight there, and
+        // marks in o may not fall on a query that is still to be read.
+        const long long blocks = (long long)m * grid.y;
+        const uintptr_t q0 = (uintptr_t)q, o0 = (uintptr_t)o, bytes = (uintptr_t)m * h * kGaD * sizeof(float);
+        const bool wide = a.n_splits == 1 && blocks > kGaTargetGroups && topk > kGwTile && fabsf(scale) > 0.0f && fabsf(scale) < INFINITY &&
+                          (q0 + bytes <= o0 || o0 + bytes <= q0);
+        if (wide) {
+            const dim3 rest((unsigned)kGaTargetGroups);
+            if (precise >= 2) {
+                hipLaunchKernelGGL((gather_attn_wide_kernel<2, 2>), grid, dim3(kGwThreads), 0, stream, a);
+                hipLaunchKernelGGL((gather_attn_marked_kernel<2, 2>), rest, dim3(kGaThreads), 0, stream, a, blocks, (int)grid.y);
+            } else if (precise == 1) {
+                hipLaunchKernelGGL((gather_attn_wide_kernel<2, 1>), grid, dim3(kGwThreads), 0, stream, a);
+                hipLaunchKernelGGL((gather_attn_marked_kernel<2, 1>), rest, dim3(kGaThreads), 0, stream, a, blocks, (int)grid.y);
+            } else {
+                hipLaunchKernelGGL((gather_attn_wide_kernel<1, 1>), grid, dim3(kGwThreads), 0, stream, a);
+            }
+        } else if (precise >= 2)
             hipLaunchKernelGGL((gather_attn_d512_kernel<2, 2>), grid, dim3(kGaThreads), 0, stream, a);
         else if (precise == 1)
             hipLaunchKernelGGL((gather_attn_d512_kernel<2, 1>), grid, dim3(kGaThreads), 0, stream, a);

@@ -78,6 +78,57 @@ def test_queries_with_and_without_a_bf16_remainder_in_one_call(oracle):
         float(np.max(np.abs(got - exact)))
 
 
+@pytest.mark.parametrize("m,h,topk,precise,scale,q_scale,remainder", [
+    (257, 64, 33, 2, 512 ** -0.5, 1.0, False),      # two tiles, the second of one slot
+    (300, 5, 64, 2, 512 ** -0.5, 1.0, False), (260, 40, 640, 2, 512 ** -0.5, 1.0, False),
+    (130, 100, 129, 1, 512 ** -0.5, 1.0, False), (513, 33, 96, 0, 512 ** -0.5, 1.0, False),
+    (257, 64, 577, 2, 512 ** -0.5, 30.0, False),    # logits far apart: the reference maximum moves
+    (257, 64, 200, 2, -0.05, 1.0, False),
+    (260, 64, 100, 2, 512 ** -0.5, 1.0, True), (130, 100, 129, 1, 512 ** -0.5, 1.0, True)])
+def test_many_queries(oracle, m, h, topk, precise, scale, q_scale, remainder):
+    """More than 256 workgroups of 64 heads: the kernel of 32 heads a wave. Masked slots anywhere, lists
+    that end in masked slots (no tiles are made of those), a query with nothing live, and queries whose
+    rows have a remainder past bf16, in some heads or in all, which that kernel leaves to the other."""
+    d, rows = 512, 700
+    q, kv, sink = attend_inputs(oracle, m, h, d, rows, seed=m + topk, q_scale=q_scale)
+    rng = np.random.default_rng(h + topk)
+    idx = random_lists(rng, m, topk, rows)
+    for t in range(0, m, 3):
+        idx[t, rng.integers(1, topk + 1):] = -1
+        idx[t, 0] = 7
+    idx[4] = -1
+    if remainder:
+        noise = (rng.standard_normal(q.shape) * 2.0 ** -12).astype(np.float32)
+        q = q.copy()
+        q[2, h - 1, 300:] += noise[2, h - 1, 300:]    # one head, not the first
+        q[5:9] += noise[5:9]
+    got = device_attend(q, kv, sink, idx, scale, precise=precise, n_kv=rows)
+    assert np.isnan(got[4]).all() and np.isfinite(np.delete(got, 4, 0)).all()
+    pick = [0, 1, 2, 3, 5, 8, m // 2, m - 1]
+    exact = sparse_attn_f64(q[pick], kv, sink, idx[pick], scale)
+    top = np.abs(exact).max()
+    assert np.max(np.abs(got[pick] - exact)) <= ATTEND_TOL * top
+    if precise == 2 and q_scale == 1.0:
+        assert np.all(np.abs(got[pick] - exact) <= 2.0 ** -8 * np.abs(exact) + 2.0 ** -10 * top), \
+            float(np.max(np.abs(got[pick] - exact)))
+    # a query's result does not depend on how many others there are: the kernel of few queries agrees with it
+    few = device_attend(q[pick], kv, sink, idx[pick], scale, precise=precise, n_kv=rows)
+    assert worst_rel(few, got[pick]) <= 2.0 ** -7
+
+
+def test_many_queries_in_place(oracle):
+    """Results over the queries' own memory."""
+    m, h, topk, rows = 260, 64, 64, 100
+    q, kv, sink = attend_inputs(oracle, m, h, 512, rows, seed=12)
+    q[3] += np.float32(2.0 ** -12)
+    idx = random_lists(np.random.default_rng(3), m, topk, rows)
+    want = device_attend(q, kv, sink, idx, 512 ** -0.5)
+    buf = dev(q)
+    hip.launch_gather_attn_shared_kv(buf, dev(kv), dev(sink), dev(idx), m, h, 512, topk, 512 ** -0.5, buf)
+    got = back(buf, np.float32).reshape(m, h, 512)
+    assert worst_rel(got, want) <= 2.0 ** -7
+
+
 def test_peaked_and_flat_softmax(oracle):
     """Logits far apart (one slot holds the whole softmax; the lazily moved maximum must move)
     and logits all equal."""

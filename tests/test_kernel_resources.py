@@ -145,3 +145,46 @@ def test_the_build_refuses_an_attention_object_that_spills():
                 fine.replace("161328", "163856")):
         with pytest.raises(RuntimeError):
             build.check_resources("mla_attend.hip", bad)
+
+
+@pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
+def test_list_attention_of_32_heads_a_wave_keeps_its_operands_apart(tmp_path):
+    """Its score products are written as assembly, so the compiler does not see to their wait states:
+    a vector instruction's result may be a matrix instruction's operand two instructions later at
+    the earliest. Reads the listing; and no block with products may touch scratch memory, where the wait for
+    it would be a wait for every row on its way."""
+    out = tmp_path / "g.s"
+    cmd = [build.hipcc(), f"--offload-arch={build.offload_arch()}", "-O3", "-std=c++17", "-fPIC",
+           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-I", os.path.join(ROOT, "include")] + \
+          build.EXTRA_FLAGS.get("gather_attn.hip", []) + \
+          ["--cuda-device-only", "-S", os.path.join(build.CSRC, "gather_attn.hip"), "-o", str(out)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]
+
+    def registers(operand):
+        m = re.fullmatch(r"v\[(\d+):(\d+)\]|v(\d+)", operand)
+        if not m:
+            return set()
+        return {int(m[3])} if m[3] else set(range(int(m[1]), int(m[2]) + 1))
+
+    kernels = scores = 0
+    for body in re.findall(r"^_ZN2rk23gather_attn_wide_kernel\w+:(.*?)^\.Lfunc_end", out.read_text(), re.S | re.M):
+        kernels += 1
+        written = []                                  # (registers a vector instruction wrote, wait states since)
+        for block in re.split(r"^\.LBB\w+:", body, flags=re.M):
+            lines = [ln.split(";")[0].split() for ln in block.splitlines()]
+            lines = [ln for ln in lines if ln and not ln[0].startswith(".") and not ln[0].endswith(":")]
+            ops = [ln[0] for ln in lines]
+            if "v_mfma_f32_32x32x16_bf16" in ops and any(op.startswith("ds_read") for op in ops):
+                assert not any(op.startswith("scratch_") for op in ops)
+            for ln in lines:
+                args = [a for a in re.split(r",\s*", " ".join(ln[1:])) if a]
+                if ln[0] == "v_mfma_f32_32x32x16_bf16":
+                    scores += args[0].startswith("v")
+                    used = registers(args[1]) | registers(args[2])
+                    assert not any(used & w for w, since in written if since < 2), " ".join(ln)
+                states = int(ln[1]) + 1 if ln[0] == "s_nop" else 1
+                written = [(w, since + states) for w, since in written if since + states < 2]
+                if ln[0].startswith("v_") and not ln[0].startswith("v_mfma") and args:
+                    written.append((registers(args[0]), 0))
+    assert kernels == 3 and scores == 3 * 32, (kernels, scores)
