@@ -28,7 +28,7 @@
 // rounded to bf16) take an f32 kernel: a wave per (query, head), lanes over the dims, one
 // online-softmax pass over the list.
 // Calls of more than 256 such workgroups take another kernel, 32 heads a wave (gather_attn_wide.hpp), and this
-// one the queries that it leaves.
+// one the queries that it leaves; calls of up to 256 workgroups of 16 heads a third (gather_attn_few.hpp).
 // Launch-only; see include/rivoli_kvcache.h for the contract.
 #include "attend_common.hpp"
 
@@ -93,8 +93,27 @@ static inline int gather_attn_splits(int m, int h, int topk) {
     return n < 2 ? 1 : (int)n;
 }
 
+// Whether a call takes the workgroups of 16 heads (gather_attn_few.hpp), and in how many shares of a list: never
+// more workgroups than compute units, each has 108 KB of LDS. 32 slots of a share take them 1.35 us against 1.9 in a
+// workgroup of 64 heads, and 6 us less around it (64 heads: one query of 640 slots 17.1 -> 10.1 us, in one share 47 -> 28);
+// but with four times the workgroups a query they run out of shares four times sooner, and the shares get longer:
+// 17 queries of 640 slots, 3 shares instead of 10, 24 -> 20 us, 32 of 1500, 2 of 24 tiles instead of 8 of 6, 34 -> 41. So a share
+// that is longer than the other plan's has at most 16 tiles, or 24 where that plan takes two rounds of workgroups (40 queries
+// of 640 slots, 1 share instead of 7, 40 -> 30; of 900 47 -> 43; 33 of 900 45 -> 45).
+static inline bool gather_attn_few(int m, int h, int topk, int splits, int* few_splits) {
+    const long long groups = (long long)m * ((h + 15) / 16);
+    if (groups > kGaTargetGroups) return false;
+    const int tiles = (topk + kGaTile - 1) / kGaTile;
+    const int n = (int)(kGaTargetGroups / groups) < splits ? (int)(kGaTargetGroups / groups) : splits;
+    const bool two_rounds = (long long)m * ((h + 63) / 64) * splits > kGaTargetGroups;
+    if (n < splits && (tiles + n - 1) / n > (two_rounds ? 24 : 16)) return false;
+    *few_splits = n;
+    return true;
+}
+
 }  // namespace rk
 
+#include "gather_attn_few.hpp"
 #include "gather_attn_wide.hpp"
 
 namespace rk {
@@ -621,19 +640,28 @@ static int gather_attn_launch(const float* q, const float* kv, const float* sink
         a.h = h, a.topk = topk, a.n_kv = n_kv, a.qscale = scale * kLog2e, a.o = o;
         // a caller without a partial buffer gets the one-workgroup-per-query plan
         a.n_splits = partial && aligned16(partial) ? gather_attn_splits(m, h, topk) : 1;
+        const bool few = gather_attn_few(m, h, topk, a.n_splits, &a.n_splits);
         a.part_acc = partial;
         a.part_ml = partial ? partial + (size_t)m * a.n_splits * h * kGaD : nullptr;
         const dim3 grid((unsigned)m, (unsigned)((h + 63) / 64), (unsigned)a.n_splits);
         // Past a workgroup of 64 heads a compute unit, two of half the waves fit one (gather_attn_wide.hpp): 300 queries of
         // 640 slots 101 -> 62 us, 520 153 -> 127, 8192 1624 -> 1044. Up to there a query is the faster the more waves it
-        // has (200 queries 54 us against 58, one 47 against 50), and a list of one tile has nothing to overlap (520 queries of
+        // has (200 queries 54 us against 58), and a list of one tile has nothing to overlap (520 queries of
         // 20 slots 43 us against 44). A scale of 0 gives a masked slot's -inf no weight there, and
         // marks in o may not fall on a query that is still to be read.
         const long long blocks = (long long)m * grid.y;
         const uintptr_t q0 = (uintptr_t)q, o0 = (uintptr_t)o, bytes = (uintptr_t)m * h * kGaD * sizeof(float);
         const bool wide = a.n_splits == 1 && blocks > kGaTargetGroups && topk > kGwTile && fabsf(scale) > 0.0f && fabsf(scale) < INFINITY &&
                           (q0 + bytes <= o0 || o0 + bytes <= q0);
-        if (wide) {
+        if (few) {
+            const dim3 few_grid((unsigned)m, (unsigned)((h + kGfHeads - 1) / kGfHeads), (unsigned)a.n_splits);
+            if (precise >= 2)
+                hipLaunchKernelGGL((gather_attn_few_kernel<2, 2>), few_grid, dim3(kGfThreads), 0, stream, a);
+            else if (precise == 1)
+                hipLaunchKernelGGL((gather_attn_few_kernel<2, 1>), few_grid, dim3(kGfThreads), 0, stream, a);
+            else
+                hipLaunchKernelGGL((gather_attn_few_kernel<1, 1>), few_grid, dim3(kGfThreads), 0, stream, a);
+        } else if (wide) {
             const dim3 rest((unsigned)kGaTargetGroups);
             if (precise >= 2) {
                 hipLaunchKernelGGL((gather_attn_wide_kernel<2, 2>), grid, dim3(kGwThreads), 0, stream, a);

@@ -84,9 +84,11 @@ def test_queries_with_and_without_a_bf16_remainder_in_one_call(oracle):
     (130, 100, 129, 1, 512 ** -0.5, 1.0, False), (513, 33, 96, 0, 512 ** -0.5, 1.0, False),
     (257, 64, 577, 2, 512 ** -0.5, 30.0, False),    # logits far apart: the reference maximum moves
     (257, 64, 200, 2, -0.05, 1.0, False),
-    (260, 64, 100, 2, 512 ** -0.5, 1.0, True), (130, 100, 129, 1, 512 ** -0.5, 1.0, True)])
+    (260, 64, 100, 2, 512 ** -0.5, 1.0, True), (130, 100, 129, 1, 512 ** -0.5, 1.0, True),
+    # up to 256 workgroups of 64 heads (one tile of more of them): the kernel of 16 heads and half the dims a wave
+    (100, 64, 200, 2, 512 ** -0.5, 1.0, True), (70, 128, 97, 1, 512 ** -0.5, 1.0, False), (300, 64, 31, 2, 512 ** -0.5, 1.0, True)])
 def test_many_queries(oracle, m, h, topk, precise, scale, q_scale, remainder):
-    """More than 256 workgroups of 64 heads: the kernel of 32 heads a wave. Masked slots anywhere, lists
+    """More than 256 workgroups of 64 heads: the kernel of 32 heads a wave, and the one below that. Masked slots anywhere, lists
     that end in masked slots (no tiles are made of those), a query with nothing live, and queries whose
     rows have a remainder past bf16, in some heads or in all, which that kernel leaves to the other."""
     d, rows = 512, 700
@@ -114,6 +116,34 @@ def test_many_queries(oracle, m, h, topk, precise, scale, q_scale, remainder):
     # a query's result does not depend on how many others there are: the kernel of few queries agrees with it
     few = device_attend(q[pick], kv, sink, idx[pick], scale, precise=precise, n_kv=rows)
     assert worst_rel(few, got[pick]) <= 2.0 ** -7
+
+
+@pytest.mark.parametrize("m,h,topk,precise,share", [
+    (1, 1, 1, 2, False), (2, 15, 63, 2, False), (2, 17, 64, 1, False), (3, 16, 65, 0, False), (1, 64, 129, 2, False),
+    (4, 64, 96, 2, True), (16, 64, 700, 2, True), (17, 64, 640, 1, True), (50, 40, 300, 2, True), (256, 16, 70, 2, False)])
+def test_workgroups_of_16_heads(oracle, m, h, topk, precise, share):
+    """Up to 256 workgroups of 16 heads: lists of one slot, of a tile of 64 and one more or less, shares of an odd number of
+    32-slot tiles, fewer shares than the buffer has room for, whole tiles masked, some queries with a remainder past bf16."""
+    d, rows = 512, 300
+    q, kv, sink = attend_inputs(oracle, m, h, d, rows, seed=m * 7 + topk)
+    rng = np.random.default_rng(topk)
+    q = q.copy()
+    q[m // 2] += (rng.standard_normal((h, d)) * 2.0 ** -12).astype(np.float32)
+    idx = random_lists(rng, m, topk, rows)
+    if topk > 200:
+        idx[0, 64:200] = -1
+    if m > 4:
+        idx[3] = -1
+    n = hip.gather_attn_scratch_floats(m, h, d, topk)
+    partial = dzeros(max(n, 4) * 4, 0xEE) if share else None
+    got = device_attend(q, kv, sink, idx, d ** -0.5, precise=precise, n_kv=rows, partial=partial)
+    pick = sorted({0, 1 % m, m // 2, m - 1})
+    if m > 4:
+        assert np.isnan(got[3]).all()
+    exact = sparse_attn_f64(q[pick], kv, sink, idx[pick], d ** -0.5)
+    top = np.abs(exact).max()
+    bound = 2.0 ** -8 * np.abs(exact) + 2.0 ** -10 * top if precise == 2 else ATTEND_TOL * top
+    assert np.all(np.abs(got[pick] - exact) <= bound), float(np.max(np.abs(got[pick] - exact)))
 
 
 def test_many_queries_in_place(oracle):
