@@ -7,7 +7,7 @@
 //
 // Two shapes share one selection rule.
 //
-// (1) One workgroup per query (`topk_block`): each wave owns a contiguous segment of the
+// (1) One workgroup per query (up to 16384 scores `select_few`, select_few.hpp; `topk_block_lean` and `topk_block`): each wave owns a contiguous segment of the
 //     score array and keeps its order-preserving u32 keys in registers (up to 64 per lane),
 //     so the scores are read once. Selection is a 4-pass, 8-bit, MSB-first radix select of the
 //     k-th largest key. Score arrays concentrate in a handful of exponent bytes, so each
@@ -50,6 +50,7 @@
 #include <type_traits>
 
 #include "gather_common.hpp"
+#include "select_few.hpp"
 #include "topk_common.hpp"
 
 namespace rk {
@@ -247,7 +248,7 @@ __device__ __forceinline__ void topk_block(const float* __restrict__ s, int nt, 
 constexpr int kTopkThreads = 1024;
 constexpr int kTopkWaves = kTopkThreads / kWave;
 
-// Shape (1), lean form for register-resident queries (nt <= 65536). A compute unit issues
+// Shape (1), lean form for register-resident queries of 16 385 to 65 536 scores (up to there select_few.hpp). A compute unit issues
 // about one wave-instruction per cycle, so what a single workgroup pays for is instructions
 // per key; sweeping all keys four times plus two compaction sweeps (topk_block) costs ~110 of
 // them. Here all keys are swept three times with a few instructions each — one 10-bit
@@ -569,6 +570,22 @@ __global__ __launch_bounds__(kTopkThreads) void index_topk_kernel(
         topk_block_lean<ITEMS>(s, nt, (uint32_t)min(k, nt), out, lds);
     else
         topk_block<kTopkThreads, 0>(s, nt, (uint32_t)min(k, nt), out, lds);
+}
+
+template <int ITEMS>
+__global__ __launch_bounds__(kSfThreads) void index_topk_few_kernel(
+    const float* __restrict__ scores, int stride, const int* __restrict__ nts, int nt_all, int k,
+    uint32_t* __restrict__ rows) {
+    __shared__ __attribute__((aligned(16))) uint32_t lds[kSfLdsWords];
+    const int q = blockIdx.x;
+    const int nt = nts ? min(nts[q], nt_all) : nt_all;
+    if (nt <= 0) return;
+    uint32_t* out = rows + (size_t)q * k;
+    if (nt <= k) {  // all of it
+        for (int i = threadIdx.x; i < nt; i += kSfThreads) out[i] = (uint32_t)i;
+        return;
+    }
+    select_few<ITEMS, FoldedZeroKey>(scores + (size_t)q * stride, nt, (uint32_t)k, out, lds, 0u);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1440,12 +1457,18 @@ static int index_topk_launch(const float* scores, int n_queries, int stride, con
         return launch_status();
     }
     dim3 grid((unsigned)n_queries), block(kTopkThreads);
-    if (nt <= kTopkThreads * 4)
-        hipLaunchKernelGGL(index_topk_kernel<4>, grid, block, 0, stream, scores, stride, nts,
-                           nt, k, rows);
-    else if (nt <= kTopkThreads * 16)
-        hipLaunchKernelGGL(index_topk_kernel<16>, grid, block, 0, stream, scores, stride,
-                           nts, nt, k, rows);
+#define RK_TOPK_FEW(I)                                                                              \
+    hipLaunchKernelGGL(index_topk_few_kernel<I>, grid, dim3(kSfThreads), 0, stream, scores, stride, \
+                       nts, nt, k, rows)
+    if (nt <= kSfThreads)
+        RK_TOPK_FEW(1);
+    else if (nt <= kSfThreads * 2)
+        RK_TOPK_FEW(2);
+    else if (nt <= kSfThreads * 8)
+        RK_TOPK_FEW(8);
+    else if (nt <= kSfThreads * 16)
+        RK_TOPK_FEW(16);
+#undef RK_TOPK_FEW
     else if (nt <= kTopkThreads * 64)
         hipLaunchKernelGGL(index_topk_kernel<64>, grid, block, 0, stream, scores, stride,
                            nts, nt, k, rows);
@@ -1478,11 +1501,10 @@ static int index_topk_launch(const float* scores, int n_queries, int stride, con
 // ties) is bisected over all the keys instead. The selection is then emitted in index order
 // by ballots and prefix counts.
 //
-// Sixteen waves on one row (decode) hold their keys in 8 or 16 registers a lane and are bound by
-// what the row does one after the other: colliding atomics of the histogram (half of a row's keys
-// share a few exponents) and the one wave's bisection. They resolve 12 bits (three of the
-// mantissa), which quarters both; the walk over 4096 bins is then a scan by all threads, four bins
-// each. One row of 8192 keys: 17.8 us in four waves of 10 bits, 14.3 in sixteen, 11.9 with 12 bits, 8.8 with the agreeing bits left out (below).
+// Sixteen waves on one row are bound by what the row does one after the other: colliding atomics of the
+// histogram (half of a row's keys share a few exponents) and the one wave's bisection. They resolve 12 bits
+// (three of the mantissa), which quarters both; the walk over 4096 bins is then a scan by all threads, four bins
+// each. (Up to 256 rows of up to 16 384 keys take select_few.hpp instead.)
 template <int WAVES>
 struct SelShapeOf {
     static constexpr int kBits = WAVES == 16 ? 12 : 10;  // key bits resolved by the histogram
@@ -1870,19 +1892,32 @@ __global__ __launch_bounds__(WAVES* kWave) void block_select_bisect_kernel(
                                                (uint32_t)offset);
 }
 
-// Few rows: sixteen waves each.
+// Few rows: sixteen waves each (select_few.hpp).
 template <int ITEMS>
-__global__ __launch_bounds__(1024) void block_select_few_kernel(
-    const float* __restrict__ scores, int n_comp, int ratio, int prefill, int k, int offset,
-    int32_t* __restrict__ out, int out_stride, SelWindow window) {
-    __shared__ __attribute__((aligned(16))) uint32_t lds[sel_lds_words<16>()];
+__device__ __forceinline__ void block_select_sixteen(const float* __restrict__ scores, int n_comp, int ratio, int prefill,
+                                                     int k, int offset, int32_t* __restrict__ out, int out_stride,
+                                                     const SelWindow& window, uint32_t* lds) {
     const int t = blockIdx.x;
     const int limit = select_row_limit(t, n_comp, ratio, prefill);
     int32_t* o = out + (size_t)t * out_stride;
-    write_window<1024>(window, t, o);
-    if (select_positional<1024>(o, limit, k, offset)) return;
-    select_bisect<16, ITEMS, TotalOrderKey>(scores + (size_t)t * n_comp, limit, (uint32_t)k,
-                                            reinterpret_cast<uint32_t*>(o), lds, (uint32_t)offset);
+    write_window<kSfThreads>(window, t, o);
+    if (select_positional<kSfThreads>(o, limit, k, offset)) return;
+    select_few<ITEMS, TotalOrderKey>(scores + (size_t)t * n_comp, limit, (uint32_t)k,
+                                     reinterpret_cast<uint32_t*>(o), lds, (uint32_t)offset);
+}
+template <int ITEMS>
+__global__ __launch_bounds__(kSfThreads) void block_select_few_kernel(
+    const float* __restrict__ scores, int n_comp, int ratio, int prefill, int k, int offset,
+    int32_t* __restrict__ out, int out_stride, SelWindow window) {
+    __shared__ __attribute__((aligned(16))) uint32_t lds[kSfLdsWords];
+    block_select_sixteen<ITEMS>(scores, n_comp, ratio, prefill, k, offset, out, out_stride, window, lds);
+}
+template <int ITEMS>  // rows of one or two keys a lane
+__global__ __launch_bounds__(kSfThreads) void block_select_short_kernel(
+    const float* __restrict__ scores, int n_comp, int ratio, int prefill, int k, int offset,
+    int32_t* __restrict__ out, int out_stride, SelWindow window) {
+    __shared__ __attribute__((aligned(16))) uint32_t lds[kSfLdsWords];
+    block_select_sixteen<ITEMS>(scores, n_comp, ratio, prefill, k, offset, out, out_stride, window, lds);
 }
 
 // Rows too long for the register form: the single-query radix select, one workgroup per row.
@@ -1920,18 +1955,23 @@ static int block_select_launch(const float* scores, int rows, int n_comp, int ra
 #define RK_BISECT(WV, I)                                                                     \
     hipLaunchKernelGGL((block_select_bisect_kernel<WV, I>), grid, dim3(WV* kWave), 0, stream, \
                        scores, n_comp, ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
-#define RK_FEW(I)                                                                             \
-    hipLaunchKernelGGL((block_select_few_kernel<I>), grid, dim3(1024), 0, stream, scores, n_comp, \
-                       ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
+#define RK_FEW(KERNEL, I)                                                                     \
+    hipLaunchKernelGGL((KERNEL<I>), grid, dim3(kSfThreads), 0, stream, scores, n_comp, ratio, \
+                       prefill ? 1 : 0, k, offset, out, out_stride, window)
 #define RK_SELECT(T, I)                                                                       \
     hipLaunchKernelGGL((block_select_kernel<T, I>), grid, dim3(T), 0, stream, scores, n_comp, \
                        ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
-    // Few rows (decode: one) leave the chip to one workgroup each, and a row's time is its
-    // longest wave's: sixteen waves, 8 keys a lane. One row of 8192: 17.8 -> 8.8 us.
-    if (rows <= kSelFewRows && n_comp > 64 * 8 && n_comp <= 1024 * 8)
-        RK_FEW(8);
-    else if (rows <= kSelFewRows && n_comp > 1024 * 8 && n_comp <= 1024 * 16)
-        RK_FEW(16);
+    // Few rows (decode: one) leave the chip to one workgroup each, and a row's time is its longest wave's: sixteen waves,
+    // as few keys a lane as there are. One row of 8192 (sums of a ReLU): in four waves 17.8 us, by leading bits and
+    // bisection in sixteen 10.6, over the range that the keys take 5.8; of 1000 7.6 -> 4.
+    if (rows <= kSelFewRows && n_comp > 64 * 8 && n_comp <= kSfThreads)
+        RK_FEW(block_select_short_kernel, 1);
+    else if (rows <= kSelFewRows && n_comp > kSfThreads && n_comp <= kSfThreads * 2)
+        RK_FEW(block_select_short_kernel, 2);
+    else if (rows <= kSelFewRows && n_comp > kSfThreads * 2 && n_comp <= kSfThreads * 8)
+        RK_FEW(block_select_few_kernel, 8);
+    else if (rows <= kSelFewRows && n_comp > kSfThreads * 8 && n_comp <= kSfThreads * 16)
+        RK_FEW(block_select_few_kernel, 16);
     // otherwise up to 32 keys per lane; a row takes as few waves as hold it
     else if (n_comp <= 64 * 8)
         RK_BISECT(1, 8);
