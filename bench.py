@@ -768,7 +768,7 @@ def bench_v4_attend(a, torch, hip):
                       "slots_per_query": cols, "live_slots": live, "precise": a.precise},
            "queries_per_s": round(n / (ms * 1e-3), 1),
            "kernels_ms": {k_: round(v, 5) for k_, v in per.items()},
-           "roofline": {"bound": "mfma", "kernel": "gather_attn_d512_kernel",
+           "roofline": {"bound": "mfma", "kernel": "gather_attn_wide_kernel",
                         "achieved": round(flops / att / 1e12, 2), "peak": 2500.0, "unit": "TFLOP/s",
                         "frac": round(flops / att / 2.5e15, 4), "avg_launch_ms": round(per["attend"], 5),
                         "flops_per_launch": flops,
@@ -931,7 +931,7 @@ def bench_dsa(a, torch, hip, scored=False, attend=False):
            "kernels_ms": {n: round(v, 5) for n, v in per.items()},
            "roofline": {"bound": "hbm",
                         # (short calls run in workgroups of 16 heads: rivoli_amd/csrc/mla_attend_plan.hpp)
-                        "kernel": ("mla_attend_heads16_kernel"
+                        "kernel": ("mla_attend_few_kernel"
                                    if B * -(-k // 32) * -(-H // 16) <= (4096 if a.precise > 2 else 8192)
                                    else "mla_attend_paged_kernel") if attend else
                                   ("topk_hist + topk_cand + topk_finish_bits (select and gather)" if fused

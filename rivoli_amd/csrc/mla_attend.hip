@@ -630,6 +630,7 @@ __device__ __forceinline__ void attend_part(const AttendArgs& a, int seq, int hb
 }  // namespace rk
 #include "mla_attend_f8.hpp"
 #include "mla_attend_heads16.hpp"
+#include "mla_attend_few.hpp"
 namespace rk {
 
 // Rows of sequence s that are attended.
@@ -875,6 +876,57 @@ __global__ __launch_bounds__(kH16Threads, 1) void mla_attend_heads16_kernel(cons
     }
 }
 
+// The same walk for 16 heads per workgroup by eight waves (mla_attend_few.hpp).
+template <int QSPLIT, int PSPLIT, int MODE>
+__global__ __launch_bounds__(kFewThreads) void mla_attend_few_kernel(const AttendArgs a) {
+    __shared__ int pre[kDealMaxSeqs + 8];
+    __shared__ int wave_total[kFewWaves];
+    // Workgroups are dealt to the eight dies in turn: the head groups of one work item follow each
+    // other on one die, whose cache then serves the item's rows to all but the first of them.
+    const int groups = (a.H + kH16Heads - 1) / kH16Heads, turn = (int)blockIdx.x >> 3;
+    const int item = (turn / groups) * 8 + ((int)blockIdx.x & 7), hg = turn % groups;
+    long long t_lo, t_hi;
+    int seq = item;
+    if (item >= (a.n_items > 0 ? a.n_items : a.n_seqs)) return;
+    if (a.by_seq) {
+        const SeqDeal d = seq_deal(MODE == kLinear ? nullptr : (MODE == kSparse ? a.n_rows : a.seq_lens), a.k, a.n_seqs, a.n_items);
+        const unsigned long long past = __ballot(d.first + d.parts > item);
+        if (!past) return;  // more work items than runs
+        seq = __builtin_ctzll(past);
+        const int first = __builtin_amdgcn_readlane(d.first, seq), parts = __builtin_amdgcn_readlane(d.parts, seq);
+        // of a sequence's work items none is longer than the run: its tiles in `parts` even shares
+        const int tiles = __builtin_amdgcn_readlane(d.tiles, seq), part = item - first;
+        const int r_begin = (int)((unsigned)(part * tiles) / (unsigned)parts) * kTile;
+        const int r_end = min(attended_rows<MODE>(a, seq), (int)((unsigned)((part + 1) * tiles) / (unsigned)parts) * kTile);
+        const size_t rec = (size_t)item + seq;
+        attend_part_few<QSPLIT, PSPLIT, MODE>(a, seq, hg, r_begin, r_end, parts == 1, a.part_acc + rec * a.H * kKvl,
+                                                  a.part_ml + rec * a.H * 2);
+        return;
+    }
+    if (!dealt_range<kFewThreads, MODE>(a, item, pre, wave_total, t_lo, t_hi, seq)) return;
+    for (;; ++seq) {
+        int r_begin = 0, r_end;
+        bool whole = true;
+        float *pa = a.part_acc, *pml = a.part_ml;
+        if (a.n_items > 0) {
+            if (t_lo >= t_hi || seq >= a.n_seqs) break;
+            if (!dealt_part<MODE>(a, item, pre, seq, t_lo, t_hi, r_begin, r_end, whole, pa, pml)) continue;
+            __syncthreads();
+        } else {
+            r_end = attended_rows<MODE>(a, seq);
+            if (r_end <= 0) {
+                for (int i = threadIdx.x; i < kH16Heads * kKvl; i += kFewThreads) {
+                    const int h = hg * kH16Heads + i / kKvl;
+                    if (h < a.H) a.clat[((size_t)seq * a.H + h) * kKvl + (i % kKvl)] = 0.0f;
+                }
+                return;
+            }
+        }
+        attend_part_few<QSPLIT, PSPLIT, MODE>(a, seq, hg, r_begin, r_end, whole, pa, pml);
+        if (a.n_items == 0) break;
+    }
+}
+
 // Dealt plan: clat[seq][head] = sum_r w_r acc_r / sum_r w_r l_r over the sequence's partial
 // records, w_r = 2^(m_r - max m), in ascending work-item order (the reference's combine,
 // crates/backend/kernels/attn.hip:235-277, in base 2). A sequence that one work item covered
@@ -990,13 +1042,19 @@ static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_row
         const dim3 grid((unsigned)(((items + 7) / 8 * 8) * (long long)((a.H + kH16Heads - 1) / kH16Heads)));
         (void)hipGetLastError();
         constexpr int M = MODE == kDensePaged ? kDense : MODE;  // the rows are looked up one by one
-        if (precise >= 2 || MODE == kLinear)
-            hipLaunchKernelGGL((mla_attend_heads16_kernel<2, 2, M>), grid, dim3(kH16Threads), 0, st, a);
-        else if constexpr (MODE != kLinear) {
-            if (precise == 1)
-                hipLaunchKernelGGL((mla_attend_heads16_kernel<2, 1, M>), grid, dim3(kH16Threads), 0, st, a);
-            else
-                hipLaunchKernelGGL((mla_attend_heads16_kernel<1, 1, M>), grid, dim3(kH16Threads), 0, st, a);
+        const bool few = route.few;  // (always, for the linear slabs)
+        const dim3 block(few ? kFewThreads : kH16Threads);
+        if (precise >= 2 || MODE == kLinear) {
+            if (few) hipLaunchKernelGGL((mla_attend_few_kernel<2, 2, M>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((mla_attend_heads16_kernel<2, 2, M>), grid, block, 0, st, a);
+        } else if constexpr (MODE != kLinear) {
+            if (precise == 1) {
+                if (few) hipLaunchKernelGGL((mla_attend_few_kernel<2, 1, M>), grid, block, 0, st, a);
+                else hipLaunchKernelGGL((mla_attend_heads16_kernel<2, 1, M>), grid, block, 0, st, a);
+            } else {
+                if (few) hipLaunchKernelGGL((mla_attend_few_kernel<1, 1, M>), grid, block, 0, st, a);
+                else hipLaunchKernelGGL((mla_attend_heads16_kernel<1, 1, M>), grid, block, 0, st, a);
+            }
         }
         return attend_merge(a, plan, n_seqs, max_rows, seq_lens, n_rows, listed, st);
     }

@@ -1,7 +1,8 @@
 // MLA decode attention for calls that the 64-head workgroups of mla_attend.hip leave most of the
 // chip idle on, or keep for a few tiles only: the same arithmetic (bf16 matrix instructions, q
 // and the weights as bf16 hi + lo in the parity mode), dealt the other way. Included by
-// mla_attend.hip.
+// mla_attend.hip. Long work items of few heads take it (heads16_few); the others, and the linear slabs, take
+// mla_attend_few.hpp.
 //
 // There a workgroup's eight waves share one tile: two of them meet in LDS over every score, and
 // a barrier ends every tile. A short call is then a chain — list entry, table, rows, staging,

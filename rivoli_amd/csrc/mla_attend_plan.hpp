@@ -93,7 +93,8 @@ static inline AttendPlan heads16_plan(const AttendPlan& plan, int n_seqs, int H,
 }
 
 // Whether a call goes to the workgroups of 16 heads: its 32-token tiles times its groups of 16
-// heads, before the lengths are known. Parity mode, 64 heads: 1 x 4 096 tokens (512) 21.5 us
+// heads, before the lengths are known. (The figures of this side here and below are those of a tile a wave;
+// eight waves on a tile, heads16_few, take 2 to 50 % off them.) Parity mode, 64 heads: 1 x 4 096 tokens (512) 21.5 us
 // against 34.5 in workgroups of 64 heads, 32 x 1 000 (4 096) 33 against 39, 6 ragged of up
 // to 9 000 (6 768) 39 against 51 with the append, 32 listed sets of 2 048 rows (8 192) 45 against 48, 32 x 4 096 (16 384) 73 against 64.
 // The 8-bit modes' kernel is the faster one sooner: 8 listed sets of 2 048 rows (2 048) 24 us in
@@ -169,19 +170,37 @@ static inline bool heads16_pays(const AttendPlan& plan, bool cut, int n_seqs, in
     return work <= (spills ? (f8 ? kH16MaxWorkSpill8Bit : kH16MaxWorkSpill) : (f8 ? kH16MaxWorkFull8Bit : kH16MaxWorkFull));
 }
 
+// Which kernel the workgroups of 16 heads run. Eight waves on a tile of 64 tokens (mla_attend_few.hpp) are the faster in
+// every shape tried that has three groups of heads and more, linear slabs or short work items: linear, 64 heads, 33 rows
+// 12.6 -> 7.1 us, 300 rows 19.4 -> 13.7, 8 192 rows 31.4 -> 28.1, 300 000 rows 564 -> 524; 20 x 9 000 tokens of 64 heads 94.5 -> 90.1.
+// One or two groups of heads that walk long work items have each row from memory and wait for it; a
+// tile of its own per wave (mla_attend_heads16.hpp) keeps more of them on their way. Parity mode, 16 heads, per tile-a-wave
+// and eight waves: dense, one sequence of 100 000 tokens (49 tiles a work item) 64.4 us and 63.1, 300 000 (146) 138.5 and 139.1,
+// 800 000 (390) 325 and 340, 300 whole sequences of 6 000 (188) 314 and 324; lists, whose rows are scattered, sooner: 64 of
+// 6 000 rows (47) 68 and 66, 300 of 3 000 (94) 180 and 186, 257 of 6 000 (188) 323 and 355. With q and weights in one term
+// (precise 0) cut dense sequences too: 100 000 tokens (49) 57.6 and 57.7, 200 000 (98) 88.7 and 91.4.
+constexpr int kFewMaxTiles = 128, kFewMaxTilesOneTerm = 64, kFewMaxTilesListed = 48;  // of a work item
+static inline bool heads16_few(const AttendPlan& p, int n_seqs, int H, int max_rows, int precise, bool dense, bool linear) {
+    if (linear || H > 2 * kH16Heads) return true;
+    const long long tiles = max_rows / kTile + (max_rows % kTile != 0);
+    const long long longest = p.n_items ? (n_seqs * tiles + p.n_items - 1) / p.n_items : tiles;
+    return longest <= (!dense ? kFewMaxTilesListed : precise == 0 && p.n_items ? kFewMaxTilesOneTerm : kFewMaxTiles);
+}
+
 // A call of the shipped row widths whose rows are whole 16-byte pieces. `plan`: attend_plan's or
 // linear_plan's.
 struct AttendRoute {
     bool heads16;  // workgroups of 16 heads; else of 64
     bool by_seq;   // no work item has tiles of two sequences (SeqDeal)
+    bool few;      // eight waves on a tile, else a tile a wave
     AttendPlan plan;
 };
 static inline AttendRoute attend_route(const AttendPlan& plan, int n_seqs, int H, int max_rows, int precise, bool dense,
                                        bool linear) {
     bool by_seq;
     const AttendPlan p = heads16_plan(plan, n_seqs, H, max_rows, by_seq);
-    if (!heads16_pays(plan, p.n_items > 0, n_seqs, H, max_rows, precise, dense, linear)) return {false, false, plan};
-    return {true, by_seq, p};
+    if (!heads16_pays(plan, p.n_items > 0, n_seqs, H, max_rows, precise, dense, linear)) return {false, false, false, plan};
+    return {true, by_seq, heads16_few(p, n_seqs, H, max_rows, precise, dense, linear), p};
 }
 
 }  // namespace rk

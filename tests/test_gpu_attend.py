@@ -517,6 +517,38 @@ def test_linear_rows_past_the_lines_of_the_paged_calls(oracle, scratch):
     check_linear(run_linear(case, h, nt, KVL, ROPE, rows=rows, scratch=scratch), want, f"scratch={scratch}")
 
 
+@pytest.mark.parametrize("precise", [2, 1, 0])
+@pytest.mark.parametrize("most,listed_most", [(4096, 1536), (4097, 1537)])
+def test_both_sides_of_the_line_between_a_tile_of_eight_waves_and_a_tile_a_wave(oracle, precise, most, listed_most):
+    """Up to 16 heads, sequences kept whole: 128 tiles of 32 dense rows and 48 of listed ones, and one row
+    more. The others end one short of, at and one past the tiles of 64 and the three buffers they pass
+    through; lists have entries of all ones, in a first tile, a last one and a whole one."""
+    H, edges = 11, [1, 0, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257]
+    lens = [most] + (edges * 22)[:299]
+    route = attend_route(len(lens), H, most, precise)
+    assert route.heads16 and route.items == 0
+    c = paged_case(oracle, lens, H=H, seed=905, outlier_frac=0.0)
+    want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], None, None,
+                                   KVL, ROPE, PT, c["scale"], n_threads=8)
+    check(run_paged(c, most, precise=precise), want, precise, "dense", mild=precise == 2)
+    k = listed_most
+    rows = np.zeros((len(lens), k), np.uint32)
+    n_rows = np.array([min(n, k) for n in lens], np.int32)
+    rng = np.random.default_rng(906)
+    for s, n in enumerate(lens):
+        rows[s, :n_rows[s]] = rng.permutation(max(n, 1))[:n_rows[s]]
+    gone = rows.copy()
+    gone[0, :64] = gone[0, 130] = gone[3, 5] = gone[9, 190] = 0xffffffff
+    kept = rows.copy()
+    kept_n = n_rows.copy()
+    for s in (0, 3, 9):
+        live = rows[s, :n_rows[s]][gone[s, :n_rows[s]] != 0xffffffff]
+        kept_n[s], kept[s, :len(live)] = len(live), live
+    want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], kept, kept_n,
+                                   KVL, ROPE, PT, c["scale"], n_threads=8)
+    check(run_paged(c, k, rows=gone, n_rows=n_rows, precise=precise), want, precise, "listed", mild=precise == 2)
+
+
 @pytest.mark.parametrize("n_seqs,H", [(3, 64), (24, 128)])
 @pytest.mark.parametrize("precise", [2, 1, 0, 4, 3])
 def test_list_entries_of_all_ones_are_left_out(oracle, precise, n_seqs, H):

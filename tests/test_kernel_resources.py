@@ -109,6 +109,19 @@ def test_kernels_of_16_heads_a_workgroup_do_not_spill():
 
 
 @pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
+def test_kernels_that_count_their_transfers_do_not_spill():
+    """Eight waves on a tile of 64 tokens (rivoli_amd/csrc/mla_attend_few.hpp): a wave waits until six reads
+    are left on their way, the next tile's; a spilled register's reload would be one more."""
+    blocks = [b for b in _resource_blocks("mla_attend.hip") if "mla_attend_few_kernel" in b.split()[0]]
+    assert len(blocks) == 7
+    for b in blocks:
+        name = b.split()[0]
+        assert int(re.search(r"VGPRs Spill: (\d+)", b).group(1)) == 0, name
+        assert int(re.search(r"ScratchSize \[bytes/lane\]: (\d+)", b).group(1)) == 0, name
+        assert int(re.search(r"LDS Size \[bytes/block\]: (\d+)", b).group(1)) <= 160 * 1024, name
+
+
+@pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
 def test_the_block_scorers_matrix_kernels_and_the_few_row_selection_do_not_spill():
     """Two waves per SIMD of 252 registers in the many-query scorer (scalar registers do spill
     there, in the fold), three in the one-query scorers; a row's keys in registers and its masks
