@@ -977,39 +977,60 @@ __global__ __launch_bounds__(128) void mla_attend_combine_kernel(
         return;
     }
     if (first == last) return;  // one work item had the whole sequence and wrote it
-    // Records are fetched eight at a time, every load of a batch issued before the first use
-    // (a record past the last re-reads the last and is left out): one round trip per batch
-    // instead of one per record. The sums run in ascending record order as before.
-    constexpr int kBatch = 8;
-    float m_g = -INFINITY;
-    for (int b0 = first; b0 <= last; b0 += kBatch) {
-        float m_r[kBatch];
-#pragma unroll
-        for (int u = 0; u < kBatch; ++u)
-            m_r[u] = part_ml[((size_t)(min(b0 + u, last) + seq) * H + head) * 2];
-#pragma unroll
-        for (int u = 0; u < kBatch; ++u) m_g = fmaxf(m_g, m_r[u]);
-    }
+    // Records are fetched a batch at a time, every load of a batch issued before the first use (a record past the last
+    // re-reads the last and is left out). Up to 16 records, as many as most calls have a sequence, are one batch, and
+    // their accumulators are asked for with the maxima that weigh them: one round trip to memory, where maxima first and
+    // eight at a time took four (6 ragged sequences of up to 9 000 tokens of 64 heads 36.2 -> 35.6 us with the append,
+    // 8 listed sets of 2 048 rows with the selection 43.5 -> 42.7). The sums run in ascending record order.
     float4 sum = {0, 0, 0, 0};
     float l_g = 0.0f;
-    if (m_g != -INFINITY) {
+    auto add = [&](float w, float l, float4 v) {
+        l_g += l * w;
+        sum.x += v.x * w, sum.y += v.y * w, sum.z += v.z * w, sum.w += v.w * w;
+    };
+    auto batch = [&](auto size, int b0, float (&m_r)[decltype(size)::value], float (&l_r)[decltype(size)::value],
+                     float4 (&v)[decltype(size)::value]) {
+#pragma unroll
+        for (int u = 0; u < decltype(size)::value; ++u) {
+            const size_t rec = (size_t)min(b0 + u, last) + seq;
+            m_r[u] = part_ml[(rec * H + head) * 2];
+            l_r[u] = part_ml[(rec * H + head) * 2 + 1];
+            v[u] = reinterpret_cast<const float4*>(part_acc + (rec * H + head) * kKvl)[threadIdx.x];
+        }
+    };
+    auto merge_one = [&](auto size) {
+        constexpr int N = decltype(size)::value;
+        float m_r[N], l_r[N], m_g = -INFINITY;
+        float4 v[N];
+        batch(size, first, m_r, l_r, v);
+#pragma unroll
+        for (int u = 0; u < N; ++u) m_g = fmaxf(m_g, m_r[u]);
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+            if (first + u <= last && m_r[u] != -INFINITY) add(exp2f(m_r[u] - m_g), l_r[u], v[u]);
+    };
+    if (last - first < 8) {
+        merge_one(std::integral_constant<int, 8>{});
+    } else if (last - first < 16) {
+        merge_one(std::integral_constant<int, 16>{});
+    } else {
+        constexpr int kBatch = 8;
+        float m_g = -INFINITY;
         for (int b0 = first; b0 <= last; b0 += kBatch) {
+            float m_r[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u)
+                m_r[u] = part_ml[((size_t)(min(b0 + u, last) + seq) * H + head) * 2];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) m_g = fmaxf(m_g, m_r[u]);
+        }
+        for (int b0 = first; b0 <= last && m_g != -INFINITY; b0 += kBatch) {
             float m_r[kBatch], l_r[kBatch];
             float4 v[kBatch];
+            batch(std::integral_constant<int, kBatch>{}, b0, m_r, l_r, v);
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const size_t rec = (size_t)min(b0 + u, last) + seq;
-                m_r[u] = part_ml[(rec * H + head) * 2];
-                l_r[u] = part_ml[(rec * H + head) * 2 + 1];
-                v[u] = reinterpret_cast<const float4*>(part_acc + (rec * H + head) * kKvl)[threadIdx.x];
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                if (b0 + u > last || m_r[u] == -INFINITY) continue;
-                const float w = exp2f(m_r[u] - m_g);
-                l_g += l_r[u] * w;
-                sum.x += v[u].x * w, sum.y += v[u].y * w, sum.z += v[u].z * w, sum.w += v[u].w * w;
-            }
+            for (int u = 0; u < kBatch; ++u)
+                if (b0 + u <= last && m_r[u] != -INFINITY) add(exp2f(m_r[u] - m_g), l_r[u], v[u]);
         }
     }
     const float inv = l_g > 0.0f ? 1.0f / l_g : 0.0f;
