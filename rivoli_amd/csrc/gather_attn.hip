@@ -521,17 +521,18 @@ __global__ __launch_bounds__(kGaThreads) void gather_attn_marked_kernel(const Ga
 
 // Split plan: o[t][head] = bf16(sum_r w_r acc_r / (sum_r w_r l_r + 2^(sink * log2 e - max m))),
 // w_r = 2^(m_r - max m), over the query's shares in ascending order. Nothing live anywhere: NaN.
+template <int kBatch>
 __global__ __launch_bounds__(128) void gather_attn_combine_kernel(
     const float* __restrict__ part_acc, const float* __restrict__ part_ml,
     const float* __restrict__ sink, int n_splits, int h, float* __restrict__ o) {
     const int head = blockIdx.x;
     const size_t t = blockIdx.y;
     const size_t rec0 = t * n_splits * h + head;
-    // Shares are fetched eight at a time, all loads of a batch in flight together (a share past
+    // Shares are fetched eight (more than eight: 16) at a time, all loads of a batch in flight together (a share past
     // the last re-reads the last and is left out), and the first batch's accumulators with its
-    // maxima: two round trips for up to eight shares instead of one per share. The sums run in
-    // ascending order. 64 heads, 10 shares: 6.0 -> 3.9 us.
-    constexpr int kBatch = 8;
+    // maxima: one round trip for up to 16 shares instead of one per share. The sums run in
+    // ascending order. 64 heads, one query, with the shares' kernel: 10 shares 11.0 -> 10.0 us, 23 shares 19.6 -> 16.4, eight
+    // at a time and 16; up to eight are no different, and no slower, in batches of eight.
     float m_r[kBatch], l_r[kBatch];
     float4 v[kBatch];
     auto fetch = [&](int r0) {
@@ -680,8 +681,12 @@ static int gather_attn_launch(const float* q, const float* kv, const float* sink
             hipLaunchKernelGGL((gather_attn_d512_kernel<1, 1>), grid, dim3(kGaThreads), 0, stream, a);
         const int rc = launch_status();
         if (rc != 0 || a.n_splits == 1) return rc;  // a split plan has fewer than 256 queries
-        hipLaunchKernelGGL(gather_attn_combine_kernel, dim3((unsigned)h, (unsigned)m), dim3(128), 0, stream,
-                           a.part_acc, a.part_ml, sink, a.n_splits, h, o);
+        if (a.n_splits <= 8)
+            hipLaunchKernelGGL(gather_attn_combine_kernel<8>, dim3((unsigned)h, (unsigned)m), dim3(128), 0, stream,
+                               a.part_acc, a.part_ml, sink, a.n_splits, h, o);
+        else
+            hipLaunchKernelGGL(gather_attn_combine_kernel<16>, dim3((unsigned)h, (unsigned)m), dim3(128), 0, stream,
+                               a.part_acc, a.part_ml, sink, a.n_splits, h, o);
         return launch_status();
     }
     // the reference launcher's limits, kept (attn.hip:450-458): d within 1024, its LDS budget
