@@ -45,9 +45,12 @@ static inline AttendPlan attend_plan(int n_seqs, int H, int max_rows) {
 }
 
 // The same for the linear slabs' one sequence, cut to what the caller's scratch holds: `fit` records of
-// which one is spare.
+// which one is spare. Up to 512 heads, where its workgroups have 16 of them (heads16_pays), a call that is cut at
+// all is cut to 128 rows a work item, where the workgroups of 64 heads want 256: 64 heads, 512 rows 16.3 -> 13.1 us, 1 024
+// 16.5 -> 13.3, 1 800 20.0 -> 16.8; 256 rows are not worth a second launch, and past 2 500 the scratch decides.
 static inline AttendPlan linear_plan(int H, int nr, int fit, bool scratch) {
     AttendPlan p = attend_plan(1, H, nr);
+    if (p.n_splits > 1 && H <= kH16Heads * kAttTargetGroups / kAttDies) p.n_splits = (nr + kTile - 1) / kTile / kH16Waves;
     if (p.n_splits > fit - 1) p.n_splits = fit - 1;
     if (!scratch || p.n_splits < 2) p.n_splits = 1;
     p.n_items = p.n_splits > 1 ? p.n_splits : 0;
