@@ -106,7 +106,7 @@ struct AttendArgs {
     size_t page_bytes;
     float qscale;                 // softmax scale * log2(e)
     int n_seqs, n_items;          // n_items > 0: tiles are dealt to that many work items
-    int by_seq;                   // and no work item has tiles of two sequences (SeqDeal)
+    int by_seq;                   // and no work item has tiles of two sequences (SeqDeal): the tiles its runs are whole numbers of, or 0
     int count_ones;               // list entries of 0xffffffff count among bad_rows
     float* clat;                  // [n_seqs][H][512]
     float* part_acc;              // [n_records][H][512]
@@ -732,8 +732,10 @@ __device__ __forceinline__ bool dealt_part(const AttendArgs& a, int item, const 
 // item each, numbered through the batch, so that no work item meets two sequences. A second part costs
 // such a workgroup its query, its first rows' latency and its waves' merge again, as much as two
 // tiles a wave, and the call lasts as long as its slowest workgroup. The longest run is the shortest whole
-// number of tiles a wave with which the work items suffice. Each wave finds it for itself, a
-// sequence a lane for the lengths and then a candidate a lane, with no barrier.
+// number of units with which the work items suffice: four tiles, or for the linear slabs, which have 15 work items at most,
+// two (64 heads, 700 rows 16.5 -> 14.7 us, 2 048 16.6 -> 15.8, 8 192 27.5 -> 26.0). In paged calls more and shorter runs
+// cost the merge as much as they save: 6 x 3 000 tokens 22.6 -> 23.1, one ragged sequence of up to 16 384 13.9 -> 15.2.
+// Each wave finds it for itself, a sequence a lane for the lengths and then a candidate a lane, with no barrier.
 // 64 heads, parity mode, ragged, the tiles dealt evenly -> so (workgroups of 64 heads): 16 x up to
 // 2 959 tokens 50.9 -> 37.5 us (47.5), 25 x 1 422 45.8 -> 32.8 (44.4),
 // 24 x 934 52.0 -> 29.4 (50.1).
@@ -748,7 +750,7 @@ __device__ __forceinline__ int ceil_quotient(int t, int c, float inv) {
     return q;
 }
 // Needs n_items >= 2 * n_seqs. `lens` null: every sequence has k rows.
-__device__ __forceinline__ SeqDeal seq_deal(const int* lens, int k, int n_seqs, int n_items) {
+__device__ __forceinline__ SeqDeal seq_deal(const int* lens, int k, int n_seqs, int n_items, int unit) {
     const int lane = threadIdx.x & (kWave - 1);
     SeqDeal d;
     const int rows = lens ? max(min(lens[min(lane, n_seqs - 1)], k), 0) : k;
@@ -759,9 +761,9 @@ __device__ __forceinline__ SeqDeal seq_deal(const int* lens, int k, int n_seqs, 
         total += __shfl_xor(total, off, kWave);
         longest = max(longest, __shfl_xor(longest, off, kWave));
     }
-    // `rounds` tiles a wave: at least what an even deal gives, and then the first that suffices
-    const int least = max((total + kH16Waves * n_items - 1) / (kH16Waves * n_items), 1);
-    const int c = (least + lane) * kH16Waves;
+    // `rounds` units: at least what an even deal gives, and then the first that suffices
+    const int least = max((total + unit * n_items - 1) / (unit * n_items), 1);
+    const int c = (least + lane) * unit;
     const float c_inv = 1.0f / (float)c;
     int items = 0;
     for (int s = 0; s < n_seqs; ++s) items += ceil_quotient(__builtin_amdgcn_readlane(d.tiles, s), c, c_inv);
@@ -770,10 +772,10 @@ __device__ __forceinline__ SeqDeal seq_deal(const int* lens, int k, int n_seqs, 
     if (enough) {
         rounds = least + __builtin_ctzll(enough);
     } else {  // sum of ceil(t / run) <= total / run + n_seqs; and a run that holds the longest is one item each
-        const int spare = kH16Waves * (n_items - n_seqs);
-        rounds = max(min((total + spare - 1) / spare, (longest + kH16Waves - 1) / kH16Waves), 1);
+        const int spare = unit * (n_items - n_seqs);
+        rounds = max(min((total + spare - 1) / spare, (longest + unit - 1) / unit), 1);
     }
-    const int run = __builtin_amdgcn_readfirstlane(rounds * kH16Waves);
+    const int run = __builtin_amdgcn_readfirstlane(rounds * unit);
     d.parts = ceil_quotient(d.tiles, run, 1.0f / (float)run);
     int upto = d.parts;
 #pragma unroll
@@ -838,7 +840,7 @@ __global__ __launch_bounds__(kH16Threads, 1) void mla_attend_heads16_kernel(cons
     int seq = item;
     if (item >= (a.n_items > 0 ? a.n_items : a.n_seqs)) return;
     if (a.by_seq) {
-        const SeqDeal d = seq_deal(MODE == kLinear ? nullptr : (MODE == kSparse ? a.n_rows : a.seq_lens), a.k, a.n_seqs, a.n_items);
+        const SeqDeal d = seq_deal(MODE == kLinear ? nullptr : (MODE == kSparse ? a.n_rows : a.seq_lens), a.k, a.n_seqs, a.n_items, a.by_seq);
         const unsigned long long past = __ballot(d.first + d.parts > item);
         if (!past) return;  // more work items than runs
         seq = __builtin_ctzll(past);
@@ -889,7 +891,7 @@ __global__ __launch_bounds__(kFewThreads) void mla_attend_few_kernel(const Atten
     int seq = item;
     if (item >= (a.n_items > 0 ? a.n_items : a.n_seqs)) return;
     if (a.by_seq) {
-        const SeqDeal d = seq_deal(MODE == kLinear ? nullptr : (MODE == kSparse ? a.n_rows : a.seq_lens), a.k, a.n_seqs, a.n_items);
+        const SeqDeal d = seq_deal(MODE == kLinear ? nullptr : (MODE == kSparse ? a.n_rows : a.seq_lens), a.k, a.n_seqs, a.n_items, a.by_seq);
         const unsigned long long past = __ballot(d.first + d.parts > item);
         if (!past) return;  // more work items than runs
         seq = __builtin_ctzll(past);
@@ -940,7 +942,7 @@ __global__ __launch_bounds__(128) void mla_attend_combine_kernel(
     int first, last;       // the sequence's work items
     long long mine = 0;    // its tiles
     if (by_seq) {
-        const SeqDeal d = seq_deal(sparse ? n_rows : seq_lens, k, n_seqs, n_items);
+        const SeqDeal d = seq_deal(sparse ? n_rows : seq_lens, k, n_seqs, n_items, by_seq);
         mine = __builtin_amdgcn_readlane(d.tiles, seq);
         first = __builtin_amdgcn_readlane(d.first, seq);
         last = first + __builtin_amdgcn_readlane(d.parts, seq) - 1;
@@ -1058,7 +1060,7 @@ static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_row
                                            MODE == kLinear);
     if (!any && a.page_bytes % 16 == 0 && route.heads16) {
         plan = route.plan;
-        a.n_items = plan.n_items, a.by_seq = route.by_seq, a.count_ones = precise > 2;
+        a.n_items = plan.n_items, a.by_seq = !route.by_seq ? 0 : MODE == kLinear ? kFewTokens / kTile : kH16Waves, a.count_ones = precise > 2;
         const int items = plan.n_items ? plan.n_items : n_seqs;
         const dim3 grid((unsigned)(((items + 7) / 8 * 8) * (long long)((a.H + kH16Heads - 1) / kH16Heads)));
         (void)hipGetLastError();
