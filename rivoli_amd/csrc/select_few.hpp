@@ -24,7 +24,8 @@ constexpr int kSfBins = 1 << kSfBits;
 constexpr int kSfCopies = 4;   // of a bin, by lane: equal scores in neighbouring lanes meet a quarter as often
 constexpr int kSfList = kWave; // members of the pivot bin that are listed: up to one a lane
 constexpr int kSfHistWords = (kSfBins + 1) * kSfCopies;  // one bin more for what is no element
-constexpr int kSfLdsWords = kSfHistWords + 2 * kSfList + 4 * kSfWaves + 4;
+constexpr int kSfFillAt = kSfHistWords + 2 * kSfList + 5 * kSfWaves;  // how far the list is filled
+constexpr int kSfLdsWords = kSfFillAt + 4;
 static_assert(kSfBins == 2 * kSfThreads && kSfCopies == 4, "a thread owns two bins of four words");
 
 // min / max over the wave, as scalars
@@ -47,10 +48,14 @@ __device__ __forceinline__ void select_few_keys(const uint32_t (&key)[ITEMS], in
     uint32_t* const hist = lds;
     uint32_t* const l_key = lds + kSfHistWords;
     uint32_t* const l_idx = l_key + kSfList;
-    uint32_t* const s_a = l_idx + kSfList;   // [16] the waves' minima, then their counts above the pivot bin
-    uint32_t* const s_b = s_a + kSfWaves;    // [16] maxima, then counts in the bin
+    uint32_t* const s_a = l_idx + kSfList;   // [16] the waves' minima
+    uint32_t* const s_b = s_a + kSfWaves;    // [16] maxima
     uint32_t* const s_tot = s_b + kSfWaves;  // [16] counts of the bins that a wave owns
-    uint32_t* const s_fill = s_tot + kSfWaves;
+    // [16] their keys above the pivot bin, and in it. Words of their own: with one value in the row no barrier stands between
+    // the waves' reading of the minima and maxima and these.
+    uint32_t* const s_gt = s_tot + kSfWaves;
+    uint32_t* const s_eq = s_gt + kSfWaves;
+    uint32_t* const s_fill = lds + kSfFillAt;
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -146,7 +151,7 @@ __device__ __forceinline__ void select_few_keys(const uint32_t (&key)[ITEMS], in
             gt += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(key[j] > hi));
             eq += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in_range(j)));  // (no use when the bin is taken whole)
         });
-        if (lane == 0) s_a[wave] = gt, s_b[wave] = eq;
+        if (lane == 0) s_gt[wave] = gt, s_eq[wave] = eq;
         if (listed && eq != 0) {  // a place in the list for the wave's members: their order there is no matter
             uint32_t at = 0;
             if (lane == 0) at = atomicAdd(s_fill, eq);
@@ -167,7 +172,7 @@ __device__ __forceinline__ void select_few_keys(const uint32_t (&key)[ITEMS], in
         const uint32_t x = lane < wave ? v[lane & (kSfWaves - 1)] : 0u;
         return wave_total(wave_inclusive_sum(x));
     };
-    uint32_t run_gt = before(s_a), run_eq = 0, here_eq = 0;  // here_eq: this wave's keys == T, where there are ties
+    uint32_t run_gt = before(s_gt), run_eq = 0, here_eq = 0;  // here_eq: this wave's keys == T, where there are ties
     if (listed) {
         const bool is = lane < (int)in_bin;
         const uint32_t k = is ? l_key[lane] - lo : 0u, i = is ? l_idx[lane] : ~0u;  // (past every wave's run)
@@ -194,8 +199,8 @@ __device__ __forceinline__ void select_few_keys(const uint32_t (&key)[ITEMS], in
         }
         run_gt += count((exact ? k >= p : k > p) && i < (uint32_t)seg0);
     } else if (!whole) {
-        run_eq = before(s_b);
-        here_eq = s_b[wave];
+        run_eq = before(s_eq);
+        here_eq = s_eq[wave];
     }
     T = (uint32_t)__builtin_amdgcn_readfirstlane((int)T);
     ties = (uint32_t)__builtin_amdgcn_readfirstlane((int)ties);
@@ -257,7 +262,7 @@ __device__ __forceinline__ void select_few(const float* __restrict__ s, int nt, 
         }
         reinterpret_cast<uint4*>(lds)[tid] = uint4{0u, 0u, 0u, 0u};
         reinterpret_cast<uint4*>(lds)[kSfThreads + tid] = uint4{0u, 0u, 0u, 0u};
-        if (tid == 0) s_b[2 * kSfWaves] = 0u;  // the list's fill
+        if (tid == 0) lds[kSfFillAt] = 0u;
         uint32_t lo = ~0u, hi = 0u;
 #pragma unroll
         for (int j = 0; j < ITEMS; ++j) {

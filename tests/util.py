@@ -67,3 +67,24 @@ def attend_route(n_seqs, H, max_rows, precise, listed=False, linear=0):
 
 
 _PLAN = None
+
+
+_WAVES = None
+
+
+def select_few_waves(scores, k, total_order, add, order):
+    """The k best of a row by rivoli_amd/csrc/select_few.hpp on the CPU, its waves in the given order between two barriers
+    (tests/native/select_few_waves.cpp); None where its barriers never end."""
+    global _WAVES
+    if _WAVES is None:
+        here = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native")
+        path = os.path.join(here, "select_few_waves.so")
+        if not os.path.exists(path):
+            subprocess.run(["make", "-C", here, path], check=True, capture_output=True)
+        _WAVES = ctypes.CDLL(path)
+    scores = np.ascontiguousarray(scores, np.float32)
+    items = next(i for i in (1, 2, 8, 16) if len(scores) <= 1024 * i)
+    out = np.full(k, 0xEEEEEEEE, np.uint32)
+    ended = _WAVES.select_few_waves(scores.ctypes.data_as(ctypes.c_void_p), len(scores), k, items, int(total_order),
+                                    ctypes.c_uint32(add), order, out.ctypes.data_as(ctypes.c_void_p))
+    return out if ended >= 0 else None
