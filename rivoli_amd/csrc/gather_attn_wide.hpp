@@ -36,12 +36,12 @@ constexpr int kGwColTiles = kGaD / 32;          // 16 output column tiles
 constexpr int kGwRing = 4;                      // rows on their way to a wave: 32 registers
 constexpr int kGwSmemBytes = 2 * kGaTileBytes + 16;
 static_assert(2 * kGwSmemBytes <= 160 * 1024, "two workgroups a compute unit");
-// The reference maximum of a head is set kGwHead above a tile's maximum (log2 units) and moved when a later
-// maximum passes it by kGwGrow, a window of 100: moving it scales 256 sums through ordinary
-// registers (6000 cycles, more than a tile), and a window of 8 moves it for every outlier row. Weights lie
-// in 2^-40 .. 2^60, f32 sums of |kv| up to 2^57 in range; hi + lo of a weight have its exponent, so the
-// window costs no precision.
-constexpr float kGwHead = 40.0f, kGwGrow = 60.0f;
+// The reference maximum of a head is a tile's maximum (log2 units), moved when a later maximum passes it by kGwGrow:
+// moving it scales 256 sums through ordinary registers (6000 cycles, more than a tile), and a window of 8, the
+// other kernels', moves it for every outlier row. A head's largest weight lies in 2^0 .. 2^100; hi + lo of a weight have its
+// exponent, so the window costs no precision. What it costs is range: sums of weights of 2^100 overflow where
+// |kv| passes 2^17. Such a query is done again with the window of 8, and gives what the other kernels give.
+constexpr float kGwGrow = 100.0f;
 
 // Row of a tile buffer (1040 bytes a row) that holds slot s: sixteen lanes of a 16-byte read (slots 0-3, 12-15, 20-23,
 // 24-27, then the rest) meet in no bank, and so do the four slots of a transposing read, 64 bytes each.
@@ -98,11 +98,12 @@ struct GwList {
     }
 };
 
-// A wave's 32 heads (qh, B operand fragments) over the whole list, results to o.
+// A wave's 32 heads (qh, B operand fragments) over the whole list, results to o. False where the workgroup's
+// results are not all in range and a narrower window may have them so.
 template <int PSPLIT>
-__device__ __forceinline__ void gather_attn_wide_pass(const GatherAttnArgs& a, lds_ptr<uint8_t> kr, size_t t, int head0,
+__device__ __forceinline__ bool gather_attn_wide_pass(const GatherAttnArgs& a, lds_ptr<uint8_t> kr, size_t t, int head0,
                                                       const bf16x8 (&qh)[kGwKSteps], const GwList& list,
-                                                      int f0, int f1, int f2) {
+                                                      int f0, int f1, int f2, float window) {
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));  // what the lane's number gives is worked out here, not kept through the prologue
     const int lane = tid & 63;
@@ -209,10 +210,10 @@ __device__ __forceinline__ void gather_attn_wide_pass(const GatherAttnArgs& a, l
             auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
             tmax = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1])) * qs;
         }
-        const bool grow = tmax > m_ref + kGwGrow;  // false while everything is masked
+        const bool grow = tmax > m_ref + window;  // false while everything is masked
         if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-            const float corr = grow ? __builtin_amdgcn_exp2f(m_ref - (tmax + kGwHead)) : 1.0f;  // 2^-inf = 0 at first
-            if (grow) m_ref = tmax + kGwHead;
+            const float corr = grow ? __builtin_amdgcn_exp2f(m_ref - tmax) : 1.0f;  // 2^-inf = 0 at first
+            if (grow) m_ref = tmax;
             l_sum *= corr;
 #pragma unroll
             for (int c = 0; c < kGwColTiles; ++c) {
@@ -303,12 +304,18 @@ __device__ __forceinline__ void gather_attn_wide_pass(const GatherAttnArgs& a, l
     // columns at a time measured 2 us more a workgroup). Columns 32 c + 8 u + 4 g .. +3 of the products are dims
     // 4 (4 c + u) + 256 g .. +3: a staged row holds dims 4 lane .. and 256 + 4 lane .. side by side.
     const lds_ptr<uint8_t> own = kr + wave * kGaTileBytes;
+    float most = 0.0f;  // the largest result, NaN where one is (the instruction takes three operands: half of one a result)
 #pragma unroll
     for (int c = 0; c < kGwColTiles; ++c) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const u32x2 w = {pack_bf16x2(o[c][4 * u] * l_inv, o[c][4 * u + 1] * l_inv),
-                             pack_bf16x2(o[c][4 * u + 2] * l_inv, o[c][4 * u + 3] * l_inv)};
+            float x[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = o[c][4 * u + i] * l_inv;
+#pragma unroll
+            for (int i = 0; i < 4; i += 2)
+                most = __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(x[i]), fabsf(x[i + 1])), most);
+            const u32x2 w = {pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3])};
             *(lds_ptr<u32x2>)(own + n32 * kGaRowBytes + 8 * (4 * c + u) + 512 * g) = w;
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -325,6 +332,13 @@ __device__ __forceinline__ void gather_attn_wide_pass(const GatherAttnArgs& a, l
                 f32x4{bf16_lo_to_f32(w.x), bf16_hi_to_f32(w.x), bf16_lo_to_f32(w.y), bf16_hi_to_f32(w.y)};
         }
     }
+    // Sums that overflowed, or a sink so far above the reference maximum that the quotient's factor is no normal number.
+    if (window == kLazyRescale || list.end_tile == 0) return true;
+    const lds_ptr<int> over = (lds_ptr<int>)(kr + 2 * kGaTileBytes) + 2;
+    const bool bad = __builtin_amdgcn_ballot_w64(!(most < INFINITY && l_inv >= 0x1p-126f)) != 0;
+    if (lane == 0) over[wave] = bad;
+    __syncthreads();  // (and both buffers are read)
+    return __builtin_amdgcn_readfirstlane(over[0] | over[1]) == 0;
 }
 
 // QSPLIT 2 keeps what bf16 leaves of a query that is not bf16-valued. The model's query is (its rotary stores bf16,
@@ -336,13 +350,13 @@ __device__ __forceinline__ void gather_attn_wide_pass(const GatherAttnArgs& a, l
 constexpr uint32_t kGwMark = 0x7fc0a55au;
 
 template <int QSPLIT, int PSPLIT>
-__global__ __launch_bounds__(kGwThreads, 1) void gather_attn_wide_kernel(const GatherAttnArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t smem[kGwSmemBytes];
-    const lds_ptr<uint8_t> kr = (lds_ptr<uint8_t>)smem;
+__device__ __forceinline__ bool gather_attn_wide_query(const GatherAttnArgs& a, lds_ptr<uint8_t> kr, float window) {
     const lds_ptr<int> flag = (lds_ptr<int>)(kr + 2 * kGaTileBytes);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // nothing of it is kept for a second time
     const size_t t = blockIdx.x;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 5, n32 = lane & 31;
     const int head0 = blockIdx.y * 64 + kGwHeads * wave;
     const global_bytes q_at = (global_bytes)(uintptr_t)(a.q + t * a.h * kGaD);
@@ -384,7 +398,7 @@ __global__ __launch_bounds__(kGwThreads, 1) void gather_attn_wide_kernel(const G
         ask_query(v, 0);
         if (QSPLIT == 2 && __builtin_amdgcn_ballot_w64((first.bits() & 0xffffu) != 0) != 0) {  // the same in both waves
             if (threadIdx.x == 0) *mark = kGwMark;
-            return;
+            return true;
         }
         stage_query(v, 0);
         ask_query(v, 16);
@@ -424,9 +438,16 @@ __global__ __launch_bounds__(kGwThreads, 1) void gather_attn_wide_kernel(const G
     __syncthreads();  // the query is read: the first tile may take its place
     if (QSPLIT == 2 && __builtin_amdgcn_readfirstlane(flag[0] | flag[1]) != 0) {
         if (threadIdx.x == 0) *mark = kGwMark;
-        return;
+        return true;
     }
-    gather_attn_wide_pass<PSPLIT>(a, kr, t, head0, qh, list, f0, f1, f2);
+    return gather_attn_wide_pass<PSPLIT>(a, kr, t, head0, qh, list, f0, f1, f2, window);
+}
+
+template <int QSPLIT, int PSPLIT>
+__global__ __launch_bounds__(kGwThreads, 1) void gather_attn_wide_kernel(const GatherAttnArgs a) {
+    __shared__ __attribute__((aligned(16))) uint8_t smem[kGwSmemBytes];
+    // (the second time from the query on: kept for it through the epilogue, its 128 registers would spill)
+    for (float window = kGwGrow; !gather_attn_wide_query<QSPLIT, PSPLIT>(a, (lds_ptr<uint8_t>)smem, window);) window = kLazyRescale;
 }
 
 }  // namespace rk

@@ -7,7 +7,7 @@ import pytest
 
 from rivoli_amd import hip
 from tests.gpu_util import back, dev, dzeros, need_ref
-from tests.v4_cases import attend_inputs, sparse_attn_f64
+from tests.v4_cases import attend_inputs, bf16_round, sparse_attn_f64
 
 pytestmark = pytest.mark.gpu
 ATTEND_TOL = 1.0 / 128.0
@@ -114,6 +114,35 @@ def test_many_queries(oracle, m, h, topk, precise, scale, q_scale, remainder):
         assert np.all(np.abs(got[pick] - exact) <= 2.0 ** -8 * np.abs(exact) + 2.0 ** -10 * top), \
             float(np.max(np.abs(got[pick] - exact)))
     # a query's result does not depend on how many others there are: the kernel of few queries agrees with it
+    few = device_attend(q[pick], kv, sink, idx[pick], scale, precise=precise, n_kv=rows)
+    assert worst_rel(few, got[pick]) <= 2.0 ** -7
+
+
+@pytest.mark.parametrize("precise", [2, 0])
+@pytest.mark.parametrize("power,rise,sink_at", [(-100, 0, 0), (100, 0, 0), (100, 90, 0), (0, 90, 0), (0, 90, 200), (-60, 99, 60)])
+def test_many_queries_keep_the_range_of_few(oracle, power, rise, sink_at, precise):
+    """The kernel of 32 heads a wave lets a head's weights grow by 2^100 before it moves the maximum they refer to. Rows of
+    2^-100 and of 2^100; logits that rise by `rise` (log2 units) after the first tile, with rows whose sums overflow under such
+    weights; a sink `sink_at` above the first logits, under which such sums are no normal number. Each is what it is in a
+    call of few queries: within bf16's rounding of the value in 64 bits."""
+    m, h, topk, rows, scale = 258, 33, 96, 200, 512 ** -0.5
+    q, kv, sink = attend_inputs(oracle, m, h, 512, rows, seed=17)
+    kv[:, 0] = 0.0
+    kv[rows // 2:, 0] = 1.0
+    q[:, :, 0] = bf16_round(np.float32(rise / (scale * np.log2(np.e))))
+    kv, q = np.ldexp(kv, power), np.ldexp(q, -power)
+    sink = sink + np.float32(sink_at * np.log(2.0))
+    rng = np.random.default_rng(power + 200)
+    idx = rng.integers(0, rows, (m, topk)).astype(np.int32)
+    idx[:, :32] %= rows // 2
+    idx[::5, 40] = -1
+    got = device_attend(q, kv, sink, idx, scale, precise=precise, n_kv=rows)
+    pick = [0, 1, 2, m // 2, m - 1]
+    exact = sparse_attn_f64(q[pick], kv, sink, idx[pick], scale)
+    top = np.abs(exact).max()
+    assert top > 0
+    bound = 2.0 ** -8 * np.abs(exact) + 2.0 ** -10 * top if precise == 2 else ATTEND_TOL * top
+    assert np.all(np.abs(got[pick] - exact) <= bound), float(np.max(np.abs(got[pick] - exact)) / top)
     few = device_attend(q[pick], kv, sink, idx[pick], scale, precise=precise, n_kv=rows)
     assert worst_rel(few, got[pick]) <= 2.0 ** -7
 
