@@ -31,6 +31,7 @@
 // one the queries that it leaves; calls of up to 256 workgroups of 16 heads a third (gather_attn_few.hpp).
 // Launch-only; see include/rivoli_kvcache.h for the contract.
 #include "attend_common.hpp"
+#include "gather_attn_plan.hpp"
 
 namespace rk {
 
@@ -81,7 +82,6 @@ struct GatherAttnArgs {
 // How many workgroups share one query's list: a pure function of the call's shape. Splitting
 // pays when the queries alone cannot fill the part (decode: one query) and a share still
 // holds a couple of tiles.
-constexpr int kGaTargetGroups = 256;
 constexpr int kGaMinTilesPerSplit = 2;
 constexpr int kGaMaxSplits = 32;
 static inline int gather_attn_splits(int m, int h, int topk) {
@@ -127,7 +127,8 @@ __device__ __forceinline__ void gather_attn_d512(const GatherAttnArgs& a, uint8_
     const lds_ptr<float> sbias = (lds_ptr<float>)(kr + kGaBufs * kGaTileBytes);  // [kGaBufs][32]: 0 or -inf
     const lds_ptr<f32x4> xch = (lds_ptr<f32x4>)(sbias + kGaBufs * kGaTile);  // [2 parities][8 waves][64 lanes][2]
 
-    const int tid = threadIdx.x;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // worked out here, not kept from one block to the next
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hw = wave & 3;     // which 16 heads of the block
@@ -488,31 +489,39 @@ __global__ __launch_bounds__(kGaThreads) void gather_attn_d512_kernel(const Gath
     gather_attn_d512<QSPLIT, PSPLIT>(a, smem, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
-// The blocks that the kernel of 32 heads a wave marked, one after another: a workgroup looks at 512 marks at a time,
-// which is all that it does when there are none (8192 queries: 3 us).
+// The blocks that the kernel of 32 heads a wave marked: a workgroup does those that are its own (marked_block), one after
+// another. No other looks at their marks, which its results replace. It looks at 512 marks at a time, which is all
+// that it does when there are none (2 us behind the other kernel).
+// All of 8192 queries x 640 slots marked 1772 -> 1720 us with the other kernel's look at them (1645 without), every 256th
+// 2815 -> 1177, each as dealt to group block mod 256 by addresses in vector registers -> so.
 template <int QSPLIT, int PSPLIT>
 __global__ __launch_bounds__(kGaThreads) void gather_attn_marked_kernel(const GatherAttnArgs a, long long blocks, int per_query) {
     __shared__ __attribute__((aligned(16))) uint8_t smem[kGaSmemBytes];
     __shared__ uint64_t marked[kGaWaves];
-    for (long long base = 0; base < blocks; base += (long long)gridDim.x * kGaThreads) {
-        const long long mine = base + (long long)threadIdx.x * gridDim.x + blockIdx.x;
+    const unsigned rows = (unsigned)((blocks + kGaTargetGroups - 1) / kGaTargetGroups);
+    for (unsigned row0 = 0; row0 < rows; row0 += kGaThreads) {
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));  // nothing of it is kept through a block's work
+        const long long mine = marked_block(row0 + tid, blockIdx.x);
         bool is = false;
         if (mine < blocks) {
             const size_t t = mine / per_query;
-            const int hb = mine % per_query;
-            is = reinterpret_cast<const uint32_t*>(a.o)[(t * a.h + hb * 64) * kGaD] == kGwMark;
+            is = reinterpret_cast<const uint32_t*>(a.o)[(t * a.h + (mine - t * per_query) * 64) * kGaD] == kGwMark;
         }
         const uint64_t word = __builtin_amdgcn_ballot_w64(is);
         __syncthreads();  // the words of the round before are read
-        if ((threadIdx.x & 63) == 0) marked[threadIdx.x >> 6] = word;
+        if ((tid & 63) == 0) marked[tid >> 6] = word;
         __syncthreads();
         for (int w = 0; w < kGaWaves; ++w) {
-            uint64_t todo = marked[w];
-            while (todo != 0) {
-                const int bit = __builtin_ctzll(todo);
-                todo &= todo - 1;
-                const long long block = base + (long long)(64 * w + bit) * gridDim.x + blockIdx.x;
-                gather_attn_d512<QSPLIT, PSPLIT>(a, smem, block / per_query, (int)(block % per_query), 0);
+            const uint64_t m = marked[w];
+            uint32_t lo = __builtin_amdgcn_readfirstlane((int)m), hi = __builtin_amdgcn_readfirstlane((int)(m >> 32));
+            while ((lo | hi) != 0) {
+                const unsigned bit = lo != 0 ? __builtin_ctz(lo) : 32 + __builtin_ctz(hi);
+                if (lo != 0) lo &= lo - 1;
+                else hi &= hi - 1;
+                const long long block = marked_block(row0 + 64 * w + bit, blockIdx.x);
+                const long long t = block / per_query;
+                gather_attn_d512<QSPLIT, PSPLIT>(a, smem, (size_t)t, (int)(block - t * per_query), 0);
                 __syncthreads();  // its LDS is read
             }
         }
@@ -646,13 +655,16 @@ static int gather_attn_launch(const float* q, const float* kv, const float* sink
         a.part_ml = partial ? partial + (size_t)m * a.n_splits * h * kGaD : nullptr;
         const dim3 grid((unsigned)m, (unsigned)((h + 63) / 64), (unsigned)a.n_splits);
         // Past a workgroup of 64 heads a compute unit, two of half the waves fit one (gather_attn_wide.hpp): 300 queries of
-        // 640 slots 101 -> 62 us, 520 153 -> 127, 8192 1624 -> 1044. Up to there a query is the faster the more waves it
-        // has (200 queries 54 us against 58), and a list of one tile has nothing to overlap (520 queries of
-        // 20 slots 43 us against 44). A scale of 0 gives a masked slot's -inf no weight there, and
-        // marks in o may not fall on a query that is still to be read.
+        // 640 slots 96 -> 62 us, 520 145 -> 127, 8192 1578 -> 1163; of 128 slots 257 34.5 -> 28.7, 600 57 -> 53. Up to there a
+        // query is the faster the more waves it has (200 queries 54 us against 58). A list of one or two tiles has little
+        // to overlap (64 slots: 600 queries 45.7 us against 48.5, 1000 66 and 61, 2049 151 and 141, 8192 542 and 448).
+        // A call whose queries all have a remainder past bf16 pays for the other kernel's look at them, 7 to 13 us and 5 %
+        // (640 slots: 300 queries 97 -> 102 us, 600 149 -> 160, 8192 1645 -> 1720; 1000 of 64 slots 66 -> 80, which is the other
+        // half of that line); one with a few of them for their pass (one in 256: 300 queries 96 -> 110, 520 145 -> 171, 2048 409 -> 349).
+        // A scale of 0 gives a masked slot's -inf no weight there, and marks in o may not fall on a query that is still to be read.
         const long long blocks = (long long)m * grid.y;
         const uintptr_t q0 = (uintptr_t)q, o0 = (uintptr_t)o, bytes = (uintptr_t)m * h * kGaD * sizeof(float);
-        const bool wide = a.n_splits == 1 && blocks > kGaTargetGroups && topk > kGwTile && fabsf(scale) > 0.0f && fabsf(scale) < INFINITY &&
+        const bool wide = a.n_splits == 1 && blocks > kGaTargetGroups && topk > (blocks > 8 * kGaTargetGroups ? 1 : 2) * kGwTile && fabsf(scale) > 0.0f && fabsf(scale) < INFINITY &&
                           (q0 + bytes <= o0 || o0 + bytes <= q0);
         if (few) {
             const dim3 few_grid((unsigned)m, (unsigned)((h + kGfHeads - 1) / kGfHeads), (unsigned)a.n_splits);

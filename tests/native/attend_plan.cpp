@@ -1,4 +1,5 @@
-// The attention launchers' routing rules (rivoli_amd/csrc/mla_attend_plan.hpp) as a C function.
+// The attention launchers' routing rules (rivoli_amd/csrc/mla_attend_plan.hpp, gather_attn_plan.hpp) as C functions.
+#include "../../rivoli_amd/csrc/gather_attn_plan.hpp"
 #include "../../rivoli_amd/csrc/mla_attend_plan.hpp"
 
 // 1: workgroups of 16 heads, 0: of 64. out: items, by_seq, records of the route; items, records the
@@ -11,3 +12,5 @@ extern "C" int attend_route(int n_seqs, int H, int max_rows, int precise, int li
     out[3] = plan.n_items, out[4] = plan.n_records;
     return r.heads16;
 }
+
+extern "C" long long marked_block(unsigned row, unsigned group) { return rk::marked_block(row, group); }

@@ -1,8 +1,9 @@
 """Which kernel an attention call takes and how its tiles are shared
 (rivoli_amd/csrc/mla_attend_plan.hpp, compiled for the host by tests/native/Makefile)."""
+import numpy as np
 import pytest
 
-from tests.util import attend_route
+from tests.util import attend_route, marked_block
 
 
 @pytest.mark.parametrize("listed", [False, True])
@@ -101,3 +102,19 @@ def test_list_positions_looked_up_ahead_stay_in_the_list(r_end):
                 assert min(wrapped(tile * 32 + lane, False), r_end - 1) in range(r_end)
     if r_end > 2 ** 31 - 384:
         assert min(wrapped((n_tiles + 11) * 32, True), r_end - 1) < 0
+
+
+def test_blocks_left_to_a_second_pass_spread_over_its_groups():
+    """The index-list attention's second pass: every block is one group's, all blocks are dealt evenly, and of blocks at
+    any regular distance (a remainder in every 256th query) the fullest group has a few more than its share, not all."""
+    rows = 32
+    owner = np.full(rows * 256, -1)
+    for row in range(rows):
+        for group in range(256):
+            block = marked_block(row, group)
+            assert block // 256 == row and owner[block] == -1
+            owner[block] = group
+    assert marked_block(2 ** 24, 7) // 256 == 2 ** 24
+    for stride in range(1, 2049):
+        most = np.bincount(owner[::stride]).max()
+        assert most <= -(-len(owner[::stride]) // 256) + 6, stride

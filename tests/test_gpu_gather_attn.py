@@ -79,13 +79,15 @@ def test_queries_with_and_without_a_bf16_remainder_in_one_call(oracle):
 
 
 @pytest.mark.parametrize("m,h,topk,precise,scale,q_scale,remainder", [
-    (257, 64, 33, 2, 512 ** -0.5, 1.0, False),      # two tiles, the second of one slot
+    (2060, 3, 33, 2, 512 ** -0.5, 1.0, False),      # two tiles, the second of one slot: past 2048 workgroups
+    (2049, 5, 64, 2, 512 ** -0.5, 1.0, True), (257, 64, 65, 2, 512 ** -0.5, 1.0, False), (1025, 100, 34, 1, 512 ** -0.5, 1.0, True),
+    (257, 64, 33, 2, 512 ** -0.5, 1.0, False),
     (300, 5, 64, 2, 512 ** -0.5, 1.0, False), (260, 40, 640, 2, 512 ** -0.5, 1.0, False),
     (130, 100, 129, 1, 512 ** -0.5, 1.0, False), (513, 33, 96, 0, 512 ** -0.5, 1.0, False),
     (257, 64, 577, 2, 512 ** -0.5, 30.0, False),    # logits far apart: the reference maximum moves
     (257, 64, 200, 2, -0.05, 1.0, False),
     (260, 64, 100, 2, 512 ** -0.5, 1.0, True), (130, 100, 129, 1, 512 ** -0.5, 1.0, True),
-    # up to 256 workgroups of 64 heads (one tile of more of them): the kernel of 16 heads and half the dims a wave
+    # up to 256 workgroups of 64 heads (one or two tiles of more of them): the kernel of 16 heads and half the dims a wave
     (100, 64, 200, 2, 512 ** -0.5, 1.0, True), (70, 128, 97, 1, 512 ** -0.5, 1.0, False), (300, 64, 31, 2, 512 ** -0.5, 1.0, True)])
 def test_many_queries(oracle, m, h, topk, precise, scale, q_scale, remainder):
     """More than 256 workgroups of 64 heads: the kernel of 32 heads a wave, and the one below that. Masked slots anywhere, lists
@@ -173,6 +175,34 @@ def test_workgroups_of_16_heads(oracle, m, h, topk, precise, share):
     top = np.abs(exact).max()
     bound = 2.0 ** -8 * np.abs(exact) + 2.0 ** -10 * top if precise == 2 else ATTEND_TOL * top
     assert np.all(np.abs(got[pick] - exact) <= bound), float(np.max(np.abs(got[pick] - exact)))
+
+
+@pytest.mark.parametrize("m,h,topk,precise", [(131200, 1, 65, 2), (1200, 100, 40, 1)])
+def test_queries_with_a_remainder_anywhere_in_a_large_call(m, h, topk, precise):
+    """The second pass looks at 512 rows of 256 blocks at a time (131 072 blocks, and some) and has one block in each: every
+    query is done, by that pass or before it, as in a call of its own neighbours alone."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m)
+    rand = lambda *n: torch.randn(*n, generator=g, device="cuda")
+    d, rows = 512, 400
+    q, kv, sink = rand(m, h, d).bfloat16().float(), rand(rows, d).bfloat16().float(), rand(h)
+    idx = torch.randint(-40, rows, (m, topk), generator=g, device="cuda", dtype=torch.int32).clamp_(min=-1)
+    idx[:, 0] = 3
+    left = torch.rand(m, generator=g, device="cuda") < 0.02
+    left[::256] = left[-150:] = True
+    q[left, -1] += rand(int(left.sum()), d) * 2.0 ** -12
+    out = torch.full((m, h, d), float("nan"), device="cuda")
+    launch = lambda a, b, o: hip.launch_gather_attn_shared_kv(
+        q[a:b], kv, sink, idx[a:b], b - a, h, d, topk, d ** -0.5, o, torch.cuda.current_stream().cuda_stream, n_kv=rows, precise=precise)
+    launch(0, m, out)
+    assert not (out.view(torch.int32) & 0xFFFF).any()          # bf16 values: no mark is left
+    step = 250 // -(-h // 64)
+    starts = [*range(0, 1000, step), m // 2, *range(m - 700, m - step, step), m - step] if m > 10000 else [*range(0, m - step, step), m - step]
+    for a in starts:
+        want = torch.empty(step, h, d, device="cuda")
+        launch(a, a + step, want)
+        assert float((out[a:a + step] - want).abs().max() / want.abs().max()) <= 2.0 ** -7, a
 
 
 def test_many_queries_in_place(oracle):

@@ -54,7 +54,7 @@ class AttendRoute:
         self.items, self.by_seq, self.records, self.scratch_items, self.scratch_records = list(out)
 
 
-def attend_route(n_seqs, H, max_rows, precise, listed=False, linear=0):
+def _plan():
     global _PLAN
     if _PLAN is None:
         here = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native")
@@ -62,8 +62,18 @@ def attend_route(n_seqs, H, max_rows, precise, listed=False, linear=0):
         if not os.path.exists(path):
             subprocess.run(["make", "-C", here, path], check=True, capture_output=True)
         _PLAN = ctypes.CDLL(path)
+        _PLAN.marked_block.restype = ctypes.c_longlong
+    return _PLAN
+
+
+def attend_route(n_seqs, H, max_rows, precise, listed=False, linear=0):
     out = (ctypes.c_int * 5)()
-    return AttendRoute(_PLAN.attend_route(n_seqs, H, max_rows, precise, int(listed), linear, out), out)
+    return AttendRoute(_plan().attend_route(n_seqs, H, max_rows, precise, int(listed), linear, out), out)
+
+
+def marked_block(row, group):
+    """rivoli_amd/csrc/gather_attn_plan.hpp: the group's block in a row of 256."""
+    return _plan().marked_block(row, group)
 
 
 _PLAN = None
