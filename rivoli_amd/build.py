@@ -26,12 +26,13 @@ EXTRA_FLAGS = {"mla_attend.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 HOST_SOURCES = ["pagepool.cpp"]
 # Kernels whose design rests on "no scratch memory": source file -> (substring of the mangled
 # name, suffix of it) of each family. The 8-bit attention kernels and those of 16 heads a workgroup
-# run one wave per SIMD on the whole register file and order their own LDS transfers (hand-placed
-# waits, an m0 swap around each transfer): a build of them that spills is a different program, so
-# the build refuses to produce one (a compile without EXTRA_FLAGS, an ablation with a piece
-# compiled out).
+# run one wave per SIMD on the whole register file, or two on half of it each, and order their own LDS transfers
+# (hand-placed waits, an m0 swap around each transfer; a reload would be waited for with them): a build of them that
+# spills is a different program, so the build refuses to produce one (a compile without EXTRA_FLAGS, an ablation
+# with a piece compiled out).
 NO_SCRATCH = {"mla_attend.hip": [("mla_attend_paged_kernel", "Lb1EEEvNS_10AttendArgsE"),
-                                 ("mla_attend_heads16_kernel", "EEEvNS_10AttendArgsE")]}
+                                 ("mla_attend_heads16_kernel", "EEEvNS_10AttendArgsE"),
+                                 ("mla_attend_few_kernel", "EEEvNS_10AttendArgsE")]}
 
 
 def check_resources(k: str, report: str) -> None:
