@@ -840,7 +840,7 @@ __global__ __launch_bounds__(kH16Threads, 1) void mla_attend_heads16_kernel(cons
     int seq = item;
     if (item >= (a.n_items > 0 ? a.n_items : a.n_seqs)) return;
     if (a.by_seq) {
-        const SeqDeal d = seq_deal(MODE == kLinear ? nullptr : (MODE == kSparse ? a.n_rows : a.seq_lens), a.k, a.n_seqs, a.n_items, a.by_seq);
+        const SeqDeal d = seq_deal(MODE == kSparse ? a.n_rows : a.seq_lens, a.k, a.n_seqs, a.n_items, a.by_seq);
         const unsigned long long past = __ballot(d.first + d.parts > item);
         if (!past) return;  // more work items than runs
         seq = __builtin_ctzll(past);
@@ -1065,19 +1065,19 @@ static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_row
         const dim3 grid((unsigned)(((items + 7) / 8 * 8) * (long long)((a.H + kH16Heads - 1) / kH16Heads)));
         (void)hipGetLastError();
         constexpr int M = MODE == kDensePaged ? kDense : MODE;  // the rows are looked up one by one
-        const bool few = route.few;  // (always, for the linear slabs)
+        const bool few = route.few;
         const dim3 block(few ? kFewThreads : kH16Threads);
-        if (precise >= 2 || MODE == kLinear) {
+        if constexpr (MODE == kLinear) {  // always the eight waves on a tile (heads16_few)
+            hipLaunchKernelGGL((mla_attend_few_kernel<2, 2, kLinear>), grid, dim3(kFewThreads), 0, st, a);
+        } else if (precise >= 2) {
             if (few) hipLaunchKernelGGL((mla_attend_few_kernel<2, 2, M>), grid, block, 0, st, a);
             else hipLaunchKernelGGL((mla_attend_heads16_kernel<2, 2, M>), grid, block, 0, st, a);
-        } else if constexpr (MODE != kLinear) {
-            if (precise == 1) {
-                if (few) hipLaunchKernelGGL((mla_attend_few_kernel<2, 1, M>), grid, block, 0, st, a);
-                else hipLaunchKernelGGL((mla_attend_heads16_kernel<2, 1, M>), grid, block, 0, st, a);
-            } else {
-                if (few) hipLaunchKernelGGL((mla_attend_few_kernel<1, 1, M>), grid, block, 0, st, a);
-                else hipLaunchKernelGGL((mla_attend_heads16_kernel<1, 1, M>), grid, block, 0, st, a);
-            }
+        } else if (precise == 1) {
+            if (few) hipLaunchKernelGGL((mla_attend_few_kernel<2, 1, M>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((mla_attend_heads16_kernel<2, 1, M>), grid, block, 0, st, a);
+        } else {
+            if (few) hipLaunchKernelGGL((mla_attend_few_kernel<1, 1, M>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((mla_attend_heads16_kernel<1, 1, M>), grid, block, 0, st, a);
         }
         return attend_merge(a, plan, n_seqs, max_rows, seq_lens, n_rows, listed, st);
     }

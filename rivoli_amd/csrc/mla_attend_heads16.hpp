@@ -2,7 +2,7 @@
 // chip idle on, or keep for a few tiles only: the same arithmetic (bf16 matrix instructions, q
 // and the weights as bf16 hi + lo in the parity mode), dealt the other way. Included by
 // mla_attend.hip. Long work items of few heads take it (heads16_few); the others, and the linear slabs, take
-// mla_attend_few.hpp.
+// mla_attend_few.hpp, which came later: figures of other calls here are from before that.
 //
 // There a workgroup's eight waves share one tile: two of them meet in LDS over every score, and
 // a barrier ends every tile. A short call is then a chain — list entry, table, rows, staging,
@@ -18,8 +18,7 @@
 // quarter of the LDS traffic of a tile staged as bf16, which is what a first form of this kernel
 // was bound by (16 heads use a tile a quarter as often as 64 do).
 // Measured, parity mode, 64 heads, with the merge of the records: one sequence of 4 096 tokens
-// 34.5 -> 21 us, 8 x 2 048 listed rows 38 -> 24 us, one token over 2 048 rows of the linear slabs
-// 52 -> 20.7 us. A wave of two listed tiles lives 39 500 cycles, by counter: matrix instructions (272)
+// 34.5 -> 21 us, 8 x 2 048 listed rows 38 -> 24 us. A wave of two listed tiles lives 39 500 cycles, by counter: matrix instructions (272)
 // 4 350, vector instructions 11 700, waits 17 100 (the first rows, the merge), the rest transfers, LDS and
 // scalar instructions.
 #pragma once
@@ -33,34 +32,28 @@ constexpr int kH16Chunks = kKSteps / 2;  // 16-byte pieces of a row per lane gro
 // A wave's tile in LDS: rows of codes with one 16-byte granule of padding, so that sixteen rows'
 // 16-byte reads meet in no bank, and the second sixteen rows 128 bytes further on, so that the
 // transposing reads, which take rows r and r + 16 together, do not either.
-// LINEAR: the slabs' roped keys are bf16 and sit in an area of their own.
-template <bool LINEAR>
 struct H16Tile {
-    static constexpr int kGranules = (LINEAR ? kKvl : kRowW) / 16 + 1;  // of a row
+    static constexpr int kGranules = kRowW / 16 + 1;  // of a row
     static constexpr int kRow = kGranules * 16;
-    static constexpr int kGap = 8;                                      // granules between the halves
+    static constexpr int kGap = 8;                    // granules between the halves
     static constexpr int kAll = kTile * kGranules + kGap;
     static constexpr int kBytes = kAll * 16;
     static constexpr int kRequests = (kAll + kWave - 1) / kWave;
-    static constexpr int kRopeRow = kRopeW * 2 + 16;
-    static constexpr int kRopeBytes = LINEAR ? kTile * kRopeRow : 0;
-    static constexpr int kWaveBytes = 2 * kBytes + kRopeBytes;
+    static constexpr int kWaveBytes = 2 * kBytes;
     static __device__ __forceinline__ int at(int row) { return row * kRow + (row >> 4) * (kGap * 16); }
 };
-static_assert(kH16ColTiles * kWave * 16 <= 2 * H16Tile<true>::kBytes && kH16ColTiles * kWave * 16 <= 2 * H16Tile<false>::kBytes,
-              "a wave's accumulators pass through its tiles' room");
-static_assert(5 * 2048 <= H16Tile<true>::kBytes, "five K-steps of the query's operands fit a second buffer");
+static_assert(kH16ColTiles * kWave * 16 <= 2 * H16Tile::kBytes, "a wave's accumulators pass through its tiles' room");
+static_assert(5 * 2048 <= H16Tile::kBytes, "five K-steps of the query's operands fit a second buffer");
 
 // One part of a workgroup's work, as attend_part: rows [r_begin, r_end) of sequence `seq`, heads
 // 16 * hg .. +15.
 template <int QSPLIT, int PSPLIT, int MODE>
 __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq, int hg, int r_begin, int r_end,
                                                     bool whole, float* pa, float* pml) {
-    constexpr bool LINEAR = MODE == kLinear;
-    static_assert(!LINEAR || (QSPLIT == 2 && PSPLIT == 2), "the linear slabs run in the parity mode");
-    using T = H16Tile<LINEAR>;
+    static_assert(MODE == kDense || MODE == kSparse, "paged rows, looked up one by one");
+    using T = H16Tile;
     __shared__ __attribute__((aligned(16))) uint8_t smem[kH16Waves * T::kWaveBytes];
-    __shared__ __attribute__((aligned(16))) float token_scale[kH16Waves][kTile * (LINEAR ? 4 : 1)];
+    __shared__ __attribute__((aligned(16))) float token_scale[kH16Waves][kTile];
     __shared__ float wave_ml[kH16Waves][kH16Heads][2];
 
     const int tid = threadIdx.x;
@@ -70,13 +63,12 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
     const int n_tiles = (r_end - r_begin + kTile - 1) / kTile;
     const lds_ptr<uint8_t> room = (lds_ptr<uint8_t>)smem;
     const lds_ptr<uint8_t> own = room + wave * T::kWaveBytes;
-    const lds_ptr<uint8_t> ropes = own + 2 * T::kBytes;
     const lds_ptr<float> scl_lds = (lds_ptr<float>)token_scale[wave];
 
     // ---- where a tile's rows are: lane r < 32 resolves row r ----------------------------------
     constexpr unsigned long long kNone = ~0ull;
-    const unsigned int* const rows_g = MODE == kSparse ? a.rows + (size_t)seq * a.k : (LINEAR ? a.rows : nullptr);
-    const int* const table_g = LINEAR ? nullptr : a.block_table + (size_t)seq * a.max_blocks;
+    const unsigned int* const rows_g = MODE == kSparse ? a.rows + (size_t)seq * a.k : nullptr;
+    const int* const table_g = a.block_table + (size_t)seq * a.max_blocks;
     // the list entry (or position) of the lane's row; the read is unconditional and clamped
     auto token_of = [&](int tile) -> unsigned int {
         // (unsigned: three rounds of tiles past the end of 2^31 - 32 rows is past what an int holds)
@@ -85,23 +77,18 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
     };
     // the row's page, likewise (-1: the block table has no entry for it)
     auto page_of = [&](unsigned int tok) -> int {
-        if (LINEAR) return 0;
         const unsigned int blk = a.page_shift >= 0 ? tok >> a.page_shift : tok / (unsigned)a.page_tokens;
         const int page = table_g[min(blk, (unsigned)a.max_blocks - 1)];
         return blk < (unsigned)a.max_blocks ? page : -1;
     };
     struct Where {
-        unsigned long long code, scale;  // linear slabs: the token, twice
+        unsigned long long code, scale;
     };
     auto resolve = [&](int tile, unsigned int tok, int page) -> Where {
         Where w = {kNone, 0};
         if (lane >= kTile || tile >= n_tiles || r_begin + tile * kTile + lane >= r_end) return w;
         // a list entry of all ones is nobody's token, and only the 8-bit modes count it (as attend_part)
-        if (MODE != kDense && tok == 0xffffffffu && (LINEAR || !a.count_ones)) return w;
-        if (LINEAR) {
-            w.code = (unsigned long long)tok * kKvl, w.scale = tok;
-            return w;
-        }
+        if (MODE != kDense && tok == 0xffffffffu && !a.count_ones) return w;
         if ((unsigned)page < (unsigned)a.n_pages) {
             const unsigned int off =
                 a.page_shift >= 0 ? tok & (unsigned)(a.page_tokens - 1) : tok % (unsigned)a.page_tokens;
@@ -126,11 +113,9 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
         from[i] = (uint32_t)row | (uint32_t)(16 * c) << 8;
     }
     unsigned int there_next = 0;      // bit r: row r of the requested tile exists
-    f32x4 scale_next = {0, 0, 0, 0};  // lanes 0..31: its scale (linear slabs: its four)
-    u32x4 rope_next[4];               // linear slabs: eight bf16 of the roped keys a lane, eight rows a load
+    float scale_next = 0.0f;          // lanes 0..31: its scale
     auto request = [&](const Where& w, int buf) {
         there_next = (unsigned int)__builtin_amdgcn_ballot_w64(w.code != kNone);
-        const uint8_t* const codes = LINEAR ? a.lc8 : a.pool;
         const unsigned long long at = w.code != kNone ? w.code : 0;  // a row that is not there reads the first one
         const uint32_t lo = (uint32_t)at, hi = (uint32_t)(at >> 32);
         // (scalar by construction: the transfer takes its LDS base from a scalar register)
@@ -141,19 +126,9 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
             const int row = (int)(from[i] & 0xffu);
             const unsigned long long b = ((unsigned long long)(uint32_t)__shfl((int)hi, row, kWave) << 32) | (uint32_t)__shfl((int)lo, row, kWave);
             if (kWave * (i + 1) <= T::kAll || lane < T::kAll - kWave * i)
-                dma16(codes + b + (from[i] >> 8), to + 1024 * i);
+                dma16(a.pool + b + (from[i] >> 8), to + 1024 * i);
         }
-        if constexpr (LINEAR) {
-            const int tok = (int)w.scale;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const size_t t = (unsigned)__shfl(tok, 8 * i + (lane >> 3), kWave);
-                rope_next[i] = *reinterpret_cast<const u32x4*>(a.rc + t * kRopeW + 8 * (lane & 7));
-            }
-            scale_next = *reinterpret_cast<const f32x4*>(a.lscale + (size_t)w.scale * 4);
-        } else {
-            scale_next[0] = *reinterpret_cast<const float*>(a.pool + w.scale);
-        }
+        scale_next = *reinterpret_cast<const float*>(a.pool + w.scale);
     };
 
     // ---- prologue -------------------------------------------------------------------------------
@@ -162,13 +137,12 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
     unsigned int tok0 = token_of(wave), tok1 = token_of(wave + kH16Waves), tok2 = token_of(wave + 2 * kH16Waves);
     const int head = hg * kH16Heads + n16;
     // dims of K-step j, lane group g: eight from dim_of(j). A lane's two K-steps 2c, 2c + 1 are one
-    // 16-byte piece of a row. Paged: the pieces of lane groups 0, 1 (and 2, 3), read together, lie
-    // 256 bytes apart, in the same banks of different rows; the linear slabs' block scales want a
-    // K-step inside one block of 128 dims, and their roped keys are bf16 (32 dims a K-step).
+    // 16-byte piece of a row. The pieces of lane groups 0, 1 (and 2, 3), read together, lie
+    // 256 bytes apart, in the same banks of different rows.
     auto dim_of = [&](int j) -> int {
         const int c = j >> 1, s = j & 1;
-        if (c == 8) return kKvl + (LINEAR ? 32 * s + 8 * g : 16 * g + 8 * s);
-        return (LINEAR ? 64 * c + 16 * g : 256 * (g & 1) + 128 * (g >> 1) + 16 * c) + 8 * s;
+        if (c == 8) return kKvl + 16 * g + 8 * s;
+        return 256 * (g & 1) + 128 * (g >> 1) + 16 * c + 8 * s;
     };
     constexpr int kMine = (kKSteps + kH16Waves - 1) / kH16Waves;
     float4 qv[kMine][2];
@@ -230,15 +204,8 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
         const unsigned int here = there_next;
         if (lane < kTile) {
             // a scale that is not a positive number cannot come from the append: such a token is
-            // left out like one that is not there (linear slabs: a token is there or it is not)
-            const bool ok = (here >> lane) & 1u;
-            if constexpr (LINEAR) *(lds_ptr<f32x4>)(scl_lds + 4 * lane) = ok ? scale_next : f32x4{0, 0, 0, 0};
-            else scl_lds[lane] = ok && scale_next[0] > 0.0f ? scale_next[0] : 0.0f;
-        }
-        if constexpr (LINEAR) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                *(lds_ptr<u32x4>)(ropes + (8 * i + (lane >> 3)) * T::kRopeRow + 16 * (lane & 7)) = rope_next[i];
+            // left out like one that is not there
+            scl_lds[lane] = ((here >> lane) & 1u) && scale_next > 0.0f ? scale_next : 0.0f;
         }
         // rows that are not there: their codes must be finite, they meet a zero weight
         for (unsigned int gone = ~here; gone; gone &= gone - 1)
@@ -250,17 +217,9 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
         tok2 = token_of(tile + 3 * kH16Waves);
 
         // ---- scores: S^T[token][head], two 16-token halves ------------------------------------
-        f32x4 s0 = {0, 0, 0, 0}, s1 = {0, 0, 0, 0}, t0 = {0, 0, 0, 0}, t1 = {0, 0, 0, 0};
-        f32x4 sa, sb, sa4[4], sb4[4];  // the lane's tokens' scales: 4g + i, 16 + 4g + i
-        if constexpr (LINEAR) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                sa4[i] = *(lds_ptr<f32x4>)(scl_lds + 4 * (4 * g + i));
-                sb4[i] = *(lds_ptr<f32x4>)(scl_lds + 4 * (16 + 4 * g + i));
-            }
-        } else {
-            sa = *(lds_ptr<f32x4>)(scl_lds + 4 * g), sb = *(lds_ptr<f32x4>)(scl_lds + 16 + 4 * g);
-        }
+        f32x4 s0 = {0, 0, 0, 0}, s1 = {0, 0, 0, 0};
+        // the lane's tokens' scales: 4g + i, 16 + 4g + i
+        const f32x4 sa = *(lds_ptr<f32x4>)(scl_lds + 4 * g), sb = *(lds_ptr<f32x4>)(scl_lds + 16 + 4 * g);
         const lds_ptr<uint8_t> a0p = codes + T::at(n16), a1p = codes + T::at(16 + n16);
         auto as_bf16 = [](uint32_t x, uint32_t y) -> bf16x8 {
             u32x4 d;
@@ -278,12 +237,11 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
                 s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f1, ql[j], s1, 0, 0, 0);
             }
         };
-        constexpr int kCodeChunks = LINEAR ? kH16Chunks - 1 : kH16Chunks;
         u32x4 c0[2], c1[2];
         c0[0] = *(lds_ptr<u32x4>)(a0p + dim_of(0)), c1[0] = *(lds_ptr<u32x4>)(a1p + dim_of(0));
 #pragma unroll
-        for (int c = 0; c < kCodeChunks; ++c) {
-            if (c + 1 < kCodeChunks) {
+        for (int c = 0; c < kH16Chunks; ++c) {
+            if (c + 1 < kH16Chunks) {
                 c0[(c + 1) & 1] = *(lds_ptr<u32x4>)(a0p + dim_of(2 * c + 2));
                 c1[(c + 1) & 1] = *(lds_ptr<u32x4>)(a1p + dim_of(2 * c + 2));
             }
@@ -291,19 +249,7 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
             const u32x4 x = c0[c & 1], y = c1[c & 1];
             step(2 * c, as_bf16(x.x, x.y), as_bf16(y.x, y.y));
             step(2 * c + 1, as_bf16(x.z, x.w), as_bf16(y.z, y.w));
-            if (LINEAR && (c & 1)) {  // the block's dots under its scales
-#pragma unroll
-                for (int e = 0; e < 4; ++e) t0[e] += s0[e] * sa4[e][c >> 1], t1[e] += s1[e] * sb4[e][c >> 1];
-                s0 = f32x4{0, 0, 0, 0}, s1 = f32x4{0, 0, 0, 0};
-            }
             __builtin_amdgcn_sched_barrier(0);
-        }
-        if constexpr (LINEAR) {
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const lds_ptr<uint8_t> r = ropes + n16 * T::kRopeRow + 64 * s + 16 * g;
-                step(16 + s, *(lds_ptr<bf16x8>)r, *(lds_ptr<bf16x8>)(r + 16 * T::kRopeRow));
-            }
         }
 
         // The first value-side operands come out of LDS under the softmax. Operand of column tile
@@ -321,13 +267,8 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
         float v[8];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            if constexpr (LINEAR) {
-                v[i] = (here >> (4 * g + i)) & 1u ? t0[i] + s0[i] : -INFINITY;
-                v[4 + i] = (here >> (16 + 4 * g + i)) & 1u ? t1[i] + s1[i] : -INFINITY;
-            } else {
-                v[i] = sa[i] > 0.0f ? s0[i] * sa[i] : -INFINITY;
-                v[4 + i] = sb[i] > 0.0f ? s1[i] * sb[i] : -INFINITY;
-            }
+            v[i] = sa[i] > 0.0f ? s0[i] * sa[i] : -INFINITY;
+            v[4 + i] = sb[i] > 0.0f ? s1[i] * sb[i] : -INFINITY;
         }
         float tmax = fmaxf(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])), fmaxf(fmaxf(v[4], v[5]), fmaxf(v[6], v[7])));
         tmax = rows_max(tmax);
@@ -346,27 +287,22 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
         if (grow) m_ref = tmax;
         l_sum *= corr;
         const float mu = m_ref == -INFINITY ? 0.0f : m_ref;
-        float e[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) e[i] = __builtin_amdgcn_exp2f(v[i] - mu);  // not there -> 0
-        // the weights under the scales of column block b (paged: the token's one scale)
+        // the weights under their tokens' scales
         bf16x8 p, p_lo;
-        auto weights = [&](int b) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float scl = LINEAR ? (i < 4 ? sa4[i & 3][b] : sb4[i & 3][b]) : (i < 4 ? sa[i & 3] : sb[i & 3]);
-                const float x = e[i] * scl;
-                const __bf16 w = (__bf16)x;
-                p[i] = w;
-                if (PSPLIT == 2) {
-                    p_lo[i] = (__bf16)(x - (float)w);
-                    if (b == 0) l_sum += e[i];
-                } else {
-                    l_sum += (float)w * (scl > 0.0f ? __builtin_amdgcn_rcpf(scl) : 0.0f);
-                }
+        for (int i = 0; i < 8; ++i) {
+            const float e = __builtin_amdgcn_exp2f(v[i] - mu);  // not there -> 0
+            const float scl = i < 4 ? sa[i & 3] : sb[i & 3];
+            const float x = e * scl;
+            const __bf16 w = (__bf16)x;
+            p[i] = w;
+            if (PSPLIT == 2) {
+                p_lo[i] = (__bf16)(x - (float)w);
+                l_sum += e;
+            } else {
+                l_sum += (float)w * (scl > 0.0f ? __builtin_amdgcn_rcpf(scl) : 0.0f);
             }
-        };
-        weights(0);
+        }
 
         // ---- values: O[head][col] += P . V ----------------------------------------------------
 #pragma unroll
@@ -377,7 +313,6 @@ __device__ __forceinline__ void attend_part_heads16(const AttendArgs& a, int seq
                 for (int i = 0; i < kValueAhead; ++i)
                     fb[cur ^ 1][i] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_ptr<i32x2>)(vrow + 16 * (n0 + kValueAhead + i)));
             }
-            if (LINEAR && n0 > 0 && n0 % 8 == 0) weights(n0 / 8);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < kValueAhead; ++i) {
