@@ -827,62 +827,10 @@ __global__ __launch_bounds__(F8 ? kF8Threads : kAttThreads) void mla_attend_page
   }  // parts of this workgroup
 }
 
-// The same walk for 16 heads per workgroup (mla_attend_heads16.hpp).
-template <int QSPLIT, int PSPLIT, int MODE>
-__global__ __launch_bounds__(kH16Threads, 1) void mla_attend_heads16_kernel(const AttendArgs a) {
-    __shared__ int pre[kDealMaxSeqs + 8];
-    __shared__ int wave_total[kH16Waves];
-    // Workgroups are dealt to the eight dies in turn: the head groups of one work item follow each
-    // other on one die, whose cache then serves the item's rows to all but the first of them.
-    const int groups = (a.H + kH16Heads - 1) / kH16Heads, turn = (int)blockIdx.x >> 3;
-    const int item = (turn / groups) * 8 + ((int)blockIdx.x & 7), hg = turn % groups;
-    long long t_lo, t_hi;
-    int seq = item;
-    if (item >= (a.n_items > 0 ? a.n_items : a.n_seqs)) return;
-    if (a.by_seq) {
-        const SeqDeal d = seq_deal(MODE == kSparse ? a.n_rows : a.seq_lens, a.k, a.n_seqs, a.n_items, a.by_seq);
-        const unsigned long long past = __ballot(d.first + d.parts > item);
-        if (!past) return;  // more work items than runs
-        seq = __builtin_ctzll(past);
-        const int first = __builtin_amdgcn_readlane(d.first, seq), parts = __builtin_amdgcn_readlane(d.parts, seq);
-        // of a sequence's work items none is longer than the run: its tiles in `parts` even shares
-        const int tiles = __builtin_amdgcn_readlane(d.tiles, seq), part = item - first;
-        const int r_begin = (int)((unsigned)(part * tiles) / (unsigned)parts) * kTile;
-        const int r_end = min(attended_rows<MODE>(a, seq), (int)((unsigned)((part + 1) * tiles) / (unsigned)parts) * kTile);
-        const size_t rec = (size_t)item + seq;
-        attend_part_heads16<QSPLIT, PSPLIT, MODE>(a, seq, hg, r_begin, r_end, parts == 1, a.part_acc + rec * a.H * kKvl,
-                                                  a.part_ml + rec * a.H * 2);
-        return;
-    }
-    if (!dealt_range<kH16Threads, MODE>(a, item, pre, wave_total, t_lo, t_hi, seq)) return;
-    for (;; ++seq) {
-        int r_begin = 0, r_end;
-        bool whole = true;
-        float *pa = a.part_acc, *pml = a.part_ml;
-        if (a.n_items > 0) {
-            if (t_lo >= t_hi || seq >= a.n_seqs) break;
-            if (!dealt_part<MODE>(a, item, pre, seq, t_lo, t_hi, r_begin, r_end, whole, pa, pml)) continue;
-            __syncthreads();
-        } else {
-            r_end = attended_rows<MODE>(a, seq);
-            if (r_end <= 0) {
-                for (int i = threadIdx.x; i < kH16Heads * kKvl; i += kH16Threads) {
-                    const int h = hg * kH16Heads + i / kKvl;
-                    if (h < a.H) a.clat[((size_t)seq * a.H + h) * kKvl + (i % kKvl)] = 0.0f;
-                }
-                return;
-            }
-        }
-        attend_part_heads16<QSPLIT, PSPLIT, MODE>(a, seq, hg, r_begin, r_end, whole, pa, pml);
-        if (a.n_items == 0) break;
-    }
-}
-
-// The same walk for 16 heads per workgroup by eight waves (mla_attend_few.hpp).
-template <int QSPLIT, int PSPLIT, int MODE>
-__global__ __launch_bounds__(kFewThreads) void mla_attend_few_kernel(const AttendArgs a) {
-    __shared__ int pre[kDealMaxSeqs + 8];
-    __shared__ int wave_total[kFewWaves];
+// The same walk for 16 heads per workgroup of THREADS: `part` is called with each part of its work as attend_part's, a
+// part of several sequences' with a barrier before it.
+template <int THREADS, int MODE, class PART>
+__device__ __forceinline__ void heads16_walk(const AttendArgs& a, int (&pre)[kDealMaxSeqs + 8], int (&wave_total)[THREADS / kWave], PART part_of) {
     // Workgroups are dealt to the eight dies in turn: the head groups of one work item follow each
     // other on one die, whose cache then serves the item's rows to all but the first of them.
     const int groups = (a.H + kH16Heads - 1) / kH16Heads, turn = (int)blockIdx.x >> 3;
@@ -901,11 +849,10 @@ __global__ __launch_bounds__(kFewThreads) void mla_attend_few_kernel(const Atten
         const int r_begin = (int)((unsigned)(part * tiles) / (unsigned)parts) * kTile;
         const int r_end = min(attended_rows<MODE>(a, seq), (int)((unsigned)((part + 1) * tiles) / (unsigned)parts) * kTile);
         const size_t rec = (size_t)item + seq;
-        attend_part_few<QSPLIT, PSPLIT, MODE>(a, seq, hg, r_begin, r_end, parts == 1, a.part_acc + rec * a.H * kKvl,
-                                                  a.part_ml + rec * a.H * 2);
+        part_of(seq, hg, r_begin, r_end, parts == 1, a.part_acc + rec * a.H * kKvl, a.part_ml + rec * a.H * 2);
         return;
     }
-    if (!dealt_range<kFewThreads, MODE>(a, item, pre, wave_total, t_lo, t_hi, seq)) return;
+    if (!dealt_range<THREADS, MODE>(a, item, pre, wave_total, t_lo, t_hi, seq)) return;
     for (;; ++seq) {
         int r_begin = 0, r_end;
         bool whole = true;
@@ -917,16 +864,32 @@ __global__ __launch_bounds__(kFewThreads) void mla_attend_few_kernel(const Atten
         } else {
             r_end = attended_rows<MODE>(a, seq);
             if (r_end <= 0) {
-                for (int i = threadIdx.x; i < kH16Heads * kKvl; i += kFewThreads) {
+                for (int i = threadIdx.x; i < kH16Heads * kKvl; i += THREADS) {
                     const int h = hg * kH16Heads + i / kKvl;
                     if (h < a.H) a.clat[((size_t)seq * a.H + h) * kKvl + (i % kKvl)] = 0.0f;
                 }
                 return;
             }
         }
-        attend_part_few<QSPLIT, PSPLIT, MODE>(a, seq, hg, r_begin, r_end, whole, pa, pml);
+        part_of(seq, hg, r_begin, r_end, whole, pa, pml);
         if (a.n_items == 0) break;
     }
+}
+
+// A tile a wave (mla_attend_heads16.hpp).
+template <int QSPLIT, int PSPLIT, int MODE>
+__global__ __launch_bounds__(kH16Threads, 1) void mla_attend_heads16_kernel(const AttendArgs a) {
+    __shared__ int pre[kDealMaxSeqs + 8];
+    __shared__ int wave_total[kH16Waves];
+    heads16_walk<kH16Threads, MODE>(a, pre, wave_total, [&](auto... part) { attend_part_heads16<QSPLIT, PSPLIT, MODE>(a, part...); });
+}
+
+// Eight waves on a tile (mla_attend_few.hpp).
+template <int QSPLIT, int PSPLIT, int MODE>
+__global__ __launch_bounds__(kFewThreads) void mla_attend_few_kernel(const AttendArgs a) {
+    __shared__ int pre[kDealMaxSeqs + 8];
+    __shared__ int wave_total[kFewWaves];
+    heads16_walk<kFewThreads, MODE>(a, pre, wave_total, [&](auto... part) { attend_part_few<QSPLIT, PSPLIT, MODE>(a, part...); });
 }
 
 // Dealt plan: clat[seq][head] = sum_r w_r acc_r / sum_r w_r l_r over the sequence's partial
