@@ -3,13 +3,13 @@
 #include "../../rivoli_amd/csrc/mla_attend_plan.hpp"
 
 // 1: workgroups of 16 heads, 0: of 64. out: items, by_seq, records of the route; items, records the
-// caller's scratch is sized by. linear: 0 a paged call, 1 the linear slabs with scratch, 2 without.
-extern "C" int attend_route(int n_seqs, int H, int max_rows, int precise, int listed, int linear, int out[5]) {
+// caller's scratch is sized by; whether eight waves share a tile. linear: 0 a paged call, 1 the linear slabs with scratch, 2 without.
+extern "C" int attend_route(int n_seqs, int H, int max_rows, int precise, int listed, int linear, int out[6]) {
     const rk::AttendPlan plan = linear ? rk::linear_plan(H, max_rows, rk::kRefMaxSplits, linear == 1)
                                        : rk::attend_plan(n_seqs, H, max_rows);
     const rk::AttendRoute r = rk::attend_route(plan, n_seqs, H, max_rows, precise, !listed && !linear, linear != 0);
     out[0] = r.plan.n_items, out[1] = r.by_seq, out[2] = r.plan.n_records;
-    out[3] = plan.n_items, out[4] = plan.n_records;
+    out[3] = plan.n_items, out[4] = plan.n_records, out[5] = r.few;
     return r.heads16;
 }
 

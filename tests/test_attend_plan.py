@@ -104,6 +104,24 @@ def test_list_positions_looked_up_ahead_stay_in_the_list(r_end):
         assert min(wrapped((n_tiles + 11) * 32, True), r_end - 1) < 0
 
 
+def test_which_calls_of_16_heads_a_workgroup_share_a_tile_among_eight_waves():
+    """All with three groups of heads, all over the linear slabs, and short work items: of the sequences kept
+    whole up to 128 tiles of 32 dense rows and 48 of listed ones, of cut ones as many a work item, or 64 where q and weights
+    are carried once."""
+    for rows in (64, 512, 4096, 40000):
+        for H in (33, 64, 512):
+            r = attend_route(1, H, rows, 2)
+            assert r.few == r.heads16
+        for linear in (1, 2):
+            assert all(attend_route(1, H, rows, 2, linear=linear).few for H in (1, 16, 32, 64, 512))
+    for precise, dense, cut in ((2, 128, 128), (1, 128, 128), (0, 128, 64)):
+        for n, rows, tiles, listed in ((300, 32 * dense, dense, False), (300, 32 * 48, 48, True), (1, 32 * cut * 64, cut, False),
+                                       (64, 32 * cut * 4, cut, False), (64, 32 * 48 * 4, 48, True), (1, 32 * 48 * 64, 48, True)):
+            at, past = attend_route(n, 16, rows, precise, listed), attend_route(n, 16, rows + 32 * 64, precise, listed)
+            assert at.heads16 and at.few and past.heads16 and not past.few, (precise, n, rows, listed)
+            assert not at.items or -(-n * -(-rows // 32) // at.items) == tiles
+
+
 def test_blocks_left_to_a_second_pass_spread_over_its_groups():
     """The index-list attention's second pass: every block is one group's, all blocks are dealt evenly, and of blocks at
     any regular distance (a remainder in every 256th query) the fullest group has a few more than its share, not all."""

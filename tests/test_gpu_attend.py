@@ -526,7 +526,8 @@ def test_both_sides_of_the_line_between_a_tile_of_eight_waves_and_a_tile_a_wave(
     H, edges = 11, [1, 0, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257]
     lens = [most] + (edges * 22)[:299]
     route = attend_route(len(lens), H, most, precise)
-    assert route.heads16 and route.items == 0
+    assert route.heads16 and route.items == 0 and route.few == (most == 4096)
+    assert attend_route(len(lens), H, listed_most, precise, True).few == (listed_most == 1536)
     c = paged_case(oracle, lens, H=H, seed=905, outlier_frac=0.0)
     want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], None, None,
                                    KVL, ROPE, PT, c["scale"], n_threads=8)
@@ -608,6 +609,38 @@ def test_few_heads_and_more_sequences_than_half_the_work_items(oracle, H):
         want = oracle.mla_attend_paged(*args, claimed, None, None, KVL, ROPE, 16, c["scale"], n_threads=8)
         got = run_paged(dict(c, lens=claimed), max(lens), pt=16)
         check(got, want, 2, "dense", mild=True)
+
+
+@pytest.mark.parametrize("precise", [2, 1, 0])
+@pytest.mark.parametrize("n,H,top,by_seq", [(64, 16, 16700, True), (7, 5, 150000, True), (200, 16, 4800, False)])
+def test_a_tile_a_wave_over_cut_work_items(oracle, n, H, top, by_seq, precise):
+    """The kernel of long work items where sequences are cut and merged: no work item with two sequences, and several
+    to one. The launcher knows the most that a sequence may have, so a few hundred tokens do: one short of, at
+    and one past a tile, a round of four waves' tiles and a run; empty ones; lists with entries of all ones, pages that the table
+    does not have."""
+    lens = ([1500, 31, 0, 129, 511, 33, 640, 1, 128, 127, 257, 96] * 17)[:n]
+    for is_listed in (False, True):
+        route = attend_route(n, H, top, precise, is_listed)
+        assert route.heads16 and not route.few and route.by_seq == by_seq and route.items >= n
+    c = paged_case(oracle, lens, H=H, seed=960 + n, outlier_frac=0.0)
+    args = (c["qabs"], c["qrope"], c["pool"], c["table"])
+    want = oracle.mla_attend_paged(*args, c["lens"], None, None, KVL, ROPE, PT, c["scale"], n_threads=8)
+    check(run_paged(c, top, precise=precise), want, precise, "dense", mild=precise == 2)
+    rng = np.random.default_rng(n)
+    tokens = [rng.permutation(k).astype(np.uint32) for k in lens]
+    rows, n_rows = listed(tokens, top)
+    for s in range(0, n, 6):  # three entries in the first tile, a whole tile, the last one
+        for at in (slice(1, 4), slice(64, 96), slice(1499, 1500)):
+            rows[s, at] = 0xFFFFFFFF
+    table = c["table"].copy()
+    table[3, 1] = -1                                     # tokens 64 .. 127 of 129
+    live = [[t for t in rows[s, :k] if t != 0xFFFFFFFF and not (s == 3 and 64 <= t < 128)] for s, k in enumerate(lens)]
+    kept, kept_n = listed(live, max(lens))
+    want = oracle.mla_attend_paged(*args, None, kept, kept_n, KVL, ROPE, PT, c["scale"], n_threads=8)
+    bad = dzeros(4)
+    got = run_paged(dict(c, table=table), top, rows=rows, n_rows=n_rows, use_lens=False, precise=precise, bad=bad)
+    check(got, want, precise, "listed", mild=precise == 2)
+    assert back(bad, np.uint32)[0] == 64
 
 
 def listed(tokens, width):

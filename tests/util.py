@@ -47,11 +47,12 @@ def slots_for(table_row, positions, page_tokens=64):
 
 class AttendRoute:
     """attend_route of rivoli_amd/csrc/mla_attend_plan.hpp: which workgroups a call of the shipped row
-    widths takes, and its work items. `linear`: over the linear slabs, 1 with scratch, 2 without."""
+    widths takes, and its work items; `few`: of 16 heads, with eight waves on a tile. `linear`: over the linear slabs, 1 with scratch, 2 without."""
 
     def __init__(self, heads16, out):
         self.heads16 = bool(heads16)
-        self.items, self.by_seq, self.records, self.scratch_items, self.scratch_records = list(out)
+        self.items, self.by_seq, self.records, self.scratch_items, self.scratch_records, few = list(out)
+        self.few = bool(few)
 
 
 def _plan():
@@ -67,7 +68,7 @@ def _plan():
 
 
 def attend_route(n_seqs, H, max_rows, precise, listed=False, linear=0):
-    out = (ctypes.c_int * 5)()
+    out = (ctypes.c_int * 6)()
     return AttendRoute(_plan().attend_route(n_seqs, H, max_rows, precise, int(listed), linear, out), out)
 
 
