@@ -1894,9 +1894,10 @@ __global__ __launch_bounds__(WAVES* kWave) void block_select_bisect_kernel(
 
 // Few rows: sixteen waves each (select_few.hpp).
 template <int ITEMS>
-__device__ __forceinline__ void block_select_sixteen(const float* __restrict__ scores, int n_comp, int ratio, int prefill,
-                                                     int k, int offset, int32_t* __restrict__ out, int out_stride,
-                                                     const SelWindow& window, uint32_t* lds) {
+__global__ __launch_bounds__(kSfThreads) void block_select_few_kernel(
+    const float* __restrict__ scores, int n_comp, int ratio, int prefill, int k, int offset,
+    int32_t* __restrict__ out, int out_stride, SelWindow window) {
+    __shared__ __attribute__((aligned(16))) uint32_t lds[kSfLdsWords];
     const int t = blockIdx.x;
     const int limit = select_row_limit(t, n_comp, ratio, prefill);
     int32_t* o = out + (size_t)t * out_stride;
@@ -1904,20 +1905,6 @@ __device__ __forceinline__ void block_select_sixteen(const float* __restrict__ s
     if (select_positional<kSfThreads>(o, limit, k, offset)) return;
     select_few<ITEMS, TotalOrderKey>(scores + (size_t)t * n_comp, limit, (uint32_t)k,
                                      reinterpret_cast<uint32_t*>(o), lds, (uint32_t)offset);
-}
-template <int ITEMS>
-__global__ __launch_bounds__(kSfThreads) void block_select_few_kernel(
-    const float* __restrict__ scores, int n_comp, int ratio, int prefill, int k, int offset,
-    int32_t* __restrict__ out, int out_stride, SelWindow window) {
-    __shared__ __attribute__((aligned(16))) uint32_t lds[kSfLdsWords];
-    block_select_sixteen<ITEMS>(scores, n_comp, ratio, prefill, k, offset, out, out_stride, window, lds);
-}
-template <int ITEMS>  // rows of one or two keys a lane
-__global__ __launch_bounds__(kSfThreads) void block_select_short_kernel(
-    const float* __restrict__ scores, int n_comp, int ratio, int prefill, int k, int offset,
-    int32_t* __restrict__ out, int out_stride, SelWindow window) {
-    __shared__ __attribute__((aligned(16))) uint32_t lds[kSfLdsWords];
-    block_select_sixteen<ITEMS>(scores, n_comp, ratio, prefill, k, offset, out, out_stride, window, lds);
 }
 
 // Rows too long for the register form: the single-query radix select, one workgroup per row.
@@ -1955,8 +1942,8 @@ static int block_select_launch(const float* scores, int rows, int n_comp, int ra
 #define RK_BISECT(WV, I)                                                                     \
     hipLaunchKernelGGL((block_select_bisect_kernel<WV, I>), grid, dim3(WV* kWave), 0, stream, \
                        scores, n_comp, ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
-#define RK_FEW(KERNEL, I)                                                                     \
-    hipLaunchKernelGGL((KERNEL<I>), grid, dim3(kSfThreads), 0, stream, scores, n_comp, ratio, \
+#define RK_FEW(I)                                                                                             \
+    hipLaunchKernelGGL((block_select_few_kernel<I>), grid, dim3(kSfThreads), 0, stream, scores, n_comp, ratio, \
                        prefill ? 1 : 0, k, offset, out, out_stride, window)
 #define RK_SELECT(T, I)                                                                       \
     hipLaunchKernelGGL((block_select_kernel<T, I>), grid, dim3(T), 0, stream, scores, n_comp, \
@@ -1965,13 +1952,13 @@ static int block_select_launch(const float* scores, int rows, int n_comp, int ra
     // as few keys a lane as there are. One row of 8192 (sums of a ReLU): in four waves 17.8 us, by leading bits and
     // bisection in sixteen 10.6, over the range that the keys take 5.8; of 1000 7.6 -> 4.
     if (rows <= kSelFewRows && n_comp > 64 * 8 && n_comp <= kSfThreads)
-        RK_FEW(block_select_short_kernel, 1);
+        RK_FEW(1);
     else if (rows <= kSelFewRows && n_comp > kSfThreads && n_comp <= kSfThreads * 2)
-        RK_FEW(block_select_short_kernel, 2);
+        RK_FEW(2);
     else if (rows <= kSelFewRows && n_comp > kSfThreads * 2 && n_comp <= kSfThreads * 8)
-        RK_FEW(block_select_few_kernel, 8);
+        RK_FEW(8);
     else if (rows <= kSelFewRows && n_comp > kSfThreads * 8 && n_comp <= kSfThreads * 16)
-        RK_FEW(block_select_few_kernel, 16);
+        RK_FEW(16);
     // otherwise up to 32 keys per lane; a row takes as few waves as hold it
     else if (n_comp <= 64 * 8)
         RK_BISECT(1, 8);

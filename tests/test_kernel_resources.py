@@ -129,18 +129,19 @@ def test_the_block_scorers_matrix_kernels_and_the_few_row_selection_do_not_spill
     seen = []
     for src, part, waves in (("block_index.hip", "score_blocks_pair_kernel", 2),
                              ("block_index.hip", "score_blocks_one_kernel", 3),
-                             ("index_topk.hip", "block_select_few_kernel", 8)):
+                             ("index_topk.hip", "block_select_few_kernel", 8),
+                             ("index_topk.hip", "index_topk_few_kernel", 8)):
         for b in _resource_blocks(src):
             name = b.split()[0]
             if part not in name:
                 continue
             seen.append(part)
-            if part == "block_select_few_kernel":
+            if src == "index_topk.hip":
                 assert int(re.search(r"SGPRs Spill: (\d+)", b).group(1)) == 0, name
             assert int(re.search(r"VGPRs Spill: (\d+)", b).group(1)) == 0, name
             assert int(re.search(r"ScratchSize \[bytes/lane\]: (\d+)", b).group(1)) == 0, name
             assert int(re.search(r"Occupancy \[waves/SIMD\]: (\d+)", b).group(1)) >= waves, name
-    assert len(seen) == 5
+    assert len(seen) == 11 and seen.count("block_select_few_kernel") == seen.count("index_topk_few_kernel") == 4
 
 
 def test_the_build_refuses_an_attention_object_that_spills():
