@@ -179,15 +179,22 @@ static inline bool heads16_pays(const AttendPlan& plan, bool cut, int n_seqs, in
 // One or two groups of heads that walk long work items have each row from memory and wait for it; a
 // tile of its own per wave (mla_attend_heads16.hpp) keeps more of them on their way. Parity mode, 16 heads, per tile-a-wave
 // and eight waves: dense, one sequence of 100 000 tokens (49 tiles a work item) 64.4 us and 63.1, 300 000 (146) 138.5 and 139.1,
-// 800 000 (390) 325 and 340, 300 whole sequences of 6 000 (188) 314 and 324; lists, whose rows are scattered, sooner: 64 of
-// 6 000 rows (47) 68 and 66, 300 of 3 000 (94) 180 and 186, 257 of 6 000 (188) 323 and 355. With q and weights in one term
-// (precise 0) cut dense sequences too: 100 000 tokens (49) 57.6 and 57.7, 200 000 (98) 88.7 and 91.4.
-constexpr int kFewMaxTiles = 128, kFewMaxTilesOneTerm = 64, kFewMaxTilesListed = 48;  // of a work item
-static inline bool heads16_few(const AttendPlan& p, int n_seqs, int H, int max_rows, int precise, bool dense, bool linear) {
+// 800 000 (390) 325 and 340. Work items that fill the chip and cover their sequences from end to end reach that sooner, the more
+// so the more even the batch: whole sequences, 256 of 1 500 (47) 56.7 and 55.1, of 2 000 (63) 75.6 and 76.2 (of one head 69.9 and 74.4; ragged 66.0 and 63.6),
+// of 3 000 (94) 107.8 and 109.8 (88.2 and 90.7); shared evenly, 192 of 3 000 (94) 100.5 and 99.9 (87.5 and 76.7), of 4 000 (125) 124.7
+// and 128.4 (104.1 and 91.9). Lists, whose rows are scattered, sooner too: 64 of 6 000 rows (47) 68 and 66, 300 of 3 000 (94)
+// 180 and 186, 257 of 6 000 (188) 323 and 355. With q and weights in one term (precise 0) cut dense sequences: 100 000 tokens (49) 57.6
+// and 57.7, 200 000 (98) 88.7 and 91.4; whole ones 257 of 3 000 (94) 158.0 and 156.4, of 4 000 (125) 195.4 and 201.3.
+constexpr int kFewMaxTiles = 128, kFewMaxTilesShared = 96, kFewMaxTilesWhole = 56, kFewMaxTilesListed = 48;  // of a work item
+constexpr int kFewMaxTilesOneTerm = 64, kFewMaxTilesOneTermWhole = 96;
+static inline bool heads16_few(const AttendPlan& p, bool by_seq, int n_seqs, int H, int max_rows, int precise, bool dense,
+                               bool linear) {
     if (linear || H > 2 * kH16Heads) return true;
     const long long tiles = max_rows / kTile + (max_rows % kTile != 0);
     const long long longest = p.n_items ? (n_seqs * tiles + p.n_items - 1) / p.n_items : tiles;
-    return longest <= (!dense ? kFewMaxTilesListed : precise == 0 && p.n_items ? kFewMaxTilesOneTerm : kFewMaxTiles);
+    if (!dense) return longest <= kFewMaxTilesListed;
+    if (precise == 0) return longest <= (p.n_items ? kFewMaxTilesOneTerm : kFewMaxTilesOneTermWhole);
+    return longest <= (by_seq ? kFewMaxTiles : p.n_items ? kFewMaxTilesShared : kFewMaxTilesWhole);
 }
 
 // A call of the shipped row widths whose rows are whole 16-byte pieces. `plan`: attend_plan's or
@@ -203,7 +210,7 @@ static inline AttendRoute attend_route(const AttendPlan& plan, int n_seqs, int H
     bool by_seq;
     const AttendPlan p = heads16_plan(plan, n_seqs, H, max_rows, by_seq);
     if (!heads16_pays(plan, p.n_items > 0, n_seqs, H, max_rows, precise, dense, linear)) return {false, false, false, plan};
-    return {true, by_seq, heads16_few(p, n_seqs, H, max_rows, precise, dense, linear), p};
+    return {true, by_seq, heads16_few(p, by_seq, n_seqs, H, max_rows, precise, dense, linear), p};
 }
 
 }  // namespace rk

@@ -105,17 +105,18 @@ def test_list_positions_looked_up_ahead_stay_in_the_list(r_end):
 
 
 def test_which_calls_of_16_heads_a_workgroup_share_a_tile_among_eight_waves():
-    """All with three groups of heads, all over the linear slabs, and short work items: of the sequences kept
-    whole up to 128 tiles of 32 dense rows and 48 of listed ones, of cut ones as many a work item, or 64 where q and weights
-    are carried once."""
+    """All with three groups of heads, all over the linear slabs, and short work items: 48 tiles of 32 listed rows; of dense
+    ones 56 where sequences stay whole, 96 where work items share them evenly, 128 where no item meets two of them; where
+    q and weights are carried once, 96 and 64."""
     for rows in (64, 512, 4096, 40000):
         for H in (33, 64, 512):
             r = attend_route(1, H, rows, 2)
             assert r.few == r.heads16
         for linear in (1, 2):
             assert all(attend_route(1, H, rows, 2, linear=linear).few for H in (1, 16, 32, 64, 512))
-    for precise, dense, cut in ((2, 128, 128), (1, 128, 128), (0, 128, 64)):
-        for n, rows, tiles, listed in ((300, 32 * dense, dense, False), (300, 32 * 48, 48, True), (1, 32 * cut * 64, cut, False),
+    for precise, whole, shared, cut in ((2, 56, 96, 128), (1, 56, 96, 128), (0, 96, 64, 64)):
+        for n, rows, tiles, listed in ((300, 32 * whole, whole, False), (300, 32 * 48, 48, True), (1, 32 * cut * 64, cut, False),
+                                       (200, 32 * shared, shared, False),
                                        (64, 32 * cut * 4, cut, False), (64, 32 * 48 * 4, 48, True), (1, 32 * 48 * 64, 48, True)):
             at, past = attend_route(n, 16, rows, precise, listed), attend_route(n, 16, rows + 32 * 64, precise, listed)
             assert at.heads16 and at.few and past.heads16 and not past.few, (precise, n, rows, listed)

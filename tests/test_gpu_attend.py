@@ -518,15 +518,15 @@ def test_linear_rows_past_the_lines_of_the_paged_calls(oracle, scratch):
 
 
 @pytest.mark.parametrize("precise", [2, 1, 0])
-@pytest.mark.parametrize("most,listed_most", [(4096, 1536), (4097, 1537)])
+@pytest.mark.parametrize("most,listed_most", [(1792, 1536), (1793, 1537), (3073, 1537), (4096, 1536), (4097, 1537)])
 def test_both_sides_of_the_line_between_a_tile_of_eight_waves_and_a_tile_a_wave(oracle, precise, most, listed_most):
-    """Up to 16 heads, sequences kept whole: 128 tiles of 32 dense rows and 48 of listed ones, and one row
+    """Up to 16 heads, sequences kept whole: 56 tiles of 32 dense rows (96 in one term) and 48 of listed ones, and one row
     more. The others end one short of, at and one past the tiles of 64 and the three buffers they pass
     through; lists have entries of all ones, in a first tile, a last one and a whole one."""
     H, edges = 11, [1, 0, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257]
     lens = [most] + (edges * 22)[:299]
     route = attend_route(len(lens), H, most, precise)
-    assert route.heads16 and route.items == 0 and route.few == (most == 4096)
+    assert route.heads16 and route.items == 0 and route.few == (most <= (1792 if precise else 3072))
     assert attend_route(len(lens), H, listed_most, precise, True).few == (listed_most == 1536)
     c = paged_case(oracle, lens, H=H, seed=905, outlier_frac=0.0)
     want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], None, None,
@@ -612,7 +612,7 @@ def test_few_heads_and_more_sequences_than_half_the_work_items(oracle, H):
 
 
 @pytest.mark.parametrize("precise", [2, 1, 0])
-@pytest.mark.parametrize("n,H,top,by_seq", [(64, 16, 16700, True), (7, 5, 150000, True), (200, 16, 4800, False)])
+@pytest.mark.parametrize("n,H,top,by_seq", [(64, 16, 16700, True), (7, 5, 150000, True), (200, 16, 3100, False)])
 def test_a_tile_a_wave_over_cut_work_items(oracle, n, H, top, by_seq, precise):
     """The kernel of long work items where sequences are cut and merged: no work item with two sequences, and several
     to one. The launcher knows the most that a sequence may have, so a few hundred tokens do: one short of, at
