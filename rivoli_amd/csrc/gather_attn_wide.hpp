@@ -80,7 +80,7 @@ struct GwEntries {  // a tile's row addresses, slot n32's in lanes n32 and n32 +
 };
 
 // A list's tiles. The addresses of masked slots are those of a live row of the query: its weight there is 0
-// and nothing that no slot lists is ever read.
+// and nothing that no slot lists is read (but row 0, in place of a list that is masked throughout).
 struct GwList {
     const int* ix;
     uint64_t kv;

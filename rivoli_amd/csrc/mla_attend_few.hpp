@@ -16,8 +16,8 @@
 // Every read from memory in the loop is a transfer into LDS, list entries, pages and scales too: a load into a register
 // would have the compiler wait for it, and with it for the rows that were asked for before it.
 // Measured, parity mode, with the merge of the records: 64 heads, 6 ragged sequences of up to 9 000 tokens 39.2 -> 36.2 us
-// (with the append), 8 x 2 048 listed rows 24 -> 20; linear slabs, 2 048 rows 19.2 -> 17.0, 300 rows 19.4 -> 13.7, 33 rows 12.6 -> 7.1. A tile
-// takes 3 800 cycles by its stamps with three barriers, of which 1 090 are matrix instructions; the prologue's chain 7 300.
+// (with the append), 8 x 2 048 listed rows 24 -> 20; linear slabs, 2 048 rows 19.2 -> 17.0, 300 rows 19.4 -> 13.7, 33 rows 12.6 -> 7.1. Of a
+// tile's cycles 1 090 a wave are matrix instructions.
 #pragma once
 
 namespace rk {

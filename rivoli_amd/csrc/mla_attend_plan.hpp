@@ -46,8 +46,10 @@ static inline AttendPlan attend_plan(int n_seqs, int H, int max_rows) {
 
 // The same for the linear slabs' one sequence, cut to what the caller's scratch holds: `fit` records of
 // which one is spare. Up to 512 heads, where its workgroups have 16 of them (heads16_pays), a call that is cut at
-// all is cut to 128 rows a work item, where the workgroups of 64 heads want 256: 64 heads, 512 rows 16.3 -> 13.1 us, 1 024
-// 16.5 -> 13.3, 1 800 20.0 -> 16.8; 256 rows are not worth a second launch, and past 2 500 the scratch decides.
+// all is cut to 128 rows a work item, where the paged workgroups of 64 heads want 256: 64 heads, 512 rows 16.3 -> 13.1 us, 1 024
+// 16.5 -> 13.3, 1 800 20.0 -> 16.8; 256 rows are not worth a second launch, and past 2 500 the scratch decides. The general form,
+// which takes other widths and slabs off a 16-byte boundary, gains as much: 64 heads of width 256, 512 rows 43.4 -> 31.5,
+// 1 024 43.4 -> 34.4, 1 800 45.9 -> 45.6; 384 47.0 -> 35.3, 47.2 -> 35.5, 49.7 -> 41.7; 512 from 8 bytes on 50.9 -> 38.8, 51.1 -> 39.1, 53.3 -> 42.4.
 static inline AttendPlan linear_plan(int H, int nr, int fit, bool scratch) {
     AttendPlan p = attend_plan(1, H, nr);
     if (p.n_splits > 1 && H <= kH16Heads * kAttTargetGroups / kAttDies) p.n_splits = (nr + kTile - 1) / kTile / kH16Waves;

@@ -204,8 +204,10 @@ __device__ __forceinline__ void select_few_keys(const uint32_t (&key)[ITEMS], in
     }
     T = (uint32_t)__builtin_amdgcn_readfirstlane((int)T);
     ties = (uint32_t)__builtin_amdgcn_readfirstlane((int)ties);
-    // What is no element has key 0, never above T, and as a tie it is past every live one in index order. slot < kq holds
-    // by construction; the compare keeps a wrong threshold from ever turning into a write outside the caller's buffer.
+    // What is no element has key 0, never above T. It can equal T only where T is 0, the lowest key: then all that lies before a tie
+    // that is taken is taken too. In steps past a wave's run (they go in fours) such a one stands where the next wave's elements
+    // do, and what it stores is the index that stands at that place of the output anyway; past the row's end nothing is left to take:
+    // slot < kq drops it. The compare also keeps a wrong threshold from ever turning into a write outside the caller's buffer.
     if (ties == 0 || __builtin_amdgcn_readfirstlane((int)here_eq) == 0) {
         run_gt += min(run_eq, ties);
         each([&](int j) {
