@@ -149,6 +149,28 @@ def test_many_queries_keep_the_range_of_few(oracle, power, rise, sink_at, precis
     assert worst_rel(few, got[pick]) <= 2.0 ** -7
 
 
+def test_many_queries_normalise_by_the_weights_of_the_products(oracle):
+    """One slot of the second tile has nearly all of every head's weight, 2^20 to 2^60 above the first tile's, another 2^-4 of
+    it. In two bf16 terms such a weight is off by 2^-19.5 of itself, which a denominator of other weights would
+    leave in the result: on the wrong side of a bf16 boundary come 3.4e-4 of the elements that did not cancel (the same sums in
+    numpy), where f32 logits and sums alone bring 9e-5. The bar lies between."""
+    m, h, scale = 257, 64, 512 ** -0.5
+    rng = np.random.default_rng(5)
+    kv = bf16_round(rng.standard_normal((100, 512)).astype(np.float32))
+    kv[:, 0] = 0.0
+    kv[90, 0], kv[91, 0] = 1.0, 0.90625
+    q = np.zeros((m, h, 512), np.float32)
+    q[:, :, 0] = bf16_round((rng.uniform(20, 60, (m, h)) / (scale * np.log2(np.e))).astype(np.float32))
+    idx = rng.integers(0, 90, (m, 65)).astype(np.int32)
+    idx[:, 40], idx[:, 50] = 90, 91
+    sink = np.zeros(h, np.float32)
+    got = device_attend(q, kv, sink, idx, scale, precise=2, n_kv=100)
+    pick = list(range(0, m, 6))
+    exact = sparse_attn_f64(q[pick], kv, sink, idx[pick], scale)
+    off = (got[pick] != bf16_round(exact.astype(np.float32)))[np.abs(exact) >= 0.25]
+    assert off.mean() <= 2e-4, off.mean()
+
+
 @pytest.mark.parametrize("m,h,topk,precise,share", [
     (1, 1, 1, 2, False), (2, 15, 63, 2, False), (2, 17, 64, 1, False), (3, 16, 65, 0, False), (1, 64, 129, 2, False),
     (4, 64, 96, 2, True), (16, 64, 700, 2, True), (17, 64, 640, 1, True), (50, 40, 300, 2, True), (256, 16, 70, 2, False)])
