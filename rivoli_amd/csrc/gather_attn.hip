@@ -491,8 +491,8 @@ __global__ __launch_bounds__(kGaThreads) void gather_attn_d512_kernel(const Gath
 
 // The blocks that the kernel of 32 heads a wave marked: a workgroup does those that are its own (marked_block), one after
 // another. No other looks at their marks, which its results replace. It looks at 512 marks at a time, which is all
-// that it does when there are none (2 us behind the other kernel).
-// All of 8192 queries x 640 slots marked 1772 -> 1720 us with the other kernel's look at them (1645 without), every 256th
+// that it does when there are none (4 to 5 us in a trace).
+// All of 8192 queries x 640 slots marked 1772 -> 1720 us (1676 since the other kernel's look at them asks for less), every 256th
 // 2815 -> 1177, each as dealt to group block mod 256 by addresses in vector registers -> so.
 template <int QSPLIT, int PSPLIT>
 __global__ __launch_bounds__(kGaThreads) void gather_attn_marked_kernel(const GatherAttnArgs a, long long blocks, int per_query) {
@@ -655,12 +655,13 @@ static int gather_attn_launch(const float* q, const float* kv, const float* sink
         a.part_ml = partial ? partial + (size_t)m * a.n_splits * h * kGaD : nullptr;
         const dim3 grid((unsigned)m, (unsigned)((h + 63) / 64), (unsigned)a.n_splits);
         // Past a workgroup of 64 heads a compute unit, two of half the waves fit one (gather_attn_wide.hpp): 300 queries of
-        // 640 slots 96 -> 62 us, 520 145 -> 127, 8192 1578 -> 1163; of 128 slots 257 34.5 -> 28.7, 600 57 -> 53. Up to there a
+        // 640 slots 96 -> 63 us, 520 145 -> 128, 8192 1569 -> 1157; of 128 slots 257 33.8 -> 28.0, 600 57 -> 53. Up to there a
         // query is the faster the more waves it has (200 queries 54 us against 58). A list of one or two tiles has little
-        // to overlap (64 slots: 600 queries 45.7 us against 48.5, 1000 66 and 61, 2049 151 and 141, 8192 542 and 448).
-        // A call whose queries all have a remainder past bf16 pays for the other kernel's look at them, 7 to 13 us and 5 %
-        // (640 slots: 300 queries 97 -> 102 us, 600 149 -> 160, 8192 1645 -> 1720; 1000 of 64 slots 66 -> 80, which is the other
-        // half of that line); one with a few of them for their pass (one in 256: 300 queries 96 -> 110, 520 145 -> 171, 2048 409 -> 349).
+        // to overlap (64 slots: 600 queries 45.7 us against 48.5, 1000 66 and 61, 2049 153 and 144, 8192 538 and 451).
+        // A call whose queries all have a remainder past bf16 pays for the other kernel's look at them, 4 to 10 us and 2 %
+        // (640 slots: 300 queries 97 -> 101 us, 600 149 -> 157, 8192 1639 -> 1676; 600 of 128 57.6 -> 65.2; 1000 of 64 66 -> 80, which is
+        // the other half of that line); one with a few of them for their pass (one in 256: 300 queries 96 -> 109, 520 145 -> 174,
+        // 2048 412 -> 362).
         // A scale of 0 gives a masked slot's -inf no weight there, and marks in o may not fall on a query that is still to be read.
         const long long blocks = (long long)m * grid.y;
         const uintptr_t q0 = (uintptr_t)q, o0 = (uintptr_t)o, bytes = (uintptr_t)m * h * kGaD * sizeof(float);

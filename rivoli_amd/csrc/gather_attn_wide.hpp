@@ -348,10 +348,12 @@ __device__ __forceinline__ bool gather_attn_wide_pass(const GatherAttnArgs& a, l
 // QSPLIT 2 keeps what bf16 leaves of a query that is not bf16-valued. The model's query is (its rotary stores bf16,
 // crates/backend/kernels/mla.hip:432), and only such a query's 64 heads fit the registers: others are marked, for
 // gather_attn_marked_kernel (gather_attn.hip) to do. The mark is the block's first output element: results are bf16
-// values, so no result has its bits. A head's row is looked at ahead of the rest, so that a call whose queries are of
-// the other kind spends a round trip a workgroup here (two passes over the list in this kernel, 16 heads and their
-// remainders a wave, took 1.24 to 1.5 times the kernel of half the dims).
+// values, so no result has its bits. A head's row is looked at ahead of most of the rest, so that a call whose queries are of
+// the other kind spends a round trip a workgroup here and a quarter of its rows' traffic (with half of them on their way by then
+// 8192 such queries of 640 slots took 1777 us, so 1740; bf16-valued ones the same within 0.5 %). Two passes over the list
+// in this kernel, 16 heads and their remainders a wave, took 1.24 to 1.5 times the kernel of half the dims.
 constexpr uint32_t kGwMark = 0x7fc0a55au;
+constexpr int kGwFirstRows = 8;  // of a wave's, asked for with the first look
 
 template <int QSPLIT, int PSPLIT>
 __device__ __forceinline__ bool gather_attn_wide_query(const GatherAttnArgs& a, lds_ptr<uint8_t> kr, float window) {
@@ -381,32 +383,35 @@ __device__ __forceinline__ bool gather_attn_wide_query(const GatherAttnArgs& a, 
 
     // a wave's 32 heads go through its buffer like a tile's rows
     uint32_t any = 0;
-    auto ask_query = [&](GwRow (&v)[16], int r0) {
+    auto ask_query = [&](auto& v, int r0) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {  // a head past h reads head 0: its column goes nowhere
+        for (int i = 0; i < (int)(sizeof(v) / sizeof(GwRow)); ++i) {  // a head past h reads head 0: its column goes nowhere
             const int hd = head0 + r0 + i < a.h ? head0 + r0 + i : 0;
             v[i].ask(q_at + (size_t)hd * (kGaD * 4), lane);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto stage_query = [&](const GwRow (&v)[16], int r0) {
+    auto stage_query = [&](const auto& v, int r0) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
+        for (int i = 0; i < (int)(sizeof(v) / sizeof(GwRow)); ++i) {
             *(lds_ptr<u32x4>)(kr + wave * kGaTileBytes + gw_row_of_slot(r0 + i) * kGaRowBytes + 16 * lane) = v[i].bf16();
             any |= v[i].bits();
         }
         __builtin_amdgcn_sched_barrier(0);
     };
     {
-        GwRow v[16];
-        ask_query(v, 0);
+        GwRow few[kGwFirstRows];
+        ask_query(few, 0);
         if (QSPLIT == 2 && __builtin_amdgcn_ballot_w64((first.bits() & 0xffffu) != 0) != 0) {  // the same in both waves
             if (threadIdx.x == 0) *mark = kGwMark;
             return true;
         }
-        stage_query(v, 0);
-        ask_query(v, 16);
-        stage_query(v, 16);
+        stage_query(few, 0);
+    }
+    {
+        GwRow rest[kGwHeads - kGwFirstRows];
+        ask_query(rest, kGwFirstRows);
+        stage_query(rest, kGwFirstRows);
     }
     if (QSPLIT == 2) {
         const bool has = __builtin_amdgcn_ballot_w64((any & 0xffffu) != 0) != 0;
