@@ -775,7 +775,7 @@ def bench_v4_attend(a, torch, hip):
                         # HBM bytes per launch by rocprofv3 FETCH_SIZE + WRITE_SIZE on this workload,
                         # each scaled by its reading for a known 1 GiB copy (profiles/); it cannot
                         # be read from inside the process
-                        "traffic": 2893700000 if (n, h, cap) == (8192, 64, 512) else None,
+                        "traffic": 2821000000 if (n, h, cap) == (8192, 64, 512) else None,
                         "hbm": {"bytes_per_launch": hbm_bytes, "achieved_GBps": round(hbm_bytes / att / 1e9, 1),
                                 "frac": round(hbm_bytes / att / HBM_PEAK, 4)}}}
     # the reference's decode shape: ONE query row over the same 640-slot list, with the list

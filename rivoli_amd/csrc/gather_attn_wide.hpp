@@ -9,7 +9,7 @@
 // runs every softmax twice), a row is read from LDS once for 32 heads instead of 16, and the two
 // waves of a workgroup (64 heads) share only the staging of its rows. 66.5 KB of LDS: two workgroups a
 // compute unit, one in its prologue or epilogue beside the other's tiles.
-// 8192 queries x 640 slots of 64 heads: 1624 us -> 1044 us. Its 0.94 P of products (the weights' remainders counted)
+// 8192 queries x 640 slots of 64 heads: 1624 us -> 1045 us. Its 0.94 P of products (the weights' remainders counted)
 // run at 0.90 P/s; a large bf16 product sustains 1.40 here, at 1.97 GHz, where power limits it. This kernel is held to
 // 2.15 GHz by the same limit (2.4 before), so what is left to save in cycles is worth half of it in time.
 //
@@ -350,7 +350,7 @@ __device__ __forceinline__ bool gather_attn_wide_pass(const GatherAttnArgs& a, l
 // gather_attn_marked_kernel (gather_attn.hip) to do. The mark is the block's first output element: results are bf16
 // values, so no result has its bits. A head's row is looked at ahead of most of the rest, so that a call whose queries are of
 // the other kind spends a round trip a workgroup here and a quarter of its rows' traffic (with half of them on their way by then
-// 8192 such queries of 640 slots took 1777 us, so 1740; bf16-valued ones the same within 0.5 %). Two passes over the list
+// 8192 such queries of 640 slots took 1777 us, so 1740; bf16-valued ones the same within 0.6 %). Two passes over the list
 // in this kernel, 16 heads and their remainders a wave, took 1.24 to 1.5 times the kernel of half the dims.
 constexpr uint32_t kGwMark = 0x7fc0a55au;
 constexpr int kGwFirstRows = 8;  // of a wave's, asked for with the first look
