@@ -23,8 +23,9 @@
 // rows is a multiple of one power of two and fits 24 bits, so no addition rounds and EVERY order
 // gives the reference's bits. The matrix kernels (hd = 128, up to 64 heads) test that property
 // on the operands they hold (RowSpan) and take such tiles through v_mfma_f32_32x32x16_bf16; any
-// other tile of the same launch is folded term by term as below. 8 192 queries x 64 heads x
-// <= 2 048 blocks: 209 us against 3 640 term by term (the whole rectangle 361 against 7 500).
+// other tile of the same launch is folded term by term as below; rows that are fp4 codes under
+// powers of two, as spread rows are, go through the block-scaled fp4 instruction. 8 192 queries x 64 heads x
+// <= 2 048 blocks: 172 us, 226 as bf16, 3 640 term by term.
 // Operands of another kind (no such rows leave the indexer) take the same launches' fold: 3 430.
 // Term by term, what is free is where the operands come from. A lane owns block c and
 // keeps its 128-value row in registers for the whole launch; a wave's 64 lanes share the query,
@@ -421,14 +422,16 @@ __device__ __forceinline__ void fold_heads(const float* __restrict__ q, const fl
 }
 
 // A workgroup's four waves own two queries each and walk the split's blocks in tiles of 32, which
-// all four read from LDS; a wave's q rows stay in registers as matrix operands (64 heads x 2
-// queries x 128 values = 128 registers). The 32 rows of a matrix tile are 16 heads of the wave's
-// first query and the same 16 of its second, dealt so that a lane's sixteen results are sixteen
-// heads of ONE query in order (the result layout gives lanes 0-31 the rows with bit 2 clear): the
-// head sum, whose order the reference fixes, is then register arithmetic. What bounds it is
-// issue: per 64 dots of a lane 32 matrix instructions of 32 cycles and five vector instructions a
-// dot (round, relu, weight, round, sum). e4m3 operands would halve the matrix half, but that
-// instruction does not keep 24 bits of a sum (checked: it loses bits at a span of 13).
+// all four read from LDS; a wave's q rows stay in registers as matrix operands. The 32 rows of a
+// matrix tile are 16 heads of the wave's first query and the same 16 of its second, dealt so that a
+// lane's sixteen results are sixteen heads of ONE query in order (the result layout gives lanes 0-31
+// the rows with bit 2 clear): the head sum, whose order the reference fixes, is then register arithmetic.
+// Bound by issue. As bf16 a lane's 64 dots were 32 matrix instructions of 32 cycles and five vector instructions each (round,
+// relu, weight, round, sum); as fp4 codes they are 8 of 32 cycles, and clamping conversions leave four a dot, in steps of which
+// none waits for another. 8 192 queries: 226 -> 172 us, of them 107 vector issue (two thirds of it those four; the kv rows' codes, made by every workgroup,
+// and the q rows' take the rest), 15 the matrix cores and about 25 the first workgroups' q rows, all asked for at once; 4 096 82 -> 74,
+// 6 001 126 -> 111. Not kept: 16 queries a workgroup (half of the conversions; all of q at once, 231), two or three sets of q loads
+// in flight (178).
 constexpr int kPairWaves = 4;
 constexpr int kPairThreads = kPairWaves * kWave;
 constexpr int kPairQueries = kPairWaves * 2;
@@ -437,13 +440,85 @@ constexpr int kPairTile = 32;
 constexpr int kPairRow = 128 * 2 + 16;  // bytes of a bf16 row in LDS: 16-byte reads of 16 rows meet no bank twice
 constexpr int kPairSplitMax = 4096;     // blocks of a split: one bit of a 128-bit mask per tile
 
+// Spread rows are what the block-scaled fp4 instruction takes: e2m1 codes, a power of two for 32 of them. A row
+// qualifies when every block's values are exactly that (fp4_of); with the block's exponent taken
+// from its largest value, products of two rows are multiples of u = 2^(lo_q + lo_kv - 2) and 128 of them sum to
+// 128 * 36 * 2^(hi_q + hi_kv) at most, hi and lo being a row's largest and smallest block exponents: below 2^24 u for (hi_q - lo_q) +
+// (hi_kv - lo_kv) <= 9, and the instruction keeps 24 bits of a sum (checked at every such difference, with cancelling
+// and one-signed sums in either half of K: exact up to 11, 12 being the first at which sums pass 2^24 u far enough to lose a bit).
+// The e4m3 form loses bits sooner. A real row's blocks differ by one binade or two.
+constexpr int kFp4Span = 9;
+constexpr int kFp4Row = 64 + 16;   // bytes of an fp4 row in LDS
+constexpr int kFp4MinExp = 127 - 59, kFp4MaxExp = 127 + 59;  // of a row's largest block, as kExactSpan's
+// The dots come out scaled, the largest that 128 products can be to just below one, so that the conversion to bf16 clamps to [0,
+// 1] and is the relu too; scores are scaled back. Powers of two change no rounding while nothing leaves the normal numbers:
+// with weights in 2^+-50, a query's heads within 20 binades (a scaled dot is 2^-44 then, or zero) and scales back of 2^-20 to 2^40,
+// terms are at least 2^-114 scaled or not, and bf16 terms' sums are multiples of 2^-121.
+constexpr int kFp4Down = 13;       // 128 * 36 < 2^13
+constexpr int kFp4Heads = 20, kFp4Back0 = -20, kFp4Back1 = 40;
+constexpr uint32_t kFp4Weight0 = 127 - 50, kFp4Weight1 = 127 + 50;
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t max_with_lane(uint32_t x) {
+    return max(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true));
+}
+// Four values of a block that eight neighbouring lanes hold, as fp4 codes under the block's scale. expo: the biased exponent of
+// the block's largest magnitude (the scale is 2^(expo - 129): that value becomes 4 or 6), 0 for zeros; off: non-zero when
+// a value is not exactly its code.
+__device__ __forceinline__ uint32_t fp4_of(const f32x4& v, uint32_t& expo, uint32_t& off) {
+    // (assembly: the compiler's maximum quiets each operand first, an instruction more for each)
+    float top;
+    asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(top) : "v"(v.x), "v"(v.y), "v"(v.z));
+    asm("v_max_f32_e64 %0, %1, |%2|" : "=v"(top) : "v"(top), "v"(v.w));
+    uint32_t m = __float_as_uint(top);
+    m = max_with_lane<0xB1>(m);   // lane ^ 1
+    m = max_with_lane<0x4E>(m);   // lane ^ 2
+    m = max_with_lane<0x141>(m);  // lane 7 - i: the other four's
+    expo = m >> 23;
+    const float scale = __uint_as_float((max(expo, 3u) - 2u) << 23);
+    uint32_t c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, v.x, v.y, scale, 0);
+    c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, v.z, v.w, scale, 1);
+    const f32x2 lo = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, scale, 0), hi = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, scale, 1);
+    off |= (__float_as_uint(v.x) ^ __float_as_uint(lo.x)) | (__float_as_uint(v.y) ^ __float_as_uint(lo.y));
+    off |= (__float_as_uint(v.z) ^ __float_as_uint(hi.x)) | (__float_as_uint(v.w) ^ __float_as_uint(hi.y));
+    return c;
+}
+__device__ __forceinline__ f32x16 fp4_products(const u32x4& a, const u32x4& b, const f32x16& d, int a_scale, int b_scale) {
+    typedef int i32x8 __attribute__((ext_vector_type(8)));
+    const i32x8 x = {(int)a.x, (int)a.y, (int)a.z, (int)a.w, 0, 0, 0, 0}, y = {(int)b.x, (int)b.y, (int)b.z, (int)b.w, 0, 0, 0, 0};
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, y, d, 4, 4, 0, a_scale, 0, b_scale);
+}
+// f(0), f(1), .. f(N - 1), each a constant.
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void each_of(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        each_of<N, I + 1>(f);
+    }
+}
+// bf16(relu(x)), and the same for an x of at most one in magnitude. (The second reads no matrix result that the first has not waited
+// for: the compiler does not see the wait that assembly would need.)
+__device__ __forceinline__ float relu_bf16(float x) {
+    x = round_bf16(x);
+    return x > 0.0f ? x : 0.0f;
+}
+__device__ __forceinline__ float clamp_bf16(float x) {
+    float r;
+    asm("v_cvt_pk_bf16_f32 %0, 0, %1 clamp" : "=v"(r) : "v"(x));
+    return r;
+}
+
+template <bool FP4>
 __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
     const float* __restrict__ q, const float* __restrict__ kv, const float* __restrict__ w,
     float* __restrict__ score, int s, int n_comp, int heads, int split_blocks, int ratio) {
-    // q rows on their way to operands (a wave's 32 at a time), then two kv tiles
+    // q rows on their way to operands (a wave's 32 at a time), then kv rows
     __shared__ __align__(16) unsigned char stage[kPairWaves * 32 * kPairRow];
     __shared__ __align__(16) float weights[kPairWaves][2][kPairHeads];
-    __shared__ int kv_spans[2][kPairTile];
+    __shared__ int kv_spans[2][2 * kPairTile];
+    __shared__ uint32_t row_expo[kPairWaves * 32], kv_expo[4 * kPairTile];  // four block exponents a row
+    __shared__ unsigned long long left_all[kPairWaves][2];
+    __shared__ int wave_fits[kPairWaves];
     const int lane = threadIdx.x & (kWave - 1), half = lane >> 5, row = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     // the last queries of a prefill rank the most blocks: they start first
@@ -459,18 +534,249 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
     const int tiles = tiles_for(min(s, (group + 1) * kPairQueries) - 1);
     if (!tiles) return;  // workgroup-uniform
     const int my_tiles = tw < s ? tiles_for(min(s, tw + 2) - 1) : 0;
+    const int t = tw + half;
 
-    // query t exists and its selection may rank a block of c's 64
-    const auto may_rank = [&](int t, int c) { return t < s && (ratio <= 0 || ((c & ~63) + 1) * (long long)ratio - 1 <= t); };
+    // blocks of query t from here on are nobody's: it does not exist, or its selection ranks none of their 64
+    const auto limit_of = [&](int t) { return t >= s ? 0 : ratio <= 0 ? n_comp : min(n_comp, ((t + 1) / ratio + 63) & ~63); };
+    const int limit = limit_of(t);
 
+    // kv tiles: eight threads a row, 16-byte pieces; the next ones are requested before these
+    // ones' products and parked after them
+    const int kr = threadIdx.x >> 3, kp = threadIdx.x & 7;
+    const auto request = [&](int tile, f32x4 (&to)[4]) {
+        const float* const p = kv + (size_t)min(c0 + tile * kPairTile + kr, n_comp - 1) * 128 + kp * 4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) to[j] = *reinterpret_cast<const f32x4*>(p + j * 32);
+    };
+    // eight loads of the rows of heads 16 c ..: load m = 2 (j0 + j) + half is row m, head c * 16 + (m >> 3) * 4 + (m & 3) of
+    // query (m >> 2) & 1; an instruction moves two whole rows
+    const auto load_heads = [&](int tw, int c, int j0, f32x4 (&v)[8]) {
+        const bool all = c * 16 + 16 <= heads;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int hh = c * 16 + ((j0 + j) >> 2) * 4 + (2 * (j0 + j) & 3);  // and hh + 1 in the upper half
+            const float* const at = q + (size_t)min(tw + ((j0 + j) >> 1 & 1), s - 1) * heads * 128;  // uniform
+            const uint32_t mine = (uint32_t)(half * 128 + row * 4);
+            if (all) {
+                v[j] = *reinterpret_cast<const f32x4_u*>(at + hh * 128 + mine);
+            } else {
+                v[j] = *reinterpret_cast<const f32x4_u*>(at + (uint32_t)(min(hh + half, heads - 1) * 128 + row * 4));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // all eight requested before the first is waited for
+        if (!all) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (c * 16 + ((j0 + j) >> 2) * 4 + (2 * (j0 + j) & 3) + half >= heads) v[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    };
+
+    float own_weights[2];  // of head `lane`, both queries
+#pragma unroll
+    for (int i = 0; i < 2; ++i) own_weights[i] = lane < heads ? w[(size_t)min(tw + i, s - 1) * heads + lane] : 0.0f;
+    unsigned long long left[2] = {0, 0};  // one bit per tile that the fp4 products did not do
+    if constexpr (FP4) {
+        f32x4 next[2][4];  // two tiles at a time
+        request(0, next[0]);
+        request(1, next[1]);  // (past the last block: that one again)
+        unsigned char* const kv_codes = stage + kPairWaves * 32 * kFp4Row;
+        // Row 32 u + kr of buffer `buf`; whether it is made of codes.
+        const auto park = [&](int buf, int u) -> bool {
+            const int at = (2 * buf + u) * kPairTile + kr;
+            unsigned char* const to = kv_codes + at * kFp4Row + kp * 2;
+            uint32_t off = 0, e[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) *reinterpret_cast<uint16_t*>(to + j * 16) = (uint16_t)fp4_of(next[u][j], e[j], off);
+            const uint32_t hi = max(max(e[0], e[1]), max(e[2], e[3]));
+            uint32_t lo = min(min(e[0], e[1]), min(e[2], e[3]));
+            if (__any(lo == 0)) {  // a block of zeros takes the largest's scale
+#pragma unroll
+                for (int j = 0; j < 4; ++j) e[j] = e[j] ? e[j] : hi;
+                lo = min(min(e[0], e[1]), min(e[2], e[3]));
+            }
+            // 127 + e - hi in each byte (none of them borrows where the row is taken)
+            const uint32_t expo = (e[0] | e[1] << 8 | e[2] << 16 | e[3] << 24) + 0x7f7f7f7fu - __builtin_amdgcn_perm(hi, hi, 0u);
+            uint32_t span = hi - lo;
+            if (hi - (uint32_t)kFp4MinExp > (uint32_t)(kFp4MaxExp - kFp4MinExp) && hi) span = kNoSpan;
+            const unsigned long long bad = __ballot(off != 0);
+            if (bad) span = bad >> (lane & ~7) & 0xffu ? (uint32_t)kNoSpan : span;
+            // (eight threads, one word)
+            kv_expo[at] = expo;
+            kv_spans[buf][u * kPairTile + kr] = (int)(span | hi << 8);
+            return off == 0;
+        };
+        bool fits = my_tiles > 0;
+        // ---- the rows as fp4 operands: lane's row of a matrix tile, blocks half and 2 + half of its four ----
+        u32x4 a[4][2];
+        uint32_t a_expo[4] = {};
+        unsigned char* const mine = stage + wave * 32 * kFp4Row;
+        uint32_t off = 0;
+        int top = 0, bottom = 255, apart = 0;  // block exponents: the rows' largest, smallest; largest difference in a row
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (c * 16 >= heads || (c == 1 && !fits)) break;
+#pragma unroll
+            for (int j0 = 0; j0 < 16; j0 += 8) {
+                f32x4 v[8];
+                load_heads(tw, c, j0, v);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int m = 2 * (j0 + j) + half;
+                    uint32_t expo;
+                    *reinterpret_cast<uint16_t*>(mine + m * kFp4Row + row * 2) = (uint16_t)fp4_of(v[j], expo, off);
+                    // (eight lanes, one byte)
+                    reinterpret_cast<unsigned char*>(row_expo)[(wave * 32 + m) * 4 + (row >> 3)] = (unsigned char)expo;
+                }
+                asm volatile("" ::: "memory");  // no more than eight rows' loads in registers at a time
+            }
+            asm volatile("" ::: "memory");  // the rows cross lanes: LDS serves a wave in order, the compiler must keep to it
+#pragma unroll
+            for (int k = 0; k < 2; ++k) a[c][k] = *reinterpret_cast<const u32x4*>(mine + row * kFp4Row + (2 * k + half) * 16);
+            const uint32_t x = row_expo[wave * 32 + row];
+            int hi = 0, lo = 255;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int e = (int)(x >> (8 * k) & 0xffu);
+                hi = max(hi, e), lo = min(lo, e ? e : 255);
+            }
+            top = max(top, hi), bottom = min(bottom, lo), apart = max(apart, hi - lo);  // a row of zeros: -255
+            a_expo[c] = x >> (8 * half);
+            asm volatile("" ::: "memory");
+            // Where some of the first sixteen heads' values, or of the wave's own rows of the first two tiles, are no codes, hardly any are.
+            if (c == 0) {
+                const bool codes[2] = {park(0, 0), park(0, 1)};
+                if (__any(!codes[0] || !codes[1] || off != 0)) fits = false;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            weights[wave][i][lane] = own_weights[i];
+            const uint32_t e = (__float_as_uint(own_weights[i]) & 0x7fffffffu) >> 23;
+            if (own_weights[i] != 0.0f && (e < kFp4Weight0 || e > kFp4Weight1)) off = 1;  // (a NaN differs from zero)
+        }
+        asm volatile("" ::: "memory");
+        if (__any(off != 0)) fits = false;
+#pragma unroll
+        for (int m = 1; m < 32; m <<= 1) {
+            top = max(top, __shfl_xor(top, m, kWave)), bottom = min(bottom, __shfl_xor(bottom, m, kWave));
+            apart = max(apart, __shfl_xor(apart, m, kWave));
+        }
+        top = __builtin_amdgcn_readfirstlane(top), bottom = __builtin_amdgcn_readfirstlane(bottom), apart = __builtin_amdgcn_readfirstlane(apart);
+        if (top != 0 && (top > kFp4MaxExp || top < kFp4MinExp || top - bottom > kFp4Heads)) fits = false;
+        // scales relative to the largest (a block of zeros takes that)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int e0 = (int)(a_expo[c] & 0xffu), e1 = (int)(a_expo[c] >> 16 & 0xffu);
+            a_expo[c] = (uint32_t)(127 - kFp4Down + (e0 ? e0 - top : 0)) | (uint32_t)(127 - kFp4Down + (e1 ? e1 - top : 0)) << 8;
+        }
+        f32x4 wv[kPairHeads / 4];
+#pragma unroll
+        for (int i = 0; i < kPairHeads / 4; ++i) wv[i] = *reinterpret_cast<const f32x4*>(&weights[wave][half][4 * i]);
+
+        if (!fits) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+                if (my_tiles > 64 * k) left[k] = my_tiles >= 64 * (k + 1) ? ~0ull : (1ull << (my_tiles & 63)) - 1;
+        }
+        if (lane == 0) wave_fits[wave] = fits;
+        __syncthreads();
+        bool some = false;
+#pragma unroll
+        for (int i = 0; i < kPairWaves; ++i) some = some || wave_fits[i];
+        const int walk = some ? tiles : 0;
+        for (int tile = 0, buf = 0; tile < walk; tile += 2, buf ^= 1) {
+            __syncthreads();  // these tiles are parked and nobody reads the other buffer any more
+            if (tile + 2 < tiles) {
+                request(tile + 2, next[0]);
+                request(tile + 3, next[1]);  // (past the last block: that one again)
+            }
+            if (fits && tile < my_tiles) {
+                u32x4 b[2][2];
+                int b_expo[2], info[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int at = (2 * buf + u) * kPairTile + row;
+                    const unsigned char* const from = kv_codes + at * kFp4Row + half * 16;
+                    b[u][0] = *reinterpret_cast<const u32x4*>(from), b[u][1] = *reinterpret_cast<const u32x4*>(from + 32);
+                    b_expo[u] = (int)(kv_expo[at] >> (8 * half));
+                    info[u] = kv_spans[buf][u * kPairTile + row];
+                }
+                const auto products = [&](int u, int c) {
+                    f32x16 d = {};
+                    d = fp4_products(a[c][0], b[u][0], d, (int)a_expo[c], b_expo[u]);
+                    return fp4_products(a[c][1], b[u][1], d, (int)(a_expo[c] >> 8), b_expo[u] >> 16);
+                };
+                f32x16 d = products(0, 0);
+                const auto taken = [&](int u) {
+                    const int back = top + (info[u] >> 8) - 2 * 129 + kFp4Down;  // the scores' scale
+                    const bool zero = (info[u] >> 8) == 0 || top == 0;
+                    return !__any(max(apart, 0) + (info[u] & 0xff) > kFp4Span || (!zero && (back < kFp4Back0 || back > kFp4Back1)));
+                };
+                const bool take[2] = {taken(0), taken(1)};
+                float acc = 0.0f;
+                const auto finish = [&](int u, int info) {
+                    const int c = c0 + (tile + u) * kPairTile + row;
+                    if (c < limit) score[(size_t)t * n_comp + c] = round_bf16(__builtin_amdgcn_ldexpf(acc, top + (info >> 8) - 2 * 129 + kFp4Down));
+                    acc = 0.0f;
+                };
+                if (!take[0]) left[tile >> 6] |= 1ull << (tile & 63);
+                if (!take[1] && tile + 1 < my_tiles) left[tile >> 6] |= 2ull << (tile & 63);
+                if (heads > 48 && take[0] && take[1]) {
+                    // A step has a head's conversion, the weight of the one before, the rounding of the one before that and the sum's
+                    // addition of a fourth: four instructions of which none waits for another. The next sixteen
+                    // heads' products run under these heads' steps.
+                    constexpr int kSteps = 2 * kPairHeads;
+                    f32x16 sets[2];
+                    sets[0] = d;
+                    float clamped = 0.0f, weighted = 0.0f, term = 0.0f;
+                    each_of<kSteps + 3>([&](auto step) {
+                        constexpr int n = decltype(step)::value, set = n / 16;
+                        if constexpr (n % 16 == 0 && set + 1 < kSteps / 16) sets[(set + 1) & 1] = products((set + 1) / 4, (set + 1) % 4);
+                        if constexpr (n >= 3) acc = acc + term;
+                        if constexpr (n >= 2 && n < kSteps + 2) term = round_bf16(weighted);
+                        if constexpr (n >= 1 && n < kSteps + 1) weighted = clamped * wv[(n - 1) / 4 % 16][(n - 1) % 4];
+                        if constexpr (n < kSteps) clamped = n % 16 == 0 ? relu_bf16(sets[set & 1][0]) : clamp_bf16(sets[set & 1][n % 16]);
+                        if constexpr (n == kPairHeads + 2) finish(0, info[0]);
+                        if constexpr (n == kSteps + 2) finish(1, info[1]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    });
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        if (!take[u]) continue;
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            if (c * 16 >= heads) break;
+                            const f32x16 d = products(u, c);
+#pragma unroll
+                            for (int i = 0; i < 16; ++i) acc = acc + head_term(d[i], wv[4 * c + i / 4][i % 4]);
+                        }
+                        finish(u, info[u]);
+                    }
+                }
+            }
+            if (tile + 2 < tiles) park(buf ^ 1, 0), park(buf ^ 1, 1);
+        }
+    }
+    // ---- what those rows are not, tiles of any of the four waves, or all of them: as bf16 operands where those are exact -----
+    if constexpr (FP4) {
+        if (lane < 2) left_all[wave][lane] = lane ? left[1] : left[0];
+        __syncthreads();
+        bool some = false;
+#pragma unroll
+        for (int i = 0; i < kPairWaves; ++i) some = some || (left_all[i][0] | left_all[i][1]) != 0;
+        if (!some) return;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) weights[wave][i][lane] = own_weights[i];
+    }
+    f32x4 next[4];
+    int again = tw;  // (nothing of the first pass over the rows is kept for the second)
+    asm volatile("" : "+s"(again));
     bf16x8 a[4][8];
     int q_span = 0;
     {
         unsigned char* const mine = stage + wave * 32 * kPairRow;
-        for (int i = lane; i < 2 * kPairHeads; i += kWave) {
-            const int hh = i & (kPairHeads - 1), t = min(tw + (i >> 6), s - 1);
-            weights[wave][i >> 6][hh] = hh < heads ? w[(size_t)t * heads + hh] : 0.0f;
-        }
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             if (c * 16 >= heads) break;
@@ -478,25 +784,17 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
 #pragma unroll
             for (int j0 = 0; j0 < 16; j0 += 8) {
                 f32x4 v[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {  // an instruction moves two whole rows
-                    const int m = 2 * (j0 + j) + half, hh = c * 16 + (m >> 3) * 4 + (m & 3);
-                    const int t = min(tw + ((m >> 2) & 1), s - 1);
-                    v[j] = *reinterpret_cast<const f32x4_u*>(q + ((size_t)t * heads + min(hh, heads - 1)) * 128 + row * 4);
-                }
-                __builtin_amdgcn_sched_barrier(0);  // all eight requested before the first is waited for
+                load_heads(again, c, j0, v);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const int m = 2 * (j0 + j) + half, hh = c * 16 + (m >> 3) * 4 + (m & 3);
-                    if (hh >= heads) v[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                     low |= low_half_bits(v[j]);
                     const u32x2 p = {upper_halves(v[j].x, v[j].y), upper_halves(v[j].z, v[j].w)};
                     *reinterpret_cast<u32x2*>(mine + (2 * (j0 + j) + half) * kPairRow + row * 8) = p;
                 }
-                asm volatile("" ::: "memory");  // no more than eight rows' loads in registers at a time
+                asm volatile("" ::: "memory");
             }
             if (__any(low != 0)) q_span = kNoSpan;
-            asm volatile("" ::: "memory");  // the rows cross lanes: LDS serves a wave in order, the compiler must keep to it
+            asm volatile("" ::: "memory");
             RowSpan span;
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
@@ -511,18 +809,9 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
 #pragma unroll
         for (int m = 1; m < 32; m <<= 1) q_span = max(q_span, __shfl_xor(q_span, m, kWave));
     }
-
-    // kv tiles: eight threads a row, 16-byte pieces; the next tile's are requested before this
-    // one's products and parked after them
-    const int kr = threadIdx.x >> 3, kp = threadIdx.x & 7;
-    f32x4 next[4];
-    const auto request = [&](int tile) {
-        const float* const p = kv + (size_t)min(c0 + tile * kPairTile + kr, n_comp - 1) * 128 + kp * 4;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) next[j] = *reinterpret_cast<const f32x4*>(p + j * 32);
-    };
-    const auto park = [&](int tile) {
-        unsigned char* const to = stage + ((tile & 1) * kPairTile + kr) * kPairRow + kp * 8;
+    int parity = 0;
+    const auto park = [&]() {
+        unsigned char* const to = stage + (parity * kPairTile + kr) * kPairRow + kp * 8;
         RowSpan span;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -535,21 +824,41 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
         f = span_max(f, __shfl_xor(f, 1, kWave));
         f = span_max(f, __shfl_xor(f, 2, kWave));
         f = span_max(f, __shfl_xor(f, 4, kWave));
-        if (kp == 0) kv_spans[tile & 1][kr] = span_of(f);
+        if (kp == 0) kv_spans[parity][kr] = span_of(f);
     };
-    request(0);
-    __syncthreads();  // every wave's q rows are out of the stage
-    park(0);
+    if constexpr (!FP4) request(0, next);
+    __syncthreads();  // every wave's q rows are out of the stage, and its tiles in left_all
+    unsigned long long todo[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        todo[k] = 0;
+        if constexpr (FP4) {
+            for (int i = 0; i < kPairWaves; ++i) todo[k] |= left_all[i][k];
+        } else {
+            if (tiles > 64 * k) todo[k] = tiles >= 64 * (k + 1) ? ~0ull : (1ull << (tiles & 63)) - 1;
+            if (my_tiles > 64 * k) left[k] = my_tiles >= 64 * (k + 1) ? ~0ull : (1ull << (my_tiles & 63)) - 1;
+        }
+    }
+    const auto pop = [&]() {  // the next of them, or -1
+        const int k = todo[0] ? 0 : 1;
+        const unsigned long long from = k ? todo[1] : todo[0];
+        if (!from) return -1;
+        (k ? todo[1] : todo[0]) = from & (from - 1);
+        return __builtin_amdgcn_readfirstlane(64 * k + __builtin_ctzll(from));
+    };
     unsigned long long inexact[2] = {0, 0};  // one bit per tile
-    const int t = tw + half;
-    for (int tile = 0; tile < tiles; ++tile) {
-        __syncthreads();  // this tile is parked and nobody reads the other buffer any more
-        if (tile + 1 < tiles) request(tile + 1);
-        if (tile < my_tiles) {
-            if (__any(kv_spans[tile & 1][row] + q_span > kExactSpan)) {
+    int tile = pop();
+    if constexpr (FP4) request(tile, next);
+    park();
+    while (tile >= 0) {
+        __syncthreads();
+        const int after = pop();
+        if (after >= 0) request(after, next);
+        if (left[tile >> 6] >> (tile & 63) & 1) {
+            if (__any(kv_spans[parity][row] + q_span > kExactSpan)) {
                 inexact[tile >> 6] |= 1ull << (tile & 63);
             } else {
-                const unsigned char* const from = stage + ((tile & 1) * kPairTile + row) * kPairRow + half * 16;
+                const unsigned char* const from = stage + (parity * kPairTile + row) * kPairRow + half * 16;
                 bf16x8 b[8];
 #pragma unroll
                 for (int k = 0; k < 8; ++k) b[k] = *reinterpret_cast<const bf16x8*>(from + k * 32);
@@ -560,7 +869,6 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
                     if (c * 16 >= heads) break;
-                    // the next sixteen heads' products run under these heads' terms
                     if (c < 3 && (c + 1) * 16 < heads) {
                         f32x16& n = d[(c + 1) & 1];
                         n = f32x16{};
@@ -575,11 +883,13 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
                     }
                 }
                 const int c = c0 + tile * kPairTile + row;
-                if (c < n_comp && may_rank(t, c))
+                if (c < limit)
                     score[(size_t)t * n_comp + c] = round_bf16(acc);
             }
         }
-        if (tile + 1 < tiles) park(tile + 1);
+        parity ^= 1;
+        if (after >= 0) park();
+        tile = after;
     }
     // What is left, term by term: a lane owns a block of a 64-block group for both of the wave's
     // queries, or where only one of the group's tiles is left a block of that for one of them.
@@ -601,8 +911,8 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
                     acc = acc + term;
                     if (i + 1 == heads) sum = acc, acc = 0.0f;
                 });
-                if (c < n_comp && may_rank(first, c)) score[(size_t)first * n_comp + c] = round_bf16(sum);
-                if (c < n_comp && both && may_rank(tw + 1, c)) score[(size_t)(tw + 1) * n_comp + c] = round_bf16(acc);
+                if (c < limit_of(first)) score[(size_t)first * n_comp + c] = round_bf16(sum);
+                if (both && c < limit_of(tw + 1)) score[(size_t)(tw + 1) * n_comp + c] = round_bf16(acc);
             }
         }
     };
@@ -788,6 +1098,10 @@ namespace rk {
 // 10 (4 x 8 192, 512 workgroups: 11.3 against 10.4; 300 queries x 75, 600: 15 against 10). One query
 // has no second for the many-query kernel's wave: 65 536 blocks 18 us against 25.
 constexpr int kOneGroups = 384;
+// Workgroups of so many blocks turn their q rows into fp4 codes, which takes a wave 2 200 vector instructions where bf16 operands
+// take 900: 192 blocks (2 049 x 512) 37 us as bf16 and 35.5 so, 384 (3 000 x 750) 54 and 48; 128 (1 500 x 375) 26.6 and 26.2, 64 (700 x 175)
+// 10.4 and 11.5.
+constexpr int kFp4Blocks = 192;
 static int score_blocks_launch(const float* q, const float* kv, const float* w, float* score, int s,
                                int n_comp, int heads, int hd, int ratio, hipStream_t st) {
     if (s <= 0 || heads <= 0 || hd <= 0) return 1001;
@@ -816,6 +1130,7 @@ static int score_blocks_launch(const float* q, const float* kv, const float* w, 
         long long splits = t_groups >= 1024 ? 1 : 1024 / t_groups;
         if (splits > groups) splits = groups;
         int per = (int)((groups + splits - 1) / splits) * 64;
+        const bool fp4 = per >= kFp4Blocks;
         // A tile each where that leaves compute units over, or is still one round and the q rows (32 KB
         // a query) stay in a die's 4 MB of cache, which every one of a query's workgroups reads them
         // through: 300 x 75 (114 workgroups) 11.7 -> 10.5 us, 5 x 8 192 (256) 10.1 -> 8.8; but 150 x 300 (190,
@@ -824,8 +1139,12 @@ static int score_blocks_launch(const float* q, const float* kv, const float* w, 
         if (per > kPairSplitMax) per = kPairSplitMax;
         const unsigned y = (unsigned)(((long long)n_comp + per - 1) / per);
         if (y <= 65535u) {
-            hipLaunchKernelGGL(score_blocks_pair_kernel, dim3(t_groups, y), dim3(kPairThreads), 0, st, q, kv, w, score,
-                               s, n_comp, heads, per, ratio);
+            if (fp4)
+                hipLaunchKernelGGL(score_blocks_pair_kernel<true>, dim3(t_groups, y), dim3(kPairThreads), 0, st, q, kv, w, score,
+                                   s, n_comp, heads, per, ratio);
+            else
+                hipLaunchKernelGGL(score_blocks_pair_kernel<false>, dim3(t_groups, y), dim3(kPairThreads), 0, st, q, kv, w, score,
+                                   s, n_comp, heads, per, ratio);
             return launch_status();
         }
     }

@@ -324,3 +324,63 @@ def test_score_at_the_largest_and_smallest_exponents_whose_sums_are_exact(oracle
     code, want = oracle.index_score_blocks(q, kv, w)
     assert code == 0 and np.isinf(want).all() == (exponent == 60)
     assert same_bits(device_score(q, kv, w), want).size == 0
+
+
+def coded_rows(rng, rows, exponents):
+    """Rows of e2m1 codes, each block of 32 times 2 to its exponent (`exponents` [rows][4]) and with a 4 or a 6."""
+    x = rng.choice(np.array([0.0, -0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0]), (rows, 4, 32)) * rng.choice([-1.0, 1.0], (rows, 4, 32))
+    x[:, :, 5] = rng.choice([4.0, 6.0], (rows, 4))
+    return (x * 2.0 ** np.asarray(exponents, np.float64)[:, :, None]).reshape(rows, 128).astype(np.float32)
+
+
+@pytest.mark.parametrize("s,n_comp,heads", [(2060, 230, 64), (2060, 161, 49), (2060, 193, 33), (1380, 390, 64)])
+def test_score_at_the_edges_of_what_the_fp4_products_take(oracle, s, n_comp, heads):
+    """Each wave's two queries are of one kind: at and just past every bound under which dots come from the block-scaled fp4
+    instruction, clamped and scaled (block exponents 9 apart, heads 20 binades, weights 2^+-50, scores scaled back by
+    2^-20 and 2^40), rows of zeros and values that are no code. The blocks' rows likewise, in tiles of their own.
+    Bit for bit on three waves of each kind, in both forms."""
+    rng = np.random.default_rng(s + n_comp + heads)
+    def at(e):  # every row's exponents
+        return np.broadcast_to(np.asarray(e), (2 * heads, 4))
+    def one_head(e, other):  # one head apart from the others
+        x = np.full((2 * heads, 4), e)
+        x[heads // 2] = other
+        return x
+    kinds = [at([0, 0, 1, 0]), at([5, 0, 3, 1]), at([6, 0, 3, 1]), one_head(0, -20), one_head(0, -21), at([0, 0, 0, 0]), at([0, 0, 0, 0]),
+             at([30, 30, 30, 29]), at([31, 30, 30, 30]), at([-29, -29, -29, -29]), at([-30, -30, -30, -30]), at([0, 0, 0, 0]), at([1, 0, 0, 0]),
+             at([1, 0, 0, 0]), at([0, 1, 0, 0])]
+    q = np.zeros((s, heads, 128), np.float32)
+    w = bf16_round((rng.standard_normal((s, heads)) * 0.1).astype(np.float32))
+    for pair in range(s // 2):
+        k = pair % len(kinds)
+        rows = coded_rows(rng, 2 * heads, kinds[k])
+        if k == 11: rows[:] = 0.0
+        if k == 12: rows[::3, 32:64] = 0.0
+        if k == 13: rows[heads - 1, 7] = 0.75          # half of a code's smallest step
+        if k == 14: rows[1] = rng.standard_normal(128)
+        q[2 * pair:2 * pair + 2] = rows.reshape(2, heads, 128)
+        if k == 5: w[2 * pair, ::2], w[2 * pair + 1, 1::3] = 2.0 ** 50, 1.5 * 2.0 ** -50
+        if k == 6: w[2 * pair, 0], w[2 * pair + 1, 1] = 2.0 ** 51, 1.5 * 2.0 ** -51
+    kv = coded_rows(rng, n_comp, np.where(np.arange(n_comp)[:, None] // 64 == 1, [0, 4, 1, 0], [0, 0, -1, 0]))
+    kv[70] = 0.0
+    kv[75, 96:] = 0.0
+    kv[n_comp - 1] = rng.standard_normal(128)
+    kv[n_comp - 2, 3] = 0.25
+    # (the scores' scale with exponents e and f: e + f + 13; the first blocks' f is 0, 64 to 127's is 4)
+    pairs = [len(kinds) * r + k for r in (0, 40, (s // 2 - len(kinds)) // len(kinds)) for k in range(len(kinds))]
+    queries = np.array([2 * p + i for p in pairs for i in (0, 1)] + [s - 1])
+    code, want = oracle.index_score_blocks(q[queries], kv, w[queries])
+    assert code == 0 and np.isfinite(want).all()
+    qd, kd, wd = dev(q), dev(kv), dev(w)
+    for ratio in (0, 4):
+        out = dzeros(s * n_comp * 4, 0x5A)
+        if ratio:
+            hip.launch_index_score_blocks_prefill(qd, kd, wd, out, s, n_comp, heads, 128, ratio)
+        else:
+            hip.launch_index_score_blocks(qd, kd, wd, out, s, n_comp, heads, 128)
+        got = back(out, np.uint32).reshape(s, n_comp)[queries]
+        live = np.ones(got.shape, bool) if not ratio else \
+            (np.arange(n_comp)[None, :] // 64) * 64 < np.minimum((queries + 1) // ratio, n_comp)[:, None]
+        bad = np.argwhere((got != want.view(np.uint32)) & live)
+        assert bad.size == 0, (ratio, [(int(queries[i]), int(queries[i]) // 2 % len(kinds), int(c)) for i, c in bad[:6]])
+        assert (got[~live] == 0x5A5A5A5A).all()
