@@ -742,48 +742,54 @@ __device__ __forceinline__ bool dealt_part(const AttendArgs& a, int item, const 
 struct SeqDeal {
     int tiles, parts, first;  // of the lane's sequence: its tiles, its work items, the first of them
 };
-__device__ __forceinline__ int ceil_quotient(int t, int c, float inv) {
+__device__ __forceinline__ int ceil_quotient(int t, int c, float inv) {  // t + c below 2^24
     const int n = t + c - 1;
-    int q = (int)((float)n * inv);  // off by one at most
+    int q = (int)((float)n * inv);  // off by one at most, with an approximate inverse too
     q -= q * c > n;
     q += (q + 1) * c <= n;
     return q;
 }
-// Needs n_items >= 2 * n_seqs. `lens` null: every sequence has k rows.
+// x summed over this lane and the ones before it
+__device__ __forceinline__ int lanes_upto(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // one, two, four, eight lanes back in its sixteen
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // the last lane of the sixteen before
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // and of the 32 before
+    return x;
+}
+// Needs n_items >= 2 * n_seqs. `lens` null: every sequence has k rows. (The workgroups and the merge wait for this before they know an
+// address: by lane shuffles and exact divisions it took 1.2 us of either: 8 listed sets of 2 048 rows 23.4 -> 22.3 us, 300 linear rows and more as much less.)
 __device__ __forceinline__ SeqDeal seq_deal(const int* lens, int k, int n_seqs, int n_items, int unit) {
     const int lane = threadIdx.x & (kWave - 1);
     SeqDeal d;
     const int rows = lens ? max(min(lens[min(lane, n_seqs - 1)], k), 0) : k;
-    d.tiles = lane < n_seqs ? (rows + kTile - 1) / kTile : 0;
-    int total = d.tiles, longest = d.tiles;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        total += __shfl_xor(total, off, kWave);
-        longest = max(longest, __shfl_xor(longest, off, kWave));
-    }
+    d.tiles = lane < n_seqs ? (int)((unsigned)rows + kTile - 1) / kTile : 0;
+    const int total = __builtin_amdgcn_readlane(lanes_upto(d.tiles), kWave - 1);
     // `rounds` units: at least what an even deal gives, and then the first that suffices
-    const int least = max((total + unit * n_items - 1) / (unit * n_items), 1);
-    const int c = (least + lane) * unit;
-    const float c_inv = 1.0f / (float)c;
-    int items = 0;
-    for (int s = 0; s < n_seqs; ++s) items += ceil_quotient(__builtin_amdgcn_readlane(d.tiles, s), c, c_inv);
-    const unsigned long long enough = __ballot(items <= n_items);
-    int rounds;
-    if (enough) {
-        rounds = least + __builtin_ctzll(enough);
-    } else {  // sum of ceil(t / run) <= total / run + n_seqs; and a run that holds the longest is one item each
-        const int spare = unit * (n_items - n_seqs);
-        rounds = max(min((total + spare - 1) / spare, (longest + unit - 1) / unit), 1);
+    const int share = unit * n_items;
+    const int least = max(ceil_quotient(total, share, __builtin_amdgcn_rcpf((float)share)), 1);
+    int rounds = least;
+    if (n_seqs > 1) {  // (of one sequence the even deal's suffice)
+        const int c = (least + lane) * unit;
+        const float c_inv = __builtin_amdgcn_rcpf((float)c);
+        int items = 0;
+        for (int s = 0; s < n_seqs; ++s) items += ceil_quotient(__builtin_amdgcn_readlane(d.tiles, s), c, c_inv);
+        const unsigned long long enough = __ballot(items <= n_items);
+        if (enough) {
+            rounds = least + __builtin_ctzll(enough);
+        } else {  // sum of ceil(t / run) <= total / run + n_seqs; and a run that holds the longest is one item each
+            int longest = d.tiles;
+#pragma unroll
+            for (int off = 1; off < kWave; off <<= 1) longest = max(longest, __shfl_xor(longest, off, kWave));
+            const int spare = unit * (n_items - n_seqs);
+            rounds = max(min((total + spare - 1) / spare, (longest + unit - 1) / unit), 1);
+        }
     }
     const int run = __builtin_amdgcn_readfirstlane(rounds * unit);
-    d.parts = ceil_quotient(d.tiles, run, 1.0f / (float)run);
-    int upto = d.parts;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const int up = __shfl_up(upto, off, kWave);
-        if (lane >= off) upto += up;
-    }
-    d.first = upto - d.parts;
+    d.parts = ceil_quotient(d.tiles, run, __builtin_amdgcn_rcpf((float)run));
+    d.first = lanes_upto(d.parts) - d.parts;
     return d;
 }
 
@@ -827,6 +833,25 @@ __global__ __launch_bounds__(F8 ? kF8Threads : kAttThreads) void mla_attend_page
   }  // parts of this workgroup
 }
 
+// The part of a work item that SeqDeal gives it, head group `hg`: part_of is called with it as attend_part.
+template <int MODE, class PART>
+__device__ __forceinline__ void seq_walk(const AttendArgs& a, int item, int hg, PART part_of) {
+    const SeqDeal d = seq_deal(MODE == kLinear ? nullptr : (MODE == kSparse ? a.n_rows : a.seq_lens), a.k, a.n_seqs, a.n_items, a.by_seq);
+    const unsigned long long past = __ballot(d.first + d.parts > item);
+    if (!past) return;  // more work items than runs
+    const int seq = __builtin_ctzll(past);
+    const int first = __builtin_amdgcn_readlane(d.first, seq), parts = __builtin_amdgcn_readlane(d.parts, seq);
+    // of a sequence's work items none is longer than the run: its tiles in `parts` even shares, the longer ones first
+    const int tiles = __builtin_amdgcn_readlane(d.tiles, seq), part = item - first;
+    const int most = ceil_quotient(tiles, parts, __builtin_amdgcn_rcpf((float)parts)), fewer = most * parts - tiles;  // of them with one tile less
+    const int t_begin = part * most - max(part - (parts - fewer), 0);
+    const int t_end = t_begin + most - (part >= parts - fewer);
+    const int r_begin = t_begin * kTile;
+    const int r_end = (int)min((unsigned)attended_rows<MODE>(a, seq), (unsigned)t_end * kTile);
+    const size_t rec = (size_t)item + seq;
+    part_of(seq, hg, r_begin, r_end, parts == 1, a.part_acc + rec * a.H * kKvl, a.part_ml + rec * a.H * 2);
+}
+
 // The same walk for 16 heads per workgroup of THREADS: `part` is called with each part of its work as attend_part's, a
 // part of several sequences' with a barrier before it.
 template <int THREADS, int MODE, class PART>
@@ -839,17 +864,7 @@ __device__ __forceinline__ void heads16_walk(const AttendArgs& a, int (&pre)[kDe
     int seq = item;
     if (item >= (a.n_items > 0 ? a.n_items : a.n_seqs)) return;
     if (a.by_seq) {
-        const SeqDeal d = seq_deal(MODE == kLinear ? nullptr : (MODE == kSparse ? a.n_rows : a.seq_lens), a.k, a.n_seqs, a.n_items, a.by_seq);
-        const unsigned long long past = __ballot(d.first + d.parts > item);
-        if (!past) return;  // more work items than runs
-        seq = __builtin_ctzll(past);
-        const int first = __builtin_amdgcn_readlane(d.first, seq), parts = __builtin_amdgcn_readlane(d.parts, seq);
-        // of a sequence's work items none is longer than the run: its tiles in `parts` even shares
-        const int tiles = __builtin_amdgcn_readlane(d.tiles, seq), part = item - first;
-        const int r_begin = (int)((unsigned)(part * tiles) / (unsigned)parts) * kTile;
-        const int r_end = min(attended_rows<MODE>(a, seq), (int)((unsigned)((part + 1) * tiles) / (unsigned)parts) * kTile);
-        const size_t rec = (size_t)item + seq;
-        part_of(seq, hg, r_begin, r_end, parts == 1, a.part_acc + rec * a.H * kKvl, a.part_ml + rec * a.H * 2);
+        seq_walk<MODE>(a, item, hg, part_of);
         return;
     }
     if (!dealt_range<THREADS, MODE>(a, item, pre, wave_total, t_lo, t_hi, seq)) return;
@@ -896,6 +911,7 @@ __global__ __launch_bounds__(kFewThreads) void mla_attend_few_kernel(const Atten
 // records, w_r = 2^(m_r - max m), in ascending work-item order (the reference's combine,
 // crates/backend/kernels/attn.hip:235-277, in base 2). A sequence that one work item covered
 // whole was written by it directly; one with nothing to attend gets zeros.
+template <int SUBS>
 __global__ __launch_bounds__(128) void mla_attend_combine_kernel(
     const float* __restrict__ part_acc, const float* __restrict__ part_ml, const int* __restrict__ seq_lens,
     const int* __restrict__ n_rows, int sparse, int k, int n_seqs, int n_items, int by_seq, int H, int kvl,
@@ -935,69 +951,73 @@ __global__ __launch_bounds__(128) void mla_attend_combine_kernel(
         first = mine ? deal_item_of(before, n_items, total) : 0;
         last = mine ? deal_item_of(before + mine - 1, n_items, total) : 0;
     }
-    if (4 * (int)threadIdx.x >= kvl) return;  // the records are 512 wide whatever the cache's width
-    float4* const dst = reinterpret_cast<float4*>(clat + ((size_t)seq * H + head) * kvl) + threadIdx.x;
+    // SUBS groups of threads share the head's columns, blockIdx.z the part of them, and take every SUBS-th record each
+    constexpr int kCols = 128 / SUBS;
+    const int sub = (int)threadIdx.x / kCols, col = (int)blockIdx.z * kCols + (int)threadIdx.x % kCols;
+    const bool mine_col = 4 * col < kvl;  // the records are 512 wide whatever the cache's width
+    float4* const dst = reinterpret_cast<float4*>(clat + ((size_t)seq * H + head) * kvl) + col;
     if (mine == 0) {
-        *dst = float4{0, 0, 0, 0};
+        if (mine_col && sub == 0) *dst = float4{0, 0, 0, 0};
         return;
     }
     if (first == last) return;  // one work item had the whole sequence and wrote it
     // Records are fetched a batch at a time, every load of a batch issued before the first use (a record past the last
-    // re-reads the last and is left out). Up to 16 records, as many as most calls have a sequence, are one batch, and
-    // their accumulators are asked for with the maxima that weigh them: one round trip to memory, where maxima first and
-    // eight at a time took four (6 ragged sequences of up to 9 000 tokens of 64 heads 36.2 -> 35.6 us with the append,
-    // 8 listed sets of 2 048 rows with the selection 43.5 -> 42.7). The sums run in ascending record order.
+    // re-reads the last and is left out), accumulators with the maxima that weigh them: one round trip to memory a batch (maxima first and
+    // eight records at a time took four where this takes one). The sums go on under the largest maximum so far, in ascending record order.
     float4 sum = {0, 0, 0, 0};
-    float l_g = 0.0f;
-    auto add = [&](float w, float l, float4 v) {
-        l_g += l * w;
-        sum.x += v.x * w, sum.y += v.y * w, sum.z += v.z * w, sum.w += v.w * w;
-    };
-    auto batch = [&](auto size, int b0, float (&m_r)[decltype(size)::value], float (&l_r)[decltype(size)::value],
-                     float4 (&v)[decltype(size)::value]) {
-#pragma unroll
-        for (int u = 0; u < decltype(size)::value; ++u) {
-            const size_t rec = (size_t)min(b0 + u, last) + seq;
-            m_r[u] = part_ml[(rec * H + head) * 2];
-            l_r[u] = part_ml[(rec * H + head) * 2 + 1];
-            v[u] = reinterpret_cast<const float4*>(part_acc + (rec * H + head) * kKvl)[threadIdx.x];
-        }
-    };
-    auto merge_one = [&](auto size) {
+    float l_g = 0.0f, m_g = -INFINITY;
+    const int n_mine = (last - first - sub + SUBS) / SUBS;  // the group's
+    auto merge = [&](auto size) {
         constexpr int N = decltype(size)::value;
-        float m_r[N], l_r[N], m_g = -INFINITY;
-        float4 v[N];
-        batch(size, first, m_r, l_r, v);
+        for (int b0 = 0; b0 < n_mine; b0 += N) {
+            float m_r[N], l_r[N], m_b = m_g;
+            float4 v[N];
 #pragma unroll
-        for (int u = 0; u < N; ++u) m_g = fmaxf(m_g, m_r[u]);
+            for (int u = 0; u < N; ++u) {
+                const size_t rec = (size_t)(first + sub + SUBS * min(b0 + u, n_mine - 1)) + seq;
+                m_r[u] = part_ml[(rec * H + head) * 2];
+                l_r[u] = part_ml[(rec * H + head) * 2 + 1];
+                v[u] = reinterpret_cast<const float4*>(part_acc + (rec * H + head) * kKvl)[col];
+            }
 #pragma unroll
-        for (int u = 0; u < N; ++u)
-            if (first + u <= last && m_r[u] != -INFINITY) add(exp2f(m_r[u] - m_g), l_r[u], v[u]);
-    };
-    if (last - first < 8) {
-        merge_one(std::integral_constant<int, 8>{});
-    } else if (last - first < 16) {
-        merge_one(std::integral_constant<int, 16>{});
-    } else {
-        constexpr int kBatch = 8;
-        float m_g = -INFINITY;
-        for (int b0 = first; b0 <= last; b0 += kBatch) {
-            float m_r[kBatch];
+            for (int u = 0; u < N; ++u) m_b = fmaxf(m_b, m_r[u]);
+            if (m_b == -INFINITY) continue;
+            const float keep = exp2f(m_g - m_b);
+            l_g *= keep, sum.x *= keep, sum.y *= keep, sum.z *= keep, sum.w *= keep;
+            m_g = m_b;
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u)
-                m_r[u] = part_ml[((size_t)(min(b0 + u, last) + seq) * H + head) * 2];
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) m_g = fmaxf(m_g, m_r[u]);
+            for (int u = 0; u < N; ++u)
+                if (b0 + u < n_mine && m_r[u] != -INFINITY) {
+                    const float w = exp2f(m_r[u] - m_g);
+                    l_g += l_r[u] * w;
+                    sum.x += v[u].x * w, sum.y += v[u].y * w, sum.z += v[u].z * w, sum.w += v[u].w * w;
+                }
         }
-        for (int b0 = first; b0 <= last && m_g != -INFINITY; b0 += kBatch) {
-            float m_r[kBatch], l_r[kBatch];
-            float4 v[kBatch];
-            batch(std::integral_constant<int, kBatch>{}, b0, m_r, l_r, v);
+    };
+    if (n_mine <= 4) merge(std::integral_constant<int, 4>{});
+    else if (n_mine <= 8) merge(std::integral_constant<int, 8>{});
+    else merge(std::integral_constant<int, 16>{});
+    if constexpr (SUBS > 1) {  // the groups' sums, in their order
+        __shared__ float4 sums[SUBS][kCols];
+        __shared__ float ml[SUBS][2];
+        sums[sub][threadIdx.x % kCols] = sum;
+        if (threadIdx.x % kCols == 0) ml[sub][0] = m_g, ml[sub][1] = l_g;
+        __syncthreads();
+        if (sub != 0) return;
+        m_g = ml[0][0];
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u)
-                if (b0 + u <= last && m_r[u] != -INFINITY) add(exp2f(m_r[u] - m_g), l_r[u], v[u]);
+        for (int u = 1; u < SUBS; ++u) m_g = fmaxf(m_g, ml[u][0]);
+        l_g = 0.0f, sum = float4{0, 0, 0, 0};
+#pragma unroll
+        for (int u = 0; u < SUBS; ++u) {
+            if (ml[u][0] == -INFINITY) continue;
+            const float w = exp2f(ml[u][0] - m_g);
+            const float4 v = sums[u][threadIdx.x];
+            l_g += ml[u][1] * w;
+            sum.x += v.x * w, sum.y += v.y * w, sum.z += v.z * w, sum.w += v.w * w;
         }
     }
+    if (!mine_col) return;
     const float inv = l_g > 0.0f ? 1.0f / l_g : 0.0f;
     *dst = float4{sum.x * inv, sum.y * inv, sum.z * inv, sum.w * inv};
 }
@@ -1007,9 +1027,16 @@ static int attend_merge(const AttendArgs& a, const AttendPlan& plan, int n_seqs,
                         const int* n_rows, bool listed, hipStream_t st) {
     const int rc = launch_status();
     if (rc != 0 || plan.n_items == 0) return rc;
-    hipLaunchKernelGGL(mla_attend_combine_kernel, dim3((unsigned)a.H, (unsigned)n_seqs), dim3(128), 0, st,
-                       a.part_acc, a.part_ml, seq_lens, n_rows, listed ? 1 : 0, max_rows, n_seqs, plan.n_items,
-                       a.by_seq, a.H, a.kvl, a.clat);
+    // Four groups of threads on a head's records while a compute unit gets at most four of their workgroups: one sequence of 16 384 tokens of 64
+    // heads, 64 records, 27.1 -> 21.9 us, two ragged ones of 8 000 22.3 -> 20.6; 3 x 3 000 of 128 heads 22.8 -> 23.2, 12 x 4 000 27.8 -> 30.9.
+    if ((long long)a.H * n_seqs <= kAttTargetGroups)
+        hipLaunchKernelGGL(mla_attend_combine_kernel<4>, dim3((unsigned)a.H, (unsigned)n_seqs, (unsigned)((a.kvl + 127) / 128)), dim3(128), 0, st,
+                           a.part_acc, a.part_ml, seq_lens, n_rows, listed ? 1 : 0, max_rows, n_seqs, plan.n_items,
+                           a.by_seq, a.H, a.kvl, a.clat);
+    else
+        hipLaunchKernelGGL(mla_attend_combine_kernel<1>, dim3((unsigned)a.H, (unsigned)n_seqs), dim3(128), 0, st,
+                           a.part_acc, a.part_ml, seq_lens, n_rows, listed ? 1 : 0, max_rows, n_seqs, plan.n_items,
+                           a.by_seq, a.H, a.kvl, a.clat);
     return launch_status();
 }
 

@@ -260,10 +260,10 @@ __device__ __forceinline__ void attend_part_few(const AttendArgs& a, int seq, in
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-            for (int c = 0; c < kFewColTiles; ++c) {
-                o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[ks][c], p[ks], o[c], 0, 0, 0);
-                if (PSPLIT == 2) o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[ks][c], p_lo[ks], o[c], 0, 0, 0);
-            }
+            for (int u = 0; u < PSPLIT; ++u)
+#pragma unroll
+                for (int c = 0; c < kFewColTiles; ++c)
+                    o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[ks][c], u ? p_lo[ks] : p[ks], o[c], 0, 0, 0);
     };
     auto take_weights = [&](float& corr, bf16x8 (&p)[2], bf16x8 (&p_lo)[2]) {
         corr = corr_smem[n16];
