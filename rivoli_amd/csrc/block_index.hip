@@ -25,7 +25,7 @@
 // on the operands they hold (RowSpan) and take such tiles through v_mfma_f32_32x32x16_bf16; any
 // other tile of the same launch is folded term by term as below; rows that are fp4 codes under
 // powers of two, as spread rows are, go through the block-scaled fp4 instruction. 8 192 queries x 64 heads x
-// <= 2 048 blocks: 172 us, 226 as bf16, 3 640 term by term.
+// <= 2 048 blocks: 164 us, 226 as bf16, 3 640 term by term.
 // Operands of another kind (no such rows leave the indexer) take the same launches' fold: 3 430.
 // Term by term, what is free is where the operands come from. A lane owns block c and
 // keeps its 128-value row in registers for the whole launch; a wave's 64 lanes share the query,
@@ -428,9 +428,9 @@ __device__ __forceinline__ void fold_heads(const float* __restrict__ q, const fl
 // the rows with bit 2 clear): the head sum, whose order the reference fixes, is then register arithmetic.
 // Bound by issue. As bf16 a lane's 64 dots were 32 matrix instructions of 32 cycles and five vector instructions each (round,
 // relu, weight, round, sum); as fp4 codes they are 8 of 32 cycles, and clamping conversions leave four a dot, in steps of which
-// none waits for another. 8 192 queries: 226 -> 172 us, of them 107 vector issue (two thirds of it those four; the kv rows' codes, made by every workgroup,
-// and the q rows' take the rest), 15 the matrix cores and about 25 the first workgroups' q rows, all asked for at once; 4 096 82 -> 74,
-// 6 001 126 -> 111. Not kept: 16 queries a workgroup (half of the conversions; all of q at once, 231), two or three sets of q loads
+// none waits for another. 8 192 queries: 226 -> 164 us, of them 107 vector issue (two thirds of it those four; the kv rows' codes, made by every workgroup,
+// and the q rows' take the rest), 15 the matrix cores and about 25 the first workgroups' q rows, all asked for at once; 4 096 82 -> 72,
+// 6 001 127 -> 103. Not kept: 16 queries a workgroup (half of the conversions; all of q at once, 231), two or three sets of q loads
 // in flight (178).
 constexpr int kPairWaves = 4;
 constexpr int kPairThreads = kPairWaves * kWave;
@@ -508,271 +508,96 @@ __device__ __forceinline__ float clamp_bf16(float x) {
     return r;
 }
 
+struct PairArgs {
+    const float *q, *kv, *w;
+    float* score;
+    int s, n_comp, heads, split_blocks, ratio;
+};
 template <bool FP4>
-__global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
-    const float* __restrict__ q, const float* __restrict__ kv, const float* __restrict__ w,
-    float* __restrict__ score, int s, int n_comp, int heads, int split_blocks, int ratio) {
-    // q rows on their way to operands (a wave's 32 at a time), then kv rows
-    __shared__ __align__(16) unsigned char stage[kPairWaves * 32 * kPairRow];
-    __shared__ __align__(16) float weights[kPairWaves][2][kPairHeads];
-    __shared__ int kv_spans[2][2 * kPairTile];
-    __shared__ uint32_t row_expo[kPairWaves * 32], kv_expo[4 * kPairTile];  // four block exponents a row
-    __shared__ unsigned long long left_all[kPairWaves][2];
-    __shared__ int wave_fits[kPairWaves];
-    const int lane = threadIdx.x & (kWave - 1), half = lane >> 5, row = lane & 31;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+struct PairShared {
+    // q rows on their way to operands (a wave's 32 at a time), and kv rows
+    __align__(16) unsigned char stage[kPairWaves * 32 * kPairRow];
+    __align__(16) float weights[kPairWaves][2][kPairHeads];
+    int kv_spans[2][FP4 ? 2 * kPairTile : kPairTile];
+    uint32_t row_expo[FP4 ? kPairWaves * 32 : 1], kv_expo[FP4 ? 4 * kPairTile : 1];  // four block exponents a row
+    unsigned long long left[kPairWaves][2];
+    int fits[kPairWaves];
+};
+// Tiles from block c0 on of 64-block groups with a block that some query up to t_last may rank (first_query).
+__device__ __forceinline__ int pair_tiles(const PairArgs& a, int c0, int t_last) {
+    int end = min(a.n_comp, c0 + a.split_blocks);
+    if (a.ratio > 0) end = min(end, ((t_last + 1) / a.ratio + 63) & ~63);
+    return end > c0 ? (end - c0 + kPairTile - 1) / kPairTile : 0;
+}
+// Blocks of query t from here on are nobody's: it does not exist, or its selection ranks none of their 64.
+__device__ __forceinline__ int pair_limit(const PairArgs& a, int t) {
+    return t >= a.s ? 0 : a.ratio <= 0 ? a.n_comp : min(a.n_comp, ((t + 1) / a.ratio + 63) & ~63);
+}
+struct PairPlace {
+    int lane, half, row, wave, kr, kp;  // kv tiles: eight threads (kp) a row (kr), 16-byte pieces
+    int tw, t, c0;                      // the wave's first query, the lane's; the workgroup's first block
+    int tiles, my_tiles;                // of the workgroup; of the wave
+};
+__device__ __forceinline__ PairPlace pair_place(const PairArgs& a, int tid) {
+    PairPlace at;
+    at.lane = tid & (kWave - 1), at.half = at.lane >> 5, at.row = at.lane & 31;
+    at.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    at.kr = tid >> 3, at.kp = tid & 7;
     // the last queries of a prefill rank the most blocks: they start first
-    const int group = ratio > 0 ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x;
-    const int tw = group * kPairQueries + wave * 2;  // the wave's first query
-    const int c0 = blockIdx.y * split_blocks;
-    // tiles of 64-block groups with a block that some query up to t_last may rank (first_query)
-    const auto tiles_for = [&](int t_last) {
-        int end = min(n_comp, c0 + split_blocks);
-        if (ratio > 0) end = min(end, ((t_last + 1) / ratio + 63) & ~63);
-        return end > c0 ? (end - c0 + kPairTile - 1) / kPairTile : 0;
-    };
-    const int tiles = tiles_for(min(s, (group + 1) * kPairQueries) - 1);
-    if (!tiles) return;  // workgroup-uniform
-    const int my_tiles = tw < s ? tiles_for(min(s, tw + 2) - 1) : 0;
-    const int t = tw + half;
+    const int group = a.ratio > 0 ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x;
+    at.tw = group * kPairQueries + at.wave * 2, at.t = at.tw + at.half;
+    at.c0 = blockIdx.y * a.split_blocks;
+    at.tiles = pair_tiles(a, at.c0, min(a.s, (group + 1) * kPairQueries) - 1);
+    at.my_tiles = at.tw < a.s ? pair_tiles(a, at.c0, min(a.s, at.tw + 2) - 1) : 0;
+    return at;
+}
+// The next kv rows are requested before these ones' products and parked after them.
+__device__ __forceinline__ void request_rows(const PairArgs& a, const PairPlace& at, int tile, f32x4 (&to)[4]) {
+    const float* const p = a.kv + (size_t)min(at.c0 + tile * kPairTile + at.kr, a.n_comp - 1) * 128 + at.kp * 4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) to[j] = *reinterpret_cast<const f32x4*>(p + j * 32);
+}
+// Eight loads of the rows of heads 16 c ..: load m = 2 (j0 + j) + half is row m, head c * 16 + (m >> 3) * 4 + (m & 3) of
+// query (m >> 2) & 1; an instruction moves two whole rows.
+__device__ __forceinline__ void request_heads(const PairArgs& a, const PairPlace& at, int c, int j0, f32x4 (&v)[8]) {
+    const bool all = c * 16 + 16 <= a.heads;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int hh = c * 16 + ((j0 + j) >> 2) * 4 + (2 * (j0 + j) & 3);  // and hh + 1 in the upper half
+        const float* const from = a.q + (size_t)min(at.tw + ((j0 + j) >> 1 & 1), a.s - 1) * a.heads * 128;  // uniform
+        if (all) v[j] = *reinterpret_cast<const f32x4_u*>(from + hh * 128 + (uint32_t)(at.half * 128 + at.row * 4));
+        else v[j] = *reinterpret_cast<const f32x4_u*>(from + (uint32_t)(min(hh + at.half, a.heads - 1) * 128 + at.row * 4));
+    }
+    __builtin_amdgcn_sched_barrier(0);  // all eight requested before the first is waited for
+    if (!all) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (c * 16 + ((j0 + j) >> 2) * 4 + (2 * (j0 + j) & 3) + at.half >= a.heads) v[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+}
+// The weights of head `lane`, both queries.
+__device__ __forceinline__ void load_weights(const PairArgs& a, const PairPlace& at, float (&x)[2]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) x[i] = at.lane < a.heads ? a.w[(size_t)min(at.tw + i, a.s - 1) * a.heads + at.lane] : 0.0f;
+}
 
-    // blocks of query t from here on are nobody's: it does not exist, or its selection ranks none of their 64
-    const auto limit_of = [&](int t) { return t >= s ? 0 : ratio <= 0 ? n_comp : min(n_comp, ((t + 1) / ratio + 63) & ~63); };
+// The tiles of `left`, of each wave its own, as bf16 operands where those are exact, the others term by term. ALL: every tile; else sh.left
+// holds what each wave has left.
+template <bool ALL, class SHARED>
+__device__ __forceinline__ void score_left(const PairArgs& a_, const PairPlace& at, SHARED& sh) {
+    const int lane = at.lane, half = at.half, row = at.row, wave = at.wave, tw = at.tw, c0 = at.c0, t = at.t, kr = at.kr, kp = at.kp;
+    const int tiles = at.tiles, my_tiles = at.my_tiles, s = a_.s, n_comp = a_.n_comp, heads = a_.heads;
+    const float* const kv = a_.kv;
+    float* const score = a_.score;
+    unsigned char* const stage = sh.stage;
+    const auto request = [&](int tile, f32x4 (&to)[4]) { request_rows(a_, at, tile, to); };
+    const auto load_heads = [&](int c, int j0, f32x4 (&v)[8]) { request_heads(a_, at, c, j0, v); };
+    const auto limit_of = [&](int t) { return pair_limit(a_, t); };
     const int limit = limit_of(t);
-
-    // kv tiles: eight threads a row, 16-byte pieces; the next ones are requested before these
-    // ones' products and parked after them
-    const int kr = threadIdx.x >> 3, kp = threadIdx.x & 7;
-    const auto request = [&](int tile, f32x4 (&to)[4]) {
-        const float* const p = kv + (size_t)min(c0 + tile * kPairTile + kr, n_comp - 1) * 128 + kp * 4;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) to[j] = *reinterpret_cast<const f32x4*>(p + j * 32);
-    };
-    // eight loads of the rows of heads 16 c ..: load m = 2 (j0 + j) + half is row m, head c * 16 + (m >> 3) * 4 + (m & 3) of
-    // query (m >> 2) & 1; an instruction moves two whole rows
-    const auto load_heads = [&](int tw, int c, int j0, f32x4 (&v)[8]) {
-        const bool all = c * 16 + 16 <= heads;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int hh = c * 16 + ((j0 + j) >> 2) * 4 + (2 * (j0 + j) & 3);  // and hh + 1 in the upper half
-            const float* const at = q + (size_t)min(tw + ((j0 + j) >> 1 & 1), s - 1) * heads * 128;  // uniform
-            const uint32_t mine = (uint32_t)(half * 128 + row * 4);
-            if (all) {
-                v[j] = *reinterpret_cast<const f32x4_u*>(at + hh * 128 + mine);
-            } else {
-                v[j] = *reinterpret_cast<const f32x4_u*>(at + (uint32_t)(min(hh + half, heads - 1) * 128 + row * 4));
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);  // all eight requested before the first is waited for
-        if (!all) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (c * 16 + ((j0 + j) >> 2) * 4 + (2 * (j0 + j) & 3) + half >= heads) v[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-    };
-
-    float own_weights[2];  // of head `lane`, both queries
-#pragma unroll
-    for (int i = 0; i < 2; ++i) own_weights[i] = lane < heads ? w[(size_t)min(tw + i, s - 1) * heads + lane] : 0.0f;
-    unsigned long long left[2] = {0, 0};  // one bit per tile that the fp4 products did not do
-    if constexpr (FP4) {
-        f32x4 next[2][4];  // two tiles at a time
-        request(0, next[0]);
-        request(1, next[1]);  // (past the last block: that one again)
-        unsigned char* const kv_codes = stage + kPairWaves * 32 * kFp4Row;
-        // Row 32 u + kr of buffer `buf`; whether it is made of codes.
-        const auto park = [&](int buf, int u) -> bool {
-            const int at = (2 * buf + u) * kPairTile + kr;
-            unsigned char* const to = kv_codes + at * kFp4Row + kp * 2;
-            uint32_t off = 0, e[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) *reinterpret_cast<uint16_t*>(to + j * 16) = (uint16_t)fp4_of(next[u][j], e[j], off);
-            const uint32_t hi = max(max(e[0], e[1]), max(e[2], e[3]));
-            uint32_t lo = min(min(e[0], e[1]), min(e[2], e[3]));
-            if (__any(lo == 0)) {  // a block of zeros takes the largest's scale
-#pragma unroll
-                for (int j = 0; j < 4; ++j) e[j] = e[j] ? e[j] : hi;
-                lo = min(min(e[0], e[1]), min(e[2], e[3]));
-            }
-            // 127 + e - hi in each byte (none of them borrows where the row is taken)
-            const uint32_t expo = (e[0] | e[1] << 8 | e[2] << 16 | e[3] << 24) + 0x7f7f7f7fu - __builtin_amdgcn_perm(hi, hi, 0u);
-            uint32_t span = hi - lo;
-            if (hi - (uint32_t)kFp4MinExp > (uint32_t)(kFp4MaxExp - kFp4MinExp) && hi) span = kNoSpan;
-            const unsigned long long bad = __ballot(off != 0);
-            if (bad) span = bad >> (lane & ~7) & 0xffu ? (uint32_t)kNoSpan : span;
-            // (eight threads, one word)
-            kv_expo[at] = expo;
-            kv_spans[buf][u * kPairTile + kr] = (int)(span | hi << 8);
-            return off == 0;
-        };
-        bool fits = my_tiles > 0;
-        // ---- the rows as fp4 operands: lane's row of a matrix tile, blocks half and 2 + half of its four ----
-        u32x4 a[4][2];
-        uint32_t a_expo[4] = {};
-        unsigned char* const mine = stage + wave * 32 * kFp4Row;
-        uint32_t off = 0;
-        int top = 0, bottom = 255, apart = 0;  // block exponents: the rows' largest, smallest; largest difference in a row
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            if (c * 16 >= heads || (c == 1 && !fits)) break;
-#pragma unroll
-            for (int j0 = 0; j0 < 16; j0 += 8) {
-                f32x4 v[8];
-                load_heads(tw, c, j0, v);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int m = 2 * (j0 + j) + half;
-                    uint32_t expo;
-                    *reinterpret_cast<uint16_t*>(mine + m * kFp4Row + row * 2) = (uint16_t)fp4_of(v[j], expo, off);
-                    // (eight lanes, one byte)
-                    reinterpret_cast<unsigned char*>(row_expo)[(wave * 32 + m) * 4 + (row >> 3)] = (unsigned char)expo;
-                }
-                asm volatile("" ::: "memory");  // no more than eight rows' loads in registers at a time
-            }
-            asm volatile("" ::: "memory");  // the rows cross lanes: LDS serves a wave in order, the compiler must keep to it
-#pragma unroll
-            for (int k = 0; k < 2; ++k) a[c][k] = *reinterpret_cast<const u32x4*>(mine + row * kFp4Row + (2 * k + half) * 16);
-            const uint32_t x = row_expo[wave * 32 + row];
-            int hi = 0, lo = 255;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int e = (int)(x >> (8 * k) & 0xffu);
-                hi = max(hi, e), lo = min(lo, e ? e : 255);
-            }
-            top = max(top, hi), bottom = min(bottom, lo), apart = max(apart, hi - lo);  // a row of zeros: -255
-            a_expo[c] = x >> (8 * half);
-            asm volatile("" ::: "memory");
-            // Where some of the first sixteen heads' values, or of the wave's own rows of the first two tiles, are no codes, hardly any are.
-            if (c == 0) {
-                const bool codes[2] = {park(0, 0), park(0, 1)};
-                if (__any(!codes[0] || !codes[1] || off != 0)) fits = false;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            weights[wave][i][lane] = own_weights[i];
-            const uint32_t e = (__float_as_uint(own_weights[i]) & 0x7fffffffu) >> 23;
-            if (own_weights[i] != 0.0f && (e < kFp4Weight0 || e > kFp4Weight1)) off = 1;  // (a NaN differs from zero)
-        }
-        asm volatile("" ::: "memory");
-        if (__any(off != 0)) fits = false;
-#pragma unroll
-        for (int m = 1; m < 32; m <<= 1) {
-            top = max(top, __shfl_xor(top, m, kWave)), bottom = min(bottom, __shfl_xor(bottom, m, kWave));
-            apart = max(apart, __shfl_xor(apart, m, kWave));
-        }
-        top = __builtin_amdgcn_readfirstlane(top), bottom = __builtin_amdgcn_readfirstlane(bottom), apart = __builtin_amdgcn_readfirstlane(apart);
-        if (top != 0 && (top > kFp4MaxExp || top < kFp4MinExp || top - bottom > kFp4Heads)) fits = false;
-        // scales relative to the largest (a block of zeros takes that)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int e0 = (int)(a_expo[c] & 0xffu), e1 = (int)(a_expo[c] >> 16 & 0xffu);
-            a_expo[c] = (uint32_t)(127 - kFp4Down + (e0 ? e0 - top : 0)) | (uint32_t)(127 - kFp4Down + (e1 ? e1 - top : 0)) << 8;
-        }
-        f32x4 wv[kPairHeads / 4];
-#pragma unroll
-        for (int i = 0; i < kPairHeads / 4; ++i) wv[i] = *reinterpret_cast<const f32x4*>(&weights[wave][half][4 * i]);
-
-        if (!fits) {
-#pragma unroll
-            for (int k = 0; k < 2; ++k)
-                if (my_tiles > 64 * k) left[k] = my_tiles >= 64 * (k + 1) ? ~0ull : (1ull << (my_tiles & 63)) - 1;
-        }
-        if (lane == 0) wave_fits[wave] = fits;
-        __syncthreads();
-        bool some = false;
-#pragma unroll
-        for (int i = 0; i < kPairWaves; ++i) some = some || wave_fits[i];
-        const int walk = some ? tiles : 0;
-        for (int tile = 0, buf = 0; tile < walk; tile += 2, buf ^= 1) {
-            __syncthreads();  // these tiles are parked and nobody reads the other buffer any more
-            if (tile + 2 < tiles) {
-                request(tile + 2, next[0]);
-                request(tile + 3, next[1]);  // (past the last block: that one again)
-            }
-            if (fits && tile < my_tiles) {
-                u32x4 b[2][2];
-                int b_expo[2], info[2];
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    const int at = (2 * buf + u) * kPairTile + row;
-                    const unsigned char* const from = kv_codes + at * kFp4Row + half * 16;
-                    b[u][0] = *reinterpret_cast<const u32x4*>(from), b[u][1] = *reinterpret_cast<const u32x4*>(from + 32);
-                    b_expo[u] = (int)(kv_expo[at] >> (8 * half));
-                    info[u] = kv_spans[buf][u * kPairTile + row];
-                }
-                const auto products = [&](int u, int c) {
-                    f32x16 d = {};
-                    d = fp4_products(a[c][0], b[u][0], d, (int)a_expo[c], b_expo[u]);
-                    return fp4_products(a[c][1], b[u][1], d, (int)(a_expo[c] >> 8), b_expo[u] >> 16);
-                };
-                f32x16 d = products(0, 0);
-                const auto taken = [&](int u) {
-                    const int back = top + (info[u] >> 8) - 2 * 129 + kFp4Down;  // the scores' scale
-                    const bool zero = (info[u] >> 8) == 0 || top == 0;
-                    return !__any(max(apart, 0) + (info[u] & 0xff) > kFp4Span || (!zero && (back < kFp4Back0 || back > kFp4Back1)));
-                };
-                const bool take[2] = {taken(0), taken(1)};
-                float acc = 0.0f;
-                const auto finish = [&](int u, int info) {
-                    const int c = c0 + (tile + u) * kPairTile + row;
-                    if (c < limit) score[(size_t)t * n_comp + c] = round_bf16(__builtin_amdgcn_ldexpf(acc, top + (info >> 8) - 2 * 129 + kFp4Down));
-                    acc = 0.0f;
-                };
-                if (!take[0]) left[tile >> 6] |= 1ull << (tile & 63);
-                if (!take[1] && tile + 1 < my_tiles) left[tile >> 6] |= 2ull << (tile & 63);
-                if (heads > 48 && take[0] && take[1]) {
-                    // A step has a head's conversion, the weight of the one before, the rounding of the one before that and the sum's
-                    // addition of a fourth: four instructions of which none waits for another. The next sixteen
-                    // heads' products run under these heads' steps.
-                    constexpr int kSteps = 2 * kPairHeads;
-                    f32x16 sets[2];
-                    sets[0] = d;
-                    float clamped = 0.0f, weighted = 0.0f, term = 0.0f;
-                    each_of<kSteps + 3>([&](auto step) {
-                        constexpr int n = decltype(step)::value, set = n / 16;
-                        if constexpr (n % 16 == 0 && set + 1 < kSteps / 16) sets[(set + 1) & 1] = products((set + 1) / 4, (set + 1) % 4);
-                        if constexpr (n >= 3) acc = acc + term;
-                        if constexpr (n >= 2 && n < kSteps + 2) term = round_bf16(weighted);
-                        if constexpr (n >= 1 && n < kSteps + 1) weighted = clamped * wv[(n - 1) / 4 % 16][(n - 1) % 4];
-                        if constexpr (n < kSteps) clamped = n % 16 == 0 ? relu_bf16(sets[set & 1][0]) : clamp_bf16(sets[set & 1][n % 16]);
-                        if constexpr (n == kPairHeads + 2) finish(0, info[0]);
-                        if constexpr (n == kSteps + 2) finish(1, info[1]);
-                        __builtin_amdgcn_sched_barrier(0);
-                    });
-                } else {
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        if (!take[u]) continue;
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) {
-                            if (c * 16 >= heads) break;
-                            const f32x16 d = products(u, c);
-#pragma unroll
-                            for (int i = 0; i < 16; ++i) acc = acc + head_term(d[i], wv[4 * c + i / 4][i % 4]);
-                        }
-                        finish(u, info[u]);
-                    }
-                }
-            }
-            if (tile + 2 < tiles) park(buf ^ 1, 0), park(buf ^ 1, 1);
-        }
-    }
-    // ---- what those rows are not, tiles of any of the four waves, or all of them: as bf16 operands where those are exact -----
-    if constexpr (FP4) {
-        if (lane < 2) left_all[wave][lane] = lane ? left[1] : left[0];
-        __syncthreads();
-        bool some = false;
-#pragma unroll
-        for (int i = 0; i < kPairWaves; ++i) some = some || (left_all[i][0] | left_all[i][1]) != 0;
-        if (!some) return;
-    } else {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) weights[wave][i][lane] = own_weights[i];
-    }
+    auto& weights = sh.weights;
+    auto& kv_spans = sh.kv_spans;
     f32x4 next[4];
-    int again = tw;  // (nothing of the first pass over the rows is kept for the second)
-    asm volatile("" : "+s"(again));
+    unsigned long long left[2] = {0, 0};
     bf16x8 a[4][8];
     int q_span = 0;
     {
@@ -784,7 +609,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
 #pragma unroll
             for (int j0 = 0; j0 < 16; j0 += 8) {
                 f32x4 v[8];
-                load_heads(again, c, j0, v);
+                load_heads(c, j0, v);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     low |= low_half_bits(v[j]);
@@ -826,14 +651,15 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
         f = span_max(f, __shfl_xor(f, 4, kWave));
         if (kp == 0) kv_spans[parity][kr] = span_of(f);
     };
-    if constexpr (!FP4) request(0, next);
+    if constexpr (ALL) request(0, next);
     __syncthreads();  // every wave's q rows are out of the stage, and its tiles in left_all
     unsigned long long todo[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         todo[k] = 0;
-        if constexpr (FP4) {
-            for (int i = 0; i < kPairWaves; ++i) todo[k] |= left_all[i][k];
+        if constexpr (!ALL) {
+            for (int i = 0; i < kPairWaves; ++i) todo[k] |= sh.left[i][k];
+            left[k] = sh.left[wave][k];
         } else {
             if (tiles > 64 * k) todo[k] = tiles >= 64 * (k + 1) ? ~0ull : (1ull << (tiles & 63)) - 1;
             if (my_tiles > 64 * k) left[k] = my_tiles >= 64 * (k + 1) ? ~0ull : (1ull << (my_tiles & 63)) - 1;
@@ -848,7 +674,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
     };
     unsigned long long inexact[2] = {0, 0};  // one bit per tile
     int tile = pop();
-    if constexpr (FP4) request(tile, next);
+    if constexpr (!ALL) request(tile, next);
     park();
     while (tile >= 0) {
         __syncthreads();
@@ -904,10 +730,10 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
                 float row_v[128];
                 load_row(row_v, kv + (size_t)min(c, n_comp - 1) * 128);
                 const int first = both ? tw : tw + half;
-                const size_t at = (size_t)min(first, s - 1) * heads;
+                const size_t from = (size_t)min(first, s - 1) * heads;
                 // (both sums first, then the stores: 8 192 x 2 048 3 475 -> 3 425 us)
                 float sum = 0.0f, acc = 0.0f;
-                fold_heads<shared>(q + at * 128, w + at, both ? min(2, s - tw) * heads : heads, row_v, [&](int i, float term) {
+                fold_heads<shared>(a_.q + from * 128, a_.w + from, both ? min(2, s - tw) * heads : heads, row_v, [&](int i, float term) {
                     acc = acc + term;
                     if (i + 1 == heads) sum = acc, acc = 0.0f;
                 });
@@ -917,10 +743,242 @@ __global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(
         }
     };
     // (a prefill's grid has a third and more workgroups without a legal block)
-    if (gridDim.x * gridDim.y <= (ratio > 0 ? 384u : 256u))
+    if (gridDim.x * gridDim.y <= (a_.ratio > 0 ? 384u : 256u))
         fold(std::false_type{});
     else
         fold(std::true_type{});
+}
+
+__global__ __launch_bounds__(kPairThreads, 2) void score_blocks_pair_kernel(const PairArgs args) {
+    __shared__ PairShared<false> sh;
+    const PairPlace at = pair_place(args, threadIdx.x);
+    if (!at.tiles) return;  // workgroup-uniform
+    float own_weights[2];
+    load_weights(args, at, own_weights);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) sh.weights[at.wave][i][at.lane] = own_weights[i];
+    score_left<true>(args, at, sh);
+}
+
+template <class SHARED>
+__device__ __forceinline__ bool score_codes(const PairArgs& a_, const PairPlace& at, SHARED& sh) {
+    const int lane = at.lane, half = at.half, row = at.row, wave = at.wave, tw = at.tw, c0 = at.c0, t = at.t, kr = at.kr, kp = at.kp;
+    const int tiles = at.tiles, my_tiles = at.my_tiles, s = a_.s, n_comp = a_.n_comp, heads = a_.heads;
+    const float* const kv = a_.kv;
+    float* const score = a_.score;
+    unsigned char* const stage = sh.stage;
+    const auto request = [&](int tile, f32x4 (&to)[4]) { request_rows(a_, at, tile, to); };
+    const auto load_heads = [&](int c, int j0, f32x4 (&v)[8]) { request_heads(a_, at, c, j0, v); };
+    const auto limit_of = [&](int t) { return pair_limit(a_, t); };
+    const int limit = limit_of(t);
+    auto& weights = sh.weights;
+    auto& kv_spans = sh.kv_spans;
+    auto& row_expo = sh.row_expo;
+    auto& kv_expo = sh.kv_expo;
+    auto& wave_fits = sh.fits;
+    float own_weights[2];
+    load_weights(a_, at, own_weights);
+    unsigned long long left[2] = {0, 0};  // one bit per tile that the fp4 products did not do
+    f32x4 next[2][4];  // two tiles at a time
+    request(0, next[0]);
+    request(1, next[1]);  // (past the last block: that one again)
+    unsigned char* const kv_codes = stage + kPairWaves * 32 * kFp4Row;
+    // Row 32 u + kr of buffer `buf`; whether it is made of codes.
+    const auto park = [&](int buf, int u) -> bool {
+        const int place = (2 * buf + u) * kPairTile + kr;
+        unsigned char* const to = kv_codes + place * kFp4Row + kp * 2;
+        uint32_t off = 0, e[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *reinterpret_cast<uint16_t*>(to + j * 16) = (uint16_t)fp4_of(next[u][j], e[j], off);
+        const uint32_t hi = max(max(e[0], e[1]), max(e[2], e[3]));
+        uint32_t lo = min(min(e[0], e[1]), min(e[2], e[3]));
+        if (__any(lo == 0)) {  // a block of zeros takes the largest's scale
+#pragma unroll
+            for (int j = 0; j < 4; ++j) e[j] = e[j] ? e[j] : hi;
+            lo = min(min(e[0], e[1]), min(e[2], e[3]));
+        }
+        // 127 + e - hi in each byte (none of them borrows where the row is taken)
+        const uint32_t expo = (e[0] | e[1] << 8 | e[2] << 16 | e[3] << 24) + 0x7f7f7f7fu - __builtin_amdgcn_perm(hi, hi, 0u);
+        uint32_t span = hi - lo;
+        if (hi - (uint32_t)kFp4MinExp > (uint32_t)(kFp4MaxExp - kFp4MinExp) && hi) span = kNoSpan;
+        const unsigned long long bad = __ballot(off != 0);
+        if (bad) span = bad >> (lane & ~7) & 0xffu ? (uint32_t)kNoSpan : span;
+        // (eight threads, one word)
+        kv_expo[place] = expo;
+        kv_spans[buf][u * kPairTile + kr] = (int)(span | hi << 8);
+        return off == 0;
+    };
+    bool fits = my_tiles > 0;
+    // ---- the rows as fp4 operands: lane's row of a matrix tile, blocks half and 2 + half of its four ----
+    u32x4 a[4][2];
+    uint32_t a_expo[4] = {};
+    unsigned char* const mine = stage + wave * 32 * kFp4Row;
+    uint32_t off = 0;
+    int top = 0, bottom = 255, apart = 0;  // block exponents: the rows' largest, smallest; largest difference in a row
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        if (c * 16 >= heads || (c == 1 && !fits)) break;
+#pragma unroll
+        for (int j0 = 0; j0 < 16; j0 += 8) {
+            f32x4 v[8];
+            load_heads(c, j0, v);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int m = 2 * (j0 + j) + half;
+                uint32_t expo;
+                *reinterpret_cast<uint16_t*>(mine + m * kFp4Row + row * 2) = (uint16_t)fp4_of(v[j], expo, off);
+                // (eight lanes, one byte)
+                reinterpret_cast<unsigned char*>(row_expo)[(wave * 32 + m) * 4 + (row >> 3)] = (unsigned char)expo;
+            }
+            asm volatile("" ::: "memory");  // no more than eight rows' loads in registers at a time
+        }
+        asm volatile("" ::: "memory");  // the rows cross lanes: LDS serves a wave in order, the compiler must keep to it
+#pragma unroll
+        for (int k = 0; k < 2; ++k) a[c][k] = *reinterpret_cast<const u32x4*>(mine + row * kFp4Row + (2 * k + half) * 16);
+        const uint32_t x = row_expo[wave * 32 + row];
+        int hi = 0, lo = 255;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int e = (int)(x >> (8 * k) & 0xffu);
+            hi = max(hi, e), lo = min(lo, e ? e : 255);
+        }
+        top = max(top, hi), bottom = min(bottom, lo), apart = max(apart, hi - lo);  // a row of zeros: -255
+        a_expo[c] = x >> (8 * half);
+        asm volatile("" ::: "memory");
+        // Where some of the first sixteen heads' values, or of the wave's own rows of the first two tiles, are no codes, hardly any are.
+        if (c == 0) {
+            const bool codes[2] = {park(0, 0), park(0, 1)};
+            if (__any(!codes[0] || !codes[1] || off != 0)) fits = false;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        weights[wave][i][lane] = own_weights[i];
+        const uint32_t e = (__float_as_uint(own_weights[i]) & 0x7fffffffu) >> 23;
+        if (own_weights[i] != 0.0f && (e < kFp4Weight0 || e > kFp4Weight1)) off = 1;  // (a NaN differs from zero)
+    }
+    asm volatile("" ::: "memory");
+    if (__any(off != 0)) fits = false;
+#pragma unroll
+    for (int m = 1; m < 32; m <<= 1) {
+        top = max(top, __shfl_xor(top, m, kWave)), bottom = min(bottom, __shfl_xor(bottom, m, kWave));
+        apart = max(apart, __shfl_xor(apart, m, kWave));
+    }
+    top = __builtin_amdgcn_readfirstlane(top), bottom = __builtin_amdgcn_readfirstlane(bottom), apart = __builtin_amdgcn_readfirstlane(apart);
+    if (top != 0 && (top > kFp4MaxExp || top < kFp4MinExp || top - bottom > kFp4Heads)) fits = false;
+    // scales relative to the largest (a block of zeros takes that)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const int e0 = (int)(a_expo[c] & 0xffu), e1 = (int)(a_expo[c] >> 16 & 0xffu);
+        a_expo[c] = (uint32_t)(127 - kFp4Down + (e0 ? e0 - top : 0)) | (uint32_t)(127 - kFp4Down + (e1 ? e1 - top : 0)) << 8;
+    }
+    f32x4 wv[kPairHeads / 4];
+#pragma unroll
+    for (int i = 0; i < kPairHeads / 4; ++i) wv[i] = *reinterpret_cast<const f32x4*>(&weights[wave][half][4 * i]);
+
+    if (!fits) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if (my_tiles > 64 * k) left[k] = my_tiles >= 64 * (k + 1) ? ~0ull : (1ull << (my_tiles & 63)) - 1;
+    }
+    if (lane == 0) wave_fits[wave] = fits;
+    __syncthreads();
+    bool some = false;
+#pragma unroll
+    for (int i = 0; i < kPairWaves; ++i) some = some || wave_fits[i];
+    const int walk = some ? tiles : 0;
+    for (int tile = 0, buf = 0; tile < walk; tile += 2, buf ^= 1) {
+        __syncthreads();  // these tiles are parked and nobody reads the other buffer any more
+        if (tile + 2 < tiles) {
+            request(tile + 2, next[0]);
+            request(tile + 3, next[1]);  // (past the last block: that one again)
+        }
+        if (fits && tile < my_tiles) {
+            u32x4 b[2][2];
+            int b_expo[2], info[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int place = (2 * buf + u) * kPairTile + row;
+                const unsigned char* const from = kv_codes + place * kFp4Row + half * 16;
+                b[u][0] = *reinterpret_cast<const u32x4*>(from), b[u][1] = *reinterpret_cast<const u32x4*>(from + 32);
+                b_expo[u] = (int)(kv_expo[place] >> (8 * half));
+                info[u] = kv_spans[buf][u * kPairTile + row];
+            }
+            const auto products = [&](int u, int c) {
+                f32x16 d = {};
+                d = fp4_products(a[c][0], b[u][0], d, (int)a_expo[c], b_expo[u]);
+                return fp4_products(a[c][1], b[u][1], d, (int)(a_expo[c] >> 8), b_expo[u] >> 16);
+            };
+            f32x16 d = products(0, 0);
+            const auto taken = [&](int u) {
+                const int back = top + (info[u] >> 8) - 2 * 129 + kFp4Down;  // the scores' scale
+                const bool zero = (info[u] >> 8) == 0 || top == 0;
+                return !__any(max(apart, 0) + (info[u] & 0xff) > kFp4Span || (!zero && (back < kFp4Back0 || back > kFp4Back1)));
+            };
+            const bool take[2] = {taken(0), taken(1)};
+            float acc = 0.0f;
+            const auto finish = [&](int u, int info) {
+                const int c = c0 + (tile + u) * kPairTile + row;
+                if (c < limit) score[(size_t)t * n_comp + c] = round_bf16(__builtin_amdgcn_ldexpf(acc, top + (info >> 8) - 2 * 129 + kFp4Down));
+                acc = 0.0f;
+            };
+            if (!take[0]) left[tile >> 6] |= 1ull << (tile & 63);
+            if (!take[1] && tile + 1 < my_tiles) left[tile >> 6] |= 2ull << (tile & 63);
+            if (heads > 48 && take[0] && take[1]) {
+                // A step has a head's conversion, the weight of the one before, the rounding of the one before that and the sum's
+                // addition of a fourth: four instructions of which none waits for another. The next sixteen
+                // heads' products run under these heads' steps.
+                constexpr int kSteps = 2 * kPairHeads;
+                f32x16 sets[2];
+                sets[0] = d;
+                float clamped = 0.0f, weighted = 0.0f, term = 0.0f;
+                each_of<kSteps + 3>([&](auto step) {
+                    constexpr int n = decltype(step)::value, set = n / 16;
+                    if constexpr (n % 16 == 0 && set + 1 < kSteps / 16) sets[(set + 1) & 1] = products((set + 1) / 4, (set + 1) % 4);
+                    if constexpr (n >= 3) acc = acc + term;
+                    if constexpr (n >= 2 && n < kSteps + 2) term = round_bf16(weighted);
+                    if constexpr (n >= 1 && n < kSteps + 1) weighted = clamped * wv[(n - 1) / 4 % 16][(n - 1) % 4];
+                    if constexpr (n < kSteps) clamped = n % 16 == 0 ? relu_bf16(sets[set & 1][0]) : clamp_bf16(sets[set & 1][n % 16]);
+                    if constexpr (n == kPairHeads + 2) finish(0, info[0]);
+                    if constexpr (n == kSteps + 2) finish(1, info[1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+            } else {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    if (!take[u]) continue;
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        if (c * 16 >= heads) break;
+                        const f32x16 d = products(u, c);
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) acc = acc + head_term(d[i], wv[4 * c + i / 4][i % 4]);
+                    }
+                    finish(u, info[u]);
+                }
+            }
+        }
+        if (tile + 2 < tiles) park(buf ^ 1, 0), park(buf ^ 1, 1);
+    }
+    if (lane < 2) sh.left[wave][lane] = lane ? left[1] : left[0];
+    __syncthreads();
+    bool some_left = false;
+#pragma unroll
+    for (int i = 0; i < kPairWaves; ++i) some_left = some_left || (sh.left[i][0] | sh.left[i][1]) != 0;
+    return some_left;
+}
+
+// Rows that are codes go through the fp4 instruction; of the others nothing that those needed is kept.
+__global__ __launch_bounds__(kPairThreads, 2) void score_blocks_codes_kernel(const PairArgs args) {
+    __shared__ PairShared<true> sh;
+    int tid = threadIdx.x;
+    {
+        const PairPlace at = pair_place(args, tid);
+        if (!at.tiles) return;  // workgroup-uniform
+        if (!score_codes(args, at, sh)) return;
+    }
+    asm volatile("" : "+v"(tid));
+    score_left<false>(args, pair_place(args, tid), sh);
 }
 
 // Few queries (a decode step: one). A workgroup owns one query's 64 heads against 32 HT blocks, a
@@ -1099,8 +1157,8 @@ namespace rk {
 // has no second for the many-query kernel's wave: 65 536 blocks 18 us against 25.
 constexpr int kOneGroups = 384;
 // Workgroups of so many blocks turn their q rows into fp4 codes, which takes a wave 2 200 vector instructions where bf16 operands
-// take 900: 192 blocks (2 049 x 512) 37 us as bf16 and 35.5 so, 384 (3 000 x 750) 54 and 48; 128 (1 500 x 375) 26.6 and 26.2, 64 (700 x 175)
-// 10.4 and 11.5.
+// take 900: 192 blocks (2 049 x 512) 37.5 us as bf16 and 33.5 so, 384 (3 000 x 750) 54 and 46; 128 (1 500 x 375) 26.6 and 26.2, 64 (700 x 175)
+// 10.4 and 11.5. Rows that are exact but no codes pay for finding that out: 8 192 queries of such q 232 -> 235, of such kv 212 -> 220, 2 049 38 -> 42.
 constexpr int kFp4Blocks = 192;
 static int score_blocks_launch(const float* q, const float* kv, const float* w, float* score, int s,
                                int n_comp, int heads, int hd, int ratio, hipStream_t st) {
@@ -1139,12 +1197,11 @@ static int score_blocks_launch(const float* q, const float* kv, const float* w, 
         if (per > kPairSplitMax) per = kPairSplitMax;
         const unsigned y = (unsigned)(((long long)n_comp + per - 1) / per);
         if (y <= 65535u) {
+            const PairArgs args = {q, kv, w, score, s, n_comp, heads, per, ratio};
             if (fp4)
-                hipLaunchKernelGGL(score_blocks_pair_kernel<true>, dim3(t_groups, y), dim3(kPairThreads), 0, st, q, kv, w, score,
-                                   s, n_comp, heads, per, ratio);
+                hipLaunchKernelGGL(score_blocks_codes_kernel, dim3(t_groups, y), dim3(kPairThreads), 0, st, args);
             else
-                hipLaunchKernelGGL(score_blocks_pair_kernel<false>, dim3(t_groups, y), dim3(kPairThreads), 0, st, q, kv, w, score,
-                                   s, n_comp, heads, per, ratio);
+                hipLaunchKernelGGL(score_blocks_pair_kernel, dim3(t_groups, y), dim3(kPairThreads), 0, st, args);
             return launch_status();
         }
     }
