@@ -631,6 +631,7 @@ __device__ __forceinline__ void attend_part(const AttendArgs& a, int seq, int hb
 #include "mla_attend_f8.hpp"
 #include "mla_attend_heads16.hpp"
 #include "mla_attend_few.hpp"
+#include "mla_attend_heads32.hpp"
 namespace rk {
 
 // Rows of sequence s that are attended.
@@ -907,6 +908,16 @@ __global__ __launch_bounds__(kFewThreads) void mla_attend_few_kernel(const Atten
     heads16_walk<kFewThreads, MODE>(a, pre, wave_total, [&](auto... part) { attend_part_few<QSPLIT, PSPLIT, MODE>(a, part...); });
 }
 
+// Eight waves on a tile for 32 heads (mla_attend_heads32.hpp): calls that SeqDeal cuts.
+template <int QSPLIT, int PSPLIT, int MODE>
+__global__ __launch_bounds__(kWideThreads) void mla_attend_wide_kernel(const AttendArgs a) {
+    // (a work item's head groups on one die, as heads16_walk)
+    const int groups = (a.H + kWideHeads - 1) / kWideHeads, turn = (int)blockIdx.x >> 3;
+    const int item = (turn / groups) * 8 + ((int)blockIdx.x & 7), hg = turn % groups;
+    if (item >= a.n_items) return;
+    seq_walk<MODE>(a, item, hg, [&](auto... part) { attend_part_wide<QSPLIT, PSPLIT, MODE>(a, part...); });
+}
+
 // Dealt plan: clat[seq][head] = sum_r w_r acc_r / sum_r w_r l_r over the sequence's partial
 // records, w_r = 2^(m_r - max m), in ascending work-item order (the reference's combine,
 // crates/backend/kernels/attn.hip:235-277, in base 2). A sequence that one work item covered
@@ -967,7 +978,7 @@ __global__ __launch_bounds__(128) void mla_attend_combine_kernel(
     float4 sum = {0, 0, 0, 0};
     float l_g = 0.0f, m_g = -INFINITY;
     const int n_mine = (last - first - sub + SUBS) / SUBS;  // the group's
-    auto merge = [&](auto size) {
+    auto merge = [&](auto size, bool once) {
         constexpr int N = decltype(size)::value;
         for (int b0 = 0; b0 < n_mine; b0 += N) {
             float m_r[N], l_r[N], m_b = m_g;
@@ -981,7 +992,10 @@ __global__ __launch_bounds__(128) void mla_attend_combine_kernel(
             }
 #pragma unroll
             for (int u = 0; u < N; ++u) m_b = fmaxf(m_b, m_r[u]);
-            if (m_b == -INFINITY) continue;
+            if (m_b == -INFINITY) {
+                if (once) break;
+                continue;
+            }
             const float keep = exp2f(m_g - m_b);
             l_g *= keep, sum.x *= keep, sum.y *= keep, sum.z *= keep, sum.w *= keep;
             m_g = m_b;
@@ -992,11 +1006,14 @@ __global__ __launch_bounds__(128) void mla_attend_combine_kernel(
                     l_g += l_r[u] * w;
                     sum.x += v[u].x * w, sum.y += v[u].y * w, sum.z += v[u].z * w, sum.w += v[u].w * w;
                 }
+            if (once) break;
         }
     };
-    if (n_mine <= 4) merge(std::integral_constant<int, 4>{});
-    else if (n_mine <= 8) merge(std::integral_constant<int, 8>{});
-    else merge(std::integral_constant<int, 16>{});
+    // (more than sixteen go by eights in a workgroup's one group: registers for more would leave fewer waves to the larger calls)
+    if (n_mine <= 4) merge(std::integral_constant<int, 4>{}, true);
+    else if (n_mine <= 8) merge(std::integral_constant<int, 8>{}, true);
+    else if (SUBS == 1 && n_mine > 16) merge(std::integral_constant<int, 8>{}, false);
+    else merge(std::integral_constant<int, 16>{}, SUBS == 1);
     if constexpr (SUBS > 1) {  // the groups' sums, in their order
         __shared__ float4 sums[SUBS][kCols];
         __shared__ float ml[SUBS][2];
@@ -1048,6 +1065,20 @@ static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_row
     // (16-byte transfers want every page to start on 16 bytes: page_tokens a multiple of 4)
     const AttendRoute route = attend_route(plan, n_seqs, a.H, max_rows, precise, MODE == kDense || MODE == kDensePaged,
                                            MODE == kLinear);
+    if constexpr (MODE != kLinear) {
+        const AttendPlan wide = heads32_route(plan, route, n_seqs, a.H, max_rows, precise, MODE != kSparse);
+        if (!any && a.page_bytes % 16 == 0 && wide.n_items) {
+            plan = wide;
+            a.n_items = plan.n_items, a.by_seq = kWideRun, a.count_ones = precise > 2;
+            const dim3 grid((unsigned)(((plan.n_items + 7) / 8 * 8) * ((a.H + kWideHeads - 1) / kWideHeads))), block(kWideThreads);
+            (void)hipGetLastError();
+            constexpr int M = MODE == kDensePaged ? kDense : MODE;
+            if (precise >= 2) hipLaunchKernelGGL((mla_attend_wide_kernel<2, 2, M>), grid, block, 0, st, a);
+            else if (precise == 1) hipLaunchKernelGGL((mla_attend_wide_kernel<2, 1, M>), grid, block, 0, st, a);
+            else hipLaunchKernelGGL((mla_attend_wide_kernel<1, 1, M>), grid, block, 0, st, a);
+            return attend_merge(a, plan, n_seqs, max_rows, seq_lens, n_rows, listed, st);
+        }
+    }
     if (!any && a.page_bytes % 16 == 0 && route.heads16) {
         plan = route.plan;
         a.n_items = plan.n_items, a.by_seq = !route.by_seq ? 0 : MODE == kLinear ? kFewTokens / kTile : kH16Waves, a.count_ones = precise > 2;

@@ -215,4 +215,49 @@ static inline AttendRoute attend_route(const AttendPlan& plan, int n_seqs, int H
     return {true, by_seq, heads16_few(p, by_seq, n_seqs, H, max_rows, precise, dense, linear), p};
 }
 
+// Workgroups of 32 heads (mla_attend_heads32.hpp) for calls that SeqDeal cuts: one a compute unit again, a die taking whole work
+// items, and no more partial records than `plan` has. n_items 0: not such a call.
+constexpr int kWideHeads = 32;
+constexpr int kWideRun = 2;  // SeqDeal's unit there: a tile of 64 tokens
+static inline AttendPlan heads32_plan(const AttendPlan& plan, int n_seqs, int H, int max_rows) {
+    const long long tiles = max_rows / kTile + (max_rows % kTile != 0);
+    const int groups = (H + kWideHeads - 1) / kWideHeads;
+    AttendPlan p = {1, 0, 0};
+    if (n_seqs > kSeqDealMax || tiles > kSeqDealMaxTiles || groups > kAttDieUnits || H <= kH16Heads) return p;
+    long long n = kAttDieUnits / groups * kAttDies;
+    const long long most = n_seqs * (tiles / kWideRun);
+    if (n > most) n = most;
+    if (n > plan.n_items) n = plan.n_items;
+    if (n < 2 * n_seqs) return p;
+    p.n_items = (int)n, p.n_splits = (int)((n + n_seqs - 1) / n_seqs), p.n_records = p.n_items + n_seqs;
+    return p;
+}
+// Whether such a call goes there; `heads16`: it would go to workgroups of 16 heads otherwise, else to those of 64. us, parity mode unless
+// said, there -> here. A tile of 32 heads costs about two of 16, and a work item 1 us more, so from 16 heads it is the finer cut of
+// a batch that pays, half as many groups making twice the work items: listed sets of 2 048 rows, 12 of 128 heads (work 6 144) 41.5 -> 37.6,
+// 32 of 64 (8 192) 44.6 -> 42.3, but 16 of 64 (4 096) 28.1 -> 30.5; dense, 17 x 7 255 ragged at precise 4 (15 436) 46.5 -> 42.5, 7 x 11 360 ragged (9 968)
+// 39.5 -> 39.2, but 20 x 3 000 ragged (7 520) 31.4 -> 32.0 and 6 x 9 000 (6 768) 34.3 -> 35.5.
+// From 64 heads: calls that those would need a second, nearly empty round for, 24 x 8 000 117 -> 77, 9 x 16 384 of 128 heads ragged 130 -> 75, 48 listed
+// sets of 2 048 rows 87 -> 66, and at precise 4 18 x 10 262 ragged 72 -> 51, 11 x 12 613 of 128 heads 96 -> 66; in one round up to 24 576: 32 x 6 000
+// (24 064) 79.1 -> 78.9, ragged 63 -> 57, 32 x 4 096 at precise 0 (16 384) 58 -> 51, but 16 x 16 384 (32 768) 94 -> 97, and the 8-bit kernel stays the faster.
+// Up to 32 heads those workgroups are half empty.
+constexpr long long kWideMinWork = 8192, kWideMinWorkListed = 5120, kWideMaxWork = 24576;
+static inline bool heads32_pays(const AttendPlan& p, const AttendPlan& plan, bool heads16, int n_seqs, int H, int max_rows, int precise,
+                                bool dense) {
+    const long long tiles = max_rows / kTile + (max_rows % kTile != 0);
+    if (heads16) return n_seqs * tiles * ((H + kH16Heads - 1) / kH16Heads) > (dense ? kWideMinWork : kWideMinWorkListed);
+    const int groups = (H + kWideHeads - 1) / kWideHeads;
+    if ((long long)plan.n_items * ((H + 63) / 64) > kAttTargetGroups) return true;
+    if (precise > 2 || 4 * p.n_items * groups < 3 * kAttTargetGroups) return false;
+    return groups == 1 || n_seqs * tiles * 2 * groups <= kWideMaxWork;
+}
+// A paged call's work items there, n_items 0 where `route`, attend_route's, stands.
+static inline AttendPlan heads32_route(const AttendPlan& plan, const AttendRoute& route, int n_seqs, int H, int max_rows, int precise,
+                                       bool dense) {
+    AttendPlan p = heads32_plan(plan, n_seqs, H, max_rows);
+    // (sequences that stay whole, or that one long one of many must not keep a workgroup with, stay where they are)
+    if (!p.n_items || (route.heads16 && !route.by_seq) || !heads32_pays(p, plan, route.heads16, n_seqs, H, max_rows, precise, dense)) p.n_items = 0;
+    return p;
+}
+
 }  // namespace rk

@@ -13,4 +13,11 @@ extern "C" int attend_route(int n_seqs, int H, int max_rows, int precise, int li
     return r.heads16;
 }
 
+// The same call's work items in workgroups of 32 heads, 0 where it stays with attend_route's.
+extern "C" int attend_wide_items(int n_seqs, int H, int max_rows, int precise, int listed) {
+    const rk::AttendPlan plan = rk::attend_plan(n_seqs, H, max_rows);
+    const rk::AttendRoute r = rk::attend_route(plan, n_seqs, H, max_rows, precise, !listed, false);
+    return rk::heads32_route(plan, r, n_seqs, H, max_rows, precise, !listed).n_items;
+}
+
 extern "C" long long marked_block(unsigned row, unsigned group) { return rk::marked_block(row, group); }

@@ -3,7 +3,7 @@
 import numpy as np
 import pytest
 
-from tests.util import attend_route, marked_block
+from tests.util import attend_route, attend_wide_items, marked_block
 
 
 @pytest.mark.parametrize("listed", [False, True])
@@ -137,3 +137,23 @@ def test_blocks_left_to_a_second_pass_spread_over_its_groups():
     for stride in range(1, 2049):
         most = np.bincount(owner[::stride]).max()
         assert most <= -(-len(owner[::stride]) // 256) + 6, stride
+
+
+@pytest.mark.parametrize("listed", [False, True])
+@pytest.mark.parametrize("precise", [0, 2, 4])
+def test_work_items_of_32_heads_fit_the_scratch_and_the_chip(precise, listed):
+    """Never more records than the caller's scratch was sized for (an item and a sequence each), two work items a sequence and
+    more, the head groups of all of them in one round of the compute units; and the calls that change sides."""
+    for H in (1, 16, 17, 32, 33, 48, 64, 80, 128, 200, 528, 1024, 4096):
+        for n in (1, 2, 7, 16, 20, 24, 33, 64, 65, 128, 1025):
+            for rows in (1, 64, 300, 1000, 4096, 40000, 2 ** 25):
+                items = attend_wide_items(n, H, rows, precise, listed)
+                if not items:
+                    continue
+                assert H > 16 and n <= 64 and 2 * n <= items <= n * (-(-rows // 32) // 2), (H, n, rows, items)
+                assert items <= attend_route(n, H, rows, precise, listed).scratch_items
+                assert -(-items // 8) * 8 * -(-H // 32) <= 256
+    wide = lambda *call: attend_wide_items(*call, precise, listed) > 0
+    assert wide(24, 64, 8000) and wide(9, 128, 16384) and wide(18, 64, 10262)  # a second round of 64 heads' workgroups
+    assert wide(6, 64, 9000) == (listed and precise < 4) and not wide(8, 64, 2048) and not wide(32, 64, 32768) and not wide(32, 16, 16384)
+    assert wide(32, 64, 6000) == (precise < 4) and wide(12, 128, 2048) == (listed and precise < 4)

@@ -18,7 +18,7 @@ import pytest
 from rivoli_amd import hip
 from tests.attend_cases import paged_case
 from tests.gpu_util import back, dev, dzeros
-from tests.util import attend_route
+from tests.util import attend_route, attend_wide_items
 
 pytestmark = pytest.mark.gpu
 KVL, ROPE, PT = 512, 64, 64
@@ -721,4 +721,61 @@ def test_peaked_softmax_in_workgroups_of_64_heads(oracle, lists):
                                    KVL, ROPE, 16, c["scale"], n_threads=8)
     rows, n_rows = listed([np.arange(k)[::-1] for k in lens], 1100)
     got = run_paged(c, 1100, rows=rows, n_rows=n_rows, pt=16) if lists else run_paged(c, 1100, pt=16)
+    check(got, want, 2, "peaked", tight_bound=False)
+
+
+@pytest.mark.parametrize("precise", [2, 1, 0, 4, 3])
+@pytest.mark.parametrize("H,pt", [(64, 64), (33, 48), (70, 4)])
+def test_workgroups_of_32_heads_over_a_ragged_batch(oracle, H, pt, precise):
+    """Lengths around every tile and run size, empty sequences and a long one, heads that do not fill a group; dense, and listed
+    with entries of all ones; then with pages the table does not have, left out and counted once each."""
+    top = 4600
+    lens = [63, 64, 65, 127, 128, 129, 1, 0, 31, 33, 191, 192, 193, 700, 2500, 32, 0, 320, 385, 511]
+    n = len(lens)
+    for is_listed in (False, True):
+        assert attend_wide_items(n, H, top, precise, is_listed)
+    c = paged_case(oracle, lens, H=H, seed=1100 + pt, page_tokens=pt, outlier_frac=0.0)
+    rng = np.random.default_rng(110)
+    width = c["table"].shape[1] * pt
+
+    def want_of(tokens):
+        rows, n_rows = listed(tokens, top)
+        return oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], None, rows, n_rows,
+                                       KVL, ROPE, pt, c["scale"], n_threads=8)
+
+    mild = precise in (2, 4)
+    every = [np.arange(k) for k in lens]
+    want = want_of(every)
+    check(run_paged(c, top, precise=precise, pt=pt), want, precise, "dense", mild=mild)
+    tokens = [np.insert(rng.permutation(t), len(t) // 2, [0xFFFFFFFF] * (len(t) % 3)) for t in every]
+    rows, n_rows = listed(tokens, top)
+    check(run_paged(c, top, rows=rows, n_rows=n_rows, use_lens=False, precise=precise, pt=pt), want, precise, "listed", mild=mild)
+    table = c["table"].copy()
+    gone = {(14, 0): -1, (14, 2400 // pt): c["n_pages"], (13, 128 // pt): c["n_pages"] + 9, (0, 0): -7}
+    for at, page in gone.items():
+        table[at] = page
+    kept = [t[[(s, b) not in gone for b in t // pt]] for s, t in enumerate(every)]
+    bad = dzeros(4)
+    check(run_paged(dict(c, table=table), top, precise=precise, pt=pt, bad=bad), want_of(kept), precise, "missing pages", mild=mild)
+    assert back(bad, np.uint32)[0] == sum(lens) - sum(len(t) for t in kept)
+    tokens = [rng.permutation(t) for t in every]
+    tokens[3][:3] = [width, 2 ** 31, 2 ** 32 - 2]
+    kept = [np.array([k for k in t if k < width and (s, k // pt) not in gone], np.int64) for s, t in enumerate(tokens)]
+    rows, n_rows = listed(tokens, top)
+    bad = dzeros(4)
+    got = run_paged(dict(c, table=table), top, rows=rows, n_rows=n_rows, use_lens=False, precise=precise, pt=pt, bad=bad)
+    check(got, want_of(kept), precise, "listed, missing pages and tokens past the table", mild=mild)
+    assert back(bad, np.uint32)[0] == sum(len(t) for t in tokens) - sum(len(t) for t in kept)
+
+
+@pytest.mark.parametrize("lists", [False, True])
+def test_peaked_softmax_in_workgroups_of_32_heads(oracle, lists):
+    """As test_peaked_softmax, where that kernel's own rescaling runs, over work items of several tiles."""
+    lens = [1100, 777, 1000, 1] * 6
+    assert attend_wide_items(24, 64, 4096, 2, lists)
+    c = paged_case(oracle, lens, H=64, seed=1190, q_gain=6.0, page_tokens=16)
+    want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], None, None,
+                                   KVL, ROPE, 16, c["scale"], n_threads=8)
+    rows, n_rows = listed([np.arange(k)[::-1] for k in lens], 4096)
+    got = run_paged(c, 4096, rows=rows, n_rows=n_rows, pt=16) if lists else run_paged(c, 4096, pt=16)
     check(got, want, 2, "peaked", tight_bound=False)

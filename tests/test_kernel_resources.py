@@ -165,6 +165,16 @@ def test_the_build_refuses_an_attention_object_that_spills():
 
 
 @pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
+def test_attention_of_32_heads_a_workgroup_fits_its_registers_and_a_compute_units_lds():
+    """Eight waves in half of the registers each, three tiles and four partial scores in nearly all of the LDS; both address modes of three modes."""
+    blocks = [b for b in _resource_blocks("mla_attend.hip") if "mla_attend_wide_kernel" in b.split()[0]]
+    assert len(blocks) == 6
+    for b in blocks:
+        assert int(re.search(r"ScratchSize \[bytes/lane\]: (\d+)", b).group(1)) == 0
+        assert int(re.search(r"LDS Size \[bytes/block\]: (\d+)", b).group(1)) <= 160 * 1024
+
+
+@pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
 def test_list_attention_of_32_heads_a_wave_keeps_its_operands_apart(tmp_path):
     """Its score products are written as assembly, so the compiler does not see to their wait states:
     a vector instruction's result may be a matrix instruction's operand two instructions later at

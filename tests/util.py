@@ -72,6 +72,11 @@ def attend_route(n_seqs, H, max_rows, precise, listed=False, linear=0):
     return AttendRoute(_plan().attend_route(n_seqs, H, max_rows, precise, int(listed), linear, out), out)
 
 
+def attend_wide_items(n_seqs, H, max_rows, precise, listed=False):
+    """heads32_route of the same file: a paged call's work items in workgroups of 32 heads, 0 where attend_route's route stands."""
+    return _plan().attend_wide_items(n_seqs, H, max_rows, precise, int(listed))
+
+
 def marked_block(row, group):
     """rivoli_amd/csrc/gather_attn_plan.hpp: the group's block in a row of 256."""
     return _plan().marked_block(row, group)
