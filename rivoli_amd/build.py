@@ -73,6 +73,9 @@ def build_kernels(verbose: bool = False) -> str:
     common = [hipcc(), f"--offload-arch={offload_arch()}", "-O3", "-std=c++17", "-fPIC",
               # packed-f32 instructions stay off: plain f32 math only
               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+              # a kernel's first arguments are in scalar registers when it starts: the short kernels of a token's
+              # chain are spared a round trip to memory each
+              "-mllvm", "-amdgpu-kernarg-preload-count=14",
               "-I", os.path.join(os.path.dirname(CSRC), "..", "include")]
 
     def compile_one(k: str) -> str:
