@@ -62,6 +62,42 @@ __device__ __forceinline__ void few_dma4(const void* src, lds_ptr<uint8_t> dst) 
                  : "memory");
 }
 
+// A lane's four pieces of a row's codes, 128 bytes apart in memory and 1024 in LDS, and its fifth, of the roped codes, for the lanes of
+// `roped`. The instruction's offset counts in memory and in LDS, so m0 makes up the difference and the address is one. All lanes are here.
+__device__ __forceinline__ void few_dma_row(const uint8_t* src, lds_ptr<uint8_t> to, lds_ptr<uint8_t> to_rope, unsigned long long roped) {
+    const uint32_t base = (uint32_t)(uintptr_t)to, rope = (uint32_t)(uintptr_t)to_rope - 512u;
+    uint32_t keep;
+    unsigned long long all;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\t"
+                 "s_add_u32 m0, m0, 896\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off offset:128\n\t"
+                 "s_add_u32 m0, m0, 896\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off offset:256\n\t"
+                 "s_add_u32 m0, m0, 896\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off offset:384\n\t"
+                 "s_mov_b32 m0, %4\n\ts_and_saveexec_b64 %1, %5\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off offset:512\n\t"
+                 "s_mov_b64 exec, %1\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep), "=&s"(all)
+                 : "v"(src), "s"(base), "s"(rope), "s"(roped)
+                 : "memory", "scc");
+}
+
+// A paged row, looked up: whether it is there, its codes and its scale (of one that is not there the first row's). bad: it should be.
+struct FewRow {
+    bool there, bad;
+    const uint8_t *codes, *scale;
+};
+__device__ __forceinline__ FewRow few_row(const AttendArgs& a, bool mine, unsigned int tok, int page) {
+    unsigned int blk, off;
+    if (a.page_shift >= 0) blk = tok >> a.page_shift, off = tok & (unsigned)(a.page_tokens - 1);
+    else blk = tok / (unsigned)a.page_tokens, off = tok - blk * (unsigned)a.page_tokens;
+    FewRow r;
+    r.there = mine & (blk < (unsigned)a.max_blocks) & ((unsigned)page < (unsigned)a.n_pages);
+    r.bad = mine & !r.there;
+    off = r.there ? off : 0u;
+    const uint8_t* const base = a.pool + (unsigned long long)(unsigned)(r.there ? page : 0) * a.page_bytes;
+    r.codes = base + (unsigned long long)off * (unsigned)kRowW;
+    r.scale = base + (size_t)a.page_tokens * kRowW + (unsigned long long)off * 4u;
+    return r;
+}
+
 // One part of a workgroup's work, as attend_part: rows [r_begin, r_end) of sequence `seq`, heads
 // 16 * hg .. +15.
 template <int QSPLIT, int PSPLIT, int MODE>
@@ -113,35 +149,31 @@ __device__ __forceinline__ void attend_part_few(const AttendArgs& a, int seq, in
         return (lds_ptr<uint8_t>)(uintptr_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)p);
     };
     const int swap = (4 * (wave & 1) + (lane >> 4)) & 7;  // (my_row >> 1) & 7
+    const unsigned long long roped = __builtin_amdgcn_ballot_w64(16 * (l8 ^ swap) < kRopeW);  // lanes with a piece of the roped codes
     auto request = [&](int tile, int buf, unsigned int tok, int page) -> bool {
         const unsigned int pos = (unsigned)tile * kFewTokens + my_row;
         // a list entry of all ones is nobody's token, and only the 8-bit modes count it (as attend_part)
         const bool nobody = MODE != kDense && tok == 0xffffffffu && (LINEAR || !a.count_ones);
-        bool there = pos < (unsigned)(r_end - r_begin) && !nobody;
-        const uint8_t *codes, *ropes, *scale;  // a row that is not there reads the first one
-        if constexpr (LINEAR) {
-            const size_t t = there ? tok : 0;
-            codes = a.lc8 + t * kKvl;
-            ropes = reinterpret_cast<const uint8_t*>(a.rc + t * kRopeW);
-            scale = reinterpret_cast<const uint8_t*>(a.lscale + t * 4 + (l8 & 3));
-        } else {
-            if (there && (block_of(tok) >= (unsigned)a.max_blocks || (unsigned)page >= (unsigned)a.n_pages)) {
-                there = false;
-                if (a.bad_rows && hg == 0 && l8 == 0) atomicAdd(a.bad_rows, 1u);
-            }
-            const unsigned int off = !there ? 0u : a.page_shift >= 0 ? tok & (unsigned)(a.page_tokens - 1) : tok % (unsigned)a.page_tokens;
-            const uint8_t* const base = a.pool + (there ? (size_t)page * a.page_bytes : 0);
-            codes = base + (size_t)off * kRowW;
-            ropes = codes + kKvl;
-            scale = base + (size_t)a.page_tokens * kRowW + (size_t)off * 4;
-        }
+        const bool mine = (pos < (unsigned)(r_end - r_begin)) & !nobody;
         const int piece = 16 * (l8 ^ swap);
         const lds_ptr<uint8_t> to = scalar(rows + buf * kFewTileBytes + wave * kFewWaveBytes);
-        few_dma4(scale, scalar((lds_ptr<uint8_t>)scale_raw[buf][wave]));
+        const lds_ptr<uint8_t> to_scale = scalar((lds_ptr<uint8_t>)scale_raw[buf][wave]);
+        if constexpr (LINEAR) {  // a row that is not there reads the first one
+            const size_t t = mine ? tok : 0;
+            few_dma4(reinterpret_cast<const uint8_t*>(a.lscale + t * 4 + (l8 & 3)), to_scale);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dma16(codes + piece + 128 * i, to + 1024 * i);
-        if (LINEAR || piece < kRopeW) dma16(ropes + piece, to + 4096);
-        return there;
+            for (int i = 0; i < 4; ++i) dma16(a.lc8 + t * kKvl + piece + 128 * i, to + 1024 * i);
+            dma16(reinterpret_cast<const uint8_t*>(a.rc + t * kRopeW) + piece, to + 4096);
+            return mine;
+        } else {
+            const FewRow r = few_row(a, mine, tok, page);
+            if (a.bad_rows && hg == 0 && __builtin_amdgcn_ballot_w64(r.bad) != 0) {
+                if (r.bad && l8 == 0) atomicAdd(a.bad_rows, 1u);
+            }
+            few_dma4(r.scale, to_scale);
+            few_dma_row(r.codes + piece, to, to + 4096, roped);
+            return r.there;
+        }
     };
 
     // ---- prologue: the query is asked for, two tiles are looked up and requested, the lookups of the third made; then

@@ -73,27 +73,19 @@ __device__ __forceinline__ void attend_part_wide(const AttendArgs& a, int seq, i
         return (lds_ptr<uint8_t>)(uintptr_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)p);
     };
     const int swap = (4 * (wave & 1) + (lane >> 4)) & 7;  // (my_row >> 1) & 7
+    const unsigned long long roped = __builtin_amdgcn_ballot_w64(16 * (l8 ^ swap) < kRopeW);  // lanes with a piece of the roped codes
     auto request = [&](int tile, int buf, unsigned int tok, int page) -> bool {
         const unsigned int pos = (unsigned)tile * kWideTokens + my_row;
         // a list entry of all ones is nobody's token, and only the 8-bit modes count it (as attend_part)
         const bool nobody = MODE != kDense && tok == 0xffffffffu && !a.count_ones;
-        bool there = pos < (unsigned)(r_end - r_begin) && !nobody;
-        if (there && (block_of(tok) >= (unsigned)a.max_blocks || (unsigned)page >= (unsigned)a.n_pages)) {
-            there = false;
-            if (a.bad_rows && hg == 0 && l8 == 0) atomicAdd(a.bad_rows, 1u);
+        const FewRow r = few_row(a, (pos < (unsigned)(r_end - r_begin)) & !nobody, tok, page);
+        if (a.bad_rows && hg == 0 && __builtin_amdgcn_ballot_w64(r.bad) != 0) {
+            if (r.bad && l8 == 0) atomicAdd(a.bad_rows, 1u);
         }
-        // a row that is not there reads the first one
-        const unsigned int off = !there ? 0u : a.page_shift >= 0 ? tok & (unsigned)(a.page_tokens - 1) : tok % (unsigned)a.page_tokens;
-        const uint8_t* const base = a.pool + (there ? (size_t)page * a.page_bytes : 0);
-        const uint8_t* const codes = base + (size_t)off * kRowW;
-        const uint8_t* const scale = base + (size_t)a.page_tokens * kRowW + (size_t)off * 4;
-        const int piece = 16 * (l8 ^ swap);
-        const lds_ptr<uint8_t> to = scalar(rows + buf * kWideTileBytes + wave * 4096);
-        few_dma4(scale, scalar((lds_ptr<uint8_t>)scale_raw[buf][wave]));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) dma16(codes + piece + 128 * i, to + 1024 * i);
-        if (piece < kRopeW) dma16(codes + kKvl + piece, scalar(rows + buf * kWideTileBytes + kWideRopeAt + (wave >> 1) * 1024));
-        return there;
+        few_dma4(r.scale, scalar((lds_ptr<uint8_t>)scale_raw[buf][wave]));
+        few_dma_row(r.codes + 16 * (l8 ^ swap), scalar(rows + buf * kWideTileBytes + wave * 4096),
+                    scalar(rows + buf * kWideTileBytes + kWideRopeAt + (wave >> 1) * 1024), roped);
+        return r.there;
     };
 
     // ---- prologue: the query is asked for, two tiles are looked up and requested, the lookups of the third made; then
