@@ -41,9 +41,19 @@ template <int CTRL>
 __device__ __forceinline__ float few_dpp(float x) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));
 }
+// max over sixteen lanes, in each of them: an instruction a step (the compiler's maximum quiets both operands first, and takes a move for
+// the other lane's). The wait before each is what a lane's value needs on its way to another.
+__device__ __forceinline__ float few_max16(float x) {
+    asm("s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:2 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:1 row_mask:0xf bank_mask:0xf"
+        : "+v"(x));
+    return x;
+}
 // max / sum over 32 lanes, in each of them
 __device__ __forceinline__ float few_max32(float x) {
-    x = fmaxf(x, few_dpp<0x128>(x)), x = fmaxf(x, few_dpp<0x124>(x)), x = fmaxf(x, few_dpp<0x122>(x)), x = fmaxf(x, few_dpp<0x121>(x));
+    x = few_max16(x);
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
 }

@@ -257,8 +257,7 @@ __device__ __forceinline__ void attend_part_wide(const AttendArgs& a, int seq, i
 #pragma unroll
             for (int i = 0; i < 4; ++i) x[i] = scl[i] > 0.0f ? ((part[0][i] + part[1][i]) + (part[2][i] + part[3][i])) * scl[i] : -INFINITY;
             float tmax = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
-            tmax = fmaxf(tmax, few_dpp<0x128>(tmax)), tmax = fmaxf(tmax, few_dpp<0x124>(tmax));
-            tmax = fmaxf(tmax, few_dpp<0x122>(tmax)), tmax = fmaxf(tmax, few_dpp<0x121>(tmax));
+            tmax = few_max16(tmax);
             const bool grow = tmax > m_ref + kLazyRescale;  // false while nothing is there
             const float corr = grow ? __builtin_amdgcn_exp2f(m_ref - tmax) : 1.0f;  // 2^-inf = 0 at first
             if (grow) m_ref = tmax;
