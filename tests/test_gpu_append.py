@@ -306,3 +306,24 @@ def test_large_batch_kernel_other_widths(oracle):
         pool = dzeros(n_pages * pb, 0x5A)
         hip.launch_kv_append_paged(dev(rows), dev(slots), pool, n, width, pt, n_pages)
         assert np.array_equal(back(pool), want), (width, pt)
+
+
+@pytest.mark.parametrize("n", [1, 3, 1024, 1025])
+@pytest.mark.parametrize("kvl,ropn", [(128, 64), (256, 1), (384, 300), (512, 64), (1024, 777)])
+def test_append_kv_rows_shared_by_four_waves_and_not(oracle, n, kvl, ropn):
+    """Up to 1 024 tokens of more than one block four waves share a token: blocks that are no multiple of four, roped keys shorter and
+    longer than the waves' first pass, and the line."""
+    nb, pos0 = kvl // 128, 2
+    rng = np.random.default_rng(n + kvl)
+    latent = (rng.standard_normal((n, kvl)) * rng.choice([0.01, 1, 30], (n, 1))).astype(np.float32)
+    rope = rng.standard_normal((n, ropn)).astype(np.float32)
+    rows = n + 4
+    first = [np.full(rows * kvl, 0xEE, np.uint8), np.full(rows * nb, 7.0, np.float32), np.full(rows * ropn, 0xABCD, np.uint16)]
+    c8, ls, rc = (dev(x) for x in first)
+    want = [x.copy() for x in first]
+    for t in range(n):
+        assert oracle.append_kv(latent[t], rope[t], *want, pos0 + t, kvl, ropn, nb) == 0
+    hip.launch_append_kv_rows(dev(latent), dev(rope), c8, ls, rc, pos0, n, kvl, ropn, nb)
+    assert np.array_equal(back(c8), want[0])
+    assert np.array_equal(back(ls, np.uint32), want[1].view(np.uint32))
+    assert np.array_equal(back(rc, np.uint16), want[2])

@@ -779,3 +779,14 @@ def test_peaked_softmax_in_workgroups_of_32_heads(oracle, lists):
     rows, n_rows = listed([np.arange(k)[::-1] for k in lens], 4096)
     got = run_paged(c, 4096, rows=rows, n_rows=n_rows, pt=16) if lists else run_paged(c, 4096, pt=16)
     check(got, want, 2, "peaked", tight_bound=False)
+
+
+@pytest.mark.parametrize("lens,H", [([16384], 64), ([16384], 7), ([9000, 40, 0, 129, 64], 64), ([7000, 33, 300, 1, 64, 64, 0, 500], 64),
+                                    ([2600, 2500, 1], 96)])
+def test_merge_of_few_and_many_records(oracle, lens, H):
+    """One sequence of up to 64 records, by four groups of threads a head (up to 256 heads times sequences) and by one, whose batches
+    are of sixteen or eight records; sequences of one record, which their work item writes, and of none."""
+    c = paged_case(oracle, lens, H=H, seed=1200 + len(lens), outlier_frac=0.01)
+    want = oracle.mla_attend_paged(c["qabs"], c["qrope"], c["pool"], c["table"], c["lens"], None, None,
+                                   KVL, ROPE, PT, c["scale"], n_threads=8)
+    check(run_paged(c, max(lens)), want, 2, "merged")

@@ -221,3 +221,15 @@ def test_select_guards():
         with pytest.raises(hip.LaunchError) as e:
             hip.launch_index_select_blocks(*args)
         assert e.value.code == code, args
+
+
+@pytest.mark.parametrize("rows,n,stride,block", [(2340, 448, 512, 64), (2341, 448, 512, 64), (1, 64, 64, 64), (5000, 64, 64, 64), (70000, 64, 64, 64),
+                                                 (300, 16 * 37, 16 * 37 + 4, 16), (997, 96, 100, 32), (40, 256 * 31, 256 * 31, 256)])
+def test_act_quant_rows_by_a_product_and_a_piece_a_thread(oracle, rows, n, stride, block):
+    """One, an odd number and a power of two of blocks a row, on both sides of the line (262 144 pieces) between one piece a
+    thread and four."""
+    rng = np.random.default_rng(rows + n)
+    x = (rng.standard_normal((rows, stride)) * np.exp(rng.uniform(-6, 6, (rows, 1)))).astype(np.float32)
+    x[rows // 2, :block] = 0.0
+    got = check_act_quant(oracle, x, n, block, what="rows")
+    assert np.array_equal(got[:, n:].view(np.uint32), x[:, n:].view(np.uint32))
