@@ -149,13 +149,13 @@ static void launch_act_quant(const float* src, float* dst, long long n_blocks, i
     const uint32_t nb_inv = nb == 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / (uint32_t)nb);
     const long long each = (n_pieces + kAqThreads - 1) / kAqThreads;  // workgroups of a piece a thread
     if (each <= kAqFewGroups) {
-        hipLaunchKernelGGL((act_quant_kernel<LANES, 1>), dim3((unsigned)each), dim3(kAqThreads), 0, stream, src, dst,
+        rk::launch_kernel((act_quant_kernel<LANES, 1>), dim3((unsigned)each), dim3(kAqThreads), 0, stream, src, dst,
                            (uint32_t)n_pieces, (uint32_t)nb, (uint32_t)row_stride, nb_inv);
         return;
     }
     long long groups = (each + kAqInFlight - 1) / kAqInFlight;
     if (groups > 256 * 16) groups = 256 * 16;
-    hipLaunchKernelGGL((act_quant_kernel<LANES, kAqInFlight>), dim3((unsigned)groups), dim3(kAqThreads), 0, stream,
+    rk::launch_kernel((act_quant_kernel<LANES, kAqInFlight>), dim3((unsigned)groups), dim3(kAqThreads), 0, stream,
                        src, dst, (uint32_t)n_pieces, (uint32_t)nb, (uint32_t)row_stride, nb_inv);
 }
 
@@ -182,7 +182,7 @@ extern "C" int rivoli_act_quant_f8_prefix(const float* src, float* dst, int rows
         case 256: rk::launch_act_quant<64>(src, dst, n_blocks, nb, row_stride, st); break;
         default: {
             const long long groups = (n_blocks + rk::kAqThreads - 1) / rk::kAqThreads;
-            hipLaunchKernelGGL(rk::act_quant_serial_kernel, dim3((unsigned)groups),
+            rk::launch_kernel(rk::act_quant_serial_kernel, dim3((unsigned)groups),
                                dim3(rk::kAqThreads), 0, st, src, dst, n_blocks, nb, row_stride,
                                block);
         }

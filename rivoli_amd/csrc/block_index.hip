@@ -1137,9 +1137,9 @@ extern "C" int rivoli_act_quant_f4_rotated(float* x, int rows, int d, void* stre
     hipStream_t st = (hipStream_t)stream;
 #define RK_SPREAD(LPR)                                                                                      \
     if (few)                                                                                                \
-        hipLaunchKernelGGL((rk::f4_rotated_kernel<LPR, 1>), grid, block, 0, st, x, (long long)rows, scale); \
+        rk::launch_kernel((rk::f4_rotated_kernel<LPR, 1>), grid, block, 0, st, x, (long long)rows, scale); \
     else                                                                                                    \
-        hipLaunchKernelGGL((rk::f4_rotated_kernel<LPR, rk::kSpreadInFlight>), grid, block, 0, st, x,        \
+        rk::launch_kernel((rk::f4_rotated_kernel<LPR, rk::kSpreadInFlight>), grid, block, 0, st, x,        \
                            (long long)rows, scale)
     switch (lpr) {
         case 8: RK_SPREAD(8); break;
@@ -1174,10 +1174,10 @@ static int score_blocks_launch(const float* q, const float* kv, const float* w, 
             // half the blocks a workgroup while there is a compute unit for each (8 192 blocks 6.1 us, 7.1 in
             // 64s; 16 384 blocks 7.1 us in 64s, 8.5 in 32s)
             if ((long long)s * 2 * groups <= 256)
-                hipLaunchKernelGGL(score_blocks_one_kernel<1>, dim3((unsigned)(((long long)n_comp + 31) / 32), (unsigned)s),
+                rk::launch_kernel(score_blocks_one_kernel<1>, dim3((unsigned)(((long long)n_comp + 31) / 32), (unsigned)s),
                                    dim3(kOneThreads), 0, st, q, kv, w, score, s, n_comp, heads, ratio);
             else
-                hipLaunchKernelGGL(score_blocks_one_kernel<2>, dim3(groups, (unsigned)s), dim3(kOneThreads), 0, st, q,
+                rk::launch_kernel(score_blocks_one_kernel<2>, dim3(groups, (unsigned)s), dim3(kOneThreads), 0, st, q,
                                    kv, w, score, s, n_comp, heads, ratio);
             return launch_status();
         }
@@ -1199,9 +1199,9 @@ static int score_blocks_launch(const float* q, const float* kv, const float* w, 
         if (y <= 65535u) {
             const PairArgs args = {q, kv, w, score, s, n_comp, heads, per, ratio};
             if (fp4)
-                hipLaunchKernelGGL(score_blocks_codes_kernel, dim3(t_groups, y), dim3(kPairThreads), 0, st, args);
+                rk::launch_kernel(score_blocks_codes_kernel, dim3(t_groups, y), dim3(kPairThreads), 0, st, args);
             else
-                hipLaunchKernelGGL(score_blocks_pair_kernel, dim3(t_groups, y), dim3(kPairThreads), 0, st, args);
+                rk::launch_kernel(score_blocks_pair_kernel, dim3(t_groups, y), dim3(kPairThreads), 0, st, args);
             return launch_status();
         }
     }
@@ -1217,15 +1217,15 @@ static int score_blocks_launch(const float* q, const float* kv, const float* w, 
     const dim3 block(kScoreThreads);
     if (hd == 128 && aligned16(kv) && (long long)s * c_groups < 256 && heads <= kSplitMaxHeads) {
         const unsigned groups = (unsigned)(((long long)n_comp + kWave - 1) / kWave);
-        hipLaunchKernelGGL(index_score_blocks_128_split_kernel, dim3(groups), dim3(kSplitWavesPerGroup * kWave),
+        rk::launch_kernel(index_score_blocks_128_split_kernel, dim3(groups), dim3(kSplitWavesPerGroup * kWave),
                            (size_t)heads * kWave * sizeof(float), st, q, kv, w, score, s, n_comp, heads, ratio);
         return launch_status();
     }
     if (hd == 128 && aligned16(kv))
-        hipLaunchKernelGGL(index_score_blocks_128_kernel, grid, block, 0, st, q, kv, w, score, s, n_comp,
+        rk::launch_kernel(index_score_blocks_128_kernel, grid, block, 0, st, q, kv, w, score, s, n_comp,
                            heads, t_per_group, ratio);
     else
-        hipLaunchKernelGGL(index_score_blocks_any_kernel, grid, block, 0, st, q, kv, w, score, s, n_comp,
+        rk::launch_kernel(index_score_blocks_any_kernel, grid, block, 0, st, q, kv, w, score, s, n_comp,
                            heads, hd, t_per_group, ratio);
     return launch_status();
 }

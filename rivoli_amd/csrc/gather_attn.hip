@@ -670,42 +670,42 @@ static int gather_attn_launch(const float* q, const float* kv, const float* sink
         if (few) {
             const dim3 few_grid((unsigned)m, (unsigned)((h + kGfHeads - 1) / kGfHeads), (unsigned)a.n_splits);
             if (precise >= 2)
-                hipLaunchKernelGGL((gather_attn_few_kernel<2, 2>), few_grid, dim3(kGfThreads), 0, stream, a);
+                rk::launch_kernel((gather_attn_few_kernel<2, 2>), few_grid, dim3(kGfThreads), 0, stream, a);
             else if (precise == 1)
-                hipLaunchKernelGGL((gather_attn_few_kernel<2, 1>), few_grid, dim3(kGfThreads), 0, stream, a);
+                rk::launch_kernel((gather_attn_few_kernel<2, 1>), few_grid, dim3(kGfThreads), 0, stream, a);
             else
-                hipLaunchKernelGGL((gather_attn_few_kernel<1, 1>), few_grid, dim3(kGfThreads), 0, stream, a);
+                rk::launch_kernel((gather_attn_few_kernel<1, 1>), few_grid, dim3(kGfThreads), 0, stream, a);
         } else if (wide) {
             const dim3 rest((unsigned)kGaTargetGroups);
             if (precise >= 2) {
-                hipLaunchKernelGGL((gather_attn_wide_kernel<2, 2>), grid, dim3(kGwThreads), 0, stream, a);
-                hipLaunchKernelGGL((gather_attn_marked_kernel<2, 2>), rest, dim3(kGaThreads), 0, stream, a, blocks, (int)grid.y);
+                rk::launch_kernel((gather_attn_wide_kernel<2, 2>), grid, dim3(kGwThreads), 0, stream, a);
+                rk::launch_kernel((gather_attn_marked_kernel<2, 2>), rest, dim3(kGaThreads), 0, stream, a, blocks, (int)grid.y);
             } else if (precise == 1) {
-                hipLaunchKernelGGL((gather_attn_wide_kernel<2, 1>), grid, dim3(kGwThreads), 0, stream, a);
-                hipLaunchKernelGGL((gather_attn_marked_kernel<2, 1>), rest, dim3(kGaThreads), 0, stream, a, blocks, (int)grid.y);
+                rk::launch_kernel((gather_attn_wide_kernel<2, 1>), grid, dim3(kGwThreads), 0, stream, a);
+                rk::launch_kernel((gather_attn_marked_kernel<2, 1>), rest, dim3(kGaThreads), 0, stream, a, blocks, (int)grid.y);
             } else {
-                hipLaunchKernelGGL((gather_attn_wide_kernel<1, 1>), grid, dim3(kGwThreads), 0, stream, a);
+                rk::launch_kernel((gather_attn_wide_kernel<1, 1>), grid, dim3(kGwThreads), 0, stream, a);
             }
         } else if (precise >= 2)
-            hipLaunchKernelGGL((gather_attn_d512_kernel<2, 2>), grid, dim3(kGaThreads), 0, stream, a);
+            rk::launch_kernel((gather_attn_d512_kernel<2, 2>), grid, dim3(kGaThreads), 0, stream, a);
         else if (precise == 1)
-            hipLaunchKernelGGL((gather_attn_d512_kernel<2, 1>), grid, dim3(kGaThreads), 0, stream, a);
+            rk::launch_kernel((gather_attn_d512_kernel<2, 1>), grid, dim3(kGaThreads), 0, stream, a);
         else
-            hipLaunchKernelGGL((gather_attn_d512_kernel<1, 1>), grid, dim3(kGaThreads), 0, stream, a);
+            rk::launch_kernel((gather_attn_d512_kernel<1, 1>), grid, dim3(kGaThreads), 0, stream, a);
         const int rc = launch_status();
         if (rc != 0 || a.n_splits == 1) return rc;  // a split plan has fewer than 256 queries
         if (a.n_splits <= 8)
-            hipLaunchKernelGGL(gather_attn_combine_kernel<8>, dim3((unsigned)h, (unsigned)m), dim3(128), 0, stream,
+            rk::launch_kernel(gather_attn_combine_kernel<8>, dim3((unsigned)h, (unsigned)m), dim3(128), 0, stream,
                                a.part_acc, a.part_ml, sink, a.n_splits, h, o);
         else
-            hipLaunchKernelGGL(gather_attn_combine_kernel<16>, dim3((unsigned)h, (unsigned)m), dim3(128), 0, stream,
+            rk::launch_kernel(gather_attn_combine_kernel<16>, dim3((unsigned)h, (unsigned)m), dim3(128), 0, stream,
                                a.part_acc, a.part_ml, sink, a.n_splits, h, o);
         return launch_status();
     }
     // the reference launcher's limits, kept (attn.hip:450-458): d within 1024, its LDS budget
     if (d > kGaRowDims * kWave || m > 65535) return 1002;
     if (((size_t)d + (size_t)topk + 256 + 2) * sizeof(float) > 65536) return 1006;
-    hipLaunchKernelGGL(gather_attn_rowwise_kernel,
+    rk::launch_kernel(gather_attn_rowwise_kernel,
                        dim3((unsigned)((h + kGaRowThreads / kWave - 1) / (kGaRowThreads / kWave)), (unsigned)m),
                        dim3(kGaRowThreads), 0, stream, q, kv, sink, idxs, h, d, topk, n_kv, scale, o);
     return launch_status();

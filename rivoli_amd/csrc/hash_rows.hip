@@ -72,7 +72,7 @@ extern "C" int rivoli_hash_rows(const float* x, int n, int stride, unsigned long
     (void)hipGetLastError();
     // Grid-stride over samples with a capped grid: one atomic per workgroup, so the cap
     // bounds the atomics whatever n is; 2048 workgroups is 8 per CU on 256 CUs.
-    hipLaunchKernelGGL(hash_rows_kernel, dim3(capped_blocks(samples, kHashThreads, 2048)),
+    rk::launch_kernel(hash_rows_kernel, dim3(capped_blocks(samples, kHashThreads, 2048)),
                        dim3(kHashThreads), 0, (hipStream_t)stream,
                        reinterpret_cast<const uint32_t*>(x), (long long)n, (long long)stride,
                        i_base, out);
@@ -83,7 +83,7 @@ extern "C" int rivoli_codec_e4m3_encode(const float* x, unsigned char* out, long
                                         void* stream) {
     if (!x || !out || n <= 0) return 1001;
     (void)hipGetLastError();
-    hipLaunchKernelGGL(rk::e4m3_encode_kernel, dim3(rk::capped_blocks(n, 256, 4096)), dim3(256), 0,
+    rk::launch_kernel(rk::e4m3_encode_kernel, dim3(rk::capped_blocks(n, 256, 4096)), dim3(256), 0,
                        (hipStream_t)stream, x, out, n);
     return rk::launch_status();
 }
@@ -92,7 +92,7 @@ extern "C" int rivoli_codec_bf16_encode(const float* x, unsigned short* out, lon
                                         void* stream) {
     if (!x || !out || n <= 0) return 1001;
     (void)hipGetLastError();
-    hipLaunchKernelGGL(rk::bf16_encode_kernel, dim3(rk::capped_blocks(n, 256, 4096)), dim3(256), 0,
+    rk::launch_kernel(rk::bf16_encode_kernel, dim3(rk::capped_blocks(n, 256, 4096)), dim3(256), 0,
                        (hipStream_t)stream, x, out, n);
     return rk::launch_status();
 }

@@ -1389,17 +1389,17 @@ static void finish_bits_launch_shape(bool fixed, int n_segs, int kmax, int n_que
     constexpr int kShort = 16 * (kSegKeys / 32) / THREADS, kLong = kBitsMaxSegs * (kSegKeys / 32) / THREADS;
     if (n_segs <= 16) {
         if (fixed)
-            hipLaunchKernelGGL((topk_finish_bits_kernel<576, 64, THREADS, SLOTS, kShort>), grid, block,
+            rk::launch_kernel((topk_finish_bits_kernel<576, 64, THREADS, SLOTS, kShort>), grid, block,
                                0, stream, args...);
         else
-            hipLaunchKernelGGL((topk_finish_bits_kernel<0, 0, THREADS, SLOTS, kShort>), grid, block, 0,
+            rk::launch_kernel((topk_finish_bits_kernel<0, 0, THREADS, SLOTS, kShort>), grid, block, 0,
                                stream, args...);
     } else {
         if (fixed)
-            hipLaunchKernelGGL((topk_finish_bits_kernel<576, 64, THREADS, SLOTS, kLong>), grid, block,
+            rk::launch_kernel((topk_finish_bits_kernel<576, 64, THREADS, SLOTS, kLong>), grid, block,
                                0, stream, args...);
         else
-            hipLaunchKernelGGL((topk_finish_bits_kernel<0, 0, THREADS, SLOTS, kLong>), grid, block, 0,
+            rk::launch_kernel((topk_finish_bits_kernel<0, 0, THREADS, SLOTS, kLong>), grid, block, 0,
                                stream, args...);
     }
 }
@@ -1426,13 +1426,13 @@ static int index_topk_launch(const float* scores, int n_queries, int stride, con
         uint32_t* ws = (uint32_t*)workspace;
         const dim3 seg_grid((unsigned)n_segs, (unsigned)n_queries), block(kSplitThreads);
         if (!hist_ready)
-            hipLaunchKernelGGL(topk_hist_kernel, seg_grid, block, 0, stream, scores, stride, nts, nt,
+            rk::launch_kernel(topk_hist_kernel, seg_grid, block, 0, stream, scores, stride, nts, nt,
                                ws, ws_stride);
         const int kmax = k < nt ? k : nt;
         const size_t page_bytes = (size_t)ga.page_tokens * ga.width + (size_t)ga.page_tokens * 4;
         const bool fixed = ga.pool && ga.width == 576 && ga.page_tokens == 64;
         if (n_segs <= kBitsMaxSegs) {
-            hipLaunchKernelGGL(topk_cand_kernel<true>, seg_grid, block, 0, stream, scores, stride,
+            rk::launch_kernel(topk_cand_kernel<true>, seg_grid, block, 0, stream, scores, stride,
                                nts, nt, k, ws, ws_stride, n_segs);
             finish_bits_launch(fixed, n_segs, kmax, n_queries, stream, nts, nt, k, rows, ws,
                                ws_stride, n_segs, ga.pool, ga.block_table, ga.out,
@@ -1440,17 +1440,17 @@ static int index_topk_launch(const float* scores, int n_queries, int stride, con
                                page_bytes, ga.bad_rows);
             return launch_status();
         }
-        hipLaunchKernelGGL(topk_cand_kernel<false>, seg_grid, block, 0, stream, scores, stride, nts,
+        rk::launch_kernel(topk_cand_kernel<false>, seg_grid, block, 0, stream, scores, stride, nts,
                            nt, k, ws, ws_stride, n_segs);
         const dim3 out_grid((unsigned)((kmax + kSlotsPerGroup - 1) / kSlotsPerGroup),
                             (unsigned)n_queries);
         if (fixed)
-            hipLaunchKernelGGL((topk_finish_kernel<576, 64>), out_grid, block, 0, stream, scores,
+            rk::launch_kernel((topk_finish_kernel<576, 64>), out_grid, block, 0, stream, scores,
                                stride, nts, nt, k, rows, ws, ws_stride, n_segs, ga.pool,
                                ga.block_table, ga.out, ga.max_blocks_per_seq, ga.width,
                                ga.page_tokens, ga.n_pages, page_bytes, ga.bad_rows);
         else
-            hipLaunchKernelGGL((topk_finish_kernel<0, 0>), out_grid, block, 0, stream, scores, stride,
+            rk::launch_kernel((topk_finish_kernel<0, 0>), out_grid, block, 0, stream, scores, stride,
                                nts, nt, k, rows, ws, ws_stride, n_segs, ga.pool, ga.block_table,
                                ga.out, ga.max_blocks_per_seq, ga.width, ga.page_tokens, ga.n_pages,
                                page_bytes, ga.bad_rows);
@@ -1458,7 +1458,7 @@ static int index_topk_launch(const float* scores, int n_queries, int stride, con
     }
     dim3 grid((unsigned)n_queries), block(kTopkThreads);
 #define RK_TOPK_FEW(I)                                                                              \
-    hipLaunchKernelGGL(index_topk_few_kernel<I>, grid, dim3(kSfThreads), 0, stream, scores, stride, \
+    rk::launch_kernel(index_topk_few_kernel<I>, grid, dim3(kSfThreads), 0, stream, scores, stride, \
                        nts, nt, k, rows)
     if (nt <= kSfThreads)
         RK_TOPK_FEW(1);
@@ -1470,10 +1470,10 @@ static int index_topk_launch(const float* scores, int n_queries, int stride, con
         RK_TOPK_FEW(16);
 #undef RK_TOPK_FEW
     else if (nt <= kTopkThreads * 64)
-        hipLaunchKernelGGL(index_topk_kernel<64>, grid, block, 0, stream, scores, stride,
+        rk::launch_kernel(index_topk_kernel<64>, grid, block, 0, stream, scores, stride,
                            nts, nt, k, rows);
     else
-        hipLaunchKernelGGL(index_topk_kernel<0>, grid, block, 0, stream, scores, stride,
+        rk::launch_kernel(index_topk_kernel<0>, grid, block, 0, stream, scores, stride,
                            nts, nt, k, rows);
     return launch_status();
 }
@@ -1940,13 +1940,13 @@ static int block_select_launch(const float* scores, int rows, int n_comp, int ra
     (void)hipGetLastError();
     const dim3 grid((unsigned)rows);
 #define RK_BISECT(WV, I)                                                                     \
-    hipLaunchKernelGGL((block_select_bisect_kernel<WV, I>), grid, dim3(WV* kWave), 0, stream, \
+    rk::launch_kernel((block_select_bisect_kernel<WV, I>), grid, dim3(WV* kWave), 0, stream, \
                        scores, n_comp, ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
 #define RK_FEW(I)                                                                                             \
-    hipLaunchKernelGGL((block_select_few_kernel<I>), grid, dim3(kSfThreads), 0, stream, scores, n_comp, ratio, \
+    rk::launch_kernel((block_select_few_kernel<I>), grid, dim3(kSfThreads), 0, stream, scores, n_comp, ratio, \
                        prefill ? 1 : 0, k, offset, out, out_stride, window)
 #define RK_SELECT(T, I)                                                                       \
-    hipLaunchKernelGGL((block_select_kernel<T, I>), grid, dim3(T), 0, stream, scores, n_comp, \
+    rk::launch_kernel((block_select_kernel<T, I>), grid, dim3(T), 0, stream, scores, n_comp, \
                        ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
     // Few rows (decode: one) leave the chip to one workgroup each, and a row's time is its longest wave's: sixteen waves,
     // as few keys a lane as there are. One row of 8192 (sums of a ReLU): in four waves 17.8 us, by leading bits and
@@ -2019,7 +2019,7 @@ static int sel_fill_launch(const SelShape& s, int win, int ratio, int start_pos,
     (void)hipGetLastError();
     const dim3 grid((unsigned)s.rows, (unsigned)((s.win_cols + n_pos + 255) / 256));
     if (grid.y > 65535) return 1002;
-    hipLaunchKernelGGL(sel_fill_kernel, grid, dim3(256), 0, stream, win, ratio, start_pos, s.win_cols,
+    rk::launch_kernel(sel_fill_kernel, grid, dim3(256), 0, stream, win, ratio, start_pos, s.win_cols,
                        n_pos, s.offset, cols, out);
     return launch_status();
 }
@@ -2188,7 +2188,7 @@ extern "C" int rivoli_dsa_select_gather_paged_noalloc(const float* scores, int n
         const int code = static_workspace(&ws);
         if (code) return code;
         (void)hipGetLastError();
-        hipLaunchKernelGGL(topk_ws_clear_kernel, dim3((unsigned)n_queries), dim3(kSplitThreads), 0,
+        rk::launch_kernel(topk_ws_clear_kernel, dim3((unsigned)n_queries), dim3(kSplitThreads), 0,
                            (hipStream_t)stream, ws, ws_stride);
         const int launched = launch_status();
         if (launched) return launched;

@@ -422,16 +422,16 @@ static RowLaunch row_launch(const CompGeom& p, bool aligned) {
 #define RK_COMPRESS_DISPATCH(KERNEL, GRID, R, ENTS, STREAM, ...)                                  \
     do {                                                                                          \
         if ((R).vec && (ENTS) <= 8)                                                               \
-            hipLaunchKernelGGL((KERNEL<4, 8>), GRID, dim3((R).threads), (R).lds, STREAM,          \
+            rk::launch_kernel((KERNEL<4, 8>), GRID, dim3((R).threads), (R).lds, STREAM,          \
                                __VA_ARGS__);                                                      \
         else if ((R).vec)                                                                         \
-            hipLaunchKernelGGL((KERNEL<4, 16>), GRID, dim3((R).threads), (R).lds, STREAM,         \
+            rk::launch_kernel((KERNEL<4, 16>), GRID, dim3((R).threads), (R).lds, STREAM,         \
                                __VA_ARGS__);                                                      \
         else if ((R).reg)                                                                         \
-            hipLaunchKernelGGL((KERNEL<1, 16>), GRID, dim3((R).threads), (R).lds, STREAM,         \
+            rk::launch_kernel((KERNEL<1, 16>), GRID, dim3((R).threads), (R).lds, STREAM,         \
                                __VA_ARGS__);                                                      \
         else                                                                                      \
-            hipLaunchKernelGGL((KERNEL<1, 0>), GRID, dim3((R).threads), (R).lds, STREAM,          \
+            rk::launch_kernel((KERNEL<1, 0>), GRID, dim3((R).threads), (R).lds, STREAM,          \
                                __VA_ARGS__);                                                      \
     } while (0)
 
@@ -461,10 +461,10 @@ extern "C" int rivoli_kv_compress_deposit(const float* kv, const float* score, c
     const size_t pieces = (carry.n + tail.n) / (vec ? 4 : 1);
     const dim3 grid((unsigned)((pieces + 255) / 256));
     if (vec)
-        hipLaunchKernelGGL(rk::kv_compress_deposit_kernel<4>, grid, dim3(256), 0, (hipStream_t)stream, kv, score,
+        rk::launch_kernel(rk::kv_compress_deposit_kernel<4>, grid, dim3(256), 0, (hipStream_t)stream, kv, score,
                            ape, kv_state, score_state, carry, tail);
     else
-        hipLaunchKernelGGL(rk::kv_compress_deposit_kernel<1>, grid, dim3(256), 0, (hipStream_t)stream, kv, score,
+        rk::launch_kernel(rk::kv_compress_deposit_kernel<1>, grid, dim3(256), 0, (hipStream_t)stream, kv, score,
                            ape, kv_state, score_state, carry, tail);
     return rk::launch_status();
 }
@@ -509,7 +509,7 @@ extern "C" int rivoli_kv_compress_decode(float* kv_state, float* score_state,
     const rk::RowLaunch r = rk::row_launch(p, aligned);
     (void)hipGetLastError();
     if (p.coff == 2 && r.vec && p.d <= rk::kCompWideMaxD) {
-        hipLaunchKernelGGL(rk::kv_compress_decode_overlap_kernel, dim3(1),
+        rk::launch_kernel(rk::kv_compress_decode_overlap_kernel, dim3(1),
                            dim3((unsigned)((p.d + rk::kWave - 1) / rk::kWave * rk::kWave)), 0, (hipStream_t)stream,
                            kv_state, score_state, *ff, p, start_pos);
         return rk::launch_status();

@@ -268,12 +268,12 @@ static int gather_paged_launch(const unsigned char* pool, const int* block_table
         if (flat) {                                                                                \
             const long long units = (total_tokens + (ROWS) - 1) / (ROWS) + n_seqs + ((APPEND) ? n_seqs : 0); \
             if (units > 0x7fffffffLL) return 1002;                                                 \
-            hipLaunchKernelGGL((kv_gather_flat_kernel<WV, PTV, FLAT_THREADS, ROWS, APPEND>),       \
+            rk::launch_kernel((kv_gather_flat_kernel<WV, PTV, FLAT_THREADS, ROWS, APPEND>),       \
                                dim3((unsigned)units), dim3(FLAT_THREADS), 0, (hipStream_t)stream, pool, \
                                block_table, seq_lens, cu_seqlens, out, n_seqs, max_blocks_per_seq, \
                                width, page_tokens, n_pages, page_bytes, bad_pages, ap);            \
         } else {                                                                                   \
-            hipLaunchKernelGGL((kv_gather_paged_kernel<WV, PTV, THREADS, ROWS, APPEND>),           \
+            rk::launch_kernel((kv_gather_paged_kernel<WV, PTV, THREADS, ROWS, APPEND>),           \
                                dim3((unsigned)max_blocks_per_seq * parts + ((APPEND) ? 1u : 0u),   \
                                     (unsigned)n_seqs),                                             \
                                dim3(THREADS), 0, (hipStream_t)stream, pool, block_table, seq_lens, \
@@ -355,11 +355,11 @@ int rk::gather_rows_launch(const unsigned char* pool, const int* block_table,
     dim3 grid((unsigned)((nr_cap + kRowsPerGroup - 1) / kRowsPerGroup), (unsigned)n_queries);
     (void)hipGetLastError();
     if (width == 576 && page_tokens == 64) {
-        hipLaunchKernelGGL((kv_gather_rows_kernel<576, 64, 9>), grid, dim3(kGatherThreads), 0,
+        rk::launch_kernel((kv_gather_rows_kernel<576, 64, 9>), grid, dim3(kGatherThreads), 0,
                            (hipStream_t)stream, pool, block_table, rows, n_rows, out, k, nr_cap,
                            max_blocks_per_seq, width, page_tokens, n_pages, page_bytes, bad_rows);
     } else {
-        hipLaunchKernelGGL((kv_gather_rows_kernel<0, 0, 4>), grid, dim3(kGatherThreads), 0,
+        rk::launch_kernel((kv_gather_rows_kernel<0, 0, 4>), grid, dim3(kGatherThreads), 0,
                            (hipStream_t)stream, pool, block_table, rows, n_rows, out, k, nr_cap,
                            max_blocks_per_seq, width, page_tokens, n_pages, page_bytes, bad_rows);
     }
@@ -381,7 +381,7 @@ extern "C" int rivoli_codec_e4m3_dequant_bf16(const unsigned char* codes, float 
     long long blocks = (n + 255) / 256;
     if (blocks > 4096) blocks = 4096;
     (void)hipGetLastError();
-    hipLaunchKernelGGL(rk::e4m3_dequant_bf16_kernel, dim3((unsigned)blocks), dim3(256), 0,
+    rk::launch_kernel(rk::e4m3_dequant_bf16_kernel, dim3((unsigned)blocks), dim3(256), 0,
                        (hipStream_t)stream, codes, scale, out, n);
     return rk::launch_status();
 }

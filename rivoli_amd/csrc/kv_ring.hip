@@ -34,11 +34,11 @@ extern "C" int rivoli_kv_ring_write(const float* kv, float* cache, int win, int 
     (void)hipGetLastError();
     const bool wide = hd % 4 == 0 && ((uintptr_t)kv | (uintptr_t)cache) % 16 == 0;
     if (wide)
-        hipLaunchKernelGGL(rk::kv_ring_write_kernel<rk::u32x4>, dim3((unsigned)n), dim3(256), 0,
+        rk::launch_kernel(rk::kv_ring_write_kernel<rk::u32x4>, dim3((unsigned)n), dim3(256), 0,
                            (hipStream_t)stream, reinterpret_cast<const rk::u32x4*>(kv),
                            reinterpret_cast<rk::u32x4*>(cache), win, hd / 4, first, src_row0);
     else
-        hipLaunchKernelGGL(rk::kv_ring_write_kernel<float>, dim3((unsigned)n), dim3(256), 0,
+        rk::launch_kernel(rk::kv_ring_write_kernel<float>, dim3((unsigned)n), dim3(256), 0,
                            (hipStream_t)stream, kv, cache, win, hd, first, src_row0);
     return rk::launch_status();
 }

@@ -1048,7 +1048,7 @@ static int attend_merge(const AttendArgs& a, const AttendPlan& plan, int n_seqs,
     // heads, 64 records, 27.1 -> 21.9 us, two ragged ones of 8 000 22.3 -> 20.6; 3 x 3 000 of 128 heads 22.8 -> 23.2, 12 x 4 000 27.8 -> 30.9.
     // Past that a call of up to eight work items a sequence has the kernel of few registers: 32 x 4 096 tokens of 128 heads 95.8 -> 94.6.
     const auto merge = [&](auto kernel, unsigned parts) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)a.H, (unsigned)n_seqs, parts), dim3(128), 0, st, a.part_acc, a.part_ml, seq_lens, n_rows,
+        rk::launch_kernel(kernel, dim3((unsigned)a.H, (unsigned)n_seqs, parts), dim3(128), 0, st, a.part_acc, a.part_ml, seq_lens, n_rows,
                            listed ? 1 : 0, max_rows, n_seqs, plan.n_items, a.by_seq, a.H, a.kvl, a.clat);
     };
     if ((long long)a.H * n_seqs <= kAttTargetGroups) merge(mla_attend_combine_kernel<4, 16>, (unsigned)((a.kvl + 127) / 128));
@@ -1073,9 +1073,9 @@ static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_row
             const dim3 grid((unsigned)(((plan.n_items + 7) / 8 * 8) * ((a.H + kWideHeads - 1) / kWideHeads))), block(kWideThreads);
             (void)hipGetLastError();
             constexpr int M = MODE == kDensePaged ? kDense : MODE;
-            if (precise >= 2) hipLaunchKernelGGL((mla_attend_wide_kernel<2, 2, M>), grid, block, 0, st, a);
-            else if (precise == 1) hipLaunchKernelGGL((mla_attend_wide_kernel<2, 1, M>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((mla_attend_wide_kernel<1, 1, M>), grid, block, 0, st, a);
+            if (precise >= 2) rk::launch_kernel((mla_attend_wide_kernel<2, 2, M>), grid, block, 0, st, a);
+            else if (precise == 1) rk::launch_kernel((mla_attend_wide_kernel<2, 1, M>), grid, block, 0, st, a);
+            else rk::launch_kernel((mla_attend_wide_kernel<1, 1, M>), grid, block, 0, st, a);
             return attend_merge(a, plan, n_seqs, max_rows, seq_lens, n_rows, listed, st);
         }
     }
@@ -1089,16 +1089,16 @@ static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_row
         const bool few = route.few;
         const dim3 block(few ? kFewThreads : kH16Threads);
         if constexpr (MODE == kLinear) {  // always the eight waves on a tile (heads16_few)
-            hipLaunchKernelGGL((mla_attend_few_kernel<2, 2, kLinear>), grid, dim3(kFewThreads), 0, st, a);
+            rk::launch_kernel((mla_attend_few_kernel<2, 2, kLinear>), grid, dim3(kFewThreads), 0, st, a);
         } else if (precise >= 2) {
-            if (few) hipLaunchKernelGGL((mla_attend_few_kernel<2, 2, M>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((mla_attend_heads16_kernel<2, 2, M>), grid, block, 0, st, a);
+            if (few) rk::launch_kernel((mla_attend_few_kernel<2, 2, M>), grid, block, 0, st, a);
+            else rk::launch_kernel((mla_attend_heads16_kernel<2, 2, M>), grid, block, 0, st, a);
         } else if (precise == 1) {
-            if (few) hipLaunchKernelGGL((mla_attend_few_kernel<2, 1, M>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((mla_attend_heads16_kernel<2, 1, M>), grid, block, 0, st, a);
+            if (few) rk::launch_kernel((mla_attend_few_kernel<2, 1, M>), grid, block, 0, st, a);
+            else rk::launch_kernel((mla_attend_heads16_kernel<2, 1, M>), grid, block, 0, st, a);
         } else {
-            if (few) hipLaunchKernelGGL((mla_attend_few_kernel<1, 1, M>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((mla_attend_heads16_kernel<1, 1, M>), grid, block, 0, st, a);
+            if (few) rk::launch_kernel((mla_attend_few_kernel<1, 1, M>), grid, block, 0, st, a);
+            else rk::launch_kernel((mla_attend_heads16_kernel<1, 1, M>), grid, block, 0, st, a);
         }
         return attend_merge(a, plan, n_seqs, max_rows, seq_lens, n_rows, listed, st);
     }
@@ -1107,20 +1107,20 @@ static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_row
     (void)hipGetLastError();
     // A cache of other widths than 512 + 64 always runs in the parity mode.
     if (any || MODE == kLinear)
-        hipLaunchKernelGGL((mla_attend_paged_kernel<2, 2, MODE, true>), grid, dim3(kAttThreads), 0, st, a);
+        rk::launch_kernel((mla_attend_paged_kernel<2, 2, MODE, true>), grid, dim3(kAttThreads), 0, st, a);
     else if constexpr (MODE != kLinear) {
         if (precise == 3)
-            hipLaunchKernelGGL((mla_attend_paged_kernel<2, 2, MODE == kSparse ? kSparse : kDense, false, true>), grid,
+            rk::launch_kernel((mla_attend_paged_kernel<2, 2, MODE == kSparse ? kSparse : kDense, false, true>), grid,
                                dim3(kF8Threads), 0, st, a);
         else if (precise == 4)
-            hipLaunchKernelGGL((mla_attend_paged_kernel<3, 2, MODE == kSparse ? kSparse : kDense, false, true>), grid,
+            rk::launch_kernel((mla_attend_paged_kernel<3, 2, MODE == kSparse ? kSparse : kDense, false, true>), grid,
                                dim3(kF8Threads), 0, st, a);
         else if (precise >= 2)
-            hipLaunchKernelGGL((mla_attend_paged_kernel<2, 2, MODE, false>), grid, dim3(kAttThreads), 0, st, a);
+            rk::launch_kernel((mla_attend_paged_kernel<2, 2, MODE, false>), grid, dim3(kAttThreads), 0, st, a);
         else if (precise == 1)
-            hipLaunchKernelGGL((mla_attend_paged_kernel<2, 1, MODE, false>), grid, dim3(kAttThreads), 0, st, a);
+            rk::launch_kernel((mla_attend_paged_kernel<2, 1, MODE, false>), grid, dim3(kAttThreads), 0, st, a);
         else
-            hipLaunchKernelGGL((mla_attend_paged_kernel<1, 1, MODE, false>), grid, dim3(kAttThreads), 0, st, a);
+            rk::launch_kernel((mla_attend_paged_kernel<1, 1, MODE, false>), grid, dim3(kAttThreads), 0, st, a);
     }
     return attend_merge(a, plan, n_seqs, max_rows, seq_lens, n_rows, listed, st);
 }
@@ -1244,7 +1244,7 @@ extern "C" int rivoli_mla_attend(const float* qabs, const float* qrope, const un
     if (!qabs || !qrope || !Lc8 || !Lscale || !Rc || !clat) return 1001;
     (void)hipGetLastError();
     if (rope > kRopeW || (reinterpret_cast<uintptr_t>(Lc8) & 7u) != 0 || H > 64 * 65535) {
-        hipLaunchKernelGGL(mla_attend_rowwise_kernel, dim3((unsigned)((H + 3) / 4)), dim3(256), 0, nullptr, qabs,
+        rk::launch_kernel(mla_attend_rowwise_kernel, dim3((unsigned)((H + 3) / 4)), dim3(256), 0, nullptr, qabs,
                            qrope, Lc8, Lscale, Rc, rows, H, nr, kvl, rope, n_blocks, scale * kLog2e, clat);
         return launch_status();
     }
