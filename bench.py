@@ -642,6 +642,9 @@ def bench_v4_index(a, torch, hip):
     scored = s * n_comp if a.full_scores else int((-(-limit // 64) * 64).clip(max=-(-n_comp // 64) * 64).sum())
     score_flops = 2 * scored * heads * hd                               # one multiply and one add per term
     score_bytes = s * heads * hd * 4 + n_comp * hd * 4 + s * n_comp * 4
+    # the launcher's rule: blocks of a workgroup's share, 192 and more of them by the fp4 instructions
+    share = -(-(-(-n_comp // 64)) // max(1, min(1024 // -(-s // 8), -(-n_comp // 64)))) * 64
+    scorer, peak = ("score_blocks_codes_kernel", 10000.0) if share >= 192 else ("score_blocks_pair_kernel", 2500.0)
     # the timed steps spread the same buffer again and again; the check runs one step on a fresh copy
     q.copy_(q_raw)
     torch.cuda.synchronize()
@@ -660,14 +663,14 @@ def bench_v4_index(a, torch, hip):
            "tokens_per_s": round(s / (ms * 1e-3), 1),
            "kernels": {"f4_rotated_kernel": {"avg_launch_ms": round(per["spread"], 5), "bytes_per_launch": spread_bytes,
                                              "GBps": round(spread_bytes / (per["spread"] * 1e-3) / 1e9, 1)},
-                       "score_blocks_pair_kernel": {"avg_launch_ms": round(per["score"], 5),
+                       scorer: {"avg_launch_ms": round(per["score"], 5),
                                                      "flops_per_launch": score_flops, "bytes_per_launch": score_bytes,
                                                      "TFLOPps": round(score_flops / (per["score"] * 1e-3) / 1e12, 2)}},
-           # rows whose sums are exact in any order, which spread rows are, go through the bf16 matrix
-           # instructions; issue of the reference's roundings, five vector instructions a dot, is the larger half
-           "roofline": {"bound": "mfma", "kernel": "score_blocks_pair_kernel",
-                        "achieved": round(score_flops / (per["score"] * 1e-3) / 1e12, 2), "peak": 2500.0,
-                        "unit": "TFLOP/s", "frac": round(score_flops / (per["score"] * 1e-3) / 2.5e15, 4),
+           # spread rows go through the fp4 matrix instructions, in small shares of the blocks through the bf16 ones;
+           # issue of the reference's roundings, four vector instructions a dot, is what bounds the launch
+           "roofline": {"bound": "mfma", "kernel": scorer,
+                        "achieved": round(score_flops / (per["score"] * 1e-3) / 1e12, 2), "peak": peak,
+                        "unit": "TFLOP/s", "frac": round(score_flops / (per["score"] * 1e-3) / (peak * 1e12), 4),
                         "avg_launch_ms": round(per["score"], 5), "traffic": None}}
     # a decode step of the same layer: one query against the ctx / ratio blocks of a long context
     d_comp = max(a.ctx // ratio, 1)
