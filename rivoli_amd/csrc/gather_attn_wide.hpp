@@ -9,7 +9,8 @@
 // runs every softmax twice), a row is read from LDS once for 32 heads instead of 16, and the two
 // waves of a workgroup (64 heads) share only the staging of its rows. 66.5 KB of LDS: two workgroups a
 // compute unit, one in its prologue or epilogue beside the other's tiles.
-// 8192 queries x 640 slots of 64 heads: 1624 us -> 1045 us. Its 0.94 P of products (the weights' remainders counted)
+// 8192 queries x 640 slots of 64 heads: 1624 us -> 1045 us, of late 1064 -> 1040 with 32 of a tile's 290 vector instructions less (a
+// conversion for two weights, row addresses from scalar registers). Its 0.94 P of products (the weights' remainders counted)
 // run at 0.90 P/s; a large bf16 product sustains 1.40 here, at 1.97 GHz, where power limits it. This kernel is held to
 // 2.15 GHz by the same limit (2.4 before), so what is left to save in cycles is worth half of it in time.
 //
@@ -62,9 +63,10 @@ typedef const __attribute__((address_space(1))) char* global_bytes;
 
 struct GwRow {  // a row on its way: dims 4 lane .. and 256 + 4 lane ..
     f32x4 v[2];
-    __device__ __forceinline__ void ask(global_bytes row, int lane) {
-        v[0] = *(const __attribute__((address_space(1))) f32x4*)(row + 16u * lane);
-        v[1] = *(const __attribute__((address_space(1))) f32x4*)(row + 16u * lane + 1024);
+    __device__ __forceinline__ void ask(global_bytes row, int lane) { ask_at(row, 16u * lane); }
+    __device__ __forceinline__ void ask_at(global_bytes row, uint32_t at) {
+        v[0] = *(const __attribute__((address_space(1))) f32x4*)(row + at);
+        v[1] = *(const __attribute__((address_space(1))) f32x4*)(row + at + 1024);
     }
     __device__ __forceinline__ u32x4 bf16() const {
         return u32x4{pack_bf16x2(v[0].x, v[0].y), pack_bf16x2(v[0].z, v[0].w),
@@ -150,7 +152,11 @@ __device__ __forceinline__ bool gather_attn_wide_pass(const GatherAttnArgs& a, l
     float m_ref = -INFINITY, l_sum = 0.0f;
     const float qs = fabsf(a.qscale);  // its sign is in the query
 
+    // A lane's place in a row, made anew at the head of each stretch without a branch: only within one does the compiler see 32 bits of
+    // it and take a row's address from scalar registers (else a 64-bit addition a row).
+    uint32_t lane_at = 16u * lane;
     for (int tile = 0; tile < list.end_tile; ++tile) {
+        asm volatile("" : "+v"(lane_at));
         const int fetched = list.fetch(n32, tile + 3);
         const int buf = tile & 1;
         const lds_ptr<uint8_t> krb = kr + buf * kGaTileBytes;
@@ -172,7 +178,7 @@ __device__ __forceinline__ bool gather_attn_wide_pass(const GatherAttnArgs& a, l
                     staged.y = pack_bf16x2(r.v[0].z, r.v[0].w);
                     deposit(buf ^ 1, kGwRowsPerWave * wave + i, staged);
                 }
-                if constexpr (part == 3) r.ask(row_at, lane);
+                if constexpr (part == 3) r.ask_at(row_at, lane_at);
             }
         };
 
@@ -232,7 +238,8 @@ __device__ __forceinline__ bool gather_attn_wide_pass(const GatherAttnArgs& a, l
         // p[ks][j] is slot 16 ks + 8 (j >> 2) + 4 g + (j & 3): the score registers in order are the value product's
         // B operand, so a weight never leaves its lane. The denominator sums what the products see, the rounded weights and their
         // remainders: a weight that is most of a head's comes out as 1 whatever its reference maximum.
-        bf16x8 p[2], p_lo[2];
+        asm volatile("" : "+v"(lane_at));
+        u32x4 p[2], p_lo[2];
         float e0 = 0.0f, e1 = 0.0f;
         auto weights = [&](auto ksc, auto pairc, auto partc) {  // two weights, in three steps
             constexpr int ks = decltype(ksc)::value, i = 2 * decltype(pairc)::value, part = decltype(partc)::value;
@@ -240,13 +247,19 @@ __device__ __forceinline__ bool gather_attn_wide_pass(const GatherAttnArgs& a, l
                 e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * ks + i], qs, -mu));  // masked -> 0
                 e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * ks + i + 1], qs, -mu));
             }
-            if constexpr (part == 1) p[ks][i] = (__bf16)e0, p[ks][i + 1] = (__bf16)e1;
+            if constexpr (part == 1) {
+                uint32_t hi = pack_bf16x2(e0, e1);
+                asm("" : "+v"(hi));  // (else a half that is taken out of the pair below is converted once more by itself)
+                p[ks][i / 2] = hi;
+            }
             if constexpr (part == 2) {
-                if (PSPLIT == 2) p_lo[ks][i] = (__bf16)(e0 - (float)p[ks][i]), p_lo[ks][i + 1] = (__bf16)(e1 - (float)p[ks][i + 1]);
+                const uint32_t hi = p[ks][i / 2];
+                const uint32_t lo = PSPLIT == 2 ? pack_bf16x2(e0 - bf16_lo_to_f32(hi), e1 - bf16_hi_to_f32(hi)) : 0u;
+                p_lo[ks][i / 2] = lo;
                 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
                 const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
-                l_sum = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{p[ks][i], p[ks][i + 1]}, ones, l_sum, false);
-                if (PSPLIT == 2) l_sum = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{p_lo[ks][i], p_lo[ks][i + 1]}, ones, l_sum, false);
+                l_sum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, hi), ones, l_sum, false);
+                if (PSPLIT == 2) l_sum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, lo), ones, l_sum, false);
                 asm volatile("" : "+v"(l_sum));  // summed here: sixteen weights kept for later are sixteen registers
             }
         };
@@ -280,10 +293,10 @@ __device__ __forceinline__ bool gather_attn_wide_pass(const GatherAttnArgs& a, l
         };
         unrolled<2 * kGwColTiles>([&](auto nc) {
             constexpr int n = decltype(nc)::value, x = n ^ 1, c = x % kGwColTiles, ks = x / kGwColTiles;
-            o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[x % 6], p[ks], o[c], 0, 0, 0);
+            o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[x % 6], __builtin_bit_cast(bf16x8, p[ks]), o[c], 0, 0, 0);
             beside(std::integral_constant<int, 2 * n>{});
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (PSPLIT == 2) o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[x % 6], p_lo[ks], o[c], 0, 0, 0);
+            if constexpr (PSPLIT == 2) o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[x % 6], __builtin_bit_cast(bf16x8, p_lo[ks]), o[c], 0, 0, 0);
             if constexpr (n + 4 < 2 * kGwColTiles) f[(n + 4) % 6] = value_frag((n + 4) % kGwColTiles, (n + 4) / kGwColTiles);
             beside(std::integral_constant<int, 2 * n + 1>{});
             __builtin_amdgcn_sched_barrier(0);
