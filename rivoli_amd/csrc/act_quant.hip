@@ -150,13 +150,13 @@ static void launch_act_quant(const float* src, float* dst, long long n_blocks, i
     const long long each = (n_pieces + kAqThreads - 1) / kAqThreads;  // workgroups of a piece a thread
     if (each <= kAqFewGroups) {
         rk::launch_kernel((act_quant_kernel<LANES, 1>), dim3((unsigned)each), dim3(kAqThreads), 0, stream, src, dst,
-                           (uint32_t)n_pieces, (uint32_t)nb, (uint32_t)row_stride, nb_inv);
+                          (uint32_t)n_pieces, (uint32_t)nb, (uint32_t)row_stride, nb_inv);
         return;
     }
     long long groups = (each + kAqInFlight - 1) / kAqInFlight;
     if (groups > 256 * 16) groups = 256 * 16;
     rk::launch_kernel((act_quant_kernel<LANES, kAqInFlight>), dim3((unsigned)groups), dim3(kAqThreads), 0, stream,
-                       src, dst, (uint32_t)n_pieces, (uint32_t)nb, (uint32_t)row_stride, nb_inv);
+                      src, dst, (uint32_t)n_pieces, (uint32_t)nb, (uint32_t)row_stride, nb_inv);
 }
 
 }  // namespace rk
@@ -183,8 +183,8 @@ extern "C" int rivoli_act_quant_f8_prefix(const float* src, float* dst, int rows
         default: {
             const long long groups = (n_blocks + rk::kAqThreads - 1) / rk::kAqThreads;
             rk::launch_kernel(rk::act_quant_serial_kernel, dim3((unsigned)groups),
-                               dim3(rk::kAqThreads), 0, st, src, dst, n_blocks, nb, row_stride,
-                               block);
+                              dim3(rk::kAqThreads), 0, st, src, dst, n_blocks, nb, row_stride,
+                              block);
         }
     }
     return rk::launch_status();

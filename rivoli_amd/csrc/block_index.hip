@@ -1137,10 +1137,10 @@ extern "C" int rivoli_act_quant_f4_rotated(float* x, int rows, int d, void* stre
     hipStream_t st = (hipStream_t)stream;
 #define RK_SPREAD(LPR)                                                                                      \
     if (few)                                                                                                \
-        rk::launch_kernel((rk::f4_rotated_kernel<LPR, 1>), grid, block, 0, st, x, (long long)rows, scale); \
+        rk::launch_kernel((rk::f4_rotated_kernel<LPR, 1>), grid, block, 0, st, x, (long long)rows, scale);  \
     else                                                                                                    \
-        rk::launch_kernel((rk::f4_rotated_kernel<LPR, rk::kSpreadInFlight>), grid, block, 0, st, x,        \
-                           (long long)rows, scale)
+        rk::launch_kernel((rk::f4_rotated_kernel<LPR, rk::kSpreadInFlight>), grid, block, 0, st, x,         \
+                          (long long)rows, scale)
     switch (lpr) {
         case 8: RK_SPREAD(8); break;
         case 16: RK_SPREAD(16); break;
@@ -1175,10 +1175,10 @@ static int score_blocks_launch(const float* q, const float* kv, const float* w, 
             // 64s; 16 384 blocks 7.1 us in 64s, 8.5 in 32s)
             if ((long long)s * 2 * groups <= 256)
                 rk::launch_kernel(score_blocks_one_kernel<1>, dim3((unsigned)(((long long)n_comp + 31) / 32), (unsigned)s),
-                                   dim3(kOneThreads), 0, st, q, kv, w, score, s, n_comp, heads, ratio);
+                                  dim3(kOneThreads), 0, st, q, kv, w, score, s, n_comp, heads, ratio);
             else
                 rk::launch_kernel(score_blocks_one_kernel<2>, dim3(groups, (unsigned)s), dim3(kOneThreads), 0, st, q,
-                                   kv, w, score, s, n_comp, heads, ratio);
+                                  kv, w, score, s, n_comp, heads, ratio);
             return launch_status();
         }
         // two workgroups per compute unit at a time; splits of the blocks while the queries alone
@@ -1218,15 +1218,15 @@ static int score_blocks_launch(const float* q, const float* kv, const float* w, 
     if (hd == 128 && aligned16(kv) && (long long)s * c_groups < 256 && heads <= kSplitMaxHeads) {
         const unsigned groups = (unsigned)(((long long)n_comp + kWave - 1) / kWave);
         rk::launch_kernel(index_score_blocks_128_split_kernel, dim3(groups), dim3(kSplitWavesPerGroup * kWave),
-                           (size_t)heads * kWave * sizeof(float), st, q, kv, w, score, s, n_comp, heads, ratio);
+                          (size_t)heads * kWave * sizeof(float), st, q, kv, w, score, s, n_comp, heads, ratio);
         return launch_status();
     }
     if (hd == 128 && aligned16(kv))
         rk::launch_kernel(index_score_blocks_128_kernel, grid, block, 0, st, q, kv, w, score, s, n_comp,
-                           heads, t_per_group, ratio);
+                          heads, t_per_group, ratio);
     else
         rk::launch_kernel(index_score_blocks_any_kernel, grid, block, 0, st, q, kv, w, score, s, n_comp,
-                           heads, hd, t_per_group, ratio);
+                          heads, hd, t_per_group, ratio);
     return launch_status();
 }
 }  // namespace rk

@@ -696,18 +696,18 @@ static int gather_attn_launch(const float* q, const float* kv, const float* sink
         if (rc != 0 || a.n_splits == 1) return rc;  // a split plan has fewer than 256 queries
         if (a.n_splits <= 8)
             rk::launch_kernel(gather_attn_combine_kernel<8>, dim3((unsigned)h, (unsigned)m), dim3(128), 0, stream,
-                               a.part_acc, a.part_ml, sink, a.n_splits, h, o);
+                              a.part_acc, a.part_ml, sink, a.n_splits, h, o);
         else
             rk::launch_kernel(gather_attn_combine_kernel<16>, dim3((unsigned)h, (unsigned)m), dim3(128), 0, stream,
-                               a.part_acc, a.part_ml, sink, a.n_splits, h, o);
+                              a.part_acc, a.part_ml, sink, a.n_splits, h, o);
         return launch_status();
     }
     // the reference launcher's limits, kept (attn.hip:450-458): d within 1024, its LDS budget
     if (d > kGaRowDims * kWave || m > 65535) return 1002;
     if (((size_t)d + (size_t)topk + 256 + 2) * sizeof(float) > 65536) return 1006;
     rk::launch_kernel(gather_attn_rowwise_kernel,
-                       dim3((unsigned)((h + kGaRowThreads / kWave - 1) / (kGaRowThreads / kWave)), (unsigned)m),
-                       dim3(kGaRowThreads), 0, stream, q, kv, sink, idxs, h, d, topk, n_kv, scale, o);
+                      dim3((unsigned)((h + kGaRowThreads / kWave - 1) / (kGaRowThreads / kWave)), (unsigned)m),
+                      dim3(kGaRowThreads), 0, stream, q, kv, sink, idxs, h, d, topk, n_kv, scale, o);
     return launch_status();
 }
 

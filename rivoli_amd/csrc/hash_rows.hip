@@ -73,9 +73,9 @@ extern "C" int rivoli_hash_rows(const float* x, int n, int stride, unsigned long
     // Grid-stride over samples with a capped grid: one atomic per workgroup, so the cap
     // bounds the atomics whatever n is; 2048 workgroups is 8 per CU on 256 CUs.
     rk::launch_kernel(hash_rows_kernel, dim3(capped_blocks(samples, kHashThreads, 2048)),
-                       dim3(kHashThreads), 0, (hipStream_t)stream,
-                       reinterpret_cast<const uint32_t*>(x), (long long)n, (long long)stride,
-                       i_base, out);
+                      dim3(kHashThreads), 0, (hipStream_t)stream,
+                      reinterpret_cast<const uint32_t*>(x), (long long)n, (long long)stride,
+                      i_base, out);
     return launch_status();
 }
 
@@ -84,7 +84,7 @@ extern "C" int rivoli_codec_e4m3_encode(const float* x, unsigned char* out, long
     if (!x || !out || n <= 0) return 1001;
     (void)hipGetLastError();
     rk::launch_kernel(rk::e4m3_encode_kernel, dim3(rk::capped_blocks(n, 256, 4096)), dim3(256), 0,
-                       (hipStream_t)stream, x, out, n);
+                      (hipStream_t)stream, x, out, n);
     return rk::launch_status();
 }
 
@@ -93,6 +93,6 @@ extern "C" int rivoli_codec_bf16_encode(const float* x, unsigned short* out, lon
     if (!x || !out || n <= 0) return 1001;
     (void)hipGetLastError();
     rk::launch_kernel(rk::bf16_encode_kernel, dim3(rk::capped_blocks(n, 256, 4096)), dim3(256), 0,
-                       (hipStream_t)stream, x, out, n);
+                      (hipStream_t)stream, x, out, n);
     return rk::launch_status();
 }

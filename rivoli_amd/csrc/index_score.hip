@@ -409,18 +409,18 @@ static int index_score_launch(const float* q, const float* w, const unsigned sho
         const size_t q_bytes = (size_t)nact * hd * sizeof(float);
         const int q_in_lds = q_bytes <= 65536;
         rk::launch_kernel(index_score_plain_kernel,
-                           dim3((unsigned)((nt + kPlainTokensPerGroup - 1) / kPlainTokensPerGroup),
+                          dim3((unsigned)((nt + kPlainTokensPerGroup - 1) / kPlainTokensPerGroup),
                                 (unsigned)n_queries),
-                           dim3(kScoreThreads), q_in_lds ? q_bytes : 0, stream, q, w, kpool, block_table,
-                           nts, heads, max_blocks_per_seq, stride, nt, nh, nact, hd, page_tokens, n_pages,
-                           wscale, dscale, scores, ws, ws_stride, q_in_lds);
+                          dim3(kScoreThreads), q_in_lds ? q_bytes : 0, stream, q, w, kpool, block_table,
+                          nts, heads, max_blocks_per_seq, stride, nt, nh, nact, hd, page_tokens, n_pages,
+                          wscale, dscale, scores, ws, ws_stride, q_in_lds);
         return launch_status();
     }
     const bool one_round = (long long)grid.x * grid.y <= kScoreTargetGroups;
 #define RK_SCORE(RBV, HDV, FIRST)                                                                  \
-    rk::launch_kernel((index_score_kernel<RBV, HDV, FIRST>), grid, dim3(kScoreThreads), 0, stream, \
-                       q, w, kpool, block_table, nts, heads, max_blocks_per_seq, stride, nt, nh,   \
-                       nact, hd, page_tokens, n_pages, wscale, dscale, scores, ws, ws_stride, blocks)
+    rk::launch_kernel((index_score_kernel<RBV, HDV, FIRST>), grid, dim3(kScoreThreads), 0, stream,  \
+                      q, w, kpool, block_table, nts, heads, max_blocks_per_seq, stride, nt, nh,    \
+                      nact, hd, page_tokens, n_pages, wscale, dscale, scores, ws, ws_stride, blocks)
 #define RK_SCORE_HD(RBV, FIRST) \
     if (hd == 128) RK_SCORE(RBV, 128, FIRST); else RK_SCORE(RBV, 0, FIRST)
     if (one_round) {
@@ -478,7 +478,7 @@ extern "C" int rivoli_index_append_paged(const float* k, const int* slot_mapping
     const long long work = (long long)n_tokens * (hd >> 3);
     (void)hipGetLastError();
     rk::launch_kernel(rk::index_append_paged_kernel, dim3((unsigned)((work + 255) / 256)),
-                       dim3(256), 0, (hipStream_t)stream, k, slot_mapping, kpool, n_tokens, hd,
-                       (long long)n_pages * page_tokens, bad_slots);
+                      dim3(256), 0, (hipStream_t)stream, k, slot_mapping, kpool, n_tokens, hd,
+                      (long long)n_pages * page_tokens, bad_slots);
     return rk::launch_status();
 }

@@ -1390,17 +1390,17 @@ static void finish_bits_launch_shape(bool fixed, int n_segs, int kmax, int n_que
     if (n_segs <= 16) {
         if (fixed)
             rk::launch_kernel((topk_finish_bits_kernel<576, 64, THREADS, SLOTS, kShort>), grid, block,
-                               0, stream, args...);
+                              0, stream, args...);
         else
             rk::launch_kernel((topk_finish_bits_kernel<0, 0, THREADS, SLOTS, kShort>), grid, block, 0,
-                               stream, args...);
+                              stream, args...);
     } else {
         if (fixed)
             rk::launch_kernel((topk_finish_bits_kernel<576, 64, THREADS, SLOTS, kLong>), grid, block,
-                               0, stream, args...);
+                              0, stream, args...);
         else
             rk::launch_kernel((topk_finish_bits_kernel<0, 0, THREADS, SLOTS, kLong>), grid, block, 0,
-                               stream, args...);
+                              stream, args...);
     }
 }
 template <class... Args>
@@ -1427,13 +1427,13 @@ static int index_topk_launch(const float* scores, int n_queries, int stride, con
         const dim3 seg_grid((unsigned)n_segs, (unsigned)n_queries), block(kSplitThreads);
         if (!hist_ready)
             rk::launch_kernel(topk_hist_kernel, seg_grid, block, 0, stream, scores, stride, nts, nt,
-                               ws, ws_stride);
+                              ws, ws_stride);
         const int kmax = k < nt ? k : nt;
         const size_t page_bytes = (size_t)ga.page_tokens * ga.width + (size_t)ga.page_tokens * 4;
         const bool fixed = ga.pool && ga.width == 576 && ga.page_tokens == 64;
         if (n_segs <= kBitsMaxSegs) {
             rk::launch_kernel(topk_cand_kernel<true>, seg_grid, block, 0, stream, scores, stride,
-                               nts, nt, k, ws, ws_stride, n_segs);
+                              nts, nt, k, ws, ws_stride, n_segs);
             finish_bits_launch(fixed, n_segs, kmax, n_queries, stream, nts, nt, k, rows, ws,
                                ws_stride, n_segs, ga.pool, ga.block_table, ga.out,
                                ga.max_blocks_per_seq, ga.width, ga.page_tokens, ga.n_pages,
@@ -1441,25 +1441,25 @@ static int index_topk_launch(const float* scores, int n_queries, int stride, con
             return launch_status();
         }
         rk::launch_kernel(topk_cand_kernel<false>, seg_grid, block, 0, stream, scores, stride, nts,
-                           nt, k, ws, ws_stride, n_segs);
+                          nt, k, ws, ws_stride, n_segs);
         const dim3 out_grid((unsigned)((kmax + kSlotsPerGroup - 1) / kSlotsPerGroup),
                             (unsigned)n_queries);
         if (fixed)
             rk::launch_kernel((topk_finish_kernel<576, 64>), out_grid, block, 0, stream, scores,
-                               stride, nts, nt, k, rows, ws, ws_stride, n_segs, ga.pool,
-                               ga.block_table, ga.out, ga.max_blocks_per_seq, ga.width,
-                               ga.page_tokens, ga.n_pages, page_bytes, ga.bad_rows);
+                              stride, nts, nt, k, rows, ws, ws_stride, n_segs, ga.pool,
+                              ga.block_table, ga.out, ga.max_blocks_per_seq, ga.width,
+                              ga.page_tokens, ga.n_pages, page_bytes, ga.bad_rows);
         else
             rk::launch_kernel((topk_finish_kernel<0, 0>), out_grid, block, 0, stream, scores, stride,
-                               nts, nt, k, rows, ws, ws_stride, n_segs, ga.pool, ga.block_table,
-                               ga.out, ga.max_blocks_per_seq, ga.width, ga.page_tokens, ga.n_pages,
-                               page_bytes, ga.bad_rows);
+                              nts, nt, k, rows, ws, ws_stride, n_segs, ga.pool, ga.block_table,
+                              ga.out, ga.max_blocks_per_seq, ga.width, ga.page_tokens, ga.n_pages,
+                              page_bytes, ga.bad_rows);
         return launch_status();
     }
     dim3 grid((unsigned)n_queries), block(kTopkThreads);
 #define RK_TOPK_FEW(I)                                                                              \
-    rk::launch_kernel(index_topk_few_kernel<I>, grid, dim3(kSfThreads), 0, stream, scores, stride, \
-                       nts, nt, k, rows)
+    rk::launch_kernel(index_topk_few_kernel<I>, grid, dim3(kSfThreads), 0, stream, scores, stride,  \
+                      nts, nt, k, rows)
     if (nt <= kSfThreads)
         RK_TOPK_FEW(1);
     else if (nt <= kSfThreads * 2)
@@ -1471,10 +1471,10 @@ static int index_topk_launch(const float* scores, int n_queries, int stride, con
 #undef RK_TOPK_FEW
     else if (nt <= kTopkThreads * 64)
         rk::launch_kernel(index_topk_kernel<64>, grid, block, 0, stream, scores, stride,
-                           nts, nt, k, rows);
+                          nts, nt, k, rows);
     else
         rk::launch_kernel(index_topk_kernel<0>, grid, block, 0, stream, scores, stride,
-                           nts, nt, k, rows);
+                          nts, nt, k, rows);
     return launch_status();
 }
 
@@ -1940,14 +1940,14 @@ static int block_select_launch(const float* scores, int rows, int n_comp, int ra
     (void)hipGetLastError();
     const dim3 grid((unsigned)rows);
 #define RK_BISECT(WV, I)                                                                     \
-    rk::launch_kernel((block_select_bisect_kernel<WV, I>), grid, dim3(WV* kWave), 0, stream, \
-                       scores, n_comp, ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
+    rk::launch_kernel((block_select_bisect_kernel<WV, I>), grid, dim3(WV* kWave), 0, stream,  \
+                      scores, n_comp, ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
 #define RK_FEW(I)                                                                                             \
-    rk::launch_kernel((block_select_few_kernel<I>), grid, dim3(kSfThreads), 0, stream, scores, n_comp, ratio, \
-                       prefill ? 1 : 0, k, offset, out, out_stride, window)
+    rk::launch_kernel((block_select_few_kernel<I>), grid, dim3(kSfThreads), 0, stream, scores, n_comp, ratio,  \
+                      prefill ? 1 : 0, k, offset, out, out_stride, window)
 #define RK_SELECT(T, I)                                                                       \
-    rk::launch_kernel((block_select_kernel<T, I>), grid, dim3(T), 0, stream, scores, n_comp, \
-                       ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
+    rk::launch_kernel((block_select_kernel<T, I>), grid, dim3(T), 0, stream, scores, n_comp,  \
+                      ratio, prefill ? 1 : 0, k, offset, out, out_stride, window)
     // Few rows (decode: one) leave the chip to one workgroup each, and a row's time is its longest wave's: sixteen waves,
     // as few keys a lane as there are. One row of 8192 (sums of a ReLU): in four waves 17.8 us, by leading bits and
     // bisection in sixteen 10.6, over the range that the keys take 5.8; of 1000 7.6 -> 4.
@@ -2020,7 +2020,7 @@ static int sel_fill_launch(const SelShape& s, int win, int ratio, int start_pos,
     const dim3 grid((unsigned)s.rows, (unsigned)((s.win_cols + n_pos + 255) / 256));
     if (grid.y > 65535) return 1002;
     rk::launch_kernel(sel_fill_kernel, grid, dim3(256), 0, stream, win, ratio, start_pos, s.win_cols,
-                       n_pos, s.offset, cols, out);
+                      n_pos, s.offset, cols, out);
     return launch_status();
 }
 
@@ -2189,7 +2189,7 @@ extern "C" int rivoli_dsa_select_gather_paged_noalloc(const float* scores, int n
         if (code) return code;
         (void)hipGetLastError();
         rk::launch_kernel(topk_ws_clear_kernel, dim3((unsigned)n_queries), dim3(kSplitThreads), 0,
-                           (hipStream_t)stream, ws, ws_stride);
+                          (hipStream_t)stream, ws, ws_stride);
         const int launched = launch_status();
         if (launched) return launched;
     }

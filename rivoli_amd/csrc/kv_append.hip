@@ -334,7 +334,7 @@ static int append_kv_rows_launch(const float* latent, const float* rope, unsigne
     (void)hipGetLastError();
     const auto launch = [&](auto kernel, int tokens) {
         rk::launch_kernel(kernel, dim3((unsigned)(((long long)n_tokens + tokens - 1) / tokens)), dim3(kAppendWaves * kWave), 0, stream,
-                           latent, rope, lc8, lscale, rc, pos0, n_tokens, kvl, ropn, n_blocks);
+                          latent, rope, lc8, lscale, rc, pos0, n_tokens, kvl, ropn, n_blocks);
     };
     if (n_tokens > kAppendShared || kvl == 128) launch(append_kv_rows_kernel<1>, kAppendWaves);
     else launch(append_kv_rows_kernel<kAppendWaves>, 1);
@@ -366,10 +366,10 @@ extern "C" int rivoli_kv_append_paged(const unsigned short* rows, const int* slo
         // chunks per thread by size (8192 tokens: 5.5 / 5.25 / 5.8 us with 1 / 2 / 4; 16384 tokens:
         // 8.4 / 8.0 / 7.7; 4096 tokens: 4.15 / 4.4 with 1 / 2)
 #define RK_WIDE(J)                                                                                     \
-    rk::launch_kernel(kv_append_paged_wide_kernel<J>,                                                 \
-                       dim3((unsigned)((n_tokens + kRowsPerWave * (J) - 1) / (kRowsPerWave * (J)))),   \
-                       dim3(kWideThreads), 0, (hipStream_t)stream, rows, slot_mapping, pool, n_tokens, \
-                       page_tokens, n_slots, page_bytes, bad_slots)
+    rk::launch_kernel(kv_append_paged_wide_kernel<J>,                                                  \
+                      dim3((unsigned)((n_tokens + kRowsPerWave * (J) - 1) / (kRowsPerWave * (J)))),    \
+                      dim3(kWideThreads), 0, (hipStream_t)stream, rows, slot_mapping, pool, n_tokens,  \
+                      page_tokens, n_slots, page_bytes, bad_slots)
         if (n_tokens < 6144)
             RK_WIDE(1);
         else if (n_tokens < 12288)
@@ -384,24 +384,24 @@ extern "C" int rivoli_kv_append_paged(const unsigned short* rows, const int* slo
         dim3 block(kAppendWaves * kWave);
         if (width <= 512)
             rk::launch_kernel(kv_append_paged_token_kernel<1>, grid, block, 0,
-                               (hipStream_t)stream, rows, slot_mapping, pool, n_tokens, width,
-                               page_tokens, n_slots, page_bytes, bad_slots);
+                              (hipStream_t)stream, rows, slot_mapping, pool, n_tokens, width,
+                              page_tokens, n_slots, page_bytes, bad_slots);
         else
             rk::launch_kernel(kv_append_paged_token_kernel<2>, grid, block, 0,
-                               (hipStream_t)stream, rows, slot_mapping, pool, n_tokens, width,
-                               page_tokens, n_slots, page_bytes, bad_slots);
+                              (hipStream_t)stream, rows, slot_mapping, pool, n_tokens, width,
+                              page_tokens, n_slots, page_bytes, bad_slots);
         return launch_status();
     }
     dim3 grid((unsigned)((n_tokens + kRowsPerWave - 1) / kRowsPerWave));
     dim3 block(kWave);
     if (width == 576) {
         rk::launch_kernel(kv_append_paged_kernel<72>, grid, block, 0, (hipStream_t)stream, rows,
-                           slot_mapping, pool, n_tokens, width, page_tokens, n_slots, page_bytes,
-                           bad_slots);
+                          slot_mapping, pool, n_tokens, width, page_tokens, n_slots, page_bytes,
+                          bad_slots);
     } else {
         rk::launch_kernel(kv_append_paged_kernel<0>, grid, block, 0, (hipStream_t)stream, rows,
-                           slot_mapping, pool, n_tokens, width, page_tokens, n_slots, page_bytes,
-                           bad_slots);
+                          slot_mapping, pool, n_tokens, width, page_tokens, n_slots, page_bytes,
+                          bad_slots);
     }
     return launch_status();
 }
@@ -424,7 +424,7 @@ extern "C" int rivoli_index_append(const float* k, unsigned short* kcache, int p
     if (hd <= 0 || pos < 0 || !k || !kcache) return 1001;
     (void)hipGetLastError();
     rk::launch_kernel(rk::index_append_kernel, dim3((unsigned)((hd + 255) / 256)), dim3(256), 0,
-                       nullptr, k, kcache, pos, hd);
+                      nullptr, k, kcache, pos, hd);
     return rk::launch_status();
 }
 

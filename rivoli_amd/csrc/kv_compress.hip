@@ -422,17 +422,17 @@ static RowLaunch row_launch(const CompGeom& p, bool aligned) {
 #define RK_COMPRESS_DISPATCH(KERNEL, GRID, R, ENTS, STREAM, ...)                                  \
     do {                                                                                          \
         if ((R).vec && (ENTS) <= 8)                                                               \
-            rk::launch_kernel((KERNEL<4, 8>), GRID, dim3((R).threads), (R).lds, STREAM,          \
-                               __VA_ARGS__);                                                      \
+            rk::launch_kernel((KERNEL<4, 8>), GRID, dim3((R).threads), (R).lds, STREAM,           \
+                              __VA_ARGS__);                                                       \
         else if ((R).vec)                                                                         \
-            rk::launch_kernel((KERNEL<4, 16>), GRID, dim3((R).threads), (R).lds, STREAM,         \
-                               __VA_ARGS__);                                                      \
+            rk::launch_kernel((KERNEL<4, 16>), GRID, dim3((R).threads), (R).lds, STREAM,          \
+                              __VA_ARGS__);                                                       \
         else if ((R).reg)                                                                         \
-            rk::launch_kernel((KERNEL<1, 16>), GRID, dim3((R).threads), (R).lds, STREAM,         \
-                               __VA_ARGS__);                                                      \
+            rk::launch_kernel((KERNEL<1, 16>), GRID, dim3((R).threads), (R).lds, STREAM,          \
+                              __VA_ARGS__);                                                       \
         else                                                                                      \
-            rk::launch_kernel((KERNEL<1, 0>), GRID, dim3((R).threads), (R).lds, STREAM,          \
-                               __VA_ARGS__);                                                      \
+            rk::launch_kernel((KERNEL<1, 0>), GRID, dim3((R).threads), (R).lds, STREAM,           \
+                              __VA_ARGS__);                                                       \
     } while (0)
 
 }  // namespace rk
@@ -462,10 +462,10 @@ extern "C" int rivoli_kv_compress_deposit(const float* kv, const float* score, c
     const dim3 grid((unsigned)((pieces + 255) / 256));
     if (vec)
         rk::launch_kernel(rk::kv_compress_deposit_kernel<4>, grid, dim3(256), 0, (hipStream_t)stream, kv, score,
-                           ape, kv_state, score_state, carry, tail);
+                          ape, kv_state, score_state, carry, tail);
     else
         rk::launch_kernel(rk::kv_compress_deposit_kernel<1>, grid, dim3(256), 0, (hipStream_t)stream, kv, score,
-                           ape, kv_state, score_state, carry, tail);
+                          ape, kv_state, score_state, carry, tail);
     return rk::launch_status();
 }
 
@@ -510,8 +510,8 @@ extern "C" int rivoli_kv_compress_decode(float* kv_state, float* score_state,
     (void)hipGetLastError();
     if (p.coff == 2 && r.vec && p.d <= rk::kCompWideMaxD) {
         rk::launch_kernel(rk::kv_compress_decode_overlap_kernel, dim3(1),
-                           dim3((unsigned)((p.d + rk::kWave - 1) / rk::kWave * rk::kWave)), 0, (hipStream_t)stream,
-                           kv_state, score_state, *ff, p, start_pos);
+                          dim3((unsigned)((p.d + rk::kWave - 1) / rk::kWave * rk::kWave)), 0, (hipStream_t)stream,
+                          kv_state, score_state, *ff, p, start_pos);
         return rk::launch_status();
     }
     RK_COMPRESS_DISPATCH(rk::kv_compress_decode_kernel, dim3(1), r, p.ents, (hipStream_t)stream,

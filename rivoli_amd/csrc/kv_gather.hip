@@ -268,17 +268,17 @@ static int gather_paged_launch(const unsigned char* pool, const int* block_table
         if (flat) {                                                                                \
             const long long units = (total_tokens + (ROWS) - 1) / (ROWS) + n_seqs + ((APPEND) ? n_seqs : 0); \
             if (units > 0x7fffffffLL) return 1002;                                                 \
-            rk::launch_kernel((kv_gather_flat_kernel<WV, PTV, FLAT_THREADS, ROWS, APPEND>),       \
-                               dim3((unsigned)units), dim3(FLAT_THREADS), 0, (hipStream_t)stream, pool, \
-                               block_table, seq_lens, cu_seqlens, out, n_seqs, max_blocks_per_seq, \
-                               width, page_tokens, n_pages, page_bytes, bad_pages, ap);            \
+            rk::launch_kernel((kv_gather_flat_kernel<WV, PTV, FLAT_THREADS, ROWS, APPEND>),        \
+                              dim3((unsigned)units), dim3(FLAT_THREADS), 0, (hipStream_t)stream, pool,  \
+                              block_table, seq_lens, cu_seqlens, out, n_seqs, max_blocks_per_seq,  \
+                              width, page_tokens, n_pages, page_bytes, bad_pages, ap);             \
         } else {                                                                                   \
-            rk::launch_kernel((kv_gather_paged_kernel<WV, PTV, THREADS, ROWS, APPEND>),           \
-                               dim3((unsigned)max_blocks_per_seq * parts + ((APPEND) ? 1u : 0u),   \
+            rk::launch_kernel((kv_gather_paged_kernel<WV, PTV, THREADS, ROWS, APPEND>),            \
+                              dim3((unsigned)max_blocks_per_seq * parts + ((APPEND) ? 1u : 0u),    \
                                     (unsigned)n_seqs),                                             \
-                               dim3(THREADS), 0, (hipStream_t)stream, pool, block_table, seq_lens, \
-                               cu_seqlens, out, max_blocks_per_seq, width, page_tokens, n_pages,   \
-                               page_bytes, bad_pages, ap);                                         \
+                              dim3(THREADS), 0, (hipStream_t)stream, pool, block_table, seq_lens,  \
+                              cu_seqlens, out, max_blocks_per_seq, width, page_tokens, n_pages,    \
+                              page_bytes, bad_pages, ap);                                          \
         }                                                                                          \
     } while (0)
 #define RK_GATHER(WV, PTV, THREADS, FLAT_THREADS, ROWS)                                            \
@@ -356,12 +356,12 @@ int rk::gather_rows_launch(const unsigned char* pool, const int* block_table,
     (void)hipGetLastError();
     if (width == 576 && page_tokens == 64) {
         rk::launch_kernel((kv_gather_rows_kernel<576, 64, 9>), grid, dim3(kGatherThreads), 0,
-                           (hipStream_t)stream, pool, block_table, rows, n_rows, out, k, nr_cap,
-                           max_blocks_per_seq, width, page_tokens, n_pages, page_bytes, bad_rows);
+                          (hipStream_t)stream, pool, block_table, rows, n_rows, out, k, nr_cap,
+                          max_blocks_per_seq, width, page_tokens, n_pages, page_bytes, bad_rows);
     } else {
         rk::launch_kernel((kv_gather_rows_kernel<0, 0, 4>), grid, dim3(kGatherThreads), 0,
-                           (hipStream_t)stream, pool, block_table, rows, n_rows, out, k, nr_cap,
-                           max_blocks_per_seq, width, page_tokens, n_pages, page_bytes, bad_rows);
+                          (hipStream_t)stream, pool, block_table, rows, n_rows, out, k, nr_cap,
+                          max_blocks_per_seq, width, page_tokens, n_pages, page_bytes, bad_rows);
     }
     return launch_status();
 }
@@ -382,6 +382,6 @@ extern "C" int rivoli_codec_e4m3_dequant_bf16(const unsigned char* codes, float 
     if (blocks > 4096) blocks = 4096;
     (void)hipGetLastError();
     rk::launch_kernel(rk::e4m3_dequant_bf16_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                       (hipStream_t)stream, codes, scale, out, n);
+                      (hipStream_t)stream, codes, scale, out, n);
     return rk::launch_status();
 }

@@ -35,10 +35,10 @@ extern "C" int rivoli_kv_ring_write(const float* kv, float* cache, int win, int 
     const bool wide = hd % 4 == 0 && ((uintptr_t)kv | (uintptr_t)cache) % 16 == 0;
     if (wide)
         rk::launch_kernel(rk::kv_ring_write_kernel<rk::u32x4>, dim3((unsigned)n), dim3(256), 0,
-                           (hipStream_t)stream, reinterpret_cast<const rk::u32x4*>(kv),
-                           reinterpret_cast<rk::u32x4*>(cache), win, hd / 4, first, src_row0);
+                          (hipStream_t)stream, reinterpret_cast<const rk::u32x4*>(kv),
+                          reinterpret_cast<rk::u32x4*>(cache), win, hd / 4, first, src_row0);
     else
         rk::launch_kernel(rk::kv_ring_write_kernel<float>, dim3((unsigned)n), dim3(256), 0,
-                           (hipStream_t)stream, kv, cache, win, hd, first, src_row0);
+                          (hipStream_t)stream, kv, cache, win, hd, first, src_row0);
     return rk::launch_status();
 }

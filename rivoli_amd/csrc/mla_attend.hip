@@ -1049,7 +1049,7 @@ static int attend_merge(const AttendArgs& a, const AttendPlan& plan, int n_seqs,
     // Past that a call of up to eight work items a sequence has the kernel of few registers: 32 x 4 096 tokens of 128 heads 95.8 -> 94.6.
     const auto merge = [&](auto kernel, unsigned parts) {
         rk::launch_kernel(kernel, dim3((unsigned)a.H, (unsigned)n_seqs, parts), dim3(128), 0, st, a.part_acc, a.part_ml, seq_lens, n_rows,
-                           listed ? 1 : 0, max_rows, n_seqs, plan.n_items, a.by_seq, a.H, a.kvl, a.clat);
+                          listed ? 1 : 0, max_rows, n_seqs, plan.n_items, a.by_seq, a.H, a.kvl, a.clat);
     };
     if ((long long)a.H * n_seqs <= kAttTargetGroups) merge(mla_attend_combine_kernel<4, 16>, (unsigned)((a.kvl + 127) / 128));
     else if (plan.n_items <= 8 * n_seqs) merge(mla_attend_combine_kernel<1, 8>, 1u);
@@ -1111,10 +1111,10 @@ static int attend_launch(AttendArgs& a, AttendPlan plan, int n_seqs, int max_row
     else if constexpr (MODE != kLinear) {
         if (precise == 3)
             rk::launch_kernel((mla_attend_paged_kernel<2, 2, MODE == kSparse ? kSparse : kDense, false, true>), grid,
-                               dim3(kF8Threads), 0, st, a);
+                              dim3(kF8Threads), 0, st, a);
         else if (precise == 4)
             rk::launch_kernel((mla_attend_paged_kernel<3, 2, MODE == kSparse ? kSparse : kDense, false, true>), grid,
-                               dim3(kF8Threads), 0, st, a);
+                              dim3(kF8Threads), 0, st, a);
         else if (precise >= 2)
             rk::launch_kernel((mla_attend_paged_kernel<2, 2, MODE, false>), grid, dim3(kAttThreads), 0, st, a);
         else if (precise == 1)
@@ -1245,7 +1245,7 @@ extern "C" int rivoli_mla_attend(const float* qabs, const float* qrope, const un
     (void)hipGetLastError();
     if (rope > kRopeW || (reinterpret_cast<uintptr_t>(Lc8) & 7u) != 0 || H > 64 * 65535) {
         rk::launch_kernel(mla_attend_rowwise_kernel, dim3((unsigned)((H + 3) / 4)), dim3(256), 0, nullptr, qabs,
-                           qrope, Lc8, Lscale, Rc, rows, H, nr, kvl, rope, n_blocks, scale * kLog2e, clat);
+                          qrope, Lc8, Lscale, Rc, rows, H, nr, kvl, rope, n_blocks, scale * kLog2e, clat);
         return launch_status();
     }
     const AttendPlan plan = linear_plan(H, nr, (int)((size_t)kRefMaxSplits * ((size_t)kvl + 2) / (kKvl + 2)), partial != nullptr);
