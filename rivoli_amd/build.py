@@ -64,24 +64,28 @@ def offload_arch() -> str:
     return os.environ.get("RIVOLI_OFFLOAD_ARCH", "gfx950")
 
 
+def compile_command(k: str) -> list[str]:
+    """The compiler and every flag that source file `k` is compiled with; what to make of it (-c, -S) is the caller's."""
+    return [hipcc(), f"--offload-arch={offload_arch()}", "-O3", "-std=c++17", "-fPIC",
+            # packed-f32 instructions stay off: plain f32 math only
+            "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+            # a kernel's first arguments are in scalar registers when it starts: the short kernels of a token's
+            # chain are spared a round trip to memory each
+            "-mllvm", "-amdgpu-kernarg-preload-count=14",
+            "-I", os.path.join(os.path.dirname(CSRC), "..", "include")] + EXTRA_FLAGS.get(k, [])
+
+
 def build_kernels(verbose: bool = False) -> str:
     """Every source to an object of its own (in parallel, under build/), then one link."""
     from concurrent.futures import ThreadPoolExecutor
 
     objdir = os.path.join(CSRC, "build")
     os.makedirs(objdir, exist_ok=True)
-    common = [hipcc(), f"--offload-arch={offload_arch()}", "-O3", "-std=c++17", "-fPIC",
-              # packed-f32 instructions stay off: plain f32 math only
-              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-              # a kernel's first arguments are in scalar registers when it starts: the short kernels of a token's
-              # chain are spared a round trip to memory each
-              "-mllvm", "-amdgpu-kernarg-preload-count=14",
-              "-I", os.path.join(os.path.dirname(CSRC), "..", "include")]
 
     def compile_one(k: str) -> str:
         obj = os.path.join(objdir, k.replace(".hip", ".o"))
         report = ["-Rpass-analysis=kernel-resource-usage"] if k in NO_SCRATCH else []
-        res = subprocess.run(common + EXTRA_FLAGS.get(k, []) + report + ["-c", os.path.join(CSRC, k), "-o", obj],
+        res = subprocess.run(compile_command(k) + report + ["-c", os.path.join(CSRC, k), "-o", obj],
                              capture_output=True, text=True)
         if res.returncode != 0 or (verbose and not report):
             sys.stderr.write(res.stdout + res.stderr)

@@ -18,15 +18,31 @@ import pytest
 
 from rivoli_amd import build
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+def test_the_build_compiles_with_the_flags_that_these_tests_compile_with(monkeypatch):
+    """The tests below ask build.compile_command for their flags: a flag that only the build had would make another program of
+    what is shipped than of what they look at."""
+    ran = []
+
+    def run(cmd, **_):
+        ran.append(cmd)
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+
+    monkeypatch.setattr(build.subprocess, "run", run)
+    monkeypatch.setattr(build, "check_resources", lambda k, report: None)
+    build.build_kernels()
+    compiles = [cmd for cmd in ran if "-c" in cmd]
+    assert sorted(os.path.basename(cmd[cmd.index("-c") + 1]) for cmd in compiles) == sorted(build.KERNELS)
+    for cmd in compiles:
+        flags = cmd[:cmd.index("-c")]
+        own = build.compile_command(os.path.basename(cmd[cmd.index("-c") + 1]))
+        assert flags[:len(own)] == own and set(flags[len(own):]) <= {"-Rpass-analysis=kernel-resource-usage"}
 
 
 @pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
 def test_eight_bit_attention_kernels_do_not_spill(tmp_path):
     src = os.path.join(build.CSRC, "mla_attend.hip")
-    cmd = [build.hipcc(), f"--offload-arch={build.offload_arch()}", "-O3", "-std=c++17", "-fPIC",
-           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-           "-I", os.path.join(ROOT, "include")] + build.EXTRA_FLAGS.get("mla_attend.hip", []) + \
+    cmd = build.compile_command("mla_attend.hip") + \
           ["-Rpass-analysis=kernel-resource-usage", "-c", src, "-o", str(tmp_path / "m.o")]
     res = subprocess.run(cmd, capture_output=True, text=True)
     assert res.returncode == 0, res.stderr[-2000:]
@@ -49,9 +65,7 @@ def test_eight_bit_attention_kernels_do_not_spill(tmp_path):
 
 def _resource_blocks(src_name):
     src = os.path.join(build.CSRC, src_name)
-    cmd = [build.hipcc(), f"--offload-arch={build.offload_arch()}", "-O3", "-std=c++17", "-fPIC",
-           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-           "-I", os.path.join(ROOT, "include")] + build.EXTRA_FLAGS.get(src_name, []) + \
+    cmd = build.compile_command(src_name) + \
           ["-Rpass-analysis=kernel-resource-usage", "-c", src, "-o", os.devnull]
     res = subprocess.run(cmd, capture_output=True, text=True)
     assert res.returncode == 0, res.stderr[-2000:]
@@ -181,9 +195,7 @@ def test_list_attention_of_32_heads_a_wave_keeps_its_operands_apart(tmp_path):
     the earliest. Reads the listing; and no block with products may touch scratch memory, where the wait for
     it would be a wait for every row on its way."""
     out = tmp_path / "g.s"
-    cmd = [build.hipcc(), f"--offload-arch={build.offload_arch()}", "-O3", "-std=c++17", "-fPIC",
-           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-I", os.path.join(ROOT, "include")] + \
-          build.EXTRA_FLAGS.get("gather_attn.hip", []) + \
+    cmd = build.compile_command("gather_attn.hip") + \
           ["--cuda-device-only", "-S", os.path.join(build.CSRC, "gather_attn.hip"), "-o", str(out)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     assert res.returncode == 0, res.stderr[-2000:]
