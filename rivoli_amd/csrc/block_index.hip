@@ -496,8 +496,8 @@ __device__ __forceinline__ void each_of(F&& f) {
         each_of<N, I + 1>(f);
     }
 }
-// bf16(relu(x)), and the same for an x of at most one in magnitude. (The second reads no matrix result that the first has not waited
-// for: the compiler does not see the wait that assembly would need.)
+// bf16(relu(x)), and the same for an x of at most one in magnitude. The second is assembly, for which the compiler keeps no distance from a
+// matrix instruction: of such an instruction's results it may read those that come out of an empty assembly with a result of the first.
 __device__ __forceinline__ float relu_bf16(float x) {
     x = round_bf16(x);
     return x > 0.0f ? x : 0.0f;
@@ -927,7 +927,8 @@ __device__ __forceinline__ bool score_codes(const PairArgs& a_, const PairPlace&
             if (heads > 48 && take[0] && take[1]) {
                 // A step has a head's conversion, the weight of the one before, the rounding of the one before that and the sum's
                 // addition of a fourth: four instructions of which none waits for another. The next sixteen
-                // heads' products run under these heads' steps.
+                // heads' products run under these heads' steps. (The sum is finished before the store's branch: used only there, the compiler
+                // would put all of its steps there, after the products.)
                 constexpr int kSteps = 2 * kPairHeads;
                 f32x16 sets[2];
                 sets[0] = d;
@@ -938,7 +939,13 @@ __device__ __forceinline__ bool score_codes(const PairArgs& a_, const PairPlace&
                     if constexpr (n >= 3) acc = acc + term;
                     if constexpr (n >= 2 && n < kSteps + 2) term = round_bf16(weighted);
                     if constexpr (n >= 1 && n < kSteps + 1) weighted = clamped * wv[(n - 1) / 4 % 16][(n - 1) % 4];
-                    if constexpr (n < kSteps) clamped = n % 16 == 0 ? relu_bf16(sets[set & 1][0]) : clamp_bf16(sets[set & 1][n % 16]);
+                    if constexpr (n < kSteps && n % 16 == 0) {
+                        clamped = relu_bf16(sets[set & 1][0]);
+                        asm volatile("" : "+v"(clamped), "+v"(sets[set & 1]));  // the other fifteen, now that this one was waited for
+                    } else if constexpr (n < kSteps) {
+                        clamped = clamp_bf16(sets[set & 1][n % 16]);
+                    }
+                    if constexpr (n == kPairHeads + 2 || n == kSteps + 2) asm volatile("" : "+v"(acc));
                     if constexpr (n == kPairHeads + 2) finish(0, info[0]);
                     if constexpr (n == kSteps + 2) finish(1, info[1]);
                     __builtin_amdgcn_sched_barrier(0);

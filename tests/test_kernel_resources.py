@@ -9,6 +9,7 @@ phases must not share per-element lane masks: 32 of them do not fit the scalar r
 when they spilled (to lanes of a vector register, a write and a read each) a quarter of the
 kernel's vector instructions were spill traffic. Compiles one file per test; needs hipcc, no
 GPU."""
+import functools
 import os
 import re
 import shutil
@@ -17,6 +18,7 @@ import subprocess
 import pytest
 
 from rivoli_amd import build
+from tests import wait_states
 
 
 def test_the_build_compiles_with_the_flags_that_these_tests_compile_with(monkeypatch):
@@ -63,13 +65,18 @@ def test_eight_bit_attention_kernels_do_not_spill(tmp_path):
     assert seen == 4, f"expected the dense and row-list kernels of both 8-bit modes, saw {seen}"
 
 
-def _resource_blocks(src_name):
-    src = os.path.join(build.CSRC, src_name)
+@functools.lru_cache(maxsize=None)
+def _compiled(src_name):
+    """The file's resource report and its listing."""
     cmd = build.compile_command(src_name) + \
-          ["-Rpass-analysis=kernel-resource-usage", "-c", src, "-o", os.devnull]
+          ["-Rpass-analysis=kernel-resource-usage", "--cuda-device-only", "-S", os.path.join(build.CSRC, src_name), "-o", "-"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     assert res.returncode == 0, res.stderr[-2000:]
-    return re.split(r"remark: Function Name: ", res.stderr)[1:]
+    return res.stderr, res.stdout
+
+
+def _resource_blocks(src_name):
+    return re.split(r"remark: Function Name: ", _compiled(src_name)[0])[1:]
 
 
 @pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
@@ -137,11 +144,12 @@ def test_kernels_that_count_their_transfers_do_not_spill():
 
 @pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
 def test_the_block_scorers_matrix_kernels_and_the_few_row_selection_do_not_spill():
-    """Two waves per SIMD of 252 registers in the many-query scorer (scalar registers do spill
+    """Two waves per SIMD of up to 255 registers in the many-query scorers (scalar registers do spill
     there, in the fold), three in the one-query scorers; a row's keys in registers and its masks
     out of memory in the few-row selection, as in the many-row one."""
     seen = []
     for src, part, waves in (("block_index.hip", "score_blocks_pair_kernel", 2),
+                             ("block_index.hip", "score_blocks_codes_kernel", 2),
                              ("block_index.hip", "score_blocks_one_kernel", 3),
                              ("index_topk.hip", "block_select_few_kernel", 8),
                              ("index_topk.hip", "index_topk_few_kernel", 8)):
@@ -155,7 +163,7 @@ def test_the_block_scorers_matrix_kernels_and_the_few_row_selection_do_not_spill
             assert int(re.search(r"VGPRs Spill: (\d+)", b).group(1)) == 0, name
             assert int(re.search(r"ScratchSize \[bytes/lane\]: (\d+)", b).group(1)) == 0, name
             assert int(re.search(r"Occupancy \[waves/SIMD\]: (\d+)", b).group(1)) >= waves, name
-    assert len(seen) == 11 and seen.count("block_select_few_kernel") == seen.count("index_topk_few_kernel") == 4
+    assert len(seen) == 12 and seen.count("block_select_few_kernel") == seen.count("index_topk_few_kernel") == 4
 
 
 def test_the_build_refuses_an_attention_object_that_spills():
@@ -227,3 +235,55 @@ def test_list_attention_of_32_heads_a_wave_keeps_its_operands_apart(tmp_path):
                 if ln[0].startswith("v_") and not ln[0].startswith("v_mfma") and args:
                     written.append((registers(args[0]), 0))
     assert kernels == 3 and scores == 3 * 32, (kernels, scores)
+
+
+@pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
+@pytest.mark.parametrize("src,with_products", [("block_index.hip", 4), ("index_score.hip", 8), ("mla_attend.hip", 36)])
+def test_no_result_of_a_matrix_instruction_is_read_before_it_is_there(src, with_products):
+    """On no way through a kernel does an instruction, inline assembly included, come sooner after the matrix instruction whose
+    result it reads than the compiler would let it."""
+    seen = 0
+    for name, body in wait_states.kernels(_compiled(src)[1]):
+        products, early = wait_states.early_uses(body)
+        seen += products > 0
+        assert not early, (name, early[:8])
+    assert seen == with_products
+
+
+def test_reads_of_matrix_results_that_come_too_soon_are_found():
+    """wait_states.early_uses on listings with and without the mistake: straight on, around a loop, over a branch, by assembly, of an
+    accumulation register, and a write over the result."""
+    product = "\tv_mfma_f32_32x32x16_bf16 v[2:17], v[20:23], v[24:27], 0\n"
+    use = "\t;;#ASMSTART\n\tv_cvt_pk_bf16_f32 v1, 0, v17 clamp\n\t;;#ASMEND\n"
+    other = "\tv_mov_b32_e32 v40, 0\n"
+    early = lambda text: [short for _, short in wait_states.early_uses(text + "\ts_endpgm\n")[1]]
+    assert early(product + use) == [12] and early(product + "\ts_nop 10\n" + use) == [1] and not early(product + "\ts_nop 11\n" + use)
+    assert not early(product + 12 * other + use) and early(product + 11 * other + use) == [1] and early(product + product + use) == [12]
+    assert early(use + product) == []
+    loop = "\ts_nop 15\n.LBB0_1:\n" + use + "%s\ts_cbranch_scc1 .LBB0_1\n"
+    assert early(loop % (product + 9 * other)) == [2] and not early(loop % (product + 11 * other))
+    over = product + "\ts_cbranch_scc1 .LBB0_2\n\ts_nop 15\n.LBB0_2:\n" + use
+    assert early(over) == [11]
+    assert early(product.replace("v[2:17]", "a[2:17]") + "\tv_accvgpr_read_b32 v1, a3\n") == [12]
+    assert early(product + "\tv_mov_b32_e32 v9, 0\n") == [12] and not early(product + "\tv_mov_b32_e32 v18, v1\n")
+    scaled = "\tv_mfma_scale_f32_32x32x64_f8f6f4 v[2:17], v[20:27], v[30:37], 0, v38, v39 op_sel_hi:[0,0,0]"
+    assert early(scaled + "\n" + use) == [20] and early(scaled + " cbsz:4 blgp:4\n" + use) == [12]
+
+
+@pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
+def test_the_code_scorers_sums_run_beside_its_conversions():
+    """Of 64 heads two tiles' clamped conversions have, between any two of them, the weight, the rounding and the addition of heads before:
+    none of these is put off to the store's branch."""
+    body, = [body for name, body in wait_states.kernels(_compiled("block_index.hip")[1]) if "score_blocks_codes_kernel" in name]
+    steps, ops = [], None
+    for instructions, _ in wait_states.blocks_of(body):
+        for op, _, line, _ in instructions:
+            if line.endswith(" clamp"):
+                steps += [ops] if ops is not None else []
+                ops = []
+            elif ops is not None:
+                ops.append(op)
+    steps = [ops for ops in steps if len(ops) < 60]  # (the store between the tiles, and the way around, are longer)
+    assert len(steps) >= 118
+    late = [ops for ops in steps[3:] if not {"v_mul_f32_e32", "v_cvt_pk_bf16_f32", "v_add_f32_e32"} <= set(ops)]
+    assert len(late) <= 3, late[:4]
