@@ -148,6 +148,11 @@ __device__ __forceinline__ bool gather_attn_wide_pass(const GatherAttnArgs& a, l
 #pragma unroll
         for (int c = 0; c < kGwColTiles; ++c)  // zeros at a sixteenth of the instructions of writing them
             asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %1, 0" : "=a"(o[c]) : "v"(z));
+        // A query without a live slot reads them next. The compiler keeps no distance from assembly, so they come out of one that does: once
+        // the last is there, all are. (Not under that condition: twelve wait states of a query's 140 000 cycles are less than a branch here.)
+        asm volatile("s_nop 11" : "+a"(o[kGwColTiles - 1]));
+#pragma unroll
+        for (int c = 0; c < kGwColTiles - 1; ++c) asm volatile("" : "+a"(o[c]));
     }
     float m_ref = -INFINITY, l_sum = 0.0f;
     const float qs = fabsf(a.qscale);  // its sign is in the query

@@ -238,7 +238,8 @@ def test_list_attention_of_32_heads_a_wave_keeps_its_operands_apart(tmp_path):
 
 
 @pytest.mark.skipif(shutil.which(build.hipcc()) is None, reason="hipcc not found")
-@pytest.mark.parametrize("src,with_products", [("block_index.hip", 4), ("index_score.hip", 8), ("mla_attend.hip", 36)])
+@pytest.mark.parametrize("src,with_products", [("block_index.hip", 4), ("index_score.hip", 8), ("mla_attend.hip", 36),
+                                               ("gather_attn.hip", 11)])
 def test_no_result_of_a_matrix_instruction_is_read_before_it_is_there(src, with_products):
     """On no way through a kernel does an instruction, inline assembly included, come sooner after the matrix instruction whose
     result it reads than the compiler would let it."""
