@@ -450,6 +450,9 @@ constexpr int kPairSplitMax = 4096;     // blocks of a split: one bit of a 128-b
 constexpr int kFp4Span = 9;
 constexpr int kFp4Row = 64 + 16;   // bytes of an fp4 row in LDS
 constexpr int kFp4MinExp = 127 - 59, kFp4MaxExp = 127 + 59;  // of a row's largest block, as kExactSpan's
+// The least exponent that a block's scale is made for. Blocks below it are out of every range above and below here; and a subnormal value, whose
+// exponent field is a zero's, is no code under that scale: it cannot pass for a zero, whether the conversions flush it or not.
+constexpr int kFp4LeastExp = 32;
 // The dots come out scaled, the largest that 128 products can be to just below one, so that the conversion to bf16 clamps to [0,
 // 1] and is the relu too; scores are scaled back. Powers of two change no rounding while nothing leaves the normal numbers:
 // with weights in 2^+-50, a query's heads within 20 binades (a scaled dot is 2^-44 then, or zero) and scales back of 2^-20 to 2^40,
@@ -457,6 +460,7 @@ constexpr int kFp4MinExp = 127 - 59, kFp4MaxExp = 127 + 59;  // of a row's large
 constexpr int kFp4Down = 13;       // 128 * 36 < 2^13
 constexpr int kFp4Heads = 20, kFp4Back0 = -20, kFp4Back1 = 40;
 constexpr uint32_t kFp4Weight0 = 127 - 50, kFp4Weight1 = 127 + 50;
+static_assert(kFp4LeastExp > 5 && kFp4MinExp - kFp4LeastExp >= kFp4Heads && kFp4Heads >= kFp4Span, "no block below kFp4LeastExp is taken");
 
 template <int CTRL>
 __device__ __forceinline__ uint32_t max_with_lane(uint32_t x) {
@@ -475,7 +479,7 @@ __device__ __forceinline__ uint32_t fp4_of(const f32x4& v, uint32_t& expo, uint3
     m = max_with_lane<0x4E>(m);   // lane ^ 2
     m = max_with_lane<0x141>(m);  // lane 7 - i: the other four's
     expo = m >> 23;
-    const float scale = __uint_as_float((max(expo, 3u) - 2u) << 23);
+    const float scale = __uint_as_float((max(expo, (uint32_t)kFp4LeastExp) - 2u) << 23);
     uint32_t c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, v.x, v.y, scale, 0);
     c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, v.z, v.w, scale, 1);
     const f32x2 lo = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, scale, 0), hi = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, scale, 1);

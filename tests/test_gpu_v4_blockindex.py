@@ -384,3 +384,125 @@ def test_score_at_the_edges_of_what_the_fp4_products_take(oracle, s, n_comp, hea
         bad = np.argwhere((got != want.view(np.uint32)) & live)
         assert bad.size == 0, (ratio, [(int(queries[i]), int(queries[i]) // 2 % len(kinds), int(c)) for i, c in bad[:6]])
         assert (got[~live] == 0x5A5A5A5A).all()
+
+
+def check_scores(q, kv, w, queries, want, what):
+    """Both forms of a launch of q [s][heads][128] against the oracle's scores of some of its queries, bit for bit; entries that the
+    prefill form has no use for stay as they were."""
+    s, heads = w.shape
+    n_comp = len(kv)
+    qd, kd, wd = dev(q), dev(kv), dev(w)
+    for ratio in (0, 4):
+        out = dzeros(s * n_comp * 4, 0x5A)
+        if ratio:
+            hip.launch_index_score_blocks_prefill(qd, kd, wd, out, s, n_comp, heads, 128, ratio)
+        else:
+            hip.launch_index_score_blocks(qd, kd, wd, out, s, n_comp, heads, 128)
+        got = back(out, np.uint32).reshape(s, n_comp)[queries]
+        live = np.ones(got.shape, bool) if not ratio else \
+            (np.arange(n_comp)[None, :] // 64) * 64 < np.minimum((queries + 1) // ratio, n_comp)[:, None]
+        bad = np.argwhere((got != want.view(np.uint32)) & live)
+        assert bad.size == 0, (what, ratio, len(bad), [(int(queries[i]), int(c)) for i, c in bad[:6]])
+        assert (got[~live] == 0x5A5A5A5A).all()
+
+
+@pytest.mark.parametrize("s,n_comp,heads", [(2060, 230, 64), (2060, 201, 33), (1380, 390, 64)])
+def test_score_of_rows_with_the_smallest_codes(oracle, s, n_comp, heads):
+    """Blocks of 0 and +-2^-127, which are half a code under the smallest normal scale and are no zeros, in rows with larger blocks and in rows
+    of nothing else; blocks whose largest value is 2^-126 to 2^-124; and spread rows of such amplitude, which is below the spread's
+    floor. Of q in waves of their own, of kv in tiles of their own."""
+    rng = np.random.default_rng(s + n_comp + heads)
+    least = np.float32(2.0 ** -127)
+
+    def spread(rows, amplitude):
+        x = bf16_round((rng.standard_normal((rows, 128)) * amplitude).astype(np.float32))
+        code, x = oracle.act_quant_f4_rotated(x)
+        assert code == 0 and (x != 0).any()
+        return x
+
+    def tiny(rows, kind):
+        if kind >= 6:
+            x = spread(rows, (0.12, 0.3, 1.0)[kind - 6] * 2.0 ** -126)
+            assert kind > 6 or np.abs(x).max() == least
+            return x
+        if kind >= 2:  # the largest value 4 or 6 times 2^-128 to 2^-125
+            return coded_rows(rng, rows, np.full((rows, 4), (-128, -127, -126, -125)[kind - 2]))
+        x = coded_rows(rng, rows, np.zeros((rows, 4)))
+        small = rng.choice(np.array([0.0, -0.0, least, -least], np.float32), (rows, 128))
+        small[:, 5::32] = least
+        if kind == 1:
+            return small
+        x[:, 32:64] = small[:, 32:64]
+        return x
+
+    q = np.zeros((s, heads, 128), np.float32)
+    w = bf16_round((rng.standard_normal((s, heads)) * 0.1).astype(np.float32))
+    rows_of = [[tiny(2 * heads, kind) if kind >= 0 else spread(2 * heads, 1.0) * np.float32(2.0 ** 20) for _ in range(6)] for kind in range(-2, 9)]
+    for pair in range(s // 2):  # (two of eleven waves with rows as usual)
+        q[2 * pair:2 * pair + 2] = rows_of[pair % 11][pair // 11 % 6].reshape(2, heads, 128)
+    kv = spread(n_comp, 1.0)
+    for kind in range(6):  # a row of each in tiles that would be taken otherwise, and whole ones
+        at = 32 * kind + 7
+        if at + 2 < n_comp:
+            kv[at:at + 2] = tiny(2, kind)
+    kv[-5:] = tiny(5, 6)
+    pairs = [11 * r + k for r in (0, 30, (s // 2 - 11) // 11) for k in range(11)]
+    queries = np.array([2 * p + i for p in pairs for i in (0, 1)])
+    code, want = oracle.index_score_blocks(q[queries], kv, w[queries])
+    assert code == 0 and np.isfinite(want).all()
+    check_scores(q, kv, w, queries, want, "smallest codes")
+    # the rest of the blocks as usual: only q has such rows
+    kv = spread(n_comp, 1.0)
+    code, want = oracle.index_score_blocks(q[queries], kv, w[queries])
+    check_scores(q, kv, w, queries, want, "smallest codes of q")
+    # and the other way round
+    q[:] = np.repeat(spread(2 * heads, 1.0), -(-s // 2), axis=0)[:s * heads].reshape(s, heads, 128)
+    kv[40:44] = tiny(4, 0)
+    kv[70:74] = tiny(4, 1)
+    kv[100:164] = tiny(64, 1)
+    kv[n_comp - 9:] = tiny(9, 6)
+    code, want = oracle.index_score_blocks(q[queries], kv, w[queries])
+    check_scores(q, kv, w, queries, want, "smallest codes of kv")
+
+
+@pytest.mark.parametrize("s,n_comp,heads", [(2060, 230, 64), (2060, 201, 33)])
+def test_score_keeps_the_last_bit_of_the_largest_sums_that_the_fp4_products_take(oracle, s, n_comp, heads):
+    """Block exponents that span 9 over both rows, three blocks at the top and one at the bottom, that one in each half of the products'
+    contraction. One-signed sums of the top blocks come to the middle between two bf16 numbers, cancelling ones to zero: the
+    bottom block's sum, down to the last unit, decides. One head a query has a weight, so that its dot is the score."""
+    rng = np.random.default_rng(s + heads)
+    n_kinds = 16  # the bottom block, whether the top blocks cancel, and 9 binades in q alone or 5 in q and 4 in kv
+    q = np.zeros((s, heads, 128), np.float32)
+    w = np.zeros((s, heads), np.float32)
+    w[np.arange(s), np.arange(s) // 2 % heads] = 1.0
+    for pair in range(s // 2):
+        low, cancel, apart = pair % 4, pair // 4 % 2, (9, 5)[pair // 8 % 2]
+        rows = np.empty((2 * heads, 128), np.float32)
+        for r in rows if pair < 5 * n_kinds else ():
+            # a sum of 4 x 96 + 2 x sixes, times a block's 4 or 6: a middle for sixes odd, or two more than a multiple of four
+            sixes = int(rng.choice(np.arange(65, 96, 2))) if rng.random() < 0.5 else int(rng.choice(np.arange(66, 96, 4)))
+            top = rng.permutation(np.where(np.arange(96) < sixes, 6.0, 4.0))
+            if cancel:
+                top = rng.permutation(np.concatenate([top[:48], -top[:48]]))
+            bottom = rng.choice([0.5, -0.5], 32)
+            bottom[rng.integers(32)] = rng.choice([4.0, -4.0])
+            values = np.insert(top, 32 * low, bottom * 2.0 ** -apart)
+            r[:] = values * (1.0 if cancel else rng.choice([1.0, 1.0, -1.0]))
+        q[2 * pair:2 * pair + 2] = rows.reshape(2, heads, 128) if pair < 5 * n_kinds else q[2 * pair - 10 * n_kinds:][:2]
+    kv = np.repeat(rng.choice(np.array([6.0, 4.0], np.float32), n_comp)[:, None], 128, axis=1)
+    for c in range(64, 128):  # of which a block is four binades down, with the smallest code in it, for the rows of 5
+        b = c % 4
+        kv[c, 32 * b:32 * b + 32] *= np.float32(2.0 ** -4)
+        kv[c, 32 * b + 1:32 * b + 9] = np.float32(0.5 * 2.0 ** -4)
+    pairs = [n_kinds * r + k for r in (0, 25, s // 2 // n_kinds - 1) for k in range(n_kinds)]
+    queries = np.array([2 * p + i for p in pairs for i in (0, 1)])
+    code, want = oracle.index_score_blocks(q[queries], kv, w[queries])
+    # the dots by themselves, and without the bottom blocks: it is these that decide
+    dots = np.einsum("thd,cd,th->tc", q[queries].astype(np.float64), kv.astype(np.float64), w[queries].astype(np.float64))
+    top_q = np.where(np.abs(q[queries]) >= 4, q[queries], 0).astype(np.float64)
+    top = np.einsum("thd,cd,th->tc", top_q, kv.astype(np.float64), w[queries].astype(np.float64))
+    taken = np.full(want.shape, True)
+    taken[:, 64:128] = (queries // 2 // 8 % 2 == 1)[:, None]
+    assert code == 0 and np.array_equal(want[taken], np.maximum(bf16_round(dots.astype(np.float32)), 0)[taken])
+    assert (bf16_round(dots.astype(np.float32)) != bf16_round(top.astype(np.float32)))[taken].mean() > 0.3
+    check_scores(q, kv, w, queries, want, "the largest sums")
