@@ -241,22 +241,53 @@ static inline AttendPlan heads32_plan(const AttendPlan& plan, int n_seqs, int H,
 // sets of 2 048 rows 87 -> 66, and at precise 4 18 x 10 262 ragged 72 -> 51, 11 x 12 613 of 128 heads 96 -> 66; in one round up to 24 576: 32 x 6 000
 // (24 064) 79.1 -> 78.9, ragged 63 -> 57, 32 x 4 096 at precise 0 (16 384) 58 -> 51, but 16 x 16 384 (32 768) 94 -> 97, and the 8-bit kernel stays the faster.
 // Up to 32 heads those workgroups are half empty.
+// What a call takes lies on a line over its longest work item, in tiles of an even batch (a thousand calls of 17 to 1 024 heads, most within
+// 3 %): here 19.5 us and 2.25 per tile of 64 tokens; by 16 heads 15.6 and 1.5; by 64 in two rounds, per tile of 32 in both of them,
+// 35 and 2.0 in the parity mode, of listed rows 44 and 1.9, but with the 8-bit instructions 43 and 1.05 (precise 3: 38 and 0.96), listed 34 and 1.7. So a
+// second round of the 8-bit kernel's is the shorter way past a length, and such calls stay there: even, precise 4, 27 x 16 384 of 128 heads 277 against 316 here, 24 x
+// 12 000 of 112 175 and 232, 6 x 16 384 of 384 175 and 304, 3 x 24 000 of 640 221 and 440, but 17 x 9 000 of 64 85 and 67, 12 x 6 000 of 128 85 and 63. Ragged
+// batches gain sooner, the more so the more sequences (22 x 6 000 of 128 heads even 112 and 124, ragged 94 and 72): the line lies between the
+// two; 17 x 13 000 of 128 heads still come here (even 0.89 of the speed, ragged 1.21), 24 x 13 000 do not (0.74 and 0.95). In the parity mode
+// only head counts that leave compute units out come to it: 3 x 16 384 of 640 268 and 304.
+// Lists whose work items come out no more than half as long again by 16 heads stay with those: 3 of 8 192 rows of 128 heads 0.94 of the speed here, 12 of
+// 4 096 of 80 0.93, 9 of 8 192 of 33 0.94. So do lists that 64 heads take in one full round of up to four work items a
+// sequence: 64 of 2 048 rows of 64 heads 0.88 of the speed, 32 of 128 heads 0.97; of eight, 16 of 4 096 of 128 heads, 1.03.
 constexpr long long kWideMinWork = 8192, kWideMinWorkListed = 5120, kWideMaxWork = 24576;
-static inline bool heads32_pays(const AttendPlan& p, const AttendPlan& plan, bool heads16, int n_seqs, int H, int max_rows, int precise,
-                                bool dense) {
+constexpr int kWideMinSplitsListed = 5;
+// Tiles of the longest of `items` work items of an even batch that SeqDeal cuts.
+static inline long long seq_deal_run(long long tiles, int n_seqs, int items) {
+    const int each = items / n_seqs;
+    return (tiles + each - 1) / each;
+}
+static inline bool heads32_pays(const AttendPlan& p, const AttendPlan& plan, const AttendRoute& route, int n_seqs, int H, int max_rows,
+                                int precise, bool dense) {
     const long long tiles = max_rows / kTile + (max_rows % kTile != 0);
-    if (heads16) return n_seqs * tiles * ((H + kH16Heads - 1) / kH16Heads) > (dense ? kWideMinWork : kWideMinWorkListed);
+    const long long run = (seq_deal_run(tiles, n_seqs, p.n_items) + kWideRun - 1) / kWideRun;  // tiles of 64 tokens
+    if (route.heads16) {
+        const long long run16 = (seq_deal_run(tiles, n_seqs, route.plan.n_items) + kWideRun - 1) / kWideRun;
+        if (!dense && precise > 0 && 2 * run16 < 3 * run + 6) return false;
+        return n_seqs * tiles * ((H + kH16Heads - 1) / kH16Heads) > (dense ? kWideMinWork : kWideMinWorkListed);
+    }
     const int groups = (H + kWideHeads - 1) / kWideHeads;
-    if ((long long)plan.n_items * ((H + 63) / 64) > kAttTargetGroups) return true;
+    const long long there = (long long)plan.n_items * ((H + 63) / 64);
+    if (there > kAttTargetGroups) {
+        if (precise == 0) return true;
+        const long long rounds = (there + kAttTargetGroups - 1) / kAttTargetGroups;
+        const long long run64 = rounds * n_seqs * tiles / plan.n_items;
+        if (precise > 2) return 100 * run <= (dense ? 47 * run64 + (n_seqs < 8 ? 1400 : 2200) : 69 * run64 + 600);
+        return 100 * run <= (dense ? 90 * run64 + 1200 : 64 * run64 + 1400);
+    }
     if (precise > 2 || 4 * p.n_items * groups < 3 * kAttTargetGroups) return false;
-    return groups == 1 || n_seqs * tiles * 2 * groups <= kWideMaxWork;
+    if (groups == 1) return true;
+    if (!dense && (precise == 2 || (precise == 1 && groups == 2)) && plan.n_splits < kWideMinSplitsListed && there == kAttTargetGroups) return false;
+    return n_seqs * tiles * 2 * groups <= kWideMaxWork;
 }
 // A paged call's work items there, n_items 0 where `route`, attend_route's, stands.
 static inline AttendPlan heads32_route(const AttendPlan& plan, const AttendRoute& route, int n_seqs, int H, int max_rows, int precise,
                                        bool dense) {
     AttendPlan p = heads32_plan(plan, n_seqs, H, max_rows);
     // (sequences that stay whole, or that one long one of many must not keep a workgroup with, stay where they are)
-    if (!p.n_items || (route.heads16 && !route.by_seq) || !heads32_pays(p, plan, route.heads16, n_seqs, H, max_rows, precise, dense)) p.n_items = 0;
+    if (!p.n_items || (route.heads16 && !route.by_seq) || !heads32_pays(p, plan, route, n_seqs, H, max_rows, precise, dense)) p.n_items = 0;
     return p;
 }
 

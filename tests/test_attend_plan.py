@@ -157,3 +157,22 @@ def test_work_items_of_32_heads_fit_the_scratch_and_the_chip(precise, listed):
     assert wide(24, 64, 8000) and wide(9, 128, 16384) and wide(18, 64, 10262)  # a second round of 64 heads' workgroups
     assert wide(6, 64, 9000) == (listed and precise < 4) and not wide(8, 64, 2048) and not wide(32, 64, 32768) and not wide(32, 16, 16384)
     assert wide(32, 64, 6000) == (precise < 4) and wide(12, 128, 2048) == (listed and precise < 4)
+
+
+def test_work_items_of_32_heads_where_they_are_the_shorter_way():
+    """Calls timed on both sides of the lines: the 8-bit modes' long ones and the parity mode's of few, uneven work items stay with
+    64 heads a workgroup, lists that 16 heads cut nearly as finely or 64 heads take in one full round with those."""
+    wide = lambda n, H, rows, precise, listed=False: attend_wide_items(n, H, rows, precise, listed) > 0
+    for precise in (3, 4):
+        for call in ((27, 128, 16384), (24, 112, 12000), (24, 128, 13000), (60, 64, 12000), (9, 256, 32768), (6, 384, 16384), (5, 384, 24000),
+                     (7, 512, 24000), (1, 640, 32768), (3, 640, 24000), (3, 768, 24000), (3, 1024, 24000)):
+            assert not wide(*call, precise), (call, precise)
+        for call in ((17, 64, 9000), (18, 64, 10262), (12, 128, 6000), (18, 128, 9000), (17, 128, 13000), (9, 160, 6000), (3, 192, 24000),
+                     (7, 256, 3000), (3, 384, 6000), (2, 768, 6000)):
+            assert wide(*call, precise), (call, precise)
+    for precise in (1, 2):
+        assert not wide(3, 640, 16384, precise) and wide(2, 768, 24000, precise) and wide(17, 160, 24000, precise) and wide(5, 512, 12000, precise)
+        assert not wide(64, 64, 2048, precise, True) and wide(16, 128, 4096, precise, True) and wide(48, 64, 2048, precise, True)
+        assert not wide(3, 128, 8192, precise, True) and not wide(12, 80, 4096, precise, True) and wide(12, 160, 2048, precise, True)
+    assert wide(3, 640, 16384, 0) and wide(64, 64, 2048, 0, True) and wide(3, 128, 8192, 0, True)
+    assert not wide(3, 640, 8192, 4, True) and wide(3, 768, 2048, 4, True)
