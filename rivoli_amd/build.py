@@ -32,15 +32,14 @@ HOST_SOURCES = ["pagepool.cpp"]
 # with a piece compiled out).
 NO_SCRATCH = {"mla_attend.hip": [("mla_attend_paged_kernel", "Lb1EEEvNS_10AttendArgsE"),
                                  ("mla_attend_heads16_kernel", "EEEvNS_10AttendArgsE"),
-                                 ("mla_attend_few_kernel", "EEEvNS_10AttendArgsE")]}
-NO_SCRATCH_WHERE_BUILT = {"mla_attend.hip": [("mla_attend_wide_kernel", "EEEvNS_10AttendArgsE")]}
+                                 ("mla_attend_few_kernel", "EEEvNS_10AttendArgsE"),
+                                 ("mla_attend_wide_kernel", "EEEvNS_10AttendArgsE")]}
 
 
 def check_resources(k: str, report: str) -> None:
     """Raises when a kernel of NO_SCRATCH[k] in hipcc's resource report uses scratch memory or
-    more LDS than a compute unit has."""
-    where_built = NO_SCRATCH_WHERE_BUILT.get(k, [])
-    for part, suffix in NO_SCRATCH.get(k, []) + where_built:
+    more LDS than a compute unit has, or a family of them is not in it."""
+    for part, suffix in NO_SCRATCH.get(k, []):
         seen = 0
         for block in re.split(r"remark: Function Name: ", report)[1:]:
             name = block.split()[0]
@@ -52,7 +51,7 @@ def check_resources(k: str, report: str) -> None:
             if scratch or lds > 160 * 1024:
                 raise RuntimeError(f"{k}: {name} uses {scratch} bytes of scratch per lane and {lds} bytes of LDS; "
                                    "this kernel must compile to 0 and at most 163840")
-        if not seen and (part, suffix) not in where_built:
+        if not seen:
             raise RuntimeError(f"{k}: no kernel matching {part}...{suffix} in the resource report")
 
 

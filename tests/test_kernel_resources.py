@@ -169,19 +169,23 @@ def test_the_block_scorers_matrix_kernels_and_the_few_row_selection_do_not_spill
 def test_the_build_refuses_an_attention_object_that_spills():
     """build.check_resources is what build_kernels applies to mla_attend.hip's resource report:
     scratch memory or too much LDS in an 8-bit attention kernel, or in one of 16 heads a workgroup (a tile a
-    wave, or eight waves on a tile), raises instead of linking, and so does a report without them."""
+    wave, or eight waves on a tile) or of 32, raises instead of linking, and so does a report without one of these families."""
     figures = "    ScratchSize [bytes/lane]: 0\n    LDS Size [bytes/block]: 85632\n"
     head = "x.hip:1:1: remark: Function Name: _ZN2rk23mla_attend_paged_kernelILi2ELi2ELi0ELb0ELb1EEEvNS_10AttendArgsE\n"
     heads16 = "x.hip:1:1: remark: Function Name: _ZN2rk25mla_attend_heads16_kernelILi2ELi2ELi3EEEvNS_10AttendArgsE\n"
     few = "x.hip:1:1: remark: Function Name: _ZN2rk21mla_attend_few_kernelILi2ELi2ELi3EEEvNS_10AttendArgsE\n"
-    fine = head + figures + heads16 + figures.replace("85632", "161328") + few + figures.replace("85632", "142912")
+    wide = "x.hip:1:1: remark: Function Name: _ZN2rk22mla_attend_wide_kernelILi2ELi2ELi0EEEvNS_10AttendArgsE\n"
+    families = [head + figures, heads16 + figures.replace("85632", "161328"), few + figures.replace("85632", "142912"),
+                wide + figures.replace("85632", "162432")]
+    fine = "".join(families)
     build.check_resources("mla_attend.hip", fine)
     build.check_resources("kv_gather.hip", "")                        # other files are not held to it
-    for bad in (fine.replace("lane]: 0", "lane]: 44", 1), fine.replace("85632", "170000"), "", head + figures,
-                head + figures + heads16 + figures.replace("lane]: 0", "lane]: 8"),
-                fine.replace("161328", "163856"), fine.replace("142912", "163856"),
-                fine.replace(few + figures.replace("85632", "142912"), ""),
-                "lane]: 4".join(fine.rsplit("lane]: 0", 1))):
+    for i, family in enumerate(families):
+        others = "".join(families[:i] + families[i + 1:])
+        for bad in (others, others + family.replace("lane]: 0", "lane]: 8"), others + re.sub(r"block\]: \d+", "block]: 163856", family)):
+            with pytest.raises(RuntimeError):
+                build.check_resources("mla_attend.hip", bad)
+    for bad in ("", families[0], fine.replace("85632", "170000"), "lane]: 4".join(fine.rsplit("lane]: 0", 1))):
         with pytest.raises(RuntimeError):
             build.check_resources("mla_attend.hip", bad)
 
