@@ -610,6 +610,16 @@ def bench_v4(a, torch, hip):
     return res
 
 
+def block_scorer(s, n_comp):
+    """The kernel that scores s queries against n_comp blocks and the peak of its matrix instructions, TFLOP/s: the launcher's rule
+    (rivoli_amd/csrc/block_index_plan.hpp), which a test compares with this one."""
+    groups = -(-n_comp // 64)
+    if s == 1 or s * groups <= 384:
+        return "score_blocks_one_kernel", 2500.0
+    share = -(-groups // max(1, min(1024 // -(-s // 8), groups))) * 64
+    return ("score_blocks_codes_kernel", 10000.0) if share >= 192 else ("score_blocks_pair_kernel", 2500.0)
+
+
 def bench_v4_index(a, torch, hip):
     """The second cache format's block indexer at prefill (crates/engine/src/v4/blocksel.rs:218-248):
     `tokens` queries x `heads` index heads of 128 are spread in place (Hadamard + simulated fp4),
@@ -642,9 +652,7 @@ def bench_v4_index(a, torch, hip):
     scored = s * n_comp if a.full_scores else int((-(-limit // 64) * 64).clip(max=-(-n_comp // 64) * 64).sum())
     score_flops = 2 * scored * heads * hd                               # one multiply and one add per term
     score_bytes = s * heads * hd * 4 + n_comp * hd * 4 + s * n_comp * 4
-    # the launcher's rule: blocks of a workgroup's share, 192 and more of them by the fp4 instructions
-    share = -(-(-(-n_comp // 64)) // max(1, min(1024 // -(-s // 8), -(-n_comp // 64)))) * 64
-    scorer, peak = ("score_blocks_codes_kernel", 10000.0) if share >= 192 else ("score_blocks_pair_kernel", 2500.0)
+    scorer, peak = block_scorer(s, n_comp)
     # the timed steps spread the same buffer again and again; the check runs one step on a fresh copy
     q.copy_(q_raw)
     torch.cuda.synchronize()

@@ -34,6 +34,7 @@
 // scores and reads 512 bytes through the scalar cache: bound by vector issue, two
 // instructions per multiply-add because the reference's rounding is two roundings.
 // Widths other than 128 re-read the block's row through the vector cache instead.
+#include "block_index_plan.hpp"
 #include "codec.hpp"
 
 #include <cmath>
@@ -434,11 +435,9 @@ __device__ __forceinline__ void fold_heads(const float* __restrict__ q, const fl
 // in flight (178).
 constexpr int kPairWaves = 4;
 constexpr int kPairThreads = kPairWaves * kWave;
-constexpr int kPairQueries = kPairWaves * 2;
+static_assert(kPairQueries == kPairWaves * 2, "a wave's two queries");
 constexpr int kPairHeads = 64;
-constexpr int kPairTile = 32;
 constexpr int kPairRow = 128 * 2 + 16;  // bytes of a bf16 row in LDS: 16-byte reads of 16 rows meet no bank twice
-constexpr int kPairSplitMax = 4096;     // blocks of a split: one bit of a 128-bit mask per tile
 
 // Spread rows are what the block-scaled fp4 instruction takes: e2m1 codes, a power of two for 32 of them. A row
 // qualifies when every block's values are exactly that (fp4_of); with the block's exponent taken
@@ -1163,14 +1162,6 @@ extern "C" int rivoli_act_quant_f4_rotated(float* x, int rows, int d, void* stre
 }
 
 namespace rk {
-// Up to here a workgroup per (query, 64 blocks) is the faster: 4 queries x 4 096 blocks 7 us against
-// 10 (4 x 8 192, 512 workgroups: 11.3 against 10.4; 300 queries x 75, 600: 15 against 10). One query
-// has no second for the many-query kernel's wave: 65 536 blocks 18 us against 25.
-constexpr int kOneGroups = 384;
-// Workgroups of so many blocks turn their q rows into fp4 codes, which takes a wave 2 200 vector instructions where bf16 operands
-// take 900: 192 blocks (2 049 x 512) 37.5 us as bf16 and 33.5 so, 384 (3 000 x 750) 54 and 46; 128 (1 500 x 375) 26.6 and 26.2, 64 (700 x 175)
-// 10.4 and 11.5. Rows that are exact but no codes pay for finding that out: 8 192 queries of such q 232 -> 235, of such kv 212 -> 220, 2 049 38 -> 42.
-constexpr int kFp4Blocks = 192;
 static int score_blocks_launch(const float* q, const float* kv, const float* w, float* score, int s,
                                int n_comp, int heads, int hd, int ratio, hipStream_t st) {
     if (s <= 0 || heads <= 0 || hd <= 0) return 1001;
@@ -1180,40 +1171,26 @@ static int score_blocks_launch(const float* q, const float* kv, const float* w, 
     if (!q || !kv || !w || !score) return 1001;
     (void)hipGetLastError();
     if (hd == 128 && aligned16(kv) && heads <= kPairHeads) {
-        const unsigned groups = (unsigned)(((long long)n_comp + kWave - 1) / kWave);
-        if (s == 1 || (long long)s * groups <= kOneGroups) {
-            // half the blocks a workgroup while there is a compute unit for each (8 192 blocks 6.1 us, 7.1 in
-            // 64s; 16 384 blocks 7.1 us in 64s, 8.5 in 32s)
-            if ((long long)s * 2 * groups <= 256)
+        const ScorePlan plan = score_plan(s, n_comp);
+        const PairArgs args = {q, kv, w, score, s, n_comp, heads, plan.split, ratio};
+        const dim3 grid(plan.groups, plan.rows);
+        switch (plan.kernel) {
+            case ScoreKernel::kOne32:
                 rk::launch_kernel(score_blocks_one_kernel<1>, dim3((unsigned)(((long long)n_comp + 31) / 32), (unsigned)s),
                                   dim3(kOneThreads), 0, st, q, kv, w, score, s, n_comp, heads, ratio);
-            else
-                rk::launch_kernel(score_blocks_one_kernel<2>, dim3(groups, (unsigned)s), dim3(kOneThreads), 0, st, q,
-                                  kv, w, score, s, n_comp, heads, ratio);
-            return launch_status();
-        }
-        // two workgroups per compute unit at a time; splits of the blocks while the queries alone
-        // give fewer than two rounds of those (a split reads its queries' rows again)
-        const unsigned t_groups = (unsigned)(((long long)s + kPairQueries - 1) / kPairQueries);
-        const long long tiles = ((long long)n_comp + kPairTile - 1) / kPairTile;
-        long long splits = t_groups >= 1024 ? 1 : 1024 / t_groups;
-        if (splits > groups) splits = groups;
-        int per = (int)((groups + splits - 1) / splits) * 64;
-        const bool fp4 = per >= kFp4Blocks;
-        // A tile each where that leaves compute units over, or is still one round and the q rows (32 KB
-        // a query) stay in a die's 4 MB of cache, which every one of a query's workgroups reads them
-        // through: 300 x 75 (114 workgroups) 11.7 -> 10.5 us, 5 x 8 192 (256) 10.1 -> 8.8; but 150 x 300 (190,
-        // 4.9 MB) 10.1 -> 11.9.
-        if (t_groups * tiles <= 128 || (t_groups * tiles <= 256 && t_groups <= 13)) per = kPairTile;
-        if (per > kPairSplitMax) per = kPairSplitMax;
-        const unsigned y = (unsigned)(((long long)n_comp + per - 1) / per);
-        if (y <= 65535u) {
-            const PairArgs args = {q, kv, w, score, s, n_comp, heads, per, ratio};
-            if (fp4)
-                rk::launch_kernel(score_blocks_codes_kernel, dim3(t_groups, y), dim3(kPairThreads), 0, st, args);
-            else
-                rk::launch_kernel(score_blocks_pair_kernel, dim3(t_groups, y), dim3(kPairThreads), 0, st, args);
-            return launch_status();
+                return launch_status();
+            case ScoreKernel::kOne64:
+                rk::launch_kernel(score_blocks_one_kernel<2>, dim3((unsigned)(((long long)n_comp + 63) / 64), (unsigned)s),
+                                  dim3(kOneThreads), 0, st, q, kv, w, score, s, n_comp, heads, ratio);
+                return launch_status();
+            case ScoreKernel::kCodes:
+                rk::launch_kernel(score_blocks_codes_kernel, grid, dim3(kPairThreads), 0, st, args);
+                return launch_status();
+            case ScoreKernel::kPair:
+                rk::launch_kernel(score_blocks_pair_kernel, grid, dim3(kPairThreads), 0, st, args);
+                return launch_status();
+            case ScoreKernel::kNone:
+                break;
         }
     }
     // enough workgroups to fill the part while a workgroup keeps its rows for several queries

@@ -1,4 +1,5 @@
-// The attention launchers' routing rules (rivoli_amd/csrc/mla_attend_plan.hpp, gather_attn_plan.hpp) as C functions.
+// The launchers' routing rules (rivoli_amd/csrc/mla_attend_plan.hpp, gather_attn_plan.hpp, block_index_plan.hpp) as C functions.
+#include "../../rivoli_amd/csrc/block_index_plan.hpp"
 #include "../../rivoli_amd/csrc/gather_attn_plan.hpp"
 #include "../../rivoli_amd/csrc/mla_attend_plan.hpp"
 
@@ -21,3 +22,10 @@ extern "C" int attend_wide_items(int n_seqs, int H, int max_rows, int precise, i
 }
 
 extern "C" long long marked_block(unsigned row, unsigned group) { return rk::marked_block(row, group); }
+
+// 0 and 1: a workgroup per query and 32 or 64 blocks; 2: many queries, bf16; 3: fp4 codes; 4: neither. out: blocks of a workgroup, the grid.
+extern "C" int score_plan(int s, int n_comp, int out[3]) {
+    const rk::ScorePlan p = rk::score_plan(s, n_comp);
+    out[0] = p.split, out[1] = (int)p.groups, out[2] = (int)p.rows;
+    return (int)p.kernel;
+}

@@ -77,6 +77,14 @@ def attend_wide_items(n_seqs, H, max_rows, precise, listed=False):
     return _plan().attend_wide_items(n_seqs, H, max_rows, precise, int(listed))
 
 
+def score_plan(s, n_comp):
+    """rivoli_amd/csrc/block_index_plan.hpp: the block scorer's kernel for a call of 128 dims and up to 64 heads, blocks of a workgroup
+    of the many-query kernels and their grid."""
+    out = (ctypes.c_int * 3)()
+    kernel = ("one 32", "one 64", "pair", "codes", "none")[_plan().score_plan(s, n_comp, out)]
+    return (kernel, *out)
+
+
 def marked_block(row, group):
     """rivoli_amd/csrc/gather_attn_plan.hpp: the group's block in a row of 256."""
     return _plan().marked_block(row, group)
