@@ -125,6 +125,9 @@ __device__ __forceinline__ bool gather_attn_wide_pass(const GatherAttnArgs& a, l
     uint32_t m_cur, m_next, m_after;  // live slots of this tile and the two after it
     const GwEntries e_first = list.entries(n32, 0, f0, m_cur);
     GwEntries e_next = list.entries(n32, 1, f1, m_next), e_after = list.entries(n32, 2, f2, m_after);
+    // O^T: a lane holds four neighbouring columns of one head in each quarter of a tile, so what scales a head
+    // is a register of its own lane. Kept in the accumulation registers ("a") throughout: 256 of them, all there are.
+    f32x16 o[kGwColTiles];
     GwRow raw[kGwRing];
 #pragma unroll
     for (int b = 0; b < kGwRowsPerWave; b += 8) {
@@ -132,6 +135,15 @@ __device__ __forceinline__ bool gather_attn_wide_pass(const GatherAttnArgs& a, l
 #pragma unroll
         for (int i = 0; i < 8; ++i) r[i].ask(row_address(e_first, b + i), lane);
         __builtin_amdgcn_sched_barrier(0);
+        if (b == 0) {  // while the first rows are on their way
+            const u32x4 z = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int c = 0; c < kGwColTiles; ++c)  // zeros at a sixteenth of the instructions of writing them
+                asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %1, 0" : "=a"(o[c]) : "v"(z));
+            // The compiler keeps no distance from assembly: a query without a live slot, which reads them first of all, does so far behind the
+            // deposits below.
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) deposit(0, kGwRowsPerWave * wave + b + i, r[i].bf16());
         __builtin_amdgcn_sched_barrier(0);
@@ -140,20 +152,6 @@ __device__ __forceinline__ bool gather_attn_wide_pass(const GatherAttnArgs& a, l
     for (int i = 0; i < kGwRing; ++i) raw[i].ask(row_address(e_next, i), lane);
     __syncthreads();
 
-    // O^T: a lane holds four neighbouring columns of one head in each quarter of a tile, so what scales a head
-    // is a register of its own lane. Kept in the accumulation registers ("a") throughout: 256 of them, all there are.
-    f32x16 o[kGwColTiles];
-    {
-        const u32x4 z = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int c = 0; c < kGwColTiles; ++c)  // zeros at a sixteenth of the instructions of writing them
-            asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %1, 0" : "=a"(o[c]) : "v"(z));
-        // A query without a live slot reads them next. The compiler keeps no distance from assembly, so they come out of one that does: once
-        // the last is there, all are. (Not under that condition: twelve wait states of a query's 140 000 cycles are less than a branch here.)
-        asm volatile("s_nop 11" : "+a"(o[kGwColTiles - 1]));
-#pragma unroll
-        for (int c = 0; c < kGwColTiles - 1; ++c) asm volatile("" : "+a"(o[c]));
-    }
     float m_ref = -INFINITY, l_sum = 0.0f;
     const float qs = fabsf(a.qscale);  // its sign is in the query
 
