@@ -212,7 +212,6 @@ __device__ __forceinline__ unsigned long long wave_xor(unsigned long long v) {
 // buffer that is not 16-byte aligned rather than let the kernel fault on it.
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Launcher epilogue shared by every entry point: 0 or -(hipError_t).
 // kernel<<<grid, block, lds, stream>>>(args...) without the configuration that the launch syntax
 // pushes for the kernel's stub and the stub pops again: 2.29 us of host time a launch, 2.44 with
 // it. The arguments are converted to the kernel's own parameter types first.
@@ -225,6 +224,7 @@ inline void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t ld
     }(args...);
 }
 
+// Launcher epilogue shared by every entry point: 0 or -(hipError_t).
 inline int launch_status() {
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : -(int)e;

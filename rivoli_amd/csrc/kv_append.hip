@@ -286,7 +286,7 @@ __global__ __launch_bounds__(kAppendWaves* kWave) void kv_append_paged_token_ker
 
 // Linear slabs, reference layout. A lane owns elements lane*2, lane*2+1 of a 128-block (so a block is exactly one
 // wave-wide butterfly). WAVES of a workgroup's four share a token, a block each at a time: what a token takes is the way from
-// memory to its codes, and one wave walked four blocks' one after another. The engine's token of 512 + 64 30.3 -> 28.7 us, 1 000 tokens 4.4 ->
+// memory to its codes, and one wave walked four blocks' one after another. The engine's token of 512 + 64 30.3 -> 29.1 us, 1 000 tokens 4.4 ->
 // 3.5; with enough tokens for the chip four times the waves only cost: 8 192 7.8 -> 10.8, so past kAppendShared a wave has a token.
 constexpr int kAppendShared = 1024;
 template <int WAVES>

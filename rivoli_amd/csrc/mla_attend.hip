@@ -743,9 +743,11 @@ __device__ __forceinline__ bool dealt_part(const AttendArgs& a, int item, const 
 struct SeqDeal {
     int tiles, parts, first;  // of the lane's sequence: its tiles, its work items, the first of them
 };
-__device__ __forceinline__ int ceil_quotient(int t, int c, float inv) {  // t + c below 2^24
+// Needs t + 2 c below 2^31 and a quotient below 2^20: n as a float, the approximate inverse and their product are each off by 2^-23 of themselves at
+// most, so q by less than one before it is cut. (A batch has up to 2^25 tiles, over two work items a sequence and more: below 2^18.)
+__device__ __forceinline__ int ceil_quotient(int t, int c, float inv) {
     const int n = t + c - 1;
-    int q = (int)((float)n * inv);  // off by one at most, with an approximate inverse too
+    int q = (int)((float)n * inv);  // off by one at most
     q -= q * c > n;
     q += (q + 1) * c <= n;
     return q;
