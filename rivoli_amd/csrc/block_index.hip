@@ -25,7 +25,7 @@
 // on the operands they hold (RowSpan) and take such tiles through v_mfma_f32_32x32x16_bf16; any
 // other tile of the same launch is folded term by term as below; rows that are fp4 codes under
 // powers of two, as spread rows are, go through the block-scaled fp4 instruction. 8 192 queries x 64 heads x
-// <= 2 048 blocks: 164 us, 226 as bf16, 3 640 term by term.
+// <= 2 048 blocks: 160 us, 226 as bf16, 3 640 term by term.
 // Operands of another kind (no such rows leave the indexer) take the same launches' fold: 3 430.
 // Term by term, what is free is where the operands come from. A lane owns block c and
 // keeps its 128-value row in registers for the whole launch; a wave's 64 lanes share the query,
@@ -429,9 +429,9 @@ __device__ __forceinline__ void fold_heads(const float* __restrict__ q, const fl
 // the rows with bit 2 clear): the head sum, whose order the reference fixes, is then register arithmetic.
 // Bound by issue. As bf16 a lane's 64 dots were 32 matrix instructions of 32 cycles and five vector instructions each (round,
 // relu, weight, round, sum); as fp4 codes they are 8 of 32 cycles, and clamping conversions leave four a dot, in steps of which
-// none waits for another. 8 192 queries: 226 -> 164 us, of them 107 vector issue (two thirds of it those four; the kv rows' codes, made by every workgroup,
-// and the q rows' take the rest), 15 the matrix cores and about 25 the first workgroups' q rows, all asked for at once; 4 096 82 -> 72,
-// 6 001 127 -> 103. Not kept: 16 queries a workgroup (half of the conversions; all of q at once, 231), two or three sets of q loads
+// none waits for another. 8 192 queries: 226 -> 160 us, of them 120 vector issue (two thirds of it those four; the kv rows' codes, made by every workgroup,
+// and the q rows' take the rest), 16 the matrix cores and about 25 the first workgroups' q rows, all asked for at once; 4 096 82 -> 73,
+// 6 001 127 -> 102. Not kept: 16 queries a workgroup (half of the conversions; all of q at once, 231), two or three sets of q loads
 // in flight (178).
 constexpr int kPairWaves = 4;
 constexpr int kPairThreads = kPairWaves * kWave;
